@@ -73,8 +73,9 @@ typedef enum tde_algo {
     TDE_ALGO_AUTO = 0,   /* = TDE_ALGO_FUSED */
     TDE_ALGO_FUSED = 1,  /* one pass per row: reduce -> residual -> norm -> quant, row kept in registers
                             (the arithmetic of the one-shot body, impl.h:450-471) */
-    TDE_ALGO_STAGED = 2, /* two launches: (A) N-way reduce of every row into `stage` (impl.h:365-377),
-                            (B) residual + norm (+quant) reading `stage` (impl.h:381-393) */
+    TDE_ALGO_STAGED = 2, /* two phases: (A) N-way reduce of every row into `stage` (impl.h:365-377),
+                            (B) residual + norm (+quant) of the rows of `stage` (impl.h:381-393); tde_reduce_rms does
+                            both in one launch, tde_stage_reduce and tde_stage_norm one each */
     TDE_ALGO_STAGED_OWNED = 3 /* as STAGED, but (A) reduces only this rank's share, rows == rank (mod nranks), as one
                             rank of the reference's two-shot does (impl.h:366); the other rows of `stage` must already
                             hold their sums (in the reference the peers write them, impl.h:373-376) */
@@ -135,7 +136,8 @@ typedef struct tde_plan_out {
                                   (0 = none); below a requested tune_workgroups_per_cu where the geometry's own LDS
                                   already admits fewer.  Also 2, without LDS padding, where the plan picks the row
                                   kernel built for two wavefronts per SIMD (eight partials, four vectors per thread,
-                                  4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its registers admit two */
+                                  4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its registers admit two.
+                                  The staged algorithms are never limited unless asked to */
     int32_t lds_bytes;         /* dynamic LDS per workgroup of the row kernel's launch, padding included */
     int64_t algorithmic_bytes; /* (N+1)*T*H*e + H*e + T*H*e + OUT, OUT as documented for the quant mode */
     int64_t scale_elems;       /* number of fp32 scales written */
@@ -171,7 +173,8 @@ int tde_reduce_rms(const tde_problem *problem, const tde_buffers *buffers, void 
    rank (mod nranks), into buffers->stage; only partial[], partial_table and stage are read from `buffers`.
    tde_stage_norm = the body after the barrier (impl.h:381-393): residual add + norm (+quant) of every row of
    buffers->stage; partial[] and partial_table are ignored.
-   tde_reduce_rms with the same problem is exactly tde_stage_reduce followed by tde_stage_norm. */
+   tde_reduce_rms with the same problem computes and stores exactly what tde_stage_reduce followed by tde_stage_norm
+   does, in one launch (in those two where `stage` overlaps another output, the residual or gamma). */
 int tde_stage_reduce(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 int tde_stage_norm(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 

@@ -1,0 +1,51 @@
+"""GPU: tde_reduce_rms with a staged algorithm is one launch that also stores (or reads) the stage.  What it leaves in every
+buffer must be what its two phases, called one at a time, leave there; a stage that overlaps an output is still correct."""
+import pytest
+import torch
+
+from oracle import eager
+from torch_dist_ext_amd import _capi
+
+from helpers import bits_equal, run_hip
+
+pytestmark = pytest.mark.gpu
+
+
+# rows around a window of the owned-rows order (1024 * N), around one compute unit's share of packed rows, and fewer rows
+# than ranks; row lengths of one wavefront, of less, and of several vectors per thread
+@pytest.mark.parametrize("n,rank,tokens,hidden,dtype,quant,vpt,rpb", [
+    (2, 0, 2047, 128, torch.bfloat16, "fp8_group", 0, 0), (2, 1, 2049, 128, torch.float32, "none", 0, 4),
+    (4, 3, 4096, 64, torch.float16, "fp8_token", 1, 3), (4, 0, 4099, 72, torch.bfloat16, "none", 2, 2),
+    (8, 7, 8191, 32, torch.float32, "fp8_static", 4, 0), (8, 3, 8200, 8, torch.bfloat16, "int8_token", 0, 0),
+    (8, 6, 5, 1000, torch.float16, "int8_token", 4, 1), (8, 1, 300, 8192, torch.bfloat16, "fp8_token", 0, 0),
+    (4, 2, 4097, 6, torch.float64, "none", 0, 0), (2, 1, 130, 2048, torch.float64, "none", 0, 0),
+])
+def test_one_launch_equals_its_phases(cuda_device, n, rank, tokens, hidden, dtype, quant, vpt, rpb):
+    print("case", n, rank, tokens, hidden, dtype, quant, vpt, rpb, flush=True)
+    p, r, g = eager.make_inputs(n, tokens, hidden, dtype, 1.0, seed=700 + n)
+    stage = torch.randn((tokens, hidden), generator=torch.Generator().manual_seed(7), dtype=torch.float64).to(dtype)
+    stage[0, 0] = -0.0   # a delivered sum is taken as it is, sign of zero included
+    kw = dict(rank=rank, stage_init=stage, vecs_per_thread=vpt, rows_per_block=rpb,
+              static_scale=0.03 if quant == "fp8_static" else 0.0)
+    for algo in (_capi.ALGO_STAGED, _capi.ALGO_STAGED_OWNED):
+        one = run_hip(p, r, g, 1e-6, quant, algo=algo, **kw)
+        two = run_hip(p, r, g, 1e-6, quant, algo=algo, calls=[(("reduce",), rank), (("norm",), rank)], **kw)
+        for k in two:
+            assert bits_equal(one[k], two[k]), (algo, k)
+
+
+@pytest.mark.parametrize("where", ["norm_out", "residual_out", "residual_in"])
+def test_stage_that_overlaps_another_buffer(cuda_device, where):
+    """Both phases then still run one after the other: the residual is read, and an output written, after all the sums."""
+    import torch_dist_ext_amd as tde
+    print("case", where, flush=True)
+    p, r, g = eager.make_inputs(4, 70, 1024, torch.bfloat16, 1.0, seed=9)
+    want = eager.reduce_rms(p, p.float().sum(0).to(p.dtype) if where == "residual_in" else r, g, 1e-6, "none")
+    parts = [p[i].to(cuda_device) for i in range(4)]
+    buf = {"residual_in": r.to(cuda_device), "residual_out": torch.empty_like(r, device=cuda_device),
+           "norm_out": torch.empty_like(r, device=cuda_device)}
+    tde.reduce_rms_local_impl(parts, buf["residual_in"], g.to(cuda_device), buf["residual_out"], buf["norm_out"], None, None,
+                              1e-6, tde.QUANT_NONE, tde.ALGO_STAGED, buf[where], 0.0)
+    torch.cuda.synchronize()
+    assert bits_equal(buf["residual_out"].cpu(), want["residual_out"])
+    assert bits_equal(buf["norm_out"].cpu(), want["norm_out"])

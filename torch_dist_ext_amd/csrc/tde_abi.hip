@@ -211,9 +211,10 @@ int validate(const tde_problem *p, tde::Geometry *geo) {
         // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
         // row kernel's two-wavefronts-per-SIMD instantiation (tde_rows.h: WIDE) is 0.2-2.2 % faster there; it is
         // reported as the limit of two workgroups per CU that its registers amount to.
-        geo->wide = p->nranks == 8 && vpt == 4 && p->dtype != TDE_F64 && !staged && wgs_per_cu == 0 &&
+        const bool wide = p->nranks == 8 && vpt == 4 && p->dtype != TDE_F64 && !staged && wgs_per_cu == 0 &&
                     p->tune_workgroups_per_cu == 0 && grid >= 4 * (int64_t)cus;
-        if (geo->wide) geo->wgs_per_cu = 2;
+        geo->form = wide ? tde::kFormWide : tde::kFormPlain;
+        if (wide) geo->wgs_per_cu = 2;
     }
     return TDE_OK;
 }
@@ -385,6 +386,18 @@ int tde_plan(const tde_problem *problem, tde_plan_out *plan) {
 namespace {
 enum : int { kPhaseReduce = 1, kPhaseNorm = 2, kTrafficOnly = 4 };
 
+// Whether the stage shares bytes with a buffer that the norm of some row reads or writes.
+bool stage_overlaps(const tde_problem *p, const tde_buffers *b) {
+    const int64_t row = p->hidden * elem_bytes(p->dtype), all = p->tokens * row;
+    const auto overlaps = [&](const void *q, int64_t bytes) {
+        const uintptr_t s = reinterpret_cast<uintptr_t>(b->stage), o = reinterpret_cast<uintptr_t>(q);
+        return q != nullptr && o < s + (uintptr_t)all && s < o + (uintptr_t)bytes;
+    };
+    const int64_t scales = p->tokens * (p->quant == TDE_QUANT_FP8_GROUP ? p->hidden / TDE_QUANT_GROUP : 1) * (int64_t)sizeof(float);
+    return overlaps(b->residual_in, all) || overlaps(b->residual_out, all) || overlaps(b->norm_out, all) ||
+           overlaps(b->gamma, row) || overlaps(b->q_out, p->tokens * p->hidden) || overlaps(b->scale_out, scales);
+}
+
 int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int phases, int probe_parts = 7) {
     tde::Geometry g{};
     const int st = validate(p, &g);
@@ -430,7 +443,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     a.gamma = b->gamma;
     a.q_out = b->q_out;
     a.scale_out = b->scale_out;
-    a.stage_out = b->stage;
+    a.owner = p->rank;
     a.tokens = p->tokens;
     a.hidden = (int32_t)p->hidden;
     a.nvec = g.nvec;
@@ -450,7 +463,18 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
         e = tde::launch_traffic(n, g.vpt, code_bytes, wn, a, g, (uint32_t)g.nvec * 16u, stream);
         return e == hipSuccess ? TDE_OK : hip_fail(e);
     }
-    if (staged && (phases & kPhaseReduce)) {
+    // The staged algorithms as a whole are one launch of the row kernel that also stores the sums to the stage (owned
+    // rows: reads the other rows' sums from it), which saves reading the sums back, a launch and the gap before it.  Both
+    // are bound by memory: 8 x [2048, 8192] bf16 -> fp8 takes 63.2 us (6.11 TB/s of what must be moved) against 70.3 us in
+    // two launches, with owned rows 28.2 us (5.35 TB/s) against 31.2; 8 x [64, 5120] 5.9 against 9.7 and 5.8 against 7.8,
+    // 4 x [13721, 532] fp32 38.5 against 47.3 and 27.3 against 36.3.  A stage that overlaps a buffer the norm reads or
+    // writes keeps the two launches, whose second only starts when every sum has been stored.
+    const bool one_launch = staged && both && !stage_overlaps(p, b);
+    if (one_launch) {
+        a.stage = b->stage;
+        g.form = p->algo == TDE_ALGO_STAGED_OWNED ? tde::kFormOwned : tde::kFormStaged;
+    } else if (staged && (phases & kPhaseReduce)) {
+        a.stage = b->stage;
         // All rows as one span of bytes, or only this rank's share (rows == rank mod nranks) row by row.
         const int64_t row_bytes = (int64_t)g.nvec * 16;
         int64_t span_bytes = p->tokens * row_bytes, first = 0, step = 1, rows = 1;
@@ -469,10 +493,11 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
         if (e != hipSuccess) return hip_fail(e);
     }
     if (!(phases & kPhaseNorm)) return TDE_OK;
-    if (staged) {
+    if (staged && !one_launch) {
         for (int r = 0; r < tde::kMaxKernelRanks; ++r) a.part[r] = nullptr;
         a.part[0] = b->stage;
         a.table = nullptr;
+        a.stage = nullptr;
         n = 0;
     }
     switch (p->dtype) {

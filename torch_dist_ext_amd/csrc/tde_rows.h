@@ -48,7 +48,7 @@ struct RowArgs {
     const void *gamma;
     void *q_out;
     float *scale_out;
-    void *stage_out; // stage A destination
+    void *stage;     // the sums' rows: written by stage A and by the one-launch staged forms, null without a stage
     int64_t tokens;
     int32_t hidden;
     int32_t nvec;           // 16-byte vectors per row
@@ -58,6 +58,7 @@ struct RowArgs {
     float eps;
     float hidden_f;
     float static_scale;
+    int32_t owner;       // OWNED row kernels: rows == owner (mod N) are summed here, the others are read from the stage
     int32_t probe_parts; // traffic skeleton only: bit 0 read the inputs, bit 1 write the T-typed rows, bit 2 write the code rows
 };
 
@@ -511,6 +512,26 @@ __device__ __forceinline__ uint32_t xcd_chunked_block(uint32_t bid, uint32_t gri
     return bid;
 }
 
+// The row that comes i-th in a launch whose rows == owner (mod N) read N partials and the others one staged sum: in each
+// window of kOwnedRun * N rows first all of the former, then the others, each in order.  In plain order the long rows
+// would meet the same few compute units again and again (workgroups go to the units of an XCD in turn, and N divides
+// their number): 8 x [2048, 8192] bf16 -> fp8 35.3 us, 28.2 us in this order.  Windows of a quarter of the length cost 0 to
+// 20 % (8 x [5000, 1024] fp16 11.1 -> 14.1 us, 4 x [2048, 8192] 30.5 -> 31.9) and gain 3-4 % on two shapes (2 x [8192, 4096]
+// 53.8 -> 52.2, fp32 rows of 532).
+constexpr int kOwnedRun = 1024;
+template <int N>
+__device__ __forceinline__ int64_t owned_first_row(int64_t i, int64_t tokens, int owner, bool &owned) {
+    const int64_t window = i / (kOwnedRun * N) * (kOwnedRun * N);
+    const int64_t left = tokens - window;
+    const int rows = left < kOwnedRun * N ? (int)left : kOwnedRun * N; // of this window; i is past the end if it is <= 0
+    const int n_owned = (rows - owner + N - 1) / N;
+    const int k = (int)(i - window), other = k - n_owned;
+    owned = other < 0;
+    if (owned) return window + k * N + owner;
+    const int in_span = other % (N - 1);
+    return window + other / (N - 1) * N + in_span + (in_span >= owner ? 1 : 0);
+}
+
 // The loads of one row: N partial vectors and one residual vector per owned 16-byte column slot.
 template <int NP, int VPT>
 struct RowLoads {
@@ -526,15 +547,22 @@ struct RowLoads {
 //   VPT    16-byte vectors per thread per row (1, 2 or 4)
 //   Q      tde_quant
 //   WN     write the T-typed normed row (always true for Q == NONE)
-//   WIDE   compiled for two wavefronts per SIMD (256 registers) instead of three, with gamma requested ahead of the
-//          row also for eight partials: two workgroups per CU whose gamma never waits.  Launched for eight partials
-//          with four vectors per thread at 4 to 24 workgroups per CU (launch_rows_nv, Geometry::wide)
+//   FORM   kFormWide: compiled for two wavefronts per SIMD (256 registers) instead of three, with gamma requested ahead
+//          of the row also for eight partials: two workgroups per CU whose gamma never waits.  Launched for eight
+//          partials with four vectors per thread at 4 to 24 workgroups per CU (launch_rows_nv, Geometry::form).
+//          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
+//          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
+//          partials and their sums stored to the stage, every other row's sum is read from the stage
 // Block layout: rows_per_block row groups of threads_per_row threads; thread t of a row group
 // owns vectors t, t + threads_per_row, ... (coalesced 1 KiB per wavefront per load).
 // ---------------------------------------------------------------------------------------------
-template <class E, int N, int VPT, int Q, bool WN, bool WIDE = false>
+enum : int { kFormPlain = 0, kFormWide = 1, kFormStaged = 2, kFormOwned = 3 };
+
+template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain>
 __global__ void __launch_bounds__(1024 / VPT)
-    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (WIDE ? 2 : 3))))) row_kernel(const RowArgs a) {
+    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))))))
+    row_kernel(const RowArgs a) {
+    constexpr bool WIDE = FORM == kFormWide, OWNED = FORM == kFormOwned;
     constexpr int VEC = E::VEC;
     constexpr int NP = (N == 0) ? 1 : N;
     // residual_out is stored together with the row's other output at the end, one write burst per row: against storing
@@ -578,11 +606,13 @@ __global__ void __launch_bounds__(1024 / VPT)
     auto issue_loads = [&](RowLoads<NP, VPT> &d, int64_t row) {
         const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
         const int64_t row_byte = row * (int64_t)row_bytes;
+        if constexpr (!OWNED) {
 #pragma unroll
-        for (int r = 0; r < NP; ++r) {
-            const rsrc_t rs = row_rsrc(part[r], row_byte, bytes);
+            for (int r = 0; r < NP; ++r) {
+                const rsrc_t rs = row_rsrc(part[r], row_byte, bytes);
 #pragma unroll
-            for (int j = 0; j < VPT; ++j) d.p[j][r] = rsrc_load16(rs, lane_off[j]);
+                for (int j = 0; j < VPT; ++j) d.p[j][r] = rsrc_load16(rs, lane_off[j]);
+            }
         }
         const rsrc_t rr = row_rsrc(a.residual_in, row_byte, bytes);
 #pragma unroll
@@ -609,7 +639,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     // -0.2 to -0.9 %), so WIDE carries gamma ahead of the row for all of them.
     const rsrc_t gamma_rsrc = row_rsrc(a.gamma, 0, row_bytes);
     constexpr bool GAMMA_FIRST =
-        VPT > 1 && N != 0 &&
+        VPT > 1 && N != 0 && !OWNED &&
         (WIDE || (N <= 4 && E::BYTES == 2 && (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN)));
     u32x4 gamma_first[GAMMA_FIRST ? VPT : 1];
     if constexpr (GAMMA_FIRST) {
@@ -619,7 +649,10 @@ __global__ void __launch_bounds__(1024 / VPT)
         __builtin_amdgcn_sched_barrier(0);
     }
     RowLoads<NP, VPT> cur;
-    issue_loads(cur, row0 + group);
+    int64_t row = row0 + group;
+    bool sum_is_new = FORM == kFormStaged; // the row's sums go to the stage as well
+    if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
+    issue_loads(cur, row);
     u32x4 gamma_early = u32x4{0, 0, 0, 0};
     if constexpr (VPT == 1) {
         __builtin_amdgcn_sched_barrier(0);
@@ -634,7 +667,6 @@ __global__ void __launch_bounds__(1024 / VPT)
 #define TDE_OFF(j) (lane0 + (uint32_t)(j) * vec_stride)
 
     {
-        const int64_t row = row0 + group;
         const bool row_ok = row < a.tokens;
         const uint32_t bytes = row_ok ? row_bytes : 0u;
         const int64_t row_byte = row * (int64_t)row_bytes; // wavefront-uniform
@@ -648,7 +680,45 @@ __global__ void __launch_bounds__(1024 / VPT)
         // vectors per thread the accumulators cost more occupancy than the overlap returns (8 partials, 1024 rows of
         // 5120: 21.5 us against 20.4), so those variants sum vector by vector.  With one vector per thread (the
         // decode-size geometries) waiting rank by rank is worth 0.5-1.5 % up to 512 rows and nothing beyond.
-        constexpr bool RANK_MAJOR = (N >= 4 && (VPT >= 4 || VPT == 1));
+        constexpr bool RANK_MAJOR = !OWNED && (N >= 4 && (VPT >= 4 || VPT == 1));
+        u32x4 sraw[VPT]; // the row's sums, rounded to T
+        if constexpr (OWNED) {
+            if (sum_is_new) {
+                // At most four partials in flight per vector: each one's registers are loaded with the partial four
+                // ranks on as soon as it has been added.  That keeps the kernel within 128 registers, four wavefronts
+                // per SIMD, which the rows that only read the stage need to have enough loads in flight (limited to
+                // two or three workgroups per CU 8 x [2048, 8192] takes 29.4 and 28.6 us instead of 28.2).
+                constexpr int B = N < 4 ? N : 4;
+                u32x4 p[VPT][B];
+                float acc[VPT][VEC];
+                auto request = [&](int r) {
+                    const rsrc_t rs = row_rsrc(part[r], row_byte, bytes);
+#pragma unroll
+                    for (int j = 0; j < VPT; ++j) p[j][r % B] = rsrc_load16(rs, TDE_OFF(j));
+                };
+#pragma unroll
+                for (int r = 0; r < B; ++r) request(r);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < N; ++r) {
+#pragma unroll
+                    for (int j = 0; j < VPT; ++j) {
+                        float v[VEC];
+                        E::unpack(p[j][r % B], v);
+#pragma unroll
+                        for (int i = 0; i < VEC; ++i) acc[j][i] = (r == 0 ? 0.0f : acc[j][i]) + v[i];
+                    }
+                    if (r + B < N) request(r + B);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < VPT; ++j) sraw[j] = E::pack(acc[j]);
+            } else {
+                const rsrc_t rs = row_rsrc(a.stage, row_byte, bytes);
+#pragma unroll
+                for (int j = 0; j < VPT; ++j) sraw[j] = rsrc_load16(rs, TDE_OFF(j));
+            }
+        }
         float racc[RANK_MAJOR ? VPT : 1][VEC];
         if constexpr (RANK_MAJOR) {
             __builtin_amdgcn_sched_barrier(0);
@@ -686,11 +756,12 @@ __global__ void __launch_bounds__(1024 / VPT)
         }
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            float s[VEC];
-            if constexpr (N == 0) {
-                E::unpack(cur.p[j][0], s);
+            if constexpr (OWNED) {
+                // above
+            } else if constexpr (N == 0) {
+                sraw[j] = cur.p[j][0];
             } else if constexpr (RANK_MAJOR) {
-                E::unpack(E::pack(racc[j]), s);
+                sraw[j] = E::pack(racc[j]);
             } else {
                 float acc[VEC];
 #pragma unroll
@@ -702,9 +773,10 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
                     for (int i = 0; i < VEC; ++i) acc[i] += p[i];
                 }
-                E::unpack(E::pack(acc), s);
+                sraw[j] = E::pack(acc);
             }
-            float res[VEC], x[VEC];
+            float s[VEC], res[VEC], x[VEC];
+            E::unpack(sraw[j], s);
             E::unpack(cur.r[j], res);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) x[i] = s[i] + res[i];
@@ -731,6 +803,13 @@ __global__ void __launch_bounds__(1024 / VPT)
                 gamma_raw[j] = __builtin_amdgcn_raw_buffer_load_b128(gamma_rsrc, (int)TDE_OFF(j), 0, kAuxDefault);
         } else {
             gamma_raw[0] = gamma_early;
+        }
+        // The stage behind the gamma request: a wavefront's loads and stores are waited for in order, and gamma would
+        // otherwise wait for these stores.
+        if (sum_is_new) {
+            const rsrc_t stage = row_rsrc(a.stage, row_byte, bytes);
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) rsrc_store16(stage, TDE_OFF(j), sraw[j]);
         }
         const float sumsq = sumsq_torch_order<VPT, VEC, E::BYTES == 2>(lds_img, lds_bs, a.hidden, TDE_T, tpr, group, TDE_LANE, xraw[VPT - 1][0]);
         const float rs = 1.0f / __builtin_sqrtf(sumsq / a.hidden_f + a.eps);
@@ -902,7 +981,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
 #pragma unroll
         for (int u = 0; u < U; ++u) raw[u][r] = rsrc_load16(rs, (uint32_t)(u * 256 + threadIdx.x) * 16u);
     }
-    const rsrc_t out = row_rsrc(a.stage_out, base, bytes);
+    const rsrc_t out = row_rsrc(a.stage, base, bytes);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         float acc[VEC];
@@ -934,7 +1013,7 @@ struct Geometry {
     int block_threads;
     int64_t grid;
     int xcd_chunk;
-    bool wide; // launch the row kernel's WIDE instantiation (eight partials, four vectors per thread)
+    int form;  // which instantiation of the row kernel (kFormPlain, kFormWide, kFormStaged, kFormOwned)
 };
 
 // Per-dtype launchers, defined in tde_rows_<dtype>.hip.
@@ -958,23 +1037,24 @@ template <class E, int N, int VPT>
 hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
+#define TDE_LAUNCH_FORM(QM, WNB, FORM)                                                                   \
+    {                                                                                                    \
+        if (lds > kDefaultMaxDynamicLds) {                                                               \
+            const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB, FORM>>();                \
+            if (e != hipSuccess) return e;                                                               \
+        }                                                                                                \
+        hipLaunchKernelGGL((row_kernel<E, N, VPT, QM, WNB, FORM>), grid, block, lds, s, a);            \
+        return hipGetLastError();                                                                        \
+    }
 #define TDE_LAUNCH(QM, WNB)                                                                              \
     if constexpr (N == 8 && VPT == 4) {                                                                  \
-        if (g.wide) {                                                                                    \
-            if (lds > kDefaultMaxDynamicLds) {                                                           \
-                const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB, true>>();            \
-                if (e != hipSuccess) return e;                                                           \
-            }                                                                                            \
-            hipLaunchKernelGGL((row_kernel<E, N, VPT, QM, WNB, true>), grid, block, lds, s, a);        \
-            return hipGetLastError();                                                                    \
-        }                                                                                                \
+        if (g.form == kFormWide) TDE_LAUNCH_FORM(QM, WNB, kFormWide)                                     \
     }                                                                                                    \
-    if (lds > kDefaultMaxDynamicLds) {                                                                   \
-        const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB>>();                          \
-        if (e != hipSuccess) return e;                                                                   \
+    if constexpr (N != 0) {                                                                              \
+        if (g.form == kFormStaged) TDE_LAUNCH_FORM(QM, WNB, kFormStaged)                                 \
+        if (g.form == kFormOwned) TDE_LAUNCH_FORM(QM, WNB, kFormOwned)                                   \
     }                                                                                                    \
-    hipLaunchKernelGGL((row_kernel<E, N, VPT, QM, WNB>), grid, block, lds, s, a);                      \
-    return hipGetLastError();
+    TDE_LAUNCH_FORM(QM, WNB, kFormPlain)
     switch (q) {
     case TDE_QUANT_NONE: TDE_LAUNCH(TDE_QUANT_NONE, true)
     case TDE_QUANT_FP8_TOKEN:
@@ -987,6 +1067,7 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
         if (wn) { TDE_LAUNCH(TDE_QUANT_FP8_STATIC, true) } else { TDE_LAUNCH(TDE_QUANT_FP8_STATIC, false) }
     }
 #undef TDE_LAUNCH
+#undef TDE_LAUNCH_FORM
     return hipErrorInvalidValue;
 }
 

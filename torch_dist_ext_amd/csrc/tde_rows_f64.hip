@@ -6,6 +6,7 @@
 //   y   = gamma * (x * double(rs))                          double                              -> norm_out
 // No quantized output for this type.  One 16-byte vector per thread, the row kernel's geometry and XCD-aware row
 // mapping.  N == 0: the sum was staged (part[0] holds it), as in the row kernel; reduce_kernel_f64 is that stage A.
+// With a stage the sums are stored to it; OWNED sums rows == owner (mod N) only and reads the others' sums from the stage.
 #include <hip/hip_runtime.h>
 
 #include "tde_rows.h"
@@ -32,7 +33,7 @@ __device__ __forceinline__ u32x4 pack_f64(const double (&d)[2]) {
     return raw;
 }
 
-template <int N>
+template <int N, bool OWNED = false>
 __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
     constexpr int NP = (N == 0) ? 1 : N;
     extern __shared__ __attribute__((aligned(16))) float lds_dyn[]; // squares (two per thread), then block sums
@@ -60,18 +61,24 @@ __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
 
     {
         // the grid covers every row; each XCD takes runs of consecutive row groups (xcd_chunked_block)
-        const int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, gridDim.x, (uint32_t)a.xcd_chunk) * a.rows_per_block + group;
+        int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, gridDim.x, (uint32_t)a.xcd_chunk) * a.rows_per_block + group;
 
+        bool sum_is_new = N != 0 && a.stage != nullptr;
+        if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
         const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
         const int64_t row_byte = row * (int64_t)row_bytes;
         u32x4 praw[NP];
+        if (!OWNED || sum_is_new) {
 #pragma unroll
-        for (int r = 0; r < NP; ++r) praw[r] = rsrc_load16(row_rsrc(part[r], row_byte, bytes), off);
+            for (int r = 0; r < NP; ++r) praw[r] = rsrc_load16(row_rsrc(part[r], row_byte, bytes), off);
+        } else {
+            praw[0] = rsrc_load16(row_rsrc(a.stage, row_byte, bytes), off);
+        }
         const u32x4 rraw = rsrc_load16(row_rsrc(a.residual_in, row_byte, bytes), off);
         const u32x4 graw = __builtin_amdgcn_raw_buffer_load_b128(gamma_rsrc, (int)off, 0, kAuxDefault);
 
         double acc[2] = {0.0, 0.0};
-        if constexpr (N == 0) {
+        if (N == 0 || (OWNED && !sum_is_new)) {
             unpack_f64(praw[0], acc); // the staged sum
         } else {
 #pragma unroll
@@ -82,6 +89,7 @@ __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
                 acc[1] += p[1];
             }
         }
+        if (sum_is_new) rsrc_store16(row_rsrc(a.stage, row_byte, bytes), off, pack_f64(acc));
         double res[2], x[2];
         unpack_f64(rraw, res);
         x[0] = acc[0] + res[0];
@@ -130,7 +138,7 @@ __global__ void __launch_bounds__(256) reduce_kernel_f64(const RowArgs a, const 
 #pragma unroll
         for (int u = 0; u < U; ++u) raw[u][r] = rsrc_load16(rs, (uint32_t)(u * 256 + threadIdx.x) * 16u);
     }
-    const rsrc_t out = row_rsrc(a.stage_out, base, bytes);
+    const rsrc_t out = row_rsrc(a.stage, base, bytes);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         double acc[2] = {0.0, 0.0};
@@ -166,11 +174,12 @@ hipError_t launch_reduce_f64(int n, const RowArgs &a, int64_t row_bytes, int64_t
 hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, 1, 2): doubles are never limited per CU
+    const bool owned = g.form == kFormOwned;
     switch (n) {
     case 0: hipLaunchKernelGGL((row_kernel_f64<0>), grid, block, lds, s, a); break;
-    case 2: hipLaunchKernelGGL((row_kernel_f64<2>), grid, block, lds, s, a); break;
-    case 4: hipLaunchKernelGGL((row_kernel_f64<4>), grid, block, lds, s, a); break;
-    case 8: hipLaunchKernelGGL((row_kernel_f64<8>), grid, block, lds, s, a); break;
+    case 2: hipLaunchKernelGGL((owned ? row_kernel_f64<2, true> : row_kernel_f64<2>), grid, block, lds, s, a); break;
+    case 4: hipLaunchKernelGGL((owned ? row_kernel_f64<4, true> : row_kernel_f64<4>), grid, block, lds, s, a); break;
+    case 8: hipLaunchKernelGGL((owned ? row_kernel_f64<8, true> : row_kernel_f64<8>), grid, block, lds, s, a); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
