@@ -435,32 +435,36 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
 
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);
     tde::RowArgs a{};
-    for (int r = 0; r < p->nranks; ++r) a.part[r] = b->partial[r];
-    a.table = b->partial_table;
-    a.residual_in = b->residual_in;
-    a.residual_out = b->residual_out;
-    a.norm_out = b->norm_out;
-    a.gamma = b->gamma;
-    a.q_out = b->q_out;
-    a.scale_out = b->scale_out;
-    a.owner = p->rank;
+    if (reads_partials) {
+        for (int r = 0; r < p->nranks; ++r) {
+            a.set(tde::kPtrPart + r, b->partial[r]);
+            if (b->partial[r] == nullptr) a.table_mask |= (uint8_t)(1u << r);
+        }
+        if (a.table_mask != 0) a.set(tde::kPtrStage, b->partial_table);
+    }
+    const uint64_t table = reinterpret_cast<uint64_t>(b->partial_table);
+    a.set(tde::kPtrResidualIn, b->residual_in);
+    a.set(tde::kPtrResidualOut, b->residual_out);
+    a.set(tde::kPtrNorm, b->norm_out);
+    a.set(tde::kPtrGamma, b->gamma);
+    a.set(tde::kPtrCodes, b->q_out);
+    a.set(tde::kPtrScale, b->scale_out);
+    a.set_hidden(p->hidden);
+    a.threads_per_row = (uint16_t)g.threads_per_row;
+    a.rows_per_block = (uint8_t)g.rows_per_block;
+    a.xcd_chunk = (uint8_t)g.xcd_chunk;
     a.tokens = p->tokens;
-    a.hidden = (int32_t)p->hidden;
-    a.nvec = g.nvec;
-    a.threads_per_row = g.threads_per_row;
-    a.rows_per_block = g.rows_per_block;
-    a.xcd_chunk = g.xcd_chunk;
     a.eps = p->eps;
-    a.hidden_f = (float)p->hidden;
     a.static_scale = p->static_scale;
-    a.probe_parts = probe_parts;
+    a.chunked_blocks = tde::chunked_blocks(g.grid, (uint32_t)g.xcd_chunk);
+    a.owner = (uint8_t)p->rank;
 
     int n = p->nranks;
     hipError_t e = hipSuccess;
     if (traffic && p->dtype == TDE_F64) return TDE_EDTYPE;
     if (traffic) {
         const int code_bytes = quant ? (elem_bytes(p->dtype) == 4 ? 4 : 8) : 0;
-        e = tde::launch_traffic(n, g.vpt, code_bytes, wn, a, g, (uint32_t)g.nvec * 16u, stream);
+        e = tde::launch_traffic(n, g.vpt, code_bytes, wn, a, g, (uint32_t)g.nvec * 16u, (uint32_t)probe_parts, stream);
         return e == hipSuccess ? TDE_OK : hip_fail(e);
     }
     // The staged algorithms as a whole are one launch of the row kernel that also stores the sums to the stage (owned
@@ -468,13 +472,14 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     // are bound by memory: 8 x [2048, 8192] bf16 -> fp8 takes 63.2 us (6.11 TB/s of what must be moved) against 70.3 us in
     // two launches, with owned rows 28.2 us (5.35 TB/s) against 31.2; 8 x [64, 5120] 5.9 against 9.7 and 5.8 against 7.8,
     // 4 x [13721, 532] fp32 38.5 against 47.3 and 27.3 against 36.3.  A stage that overlaps a buffer the norm reads or
-    // writes keeps the two launches, whose second only starts when every sum has been stored.
-    const bool one_launch = staged && both && !stage_overlaps(p, b);
+    // writes keeps the two launches, whose second only starts when every sum has been stored; so do partials that only a
+    // device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
+    const bool one_launch = staged && both && a.table_mask == 0 && !stage_overlaps(p, b);
     if (one_launch) {
-        a.stage = b->stage;
+        a.set(tde::kPtrStage, b->stage);
         g.form = p->algo == TDE_ALGO_STAGED_OWNED ? tde::kFormOwned : tde::kFormStaged;
     } else if (staged && (phases & kPhaseReduce)) {
-        a.stage = b->stage;
+        a.set(tde::kPtrStage, b->stage);
         // All rows as one span of bytes, or only this rank's share (rows == rank mod nranks) row by row.
         const int64_t row_bytes = (int64_t)g.nvec * 16;
         int64_t span_bytes = p->tokens * row_bytes, first = 0, step = 1, rows = 1;
@@ -485,19 +490,17 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
             rows = (p->tokens - p->rank + p->nranks - 1) / p->nranks;
         }
         switch (p->dtype) {
-        case TDE_BF16: e = tde::launch_reduce_bf16(n, a, span_bytes, first, step, rows, stream); break;
-        case TDE_F16: e = tde::launch_reduce_f16(n, a, span_bytes, first, step, rows, stream); break;
-        case TDE_F32: e = tde::launch_reduce_f32(n, a, span_bytes, first, step, rows, stream); break;
-        case TDE_F64: e = tde::launch_reduce_f64(n, a, span_bytes, first, step, rows, stream); break;
+        case TDE_BF16: e = tde::launch_reduce_bf16(n, a, table, span_bytes, first, step, rows, stream); break;
+        case TDE_F16: e = tde::launch_reduce_f16(n, a, table, span_bytes, first, step, rows, stream); break;
+        case TDE_F32: e = tde::launch_reduce_f32(n, a, table, span_bytes, first, step, rows, stream); break;
+        case TDE_F64: e = tde::launch_reduce_f64(n, a, table, span_bytes, first, step, rows, stream); break;
         }
         if (e != hipSuccess) return hip_fail(e);
     }
     if (!(phases & kPhaseNorm)) return TDE_OK;
     if (staged && !one_launch) {
-        for (int r = 0; r < tde::kMaxKernelRanks; ++r) a.part[r] = nullptr;
-        a.part[0] = b->stage;
-        a.table = nullptr;
-        a.stage = nullptr;
+        a.table_mask = 0;
+        a.set(tde::kPtrPart, b->stage);
         n = 0;
     }
     switch (p->dtype) {

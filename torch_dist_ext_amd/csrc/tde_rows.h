@@ -38,29 +38,63 @@ constexpr int kWave = 64;
 constexpr int kMaxWavesPerBlock = 16;
 constexpr int kMaxKernelRanks = 8;
 
-// Kernel argument block (passed by value in kernarg memory).
+// Kernel argument block, passed by value.  A launch with 128 bytes of arguments or more costs the host 0.6-0.7 us more
+// than one with less on some machines (3.6 us against 2.9; on others 2.5 either way), a tenth of a decode-size call: so
+// the device addresses are packed to the 48 bits they have -- as a buffer resource takes them, 32 low bits and 16 high --
+// and the kernels read neither the grid's nor the workgroup's size, which would come in 256 bytes of hidden arguments.
+// Unpacking is one scalar instruction per address.
+enum : int { kPtrPart = 0, kPtrResidualIn = kMaxKernelRanks, kPtrResidualOut, kPtrNorm, kPtrGamma, kPtrCodes, kPtrScale, kPtrStage, kPtrs };
+
 struct RowArgs {
-    const void *part[kMaxKernelRanks]; // host-known partial pointers (or the stage buffer in [0])
-    const void *const *table;          // optional device pointer table; entry r used when part[r] == null
-    const void *residual_in;
-    void *residual_out;
-    void *norm_out;
-    const void *gamma;
-    void *q_out;
-    float *scale_out;
-    void *stage;     // the sums' rows: written by stage A and by the one-launch staged forms, null without a stage
+    uint32_t lo[kPtrs];
+    uint32_t hi[(kPtrs + 1) / 2]; // two per word; the last half word is `hidden`
+    uint16_t threads_per_row;     // multiple of 64
+    uint8_t rows_per_block;       // at most 16
+    uint8_t xcd_chunk;            // workgroups per XCD chunk of the row mapping (power of two; 0 or 1 = rows in launch order)
     int64_t tokens;
-    int32_t hidden;
-    int32_t nvec;           // 16-byte vectors per row
-    int32_t threads_per_row; // multiple of 64
-    int32_t rows_per_block;
-    int32_t xcd_chunk; // workgroups per XCD chunk of the row mapping (power of two; 0 or 1 = rows in launch order)
     float eps;
-    float hidden_f;
     float static_scale;
-    int32_t owner;       // OWNED row kernels: rows == owner (mod N) are summed here, the others are read from the stage
-    int32_t probe_parts; // traffic skeleton only: bit 0 read the inputs, bit 1 write the T-typed rows, bit 2 write the code rows
+    uint32_t chunked_blocks; // workgroups the XCD mapping permutes: the whole groups of 8 * xcd_chunk of the grid
+    uint8_t owner;           // OWNED row kernels: rows == owner (mod N) are summed here, the others are read from the stage
+    uint8_t table_mask;      // bit r: partial r's address is entry r of a device pointer table.  The table's own address
+                             // stands in the stage's place: a launch has one or the other
+    uint16_t pad;
+
+    __host__ __device__ uint64_t address(int i) const {
+        return ((uint64_t)((i & 1) ? hi[i >> 1] >> 16 : hi[i >> 1] & 0xffffu) << 32) | lo[i];
+    }
+    __host__ __device__ void *ptr(int i) const { return reinterpret_cast<void *>(address(i)); }
+    __host__ __device__ int hidden() const { return (int)(hi[kPtrs >> 1] >> 16); }
+    void set(int i, const void *p) {
+        const uint64_t v = reinterpret_cast<uint64_t>(p);
+        lo[i] = (uint32_t)v;
+        set_half(i, (uint32_t)(v >> 32));
+    }
+    void set_hidden(int64_t h) { set_half(kPtrs, (uint32_t)h); }
+
+private:
+    void set_half(int i, uint32_t v) {
+        const int shift = (i & 1) * 16;
+        hi[i >> 1] = (hi[i >> 1] & ~(0xffffu << shift)) | ((v & 0xffffu) << shift);
+    }
 };
+static_assert(sizeof(RowArgs) == 120 && (kPtrs & 1) == 1, "below 128 bytes, and a half word left for `hidden`");
+
+// The partials' addresses: from the argument block, or (one uniform branch, batched scalar loads) from the device pointer
+// table for the entries the host does not know.
+typedef const __attribute__((address_space(4))) uint64_t *table_t;
+template <int NP>
+__device__ __forceinline__ void partial_addresses(const RowArgs &a, uint64_t table, const void *(&part)[NP]) {
+#pragma unroll
+    for (int r = 0; r < NP; ++r) part[r] = a.ptr(kPtrPart + r);
+    if (a.table_mask != 0) {
+#pragma unroll
+        for (int r = 0; r < NP; ++r) {
+            const void *from_table = reinterpret_cast<const void *>(((table_t)table)[r]);
+            part[r] = (a.table_mask >> r & 1) ? from_table : part[r];
+        }
+    }
+}
 
 // ---------------------------------------------------------------------------------------------
 // Element traits: a 16-byte vector <-> VEC floats.  pack() rounds to nearest even.
@@ -501,10 +535,12 @@ __device__ __forceinline__ float clamp_keep_nan(float q, float limit) {
 // measured 0.5-1.5 % faster with chunks of 8-16 rows (c3 58.4 -> 57.5 us), slower again beyond 64, and 2 %
 // slower when each XCD owns one contiguous eighth of the tensor.  A grid tail shorter than a group keeps
 // launch order, so the mapping stays one-to-one.
-__device__ __forceinline__ uint32_t xcd_chunked_block(uint32_t bid, uint32_t grid, uint32_t chunk) {
+// `chunked`: the workgroups in whole groups, chunked_blocks(grid, chunk).
+inline uint32_t chunked_blocks(int64_t grid, uint32_t chunk) { return chunk > 1 ? (uint32_t)grid & ~(8u * chunk - 1u) : 0u; }
+__device__ __forceinline__ uint32_t xcd_chunked_block(uint32_t bid, uint32_t chunked, uint32_t chunk) {
     if (chunk > 1) {
         const uint32_t span = 8u * chunk; // power of two
-        if (bid < (grid & ~(span - 1u))) {
+        if (bid < chunked) {
             const uint32_t w = bid & (span - 1u);
             bid = (bid - w) + (w & 7u) * chunk + (w >> 3);
         }
@@ -571,7 +607,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     // Dynamic LDS: the workgroup's squares (one float per element it holds), then 1024 floats of block sums.
     extern __shared__ __attribute__((aligned(16))) float lds_dyn[];
     float *const lds_img = lds_dyn;
-    float *const lds_bs = lds_dyn + blockDim.x * (VPT * VEC);
+    float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * (VPT * VEC);
     __shared__ uint32_t lds_max[kMaxWavesPerBlock];
 
     const int tid = threadIdx.x;
@@ -580,20 +616,10 @@ __global__ void __launch_bounds__(1024 / VPT)
     const int waves_per_row = tpr >> 6;
     const int group = __builtin_amdgcn_readfirstlane(tid / tpr); // uniform inside a wavefront
     const int first_wave = group * waves_per_row;
-    const uint32_t row_bytes = (uint32_t)a.hidden * E::BYTES;
+    const uint32_t row_bytes = (uint32_t)a.hidden() * E::BYTES;
 
-    // Partial pointers: from the argument block, or (one uniform branch, batched scalar loads)
-    // from the device pointer table for the entries the host left null.
     const void *part[NP];
-#pragma unroll
-    for (int r = 0; r < NP; ++r) part[r] = a.part[r];
-    if (a.table != nullptr) {
-#pragma unroll
-        for (int r = 0; r < NP; ++r) {
-            const void *from_table = a.table[r];
-            part[r] = (part[r] != nullptr) ? part[r] : from_table;
-        }
-    }
+    partial_addresses(a, a.address(kPtrStage), part);
 
     uint32_t lane_off[VPT]; // byte offset of this thread's vector j inside a row
 #pragma unroll
@@ -614,14 +640,14 @@ __global__ void __launch_bounds__(1024 / VPT)
                 for (int j = 0; j < VPT; ++j) d.p[j][r] = rsrc_load16(rs, lane_off[j]);
             }
         }
-        const rsrc_t rr = row_rsrc(a.residual_in, row_byte, bytes);
+        const rsrc_t rr = row_rsrc(a.ptr(kPtrResidualIn), row_byte, bytes);
 #pragma unroll
         for (int j = 0; j < VPT; ++j) d.r[j] = rsrc_load16(rr, lane_off[j]);
     };
 
     // One workgroup, one group of rows: the grid covers every row (no loop; a looping wavefront waits for its
     // own stores, a fresh workgroup does not).
-    const int64_t row0 = (int64_t)xcd_chunked_block(blockIdx.x, gridDim.x, (uint32_t)a.xcd_chunk) * a.rows_per_block;
+    const int64_t row0 = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block;
 
     // The row's loads go out before anything else touches memory -- except gamma where it pays to have it first:
     // with up to four partials of a 2-byte type, several vectors per thread and a per-token scale, the registers are
@@ -637,7 +663,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     // (where the launch is limited to two workgroups per CU anyway) and +0.8 to +1.8 % below 1024 rows.  The other
     // eight-partial kernels gain less but none loses (per-group scales -1.0 %, T-typed output -0.3 to -0.8 %, fp32 rows
     // -0.2 to -0.9 %), so WIDE carries gamma ahead of the row for all of them.
-    const rsrc_t gamma_rsrc = row_rsrc(a.gamma, 0, row_bytes);
+    const rsrc_t gamma_rsrc = row_rsrc(a.ptr(kPtrGamma), 0, row_bytes);
     constexpr bool GAMMA_FIRST =
         VPT > 1 && N != 0 && !OWNED &&
         (WIDE || (N <= 4 && E::BYTES == 2 && (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN)));
@@ -672,7 +698,7 @@ __global__ void __launch_bounds__(1024 / VPT)
         const int64_t row_byte = row * (int64_t)row_bytes; // wavefront-uniform
 
         // ---- reduce, residual add, sum of squares ------------------------------------------------
-        const rsrc_t res_out = row_rsrc(a.residual_out, row_byte, bytes);
+        const rsrc_t res_out = row_rsrc(a.ptr(kPtrResidualOut), row_byte, bytes);
         u32x4 xraw[VPT];
         // With four vectors per thread, or one, the partials are summed rank by rank as they arrive (the memory system
         // returns a wavefront's loads in the order it issued them), so that only the last partial's additions are
@@ -714,7 +740,7 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) sraw[j] = E::pack(acc[j]);
             } else {
-                const rsrc_t rs = row_rsrc(a.stage, row_byte, bytes);
+                const rsrc_t rs = row_rsrc(a.ptr(kPtrStage), row_byte, bytes);
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) sraw[j] = rsrc_load16(rs, TDE_OFF(j));
             }
@@ -807,12 +833,12 @@ __global__ void __launch_bounds__(1024 / VPT)
         // The stage behind the gamma request: a wavefront's loads and stores are waited for in order, and gamma would
         // otherwise wait for these stores.
         if (sum_is_new) {
-            const rsrc_t stage = row_rsrc(a.stage, row_byte, bytes);
+            const rsrc_t stage = row_rsrc(a.ptr(kPtrStage), row_byte, bytes);
 #pragma unroll
             for (int j = 0; j < VPT; ++j) rsrc_store16(stage, TDE_OFF(j), sraw[j]);
         }
-        const float sumsq = sumsq_torch_order<VPT, VEC, E::BYTES == 2>(lds_img, lds_bs, a.hidden, TDE_T, tpr, group, TDE_LANE, xraw[VPT - 1][0]);
-        const float rs = 1.0f / __builtin_sqrtf(sumsq / a.hidden_f + a.eps);
+        const float sumsq = sumsq_torch_order<VPT, VEC, E::BYTES == 2>(lds_img, lds_bs, a.hidden(), TDE_T, tpr, group, TDE_LANE, xraw[VPT - 1][0]);
+        const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
 
         // ---- normalize ------------------------------------------------------------------------------
         u32x4 yraw[VPT];
@@ -829,7 +855,7 @@ __global__ void __launch_bounds__(1024 / VPT)
             for (int i = 0; i < VEC; ++i) y[i] = g[i] * y[i];
             yraw[j] = E::pack(y);
             if constexpr (Q == TDE_QUANT_NONE || WN) {
-                const rsrc_t norm_out = row_rsrc(a.norm_out, row_byte, bytes);
+                const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
                 rsrc_store16(norm_out, TDE_OFF(j), yraw[j]);
             }
             if constexpr (Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC) amax[j] = amax_fold<E>(0u, yraw[j]);
@@ -846,8 +872,8 @@ __global__ void __launch_bounds__(1024 / VPT)
             float scale[VPT];
             if constexpr (Q == TDE_QUANT_FP8_GROUP) {
                 constexpr int LANES_PER_GROUP = TDE_QUANT_GROUP / VEC; // 16 (2-byte types) or 32 (fp32)
-                const int64_t groups_per_row = a.hidden / TDE_QUANT_GROUP;
-                const rsrc_t sc_out = row_rsrc(a.scale_out, row * groups_per_row * 4, row_ok ? (uint32_t)groups_per_row * 4u : 0u);
+                const int64_t groups_per_row = a.hidden() / TDE_QUANT_GROUP;
+                const rsrc_t sc_out = row_rsrc(a.ptr(kPtrScale), row * groups_per_row * 4, row_ok ? (uint32_t)groups_per_row * 4u : 0u);
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) {
                     uint32_t m = row16_max(amax_f32_bits<E>(amax[j]));
@@ -871,9 +897,9 @@ __global__ void __launch_bounds__(1024 / VPT)
                 const float sc = __builtin_bit_cast(float, m) / QMAX;
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) scale[j] = sc;
-                if (row_ok && TDE_T == 0) ((TDE_GLOBAL float *)a.scale_out)[row] = sc;
+                if (row_ok && TDE_T == 0) ((TDE_GLOBAL float *)a.ptr(kPtrScale))[row] = sc;
             }
-            const rsrc_t q_out = row_rsrc(a.q_out, row * (int64_t)a.hidden, row_ok ? (uint32_t)a.hidden : 0u);
+            const rsrc_t q_out = row_rsrc(a.ptr(kPtrCodes), row * (int64_t)a.hidden(), row_ok ? (uint32_t)a.hidden() : 0u);
 #pragma unroll
             for (int j = 0; j < VPT; ++j) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
             // One wavefront-uniform decision for all of the thread's vectors, so the common path carries no per-lane
@@ -952,6 +978,8 @@ struct ReduceSpan {
     int64_t row_step;
     int64_t spans_per_row;
     uint32_t xcd_chunk; // spans each XCD takes in a row (xcd_chunked_block); 16 over whole tensors, 1 for single rows
+    uint32_t chunked_blocks;
+    uint64_t table; // device pointer table of the partials that RowArgs::table_mask names
 };
 
 template <class E, int N, int U>
@@ -959,16 +987,8 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
     constexpr int VEC = E::VEC;
     constexpr uint32_t SPAN = 256u * U * 16u; // bytes per workgroup
     const void *part[N];
-#pragma unroll
-    for (int r = 0; r < N; ++r) part[r] = a.part[r];
-    if (a.table != nullptr) {
-#pragma unroll
-        for (int r = 0; r < N; ++r) {
-            const void *from_table = a.table[r];
-            part[r] = (part[r] != nullptr) ? part[r] : from_table;
-        }
-    }
-    const int64_t bid = xcd_chunked_block(blockIdx.x, gridDim.x, sp.xcd_chunk);
+    partial_addresses(a, sp.table, part);
+    const int64_t bid = xcd_chunked_block(blockIdx.x, sp.chunked_blocks, sp.xcd_chunk);
     const int64_t k = bid / sp.spans_per_row;
     const int64_t in_row = (bid - k * sp.spans_per_row) * SPAN;
     const int64_t base = (sp.first_row + k * sp.row_step) * sp.row_bytes + in_row;
@@ -981,7 +1001,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
 #pragma unroll
         for (int u = 0; u < U; ++u) raw[u][r] = rsrc_load16(rs, (uint32_t)(u * 256 + threadIdx.x) * 16u);
     }
-    const rsrc_t out = row_rsrc(a.stage, base, bytes);
+    const rsrc_t out = row_rsrc(a.ptr(kPtrStage), base, bytes);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         float acc[VEC];
@@ -1020,16 +1040,16 @@ struct Geometry {
 hipError_t launch_rows_bf16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_rows_f16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
-hipError_t launch_reduce_bf16(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
-hipError_t launch_reduce_f16(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
-hipError_t launch_reduce_f32(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
+hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
+hipError_t launch_reduce_f16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
+hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 
 // Rows of doubles (tde_rows_f64.hip): one vector per thread, no quantized output.
 hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s);
-hipError_t launch_reduce_f64(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
+hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 
 // Traffic skeleton of the row kernel (tde_probe.hip): same geometry and bytes, no arithmetic.
-hipError_t launch_traffic(int n, int vpt, int code_bytes, bool wn, const RowArgs &a, const Geometry &g, uint32_t row_bytes,
+hipError_t launch_traffic(int n, int vpt, int code_bytes, bool wn, const RowArgs &a, const Geometry &g, uint32_t row_bytes, uint32_t parts,
                           hipStream_t s);
 
 // Instantiation + dispatch body used by the three per-dtype translation units.
@@ -1091,32 +1111,33 @@ hipError_t launch_rows_e(int n, int vpt, int q, bool wn, const RowArgs &a, const
 }
 
 template <class E, int N, int U>
-hipError_t launch_reduce_nu(const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
+hipError_t launch_reduce_nu(const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
                             hipStream_t s) {
     constexpr int64_t span = 256 * U * 16;
-    ReduceSpan sp{row_bytes, first_row, row_step, (row_bytes + span - 1) / span, rows == 1 ? 16u : 1u};
+    ReduceSpan sp{row_bytes, first_row, row_step, (row_bytes + span - 1) / span, rows == 1 ? 16u : 1u, 0u, table};
     const int64_t blocks = rows * sp.spans_per_row;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue; // grid dimension limit
+    sp.chunked_blocks = chunked_blocks(blocks, sp.xcd_chunk);
     hipLaunchKernelGGL((reduce_kernel<E, N, U>), dim3((unsigned)blocks), dim3(256), 0, s, a, sp);
     return hipGetLastError();
 }
 
 template <class E, int N>
-hipError_t launch_reduce_n(const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
+hipError_t launch_reduce_n(const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
                            hipStream_t s) {
-    if (N >= 8 && row_bytes <= 256 * 4 * 16) return launch_reduce_nu<E, N, 2>(a, row_bytes, first_row, row_step, rows, s);
-    return launch_reduce_nu<E, N, 4>(a, row_bytes, first_row, row_step, rows, s);
+    if (N >= 8 && row_bytes <= 256 * 4 * 16) return launch_reduce_nu<E, N, 2>(a, table, row_bytes, first_row, row_step, rows, s);
+    return launch_reduce_nu<E, N, 4>(a, table, row_bytes, first_row, row_step, rows, s);
 }
 
 // Stage A over rows first_row, first_row + row_step, ... (`rows` of them), each row_bytes long.
 template <class E>
-hipError_t launch_reduce_e(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
+hipError_t launch_reduce_e(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
                            hipStream_t s) {
     switch (n) {
-    case 2: return launch_reduce_n<E, 2>(a, row_bytes, first_row, row_step, rows, s);
-    case 4: return launch_reduce_n<E, 4>(a, row_bytes, first_row, row_step, rows, s);
-    case 8: return launch_reduce_n<E, 8>(a, row_bytes, first_row, row_step, rows, s);
+    case 2: return launch_reduce_n<E, 2>(a, table, row_bytes, first_row, row_step, rows, s);
+    case 4: return launch_reduce_n<E, 4>(a, table, row_bytes, first_row, row_step, rows, s);
+    case 8: return launch_reduce_n<E, 8>(a, table, row_bytes, first_row, row_step, rows, s);
     }
     return hipErrorInvalidValue;
 }

@@ -33,37 +33,30 @@ __device__ __forceinline__ u32x4 pack_f64(const double (&d)[2]) {
     return raw;
 }
 
-template <int N, bool OWNED = false>
+template <int N, int FORM = kFormPlain>
 __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
+    constexpr bool OWNED = FORM == kFormOwned, STAGED = FORM == kFormStaged;
     constexpr int NP = (N == 0) ? 1 : N;
     extern __shared__ __attribute__((aligned(16))) float lds_dyn[]; // squares (two per thread), then block sums
     float *const lds_img = lds_dyn;
-    float *const lds_bs = lds_dyn + blockDim.x * 2;
+    float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * 2;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int tpr = a.threads_per_row;
     const int group = __builtin_amdgcn_readfirstlane(tid / tpr);
     const int t = tid - group * tpr;
-    const uint32_t row_bytes = (uint32_t)a.hidden * 8u;
+    const uint32_t row_bytes = (uint32_t)a.hidden() * 8u;
     const uint32_t off = (uint32_t)t * 16u;
 
     const void *part[NP];
-#pragma unroll
-    for (int r = 0; r < NP; ++r) part[r] = a.part[r];
-    if (a.table != nullptr) {
-#pragma unroll
-        for (int r = 0; r < NP; ++r) {
-            const void *from_table = a.table[r];
-            part[r] = (part[r] != nullptr) ? part[r] : from_table;
-        }
-    }
-    const rsrc_t gamma_rsrc = row_rsrc(a.gamma, 0, row_bytes);
+    partial_addresses(a, a.address(kPtrStage), part);
+    const rsrc_t gamma_rsrc = row_rsrc(a.ptr(kPtrGamma), 0, row_bytes);
 
     {
         // the grid covers every row; each XCD takes runs of consecutive row groups (xcd_chunked_block)
-        int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, gridDim.x, (uint32_t)a.xcd_chunk) * a.rows_per_block + group;
+        int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block + group;
 
-        bool sum_is_new = N != 0 && a.stage != nullptr;
+        bool sum_is_new = STAGED;
         if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
         const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
         const int64_t row_byte = row * (int64_t)row_bytes;
@@ -72,9 +65,9 @@ __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
 #pragma unroll
             for (int r = 0; r < NP; ++r) praw[r] = rsrc_load16(row_rsrc(part[r], row_byte, bytes), off);
         } else {
-            praw[0] = rsrc_load16(row_rsrc(a.stage, row_byte, bytes), off);
+            praw[0] = rsrc_load16(row_rsrc(a.ptr(kPtrStage), row_byte, bytes), off);
         }
-        const u32x4 rraw = rsrc_load16(row_rsrc(a.residual_in, row_byte, bytes), off);
+        const u32x4 rraw = rsrc_load16(row_rsrc(a.ptr(kPtrResidualIn), row_byte, bytes), off);
         const u32x4 graw = __builtin_amdgcn_raw_buffer_load_b128(gamma_rsrc, (int)off, 0, kAuxDefault);
 
         double acc[2] = {0.0, 0.0};
@@ -89,25 +82,25 @@ __global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
                 acc[1] += p[1];
             }
         }
-        if (sum_is_new) rsrc_store16(row_rsrc(a.stage, row_byte, bytes), off, pack_f64(acc));
+        if (sum_is_new) rsrc_store16(row_rsrc(a.ptr(kPtrStage), row_byte, bytes), off, pack_f64(acc));
         double res[2], x[2];
         unpack_f64(rraw, res);
         x[0] = acc[0] + res[0];
         x[1] = acc[1] + res[1];
-        rsrc_store16(row_rsrc(a.residual_out, row_byte, bytes), off, pack_f64(x));
+        rsrc_store16(row_rsrc(a.ptr(kPtrResidualOut), row_byte, bytes), off, pack_f64(x));
 
         const float f0 = (float)x[0], f1 = (float)x[1];
         const float sq[2] = {f0 * f0, f1 * f1};
         const uint32_t landed = __builtin_bit_cast(uint32_t, sq[0]);
         sumsq_put<1, 2>(lds_img, 0, tpr, group, t, sq, landed);
-        const float sumsq = sumsq_torch_order<1, 2, false>(lds_img, lds_bs, a.hidden, t, tpr, group, lane, landed);
-        const float rs = 1.0f / __builtin_sqrtf(sumsq / a.hidden_f + a.eps);
+        const float sumsq = sumsq_torch_order<1, 2, false>(lds_img, lds_bs, a.hidden(), t, tpr, group, lane, landed);
+        const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
 
         double g[2], y[2];
         unpack_f64(graw, g);
         y[0] = g[0] * (x[0] * (double)rs);
         y[1] = g[1] * (x[1] * (double)rs);
-        rsrc_store16(row_rsrc(a.norm_out, row_byte, bytes), off, pack_f64(y));
+        rsrc_store16(row_rsrc(a.ptr(kPtrNorm), row_byte, bytes), off, pack_f64(y));
     }
 }
 
@@ -116,16 +109,8 @@ template <int N, int U>
 __global__ void __launch_bounds__(256) reduce_kernel_f64(const RowArgs a, const ReduceSpan sp) {
     constexpr uint32_t SPAN = 256u * U * 16u; // bytes per workgroup
     const void *part[N];
-#pragma unroll
-    for (int r = 0; r < N; ++r) part[r] = a.part[r];
-    if (a.table != nullptr) {
-#pragma unroll
-        for (int r = 0; r < N; ++r) {
-            const void *from_table = a.table[r];
-            part[r] = (part[r] != nullptr) ? part[r] : from_table;
-        }
-    }
-    const int64_t bid = xcd_chunked_block(blockIdx.x, gridDim.x, sp.xcd_chunk);
+    partial_addresses(a, sp.table, part);
+    const int64_t bid = xcd_chunked_block(blockIdx.x, sp.chunked_blocks, sp.xcd_chunk);
     const int64_t k = bid / sp.spans_per_row;
     const int64_t in_row = (bid - k * sp.spans_per_row) * SPAN;
     const int64_t base = (sp.first_row + k * sp.row_step) * sp.row_bytes + in_row;
@@ -138,7 +123,7 @@ __global__ void __launch_bounds__(256) reduce_kernel_f64(const RowArgs a, const 
 #pragma unroll
         for (int u = 0; u < U; ++u) raw[u][r] = rsrc_load16(rs, (uint32_t)(u * 256 + threadIdx.x) * 16u);
     }
-    const rsrc_t out = row_rsrc(a.stage, base, bytes);
+    const rsrc_t out = row_rsrc(a.ptr(kPtrStage), base, bytes);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         double acc[2] = {0.0, 0.0};
@@ -153,14 +138,15 @@ __global__ void __launch_bounds__(256) reduce_kernel_f64(const RowArgs a, const 
     }
 }
 
-hipError_t launch_reduce_f64(int n, const RowArgs &a, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
+hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,
                              hipStream_t s) {
     constexpr int U = 4;
     constexpr int64_t span = 256 * U * 16;
-    ReduceSpan sp{row_bytes, first_row, row_step, (row_bytes + span - 1) / span, rows == 1 ? 16u : 1u};
+    ReduceSpan sp{row_bytes, first_row, row_step, (row_bytes + span - 1) / span, rows == 1 ? 16u : 1u, 0u, table};
     const int64_t blocks = rows * sp.spans_per_row;
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+    sp.chunked_blocks = chunked_blocks(blocks, sp.xcd_chunk);
     const dim3 grid((unsigned)blocks), block(256);
     switch (n) {
     case 2: hipLaunchKernelGGL((reduce_kernel_f64<2, U>), grid, block, 0, s, a, sp); break;
@@ -174,14 +160,20 @@ hipError_t launch_reduce_f64(int n, const RowArgs &a, int64_t row_bytes, int64_t
 hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, 1, 2): doubles are never limited per CU
-    const bool owned = g.form == kFormOwned;
+#define TDE_F64(N)                                                                                              \
+    case N:                                                                                                     \
+        hipLaunchKernelGGL((g.form == kFormOwned    ? row_kernel_f64<N, kFormOwned>                             \
+                            : g.form == kFormStaged ? row_kernel_f64<N, kFormStaged>                            \
+                                                    : row_kernel_f64<N>), grid, block, lds, s, a);             \
+        break;
     switch (n) {
     case 0: hipLaunchKernelGGL((row_kernel_f64<0>), grid, block, lds, s, a); break;
-    case 2: hipLaunchKernelGGL((owned ? row_kernel_f64<2, true> : row_kernel_f64<2>), grid, block, lds, s, a); break;
-    case 4: hipLaunchKernelGGL((owned ? row_kernel_f64<4, true> : row_kernel_f64<4>), grid, block, lds, s, a); break;
-    case 8: hipLaunchKernelGGL((owned ? row_kernel_f64<8, true> : row_kernel_f64<8>), grid, block, lds, s, a); break;
+    TDE_F64(2)
+    TDE_F64(4)
+    TDE_F64(8)
     default: return hipErrorInvalidValue;
     }
+#undef TDE_F64
     return hipGetLastError();
 }
 

@@ -47,28 +47,35 @@ int32_t dtype_code(const Tensor &t) {
     return -1;
 }
 
-// Pointer tables handed out by CommWorkspace::get_workspace, keyed by their device address, with the size of
-// the slots they point to.  The operators receive only the table tensor (the reference's signature), so this
-// is how they learn how many bytes of each slot exist: a call whose rows do not fit is refused instead of
-// reading past a slot.
+// Pointer tables handed out by CommWorkspace::get_workspace, keyed by their device address, with the slots they point to
+// and their size.  The operators receive only the table tensor (the reference's signature), so this is how they learn how
+// many bytes of each slot exist -- a call whose rows do not fit is refused instead of reading past a slot -- and the slots'
+// addresses, which go to the kernel as arguments: reading them from the table on the device is a memory access that every
+// wavefront's first load waits for (8 x [128, 4096] bf16: 5.20 us in the kernel with the table, 4.96 with arguments; 2 x
+// [16, 1024] 3.28 and 3.12).
+struct TableInfo {
+    int64_t slot_bytes = -1;
+    int64_t nranks = 0;
+    const void *slots[TDE_MAX_RANKS] = {};
+};
 std::mutex g_tables_mutex;
-std::unordered_map<const void *, int64_t> g_table_slot_bytes;
+std::unordered_map<const void *, TableInfo> g_tables;
 
-void register_table(const void *table, int64_t slot_bytes) {
+void register_table(const void *table, const TableInfo &info) {
     const std::lock_guard<std::mutex> lock(g_tables_mutex);
-    g_table_slot_bytes[table] = slot_bytes;
+    g_tables[table] = info;
 }
 
 void unregister_table(const void *table) {
     const std::lock_guard<std::mutex> lock(g_tables_mutex);
-    g_table_slot_bytes.erase(table);
+    g_tables.erase(table);
 }
 
-// -1 if `table` was not handed out by a live CommWorkspace.
-int64_t table_slot_bytes(const void *table) {
+// slot_bytes is -1 if `table` was not handed out by a live CommWorkspace.
+TableInfo table_info(const void *table) {
     const std::lock_guard<std::mutex> lock(g_tables_mutex);
-    const auto it = g_table_slot_bytes.find(table);
-    return it == g_table_slot_bytes.end() ? -1 : it->second;
+    const auto it = g_tables.find(table);
+    return it == g_tables.end() ? TableInfo{} : it->second;
 }
 
 void check_row_tensor(const Tensor &t, const Tensor &like, const char *name) {
@@ -140,7 +147,11 @@ public:
         check_status(tde_workspace_fill_table(ws_, reinterpret_cast<void **>(host.data_ptr()), (int32_t)entries),
                      "get_workspace");
         table_ = host.to(ref.device());
-        register_table(table_.data_ptr(), size_in_bytes_);
+        TableInfo info;
+        info.slot_bytes = size_in_bytes_;
+        info.nranks = world_size_;
+        for (int64_t r = 0; r < world_size_; ++r) info.slots[r] = tde_workspace_slot(ws_, (int32_t)r);
+        register_table(table_.data_ptr(), info);
         return table_;
     }
 
@@ -287,15 +298,16 @@ void use_table(Call &c, int64_t rank, int64_t nranks, const Tensor &allreduce_in
                     workspace.numel() >= (3 * nranks + 5) * (int64_t)sizeof(void *),
                 "workspace must be the uint8 GPU pointer table returned by get_workspace for this world size");
     TORCH_CHECK(rank >= 0 && rank < nranks && nranks <= TDE_MAX_RANKS, "rank/nranks out of range");
-    const int64_t slot_bytes = table_slot_bytes(workspace.data_ptr());
-    TORCH_CHECK(slot_bytes >= 0, "workspace is not a pointer table handed out by a live CommWorkspace's get_workspace "
+    const TableInfo info = table_info(workspace.data_ptr());
+    TORCH_CHECK(info.slot_bytes >= 0, "workspace is not a pointer table handed out by a live CommWorkspace's get_workspace "
                                  "(pass that tensor itself, not a copy)");
     TORCH_CHECK(allreduce_in.is_cuda() && allreduce_in.device() == workspace.device(),
                 "allreduce_in must live on the workspace's GPU: the pointer table holds that device's addresses");
     const int64_t bytes = allreduce_in.numel() * (int64_t)allreduce_in.element_size();
-    TORCH_CHECK(bytes <= slot_bytes, "allreduce_in has ", bytes, " bytes but the workspace slots hold ", slot_bytes,
+    TORCH_CHECK(bytes <= info.slot_bytes, "allreduce_in has ", bytes, " bytes but the workspace slots hold ", info.slot_bytes,
                 "; create the workspace (setup_env) with a larger size");
-    c.b.partial_table = reinterpret_cast<const void *const *>(workspace.data_ptr());
+    TORCH_CHECK(nranks <= info.nranks, "workspace was created for ", info.nranks, " ranks, not ", nranks);
+    for (int64_t r = 0; r < nranks; ++r) c.b.partial[r] = info.slots[r];
     c.b.partial[rank] = allreduce_in.data_ptr();
 }
 
