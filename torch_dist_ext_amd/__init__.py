@@ -33,6 +33,7 @@ CommWorkspace = torch.classes.torch_dist_ext.CommWorkspace
 allreduce_rms_fusion_impl = torch.ops.torch_dist_ext.allreduce_rms_fusion
 allreduce_rms_quant_fusion_impl = torch.ops.torch_dist_ext.allreduce_rms_quant_fusion
 reduce_rms_local_impl = torch.ops.torch_dist_ext.reduce_rms_local
+_reduce_rms_partials = torch.ops.torch_dist_ext.reduce_rms_partials.default
 
 QUANT_MODES = {"none": QUANT_NONE, "fp8_token": QUANT_FP8_TOKEN, "fp8_group": QUANT_FP8_GROUP, "int8_token": QUANT_INT8_TOKEN,
                "fp8_static": QUANT_FP8_STATIC}
@@ -112,41 +113,23 @@ def get_workspace_fake(ref: torch.Tensor) -> torch.Tensor:
 allreduce_rms_quant = torch.ops.torch_dist_ext.allreduce_rms_quant
 
 
-def _quant_out_shapes(allreduce_in: torch.Tensor, quant_mode: int):
-    hidden = allreduce_in.shape[-1]
-    lead = tuple(allreduce_in.shape[:-1])
-    if quant_mode == QUANT_FP8_GROUP:
-        scale_shape = lead + (hidden // QUANT_GROUP,)
-    elif quant_mode == QUANT_FP8_STATIC:
-        scale_shape = (0,)   # the scale is the caller's; nothing is written
-    else:
-        scale_shape = lead
-    q_dtype = torch.int8 if quant_mode == QUANT_INT8_TOKEN else torch.float8_e4m3fn
-    return q_dtype, scale_shape
-
-
 def reduce_rms(partials, residual_in, rms_gamma, eps, quant_mode=QUANT_NONE, write_norm=None, algo=ALGO_AUTO, stage=None,
                static_scale=0.0):
     """One rank's stage with the N partials passed as a list of N [tokens, hidden] GPU tensors.
 
     Returns a dict with residual_out and, depending on the mode, norm_out / q / scale."""
-    ref = partials[0]
+    partials = list(partials)
+    if not partials:
+        raise IndexError("reduce_rms: no partials")
     if write_norm is None:
         write_norm = quant_mode == QUANT_NONE
-    out = {"residual_out": torch.empty_like(residual_in)}
-    norm_out = torch.empty_like(ref) if (write_norm or quant_mode == QUANT_NONE) else None
-    q_out = scale_out = None
-    if quant_mode != QUANT_NONE:
-        q_dtype, scale_shape = _quant_out_shapes(ref, quant_mode)
-        q_out = torch.empty(ref.shape, dtype=q_dtype, device=ref.device)
-        out["q"] = q_out
-        if quant_mode != QUANT_FP8_STATIC:
-            scale_out = torch.empty(scale_shape, dtype=torch.float32, device=ref.device)
-            out["scale"] = scale_out
-    if algo in (ALGO_STAGED, ALGO_STAGED_OWNED) and stage is None:
-        stage = torch.empty_like(ref)
-    reduce_rms_local_impl(list(partials), residual_in, rms_gamma, out["residual_out"], norm_out, q_out, scale_out, eps,
-                          quant_mode, algo, stage, static_scale)
+    residual_out, norm_out, q, scale = _reduce_rms_partials(partials, residual_in, rms_gamma, eps, quant_mode, bool(write_norm), algo,
+                                                            stage, static_scale)
+    out = {"residual_out": residual_out}
+    if q is not None:
+        out["q"] = q
+        if scale is not None:
+            out["scale"] = scale
     if norm_out is not None:
         out["norm_out"] = norm_out
     return out
