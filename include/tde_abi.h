@@ -174,7 +174,8 @@ int tde_reduce_rms(const tde_problem *problem, const tde_buffers *buffers, void 
    tde_stage_norm = the body after the barrier (impl.h:381-393): residual add + norm (+quant) of every row of
    buffers->stage; partial[] and partial_table are ignored.
    tde_reduce_rms with the same problem computes and stores exactly what tde_stage_reduce followed by tde_stage_norm
-   does, in one launch (in those two where `stage` overlaps another output, the residual or gamma). */
+   does, in one launch (in those two where `stage` overlaps another output, the residual or gamma, or a partial an
+   output). */
 int tde_stage_reduce(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 int tde_stage_norm(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 

@@ -49,3 +49,28 @@ def test_stage_that_overlaps_another_buffer(cuda_device, where):
     torch.cuda.synchronize()
     assert bits_equal(buf["residual_out"].cpu(), want["residual_out"])
     assert bits_equal(buf["norm_out"].cpu(), want["norm_out"])
+
+
+@pytest.mark.parametrize("out", ["norm_out", "residual_out", "q_out"])
+@pytest.mark.parametrize("algo", [_capi.ALGO_STAGED, _capi.ALGO_STAGED_OWNED])
+def test_output_that_overlaps_a_partial(cuda_device, out, algo):
+    """A caller may reuse the partials' memory for the outputs, shifted: no output is written before the last sum is stored."""
+    import torch_dist_ext_amd as tde
+    print("case", out, algo, flush=True)
+    shift, tokens, hidden = 40, 3000, 1024
+    p, r, g = eager.make_inputs(4, tokens, hidden, torch.bfloat16, 1.0, seed=10)
+    want = eager.reduce_rms(p, r, g, 1e-6, "fp8_token")
+    stage = p.float().sum(0).to(p.dtype).to(cuda_device)   # owned rows: what the peers delivered
+    memory = torch.empty((tokens + shift, hidden), dtype=p.dtype, device=cuda_device)
+    parts = [p[0].to(cuda_device), memory[shift:].copy_(p[1]), p[2].to(cuda_device), p[3].to(cuda_device)]
+    buf = {k: torch.empty_like(r, device=cuda_device) for k in ("norm_out", "residual_out")}
+    buf["q_out"] = torch.empty((tokens, hidden), dtype=torch.float8_e4m3fn, device=cuda_device)
+    buf[out] = memory.view(torch.float8_e4m3fn).view(-1)[: tokens * hidden].view(tokens, hidden) if out == "q_out" else memory[:tokens]
+    if out == "q_out":
+        parts[1] = memory.view(-1)[: tokens * hidden].view(tokens, hidden).copy_(p[1])   # codes of row t lie on row t / 2
+    scale = torch.empty(tokens, device=cuda_device)
+    tde.reduce_rms_local_impl(parts, r.to(cuda_device), g.to(cuda_device), buf["residual_out"], buf["norm_out"], buf["q_out"], scale,
+                              1e-6, tde.QUANT_FP8_TOKEN, algo, stage, 0.0)
+    torch.cuda.synchronize()
+    for got, name in ((buf["residual_out"], "residual_out"), (buf["norm_out"], "norm_out"), (buf["q_out"], "q"), (scale, "scale")):
+        assert bits_equal(got.cpu(), want[name]), name

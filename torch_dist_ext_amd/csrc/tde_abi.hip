@@ -386,16 +386,22 @@ int tde_plan(const tde_problem *problem, tde_plan_out *plan) {
 namespace {
 enum : int { kPhaseReduce = 1, kPhaseNorm = 2, kTrafficOnly = 4 };
 
-// Whether the stage shares bytes with a buffer that the norm of some row reads or writes.
-bool stage_overlaps(const tde_problem *p, const tde_buffers *b) {
-    const int64_t row = p->hidden * elem_bytes(p->dtype), all = p->tokens * row;
-    const auto overlaps = [&](const void *q, int64_t bytes) {
-        const uintptr_t s = reinterpret_cast<uintptr_t>(b->stage), o = reinterpret_cast<uintptr_t>(q);
-        return q != nullptr && o < s + (uintptr_t)all && s < o + (uintptr_t)bytes;
-    };
+// Whether a row's norm touches bytes that another row's sum still needs, or the other way round: the stage shares bytes with a
+// buffer that the norm reads or writes, or a partial shares bytes with an output.
+bool phases_overlap(const tde_problem *p, const tde_buffers *b) {
+    const int64_t row = p->hidden * elem_bytes(p->dtype), all = p->tokens * row, codes = p->tokens * p->hidden;
     const int64_t scales = p->tokens * (p->quant == TDE_QUANT_FP8_GROUP ? p->hidden / TDE_QUANT_GROUP : 1) * (int64_t)sizeof(float);
-    return overlaps(b->residual_in, all) || overlaps(b->residual_out, all) || overlaps(b->norm_out, all) ||
-           overlaps(b->gamma, row) || overlaps(b->q_out, p->tokens * p->hidden) || overlaps(b->scale_out, scales);
+    const auto overlap = [](const void *x, int64_t x_bytes, const void *y, int64_t y_bytes) {
+        const uintptr_t u = reinterpret_cast<uintptr_t>(x), v = reinterpret_cast<uintptr_t>(y);
+        return u != 0 && v != 0 && u < v + (uintptr_t)y_bytes && v < u + (uintptr_t)x_bytes;
+    };
+    const auto meets_output = [&](const void *x) {
+        return overlap(x, all, b->residual_out, all) || overlap(x, all, b->norm_out, all) || overlap(x, all, b->q_out, codes) ||
+               overlap(x, all, b->scale_out, scales);
+    };
+    bool any = meets_output(b->stage) || overlap(b->stage, all, b->residual_in, all) || overlap(b->stage, all, b->gamma, row);
+    for (int r = 0; r < p->nranks; ++r) any = any || meets_output(b->partial[r]);
+    return any;
 }
 
 int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int phases, int probe_parts = 7) {
@@ -472,9 +478,10 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     // are bound by memory: 8 x [2048, 8192] bf16 -> fp8 takes 63.2 us (6.11 TB/s of what must be moved) against 70.3 us in
     // two launches, with owned rows 28.2 us (5.35 TB/s) against 31.2; 8 x [64, 5120] 5.9 against 9.7 and 5.8 against 7.8,
     // 4 x [13721, 532] fp32 38.5 against 47.3 and 27.3 against 36.3.  A stage that overlaps a buffer the norm reads or
-    // writes keeps the two launches, whose second only starts when every sum has been stored; so do partials that only a
+    // writes, or a partial that overlaps an output, keeps the two launches, whose second only starts when every sum has
+    // been stored; so do partials that only a
     // device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
-    const bool one_launch = staged && both && a.table_mask == 0 && !stage_overlaps(p, b);
+    const bool one_launch = staged && both && a.table_mask == 0 && !phases_overlap(p, b);
     if (one_launch) {
         a.set(tde::kPtrStage, b->stage);
         g.form = p->algo == TDE_ALGO_STAGED_OWNED ? tde::kFormOwned : tde::kFormStaged;
