@@ -77,6 +77,14 @@ def test_local_list_op_and_staged(tde, cuda_device):
         assert bits_equal(a[k].cpu(), b[k].cpu()), k
 
 
+def test_reduce_rms_outputs_require_no_gradient(tde, cuda_device):
+    """Also with gamma a parameter: the outputs are tensors that a caller can convert or write in place."""
+    p, r, g = eager.make_inputs(2, 3, 256, torch.bfloat16, 1.0, seed=33)
+    out = tde.reduce_rms([p[i].to(cuda_device) for i in range(2)], r.to(cuda_device), torch.nn.Parameter(g.to(cuda_device)), 1e-6,
+                         tde.QUANT_FP8_TOKEN, write_norm=True)
+    assert len(out) == 4 and not any(v.requires_grad for v in out.values())
+
+
 def test_error_paths_raise(tde, cuda_device):
     x = torch.zeros((4, 256), dtype=torch.bfloat16, device=cuda_device)
     g = torch.ones((256,), dtype=torch.bfloat16, device=cuda_device)

@@ -528,6 +528,10 @@ TORCH_LIBRARY_IMPL(torch_dist_ext, CUDA, m) {
     m.impl("get_workspace", &get_workspace_op);
 }
 
+// The outputs of reduce_rms are plain tensors, also where an input (gamma as a parameter) requires a gradient: without this the
+// default autograd kernel would mark them as having a gradient that is not implemented.
+TORCH_LIBRARY_IMPL(torch_dist_ext, Autograd, m) { m.impl("reduce_rms_partials", torch::CppFunction::makeFallthrough()); }
+
 TORCH_LIBRARY_IMPL(torch_dist_ext, Meta, m) {
     m.impl("allreduce_rms", &allreduce_rms_meta);
     m.impl("allreduce_rms_quant", &allreduce_rms_quant_meta);
