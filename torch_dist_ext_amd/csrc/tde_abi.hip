@@ -87,6 +87,22 @@ int compute_units() {
     return cached_cu;
 }
 
+// Vectors per thread for rows of doubles (4 partials x 2048 rows of 2048: 39.9 -> 38.4 us, 8 x 2048 rows 62.4 -> 58.8, 8 x 300
+// rows 14.7 -> 12.9, 2 x 900 rows of 1700 15.3 -> 13.2).  From a sweep over 2/4/8 partials x rows of 128 to 1024 vectors x 300 to
+// 16000 rows: four vectors per thread are 1-15 % faster than one until there are enough rows to fill the compute units
+// evenly with the wide workgroups as well; beyond, one is 1-12 % faster (more wavefronts in flight).  Rows that fill their
+// lanes or need 13 wavefronts and more gain the longest.
+int vecs_per_thread_f64(const tde_problem *p, int64_t nvec) {
+    const bool many = p->nranks >= 8;
+    // short rows, eight partials: 3-4 % at any length (300 vectors); 128 vectors 2-4 % from 8192 rows
+    if (many && p->algo != TDE_ALGO_STAGED_OWNED && nvec >= 128 && nvec <= 320 && p->tokens >= (nvec < 256 ? 8192 : 256)) return 4;
+    if (nvec < 256 || p->tokens < 256) return 1;
+    if (p->nranks == 2 && nvec > 576 && nvec <= 640) return 4; // ten wavefronts per row: 3-13 % at any length
+    if (many && p->algo == TDE_ALGO_STAGED_OWNED && nvec > 640 && nvec <= 768) return 4; // 700 vectors: 3-6 % at any length
+    const bool longest = nvec % 256 == 0 || nvec > 768;
+    return p->tokens < (longest ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
+}
+
 int validate(const tde_problem *p, tde::Geometry *geo) {
     if (p == nullptr) return TDE_EINVAL;
     const int eb = elem_bytes(p->dtype);
@@ -149,13 +165,13 @@ int validate(const tde_problem *p, tde::Geometry *geo) {
         else if (p->nranks == 4 && p->tokens >= even_from) vpt = 4;
         else if (p->nranks >= 8 && p->tokens >= 16384) vpt = 2; // eight partials, long launches: 2 % over one
     }
+    if (p->dtype == TDE_F64) vpt = vecs_per_thread_f64(p, nvec);
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
     }
     if (p->tune_rows_per_block < 0) return TDE_EINVAL;
     if (p->tune_workgroups_per_cu < -1 || p->tune_workgroups_per_cu > 8 || p->reserved != 0) return TDE_EINVAL;
-    if (p->dtype == TDE_F64) vpt = 1;
     const int64_t lanes = (nvec + vpt - 1) / vpt;
     const int tpr = (int)((lanes + 63) / 64 * 64);
     int rpb = 256 / tpr; // pack short rows so a workgroup has at least four wavefronts

@@ -4,8 +4,10 @@
 //   x   = ((0 + p_0) + ... + p_{N-1}) + residual_in        all in double, rank order          -> residual_out
 //   rs  = 1 / sqrt( sum(float(x)^2) / H + eps )             fp32: RMSNorm.forward squares x.float()
 //   y   = gamma * (x * double(rs))                          double                              -> norm_out
-// No quantized output for this type.  One 16-byte vector per thread, the row kernel's geometry and XCD-aware row
-// mapping.  N == 0: the sum was staged (part[0] holds it), as in the row kernel; reduce_kernel_f64 is that stage A.
+// No quantized output for this type.  One, two or four 16-byte vectors per thread (the plan's vecs_per_thread_f64 says which and
+// what it measured), the row kernel's geometry and XCD-aware row mapping.  Bound by memory: 4 x [2048, 2048] moves 235 MB.  As
+// in the row kernel the partials are added as they arrive, gamma of several vectors is requested once the row's registers
+// are free, and residual_out is stored with the row's other output (one write burst per row).  N == 0: the sum was staged (part[0] holds it), as in the row kernel; reduce_kernel_f64 is that stage A.
 // With a stage the sums are stored to it; OWNED sums rows == owner (mod N) only and reads the others' sums from the stage.
 #include <hip/hip_runtime.h>
 
@@ -33,75 +35,123 @@ __device__ __forceinline__ u32x4 pack_f64(const double (&d)[2]) {
     return raw;
 }
 
-template <int N, int FORM = kFormPlain>
-__global__ void __launch_bounds__(1024) row_kernel_f64(const RowArgs a) {
+// residual_out is stored as soon as it is known in launches whose rows together have this many bytes, and with the normed row
+// in shorter ones, whose rows are all in flight at once and should finish loading first.  Late against early, four vectors
+// per thread: 2 x 300 rows of 2048 -10 %, 2 x 900 of 1024 -11 %, 4 x 900 of 600 -10 %; 4 x 2048 rows of 2048 +3.3 %, 8 x 2048 of 600 +2.8 %.
+constexpr int64_t kEarlyStoreBytes = 9 << 20;
+
+template <int N, int VPT, int FORM = kFormPlain>
+__global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     constexpr bool OWNED = FORM == kFormOwned, STAGED = FORM == kFormStaged;
     constexpr int NP = (N == 0) ? 1 : N;
-    extern __shared__ __attribute__((aligned(16))) float lds_dyn[]; // squares (two per thread), then block sums
+    extern __shared__ __attribute__((aligned(16))) float lds_dyn[]; // squares (two per vector), then block sums
     float *const lds_img = lds_dyn;
-    float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * 2;
+    float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * (VPT * 2);
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int tpr = a.threads_per_row;
     const int group = __builtin_amdgcn_readfirstlane(tid / tpr);
     const int t = tid - group * tpr;
     const uint32_t row_bytes = (uint32_t)a.hidden() * 8u;
-    const uint32_t off = (uint32_t)t * 16u;
+    uint32_t off[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
 
     const void *part[NP];
     partial_addresses(a, a.address(kPtrStage), part);
     const rsrc_t gamma_rsrc = row_rsrc(a.ptr(kPtrGamma), 0, row_bytes);
 
-    {
-        // the grid covers every row; each XCD takes runs of consecutive row groups (xcd_chunked_block)
-        int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block + group;
+    // the grid covers every row; each XCD takes runs of consecutive row groups (xcd_chunked_block)
+    int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block + group;
 
-        bool sum_is_new = STAGED;
-        if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
-        const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
-        const int64_t row_byte = row * (int64_t)row_bytes;
-        u32x4 praw[NP];
-        if (!OWNED || sum_is_new) {
+    bool sum_is_new = STAGED;
+    if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
+    const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
+    const int64_t row_byte = row * (int64_t)row_bytes;
+    const auto load_row = [&](const void *base, u32x4(&v)[VPT]) {
+        const rsrc_t rs = row_rsrc(base, row_byte, bytes);
 #pragma unroll
-            for (int r = 0; r < NP; ++r) praw[r] = rsrc_load16(row_rsrc(part[r], row_byte, bytes), off);
-        } else {
-            praw[0] = rsrc_load16(row_rsrc(a.ptr(kPtrStage), row_byte, bytes), off);
-        }
-        const u32x4 rraw = rsrc_load16(row_rsrc(a.ptr(kPtrResidualIn), row_byte, bytes), off);
-        const u32x4 graw = __builtin_amdgcn_raw_buffer_load_b128(gamma_rsrc, (int)off, 0, kAuxDefault);
-
-        double acc[2] = {0.0, 0.0};
-        if (N == 0 || (OWNED && !sum_is_new)) {
-            unpack_f64(praw[0], acc); // the staged sum
-        } else {
+        for (int j = 0; j < VPT; ++j) v[j] = rsrc_load16(rs, off[j]);
+    };
+    u32x4 praw[NP][VPT], rraw[VPT], graw[VPT];
+    if (!OWNED || sum_is_new) {
 #pragma unroll
-            for (int r = 0; r < N; ++r) {
-                double p[2];
-                unpack_f64(praw[r], p);
-                acc[0] += p[0];
-                acc[1] += p[1];
-            }
-        }
-        if (sum_is_new) rsrc_store16(row_rsrc(a.ptr(kPtrStage), row_byte, bytes), off, pack_f64(acc));
-        double res[2], x[2];
-        unpack_f64(rraw, res);
-        x[0] = acc[0] + res[0];
-        x[1] = acc[1] + res[1];
-        rsrc_store16(row_rsrc(a.ptr(kPtrResidualOut), row_byte, bytes), off, pack_f64(x));
-
-        const float f0 = (float)x[0], f1 = (float)x[1];
-        const float sq[2] = {f0 * f0, f1 * f1};
-        const uint32_t landed = __builtin_bit_cast(uint32_t, sq[0]);
-        sumsq_put<1, 2>(lds_img, 0, tpr, group, t, sq, landed);
-        const float sumsq = sumsq_torch_order<1, 2, false>(lds_img, lds_bs, a.hidden(), t, tpr, group, lane, landed);
-        const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
-
-        double g[2], y[2];
-        unpack_f64(graw, g);
-        y[0] = g[0] * (x[0] * (double)rs);
-        y[1] = g[1] * (x[1] * (double)rs);
-        rsrc_store16(row_rsrc(a.ptr(kPtrNorm), row_byte, bytes), off, pack_f64(y));
+        for (int r = 0; r < NP; ++r) load_row(part[r], praw[r]);
+    } else {
+        load_row(a.ptr(kPtrStage), praw[0]);
     }
+    load_row(a.ptr(kPtrResidualIn), rraw);
+    const auto load_gamma = [&] {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) graw[j] = __builtin_amdgcn_raw_buffer_load_b128(gamma_rsrc, (int)off[j], 0, kAuxDefault);
+    };
+    if constexpr (VPT == 1) load_gamma();
+    else __builtin_amdgcn_sched_barrier(0);
+
+    // The partials are summed rank by rank, as they arrive.
+    double acc[VPT][2];
+    if (N == 0 || (OWNED && !sum_is_new)) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) unpack_f64(praw[0][j], acc[j]); // the staged sum
+    } else {
+#pragma unroll
+        for (int r = 0; r < N; ++r) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {
+                double p[2];
+                unpack_f64(praw[r][j], p);
+                acc[j][0] = (r == 0 ? 0.0 : acc[j][0]) + p[0];
+                acc[j][1] = (r == 0 ? 0.0 : acc[j][1]) + p[1];
+            }
+            if constexpr (VPT > 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    double x[VPT][2];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        double res[2];
+        unpack_f64(rraw[j], res);
+        x[j][0] = acc[j][0] + res[0];
+        x[j][1] = acc[j][1] + res[1];
+    }
+    const bool early = a.tokens * (int64_t)row_bytes >= kEarlyStoreBytes;
+    const auto store_row = [&](const void *base, const double(&v)[VPT][2]) {
+        const rsrc_t rs = row_rsrc(base, row_byte, bytes);
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) rsrc_store16(rs, off[j], pack_f64(v[j]));
+    };
+    const auto store_sums = [&] {
+        if (sum_is_new) store_row(a.ptr(kPtrStage), acc);
+        if (early) store_row(a.ptr(kPtrResidualOut), x);
+    };
+    // Behind the request for gamma: what a wavefront loads is waited for behind the stores it issued before.
+    if constexpr (VPT == 1) store_sums();
+    uint32_t landed = 0;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const float f0 = (float)x[j][0], f1 = (float)x[j][1];
+        const float sq[2] = {f0 * f0, f1 * f1};
+        landed = __builtin_bit_cast(uint32_t, sq[0]);
+        sumsq_put<VPT, 2>(lds_img, j, tpr, group, t, sq, landed);
+    }
+    if constexpr (VPT > 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_gamma();
+        store_sums();
+    }
+    const float sumsq = sumsq_torch_order<VPT, 2, false>(lds_img, lds_bs, a.hidden(), t, tpr, group, lane, landed);
+    const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
+
+    const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        double g[2], y[2];
+        unpack_f64(graw[j], g);
+        y[0] = g[0] * (x[j][0] * (double)rs);
+        y[1] = g[1] * (x[j][1] * (double)rs);
+        rsrc_store16(norm_out, off[j], pack_f64(y));
+    }
+    if (!early) store_row(a.ptr(kPtrResidualOut), x);
 }
 
 // Stage A for doubles: the reduce kernel's spans (ReduceSpan), sums in double from +0 in rank order.
@@ -157,24 +207,37 @@ hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t ro
     return hipGetLastError();
 }
 
-hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s) {
+template <int N, int VPT>
+hipError_t launch_rows_f64_nv(const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
-    const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, 1, 2): doubles are never limited per CU
-#define TDE_F64(N)                                                                                              \
-    case N:                                                                                                     \
-        hipLaunchKernelGGL((g.form == kFormOwned    ? row_kernel_f64<N, kFormOwned>                             \
-                            : g.form == kFormStaged ? row_kernel_f64<N, kFormStaged>                            \
-                                                    : row_kernel_f64<N>), grid, block, lds, s, a);             \
-        break;
-    switch (n) {
-    case 0: hipLaunchKernelGGL((row_kernel_f64<0>), grid, block, lds, s, a); break;
-    TDE_F64(2)
-    TDE_F64(4)
-    TDE_F64(8)
-    default: return hipErrorInvalidValue;
-    }
-#undef TDE_F64
+    const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, VPT, 2): doubles are never limited per CU
+    if constexpr (N == 0)
+        hipLaunchKernelGGL((row_kernel_f64<0, VPT>), grid, block, lds, s, a);
+    else
+        hipLaunchKernelGGL((g.form == kFormOwned    ? row_kernel_f64<N, VPT, kFormOwned>
+                            : g.form == kFormStaged ? row_kernel_f64<N, VPT, kFormStaged>
+                                                    : row_kernel_f64<N, VPT>), grid, block, lds, s, a);
     return hipGetLastError();
+}
+
+template <int N>
+hipError_t launch_rows_f64_n(const RowArgs &a, const Geometry &g, hipStream_t s) {
+    switch (g.vpt) {
+    case 1: return launch_rows_f64_nv<N, 1>(a, g, s);
+    case 2: return launch_rows_f64_nv<N, 2>(a, g, s);
+    case 4: return launch_rows_f64_nv<N, 4>(a, g, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s) {
+    switch (n) {
+    case 0: return launch_rows_f64_n<0>(a, g, s);
+    case 2: return launch_rows_f64_n<2>(a, g, s);
+    case 4: return launch_rows_f64_n<4>(a, g, s);
+    case 8: return launch_rows_f64_n<8>(a, g, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 } // namespace tde
