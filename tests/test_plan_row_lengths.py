@@ -20,3 +20,41 @@ def vecs(dtype, n, nvec, tokens, **kw):
 ])
 def test_doubles(n, nvec, tokens, vpt):
     assert vecs(_capi.F64, n, nvec, tokens) == vpt
+
+
+NONE, FP8, GROUP, INT8, STATIC = (_capi.QUANT_NONE, _capi.QUANT_FP8_TOKEN, _capi.QUANT_FP8_GROUP, _capi.QUANT_INT8_TOKEN,
+                                  _capi.QUANT_FP8_STATIC)
+
+
+@pytest.mark.parametrize("dtype,n,nvec,tokens,quant,vpt", [
+    # 13 wavefronts per row and more
+    (_capi.BF16, 8, 768, 1000, FP8, 1), (_capi.BF16, 8, 769, 1000, FP8, 4), (_capi.BF16, 4, 830, 256, NONE, 4),
+    (_capi.BF16, 4, 830, 255, NONE, 2), (_capi.BF16, 4, 830, 4096, NONE, 4), (_capi.BF16, 4, 830, 4097, NONE, 1), (_capi.F16, 2, 830, 2048, INT8, 2), (_capi.F16, 2, 830, 2049, INT8, 4),
+    (_capi.F16, 2, 830, 2049, NONE, 1), (_capi.F32, 2, 830, 2049, NONE, 4), (_capi.F16, 2, 896, 2049, NONE, 4),
+    # ten wavefronts
+    (_capi.BF16, 8, 577, 768, FP8, 2), (_capi.BF16, 8, 577, 1152, FP8, 1), (_capi.BF16, 8, 577, 16384, FP8, 1),
+    (_capi.BF16, 4, 600, 16384, FP8, 2), (_capi.F32, 2, 600, 32768, NONE, 2), (_capi.BF16, 4, 600, 639, FP8, 1),
+    (_capi.BF16, 4, 600, 1791, NONE, 2), (_capi.BF16, 4, 600, 1792, NONE, 1),
+    # two partials, quantized
+    (_capi.BF16, 2, 576, 1023, FP8, 1), (_capi.BF16, 2, 576, 1024, FP8, 2), (_capi.BF16, 2, 513, 4096, STATIC, 2),
+    (_capi.BF16, 2, 528, 4095, GROUP, 1), (_capi.F16, 2, 641, 768, INT8, 2), (_capi.F16, 2, 768, 1536, INT8, 1),
+    (_capi.F16, 2, 768, 2304, INT8, 2), (_capi.F32, 2, 768, 1536, INT8, 2), (_capi.BF16, 2, 384, 1536, FP8, 2),
+    (_capi.BF16, 2, 449, 1536, FP8, 1), (_capi.BF16, 2, 320, 16383, FP8, 1), (_capi.F32, 2, 320, 1536, FP8, 2),
+    (_capi.F32, 4, 513, 1536, FP8, 2), (_capi.BF16, 4, 513, 1536, FP8, 1),
+    # T-typed output: the windows of row counts
+    (_capi.BF16, 2, 641, 575, NONE, 1), (_capi.BF16, 2, 641, 576, NONE, 4), (_capi.BF16, 2, 768, 1280, NONE, 1),
+    (_capi.BF16, 2, 512, 1536, NONE, 4), (_capi.BF16, 2, 512, 1537, NONE, 1), (_capi.BF16, 4, 512, 1023, NONE, 4), (_capi.BF16, 4, 512, 1024, NONE, 1),
+    (_capi.F32, 2, 257, 1344, NONE, 4), (_capi.F32, 2, 256, 3071, NONE, 4), (_capi.F32, 4, 193, 2079, NONE, 4),
+    (_capi.F32, 4, 192, 2000, NONE, 1),
+])
+def test_row_lengths(dtype, n, nvec, tokens, quant, vpt):
+    assert vecs(dtype, n, nvec, tokens, quant=quant, static_scale=0.5 if quant == STATIC else 0.0) == vpt
+
+
+@pytest.mark.parametrize("n,nvec,tokens,quant,vpt", [
+    (2, 321, 1023, FP8, 1), (2, 321, 1024, FP8, 2), (2, 353, 5000, FP8, 1), (2, 448, 5000, FP8, 1), (4, 448, 1024, INT8, 2), (4, 512, 5000, FP8, 1),
+    (8, 513, 2048, FP8, 2), (2, 576, 4096, FP8, 2), (8, 640, 5000, FP8, 2), (8, 768, 2048, FP8, 4), (2, 768, 4096, FP8, 2),
+    (8, 700, 5000, NONE, 1),
+])
+def test_owned_row_lengths(n, nvec, tokens, quant, vpt):
+    assert vecs(_capi.BF16, n, nvec, tokens, quant=quant, algo=_capi.ALGO_STAGED_OWNED) == vpt

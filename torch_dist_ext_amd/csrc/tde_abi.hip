@@ -103,6 +103,118 @@ int vecs_per_thread_f64(const tde_problem *p, int64_t nvec) {
     return p->tokens < (longest ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
 }
 
+// TDE_ALGO_STAGED_OWNED in one launch, per-token scales: most rows read two buffers only, so a row of one vector per thread has
+// little in flight for its many wavefronts.  Swept over 2/4/8 partials x rows of 240 to 832 vectors x 300 to 16000 rows
+// against one vector per thread: two are 2-19 % faster with six wavefronts per row, 5-18 % with seven (two partials of a
+// 2-byte type: nothing), 4-24 % with nine, 8-21 % with ten; with eleven and twelve four are 3-24 % faster with four and
+// eight partials, two 4-17 % with two.
+int vecs_per_thread_owned(const tde_problem *p, int64_t nvec, int vpt) {
+    const bool few = p->nranks == 2;
+    switch ((nvec + 63) / 64) {
+    case 6: return p->tokens >= 1024 && (!few || nvec <= 352) ? 2 : vpt; // two partials, 371 vectors: +3 %
+    case 7: return p->tokens >= 1024 && (!few || p->dtype == TDE_F32) ? 2 : vpt;
+    case 9: return p->tokens >= (few ? 4096 : 2048) ? 2 : vpt;
+    case 10: return p->tokens >= 640 ? 2 : vpt;
+    case 11:
+    case 12: return p->tokens >= (few ? 4096 : 2048) ? (few ? 2 : 4) : vpt;
+    }
+    return vpt;
+}
+
+// Two and four partials in one launch, rows of up to 768 vectors: a row has few loads per wavefront to cover its reduction, so
+// fewer wavefronts with more vectors each can be faster.  From sweeps over rows of 100 to 768 vectors x 300 to 25000 rows,
+// bf16, fp16 and fp32, every output mode; each line holds where all of its measured points agree.
+int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec) {
+    const int waves = (int)((nvec + 63) / 64); // of a row, with one vector per thread
+    const int64_t t = p->tokens;
+    const bool two = p->nranks == 2, f32 = p->dtype == TDE_F32;
+    if (p->quant == TDE_QUANT_NONE) {
+        // T-typed output is bound by memory either way; what counts is whether the launch is a little more than the
+        // workgroups the compute units hold at once.  There four vectors per thread fit all rows in one go: two partials
+        // 700 to 900 rows of 656 and 768 vectors -14 %, 1400 and 1536 rows of 400 and 512 -10 to -20 %, of 304 -9 to -15 %, 2000 and
+        // 2700 rows of 200 to 256 -3 to -19 %; four partials 700 rows of 400 and 512 -4 to -11 %, 1536 and 2000 rows of 200 to 256
+        // -6 to -12 %.  1570 rows, a little more than six workgroups per compute unit, lose 2-4 % again.
+        if (two && waves >= 11) return t >= 576 && t < 1280 ? 4 : 1;
+        if (waves == 7 || waves == 8) return two ? (t >= 832 && t <= 1536 ? 4 : 1) : (t >= 640 && t < 1024 ? 4 : 1);
+        if (two && (waves == 5 || waves == 6)) return t >= 1344 && t <= 1536 ? 4 : 1;
+        if (waves == 4) return two ? (t >= 1536 && t < 3072 ? 4 : 1) : ((t >= 1472 && t <= 1536) || (t >= 1900 && t < 2080) ? 4 : 1);
+        return 1;
+    }
+    const bool per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
+    if (!two) return f32 && per_token && waves == 9 && t >= 1536 ? 2 : 1; // 3-5 %
+    if (!per_token) return ((waves == 9 || waves >= 11) && t >= 4096) || (waves >= 11 && t >= 768 && t < 1400) ? 2 : 1; // 1-14 %, 0-6 %
+    if (waves >= 11) // 2-18 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
+        return t >= 768 && (f32 || waves == 11 || t < 1536 || t >= 2304) ? 2 : 1;
+    if (waves == 9) return t >= 1024 ? 2 : 1;                           // 1-19 %
+    if (waves == 6 || waves == 7) return t >= 1536 ? 2 : 1;             // 1-14 %
+    if (waves == 5) return t >= (f32 ? 1536 : 16384) ? 2 : 1;           // fp32 3-13 %, others 0-10 %
+    return 1;
+}
+
+int vecs_per_thread(const tde_problem *p, int64_t nvec) {
+    // Vectors per thread, from sweeps on MI355X over hidden 1024..8192 in steps of 1024, 2/4/8 partials, 128..32768 rows
+    // and three output modes (bf16 and fp16 agree); only differences that held on two devices and across the row
+    // counts between the swept powers of two are in here.  Four vectors per thread (small workgroups, many loads in
+    // flight per thread, few wavefronts to synchronize per row, partials summed while the later ones are still
+    // arriving) win on long rows and wherever eight partials meet full wavefronts, two in the longest launches of
+    // mid-length rows; elsewhere one vector per thread is as fast or faster.
+    const bool staged = p->algo == TDE_ALGO_STAGED;
+    int vpt = 1;
+    if (nvec > 768) {
+        // Few rows are latency-bound and the widest row groups have the shortest dependent chain; from 256 rows
+        // up four vectors per thread are 4-13 % faster than one (8 partials, hidden 8192).  With two partials
+        // and up to 2048 rows two vectors per thread are another 2-7 % faster.
+        vpt = p->tokens >= 256 ? 4 : (p->tokens >= 128 ? 2 : 1);
+        if (p->nranks == 2 && p->tokens >= 256 && p->tokens <= 2048) vpt = 2;
+        // Rows of 13 and 14 wavefronts, 769 to 888 vectors against one per thread: quantized output up to -27 % with two
+        // partials, -22 % with four, -15 % with eight, T-typed output -1 to -13 %; but +2 to +6 % in long launches of two
+        // and four partials that move more per row (T-typed rows, the stage), and around 1300 staged rows of two partials.
+        if (nvec < 896 && p->nranks <= 4) {
+            const bool t_typed = p->quant == TDE_QUANT_NONE;
+            const int64_t until = t_typed ? (p->dtype == TDE_F32 ? 6144 : 2048 * p->nranks / 2)
+                                          : (staged || (p->nranks == 4 && p->quant == TDE_QUANT_FP8_STATIC) ? 12288 : INT64_MAX);
+            if (p->tokens > until || (staged && p->nranks == 2 && p->tokens >= 1024 && p->tokens < 1792)) vpt = 1;
+        }
+    } else if (nvec == 512 && p->nranks >= 8 && p->tokens >= 1024) {
+        vpt = p->tokens >= 16384 ? 2 : 4; // four: 3-4 % over one; from 16384 rows two are another 4-7 % ahead
+    } else if (nvec == 256 && p->nranks >= 8 && p->tokens >= 2048) {
+        // four: 3-6 % over one (with fewer partials or rows one is 3-16 % faster); from 32768 rows two: another 4-6 %
+        vpt = p->tokens >= 32768 ? 2 : 4;
+    } else if (nvec == 256 && p->nranks == 4 && p->tokens >= 32768) {
+        vpt = 2; // 3-4 % over one
+    } else if (nvec == 768 && p->nranks >= 8 && p->tokens >= 2048) {
+        // rows of 6144 2-byte elements: twelve wavefronts with one vector each lose to three with four vectors
+        // (2048 to 5600 rows: 1.5-2.3 %) and, in long launches, to six with two (3-6 % from 8192 rows)
+        if (p->tokens >= 8192) vpt = 2;
+        else if (p->tokens < 5632) vpt = 4;
+    } else if (nvec == 768 && p->nranks == 4 && p->tokens >= 1024 && p->tokens < 2048) {
+        vpt = 4; // 1-5 %
+    } else if (nvec == 384 && p->nranks >= 8 && p->tokens >= 8192 && p->quant != TDE_QUANT_NONE) {
+        vpt = p->tokens >= 32768 ? 2 : 4; // 4-5 % over one with quantized output; with T-typed output one is 2 % ahead
+    } else if (nvec == 128 && p->nranks >= 8 && p->tokens >= 4096 && p->tokens < 8192) {
+        vpt = 2; // 1-3 % over one
+    } else if (nvec > 576 && nvec <= 640) {
+        // Ten wavefronts per row leave the compute units unevenly filled: from 640 rows up five wavefronts with two
+        // vectors each are 10-21 % faster until there are enough rows to even that out (2048 with eight partials,
+        // 16384 with four; with two partials one vector per thread stays 16 % behind at any size).  With four partials
+        // and 16384+ rows all three choices are within 1 %; four vectors per thread is the one whose launches take the
+        // same time from the first on (with one, launches 5 to 50 of a cold run took up to 30 % longer); rows that do not
+        // fill four vectors per thread (592 vectors: -5 % with two, -1 % with four) keep two.  They also stop gaining sooner
+        // where a row moves more: four partials with T-typed or staged rows +3 to +6 % from 2800 rows, eight +3 % at 1300.
+        const bool full = nvec == 640, heavy = !full && (staged || (p->nranks == 4 && p->quant == TDE_QUANT_NONE));
+        const int64_t even_from = p->nranks >= 8 ? (full ? 2048 : 1152) : (p->nranks == 4 ? 16384 : INT64_MAX);
+        if (heavy) vpt = p->tokens >= 640 && p->tokens < (p->nranks == 2 ? 6144 : (p->nranks == 4 ? 1792 : 1152)) ? 2 : 1;
+        else if (p->tokens >= (full || p->nranks < 8 ? 640 : 768) && p->tokens < even_from) vpt = 2;
+        else if (p->nranks == 4 && p->tokens >= even_from) vpt = nvec == 640 ? 4 : 2;
+        else if (p->nranks >= 8 && p->tokens >= 16384 && nvec == 640) vpt = 2; // eight partials, long launches: 2 % over one
+    }
+    const bool per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
+    const bool owned = p->algo == TDE_ALGO_STAGED_OWNED, fused = !staged && !owned;
+    if (owned && per_token) vpt = vecs_per_thread_owned(p, nvec, vpt);
+    else if (fused && vpt == 1 && p->nranks <= 4) vpt = vecs_per_thread_few_partials(p, nvec);
+    return vpt;
+}
+
 int validate(const tde_problem *p, tde::Geometry *geo) {
     if (p == nullptr) return TDE_EINVAL;
     const int eb = elem_bytes(p->dtype);
@@ -123,49 +235,7 @@ int validate(const tde_problem *p, tde::Geometry *geo) {
     int64_t total_bytes = 0; // tokens * hidden * elem must be addressable with 64-bit signed offsets
     if (__builtin_mul_overflow(p->tokens, p->hidden * eb, &total_bytes)) return TDE_ESHAPE;
 
-    // Vectors per thread, from sweeps on MI355X over hidden 1024..8192 in steps of 1024, 2/4/8 partials, 128..32768 rows
-    // and three output modes (bf16 and fp16 agree); only differences that held on two devices and across the row
-    // counts between the swept powers of two are in here.  Four vectors per thread (small workgroups, many loads in
-    // flight per thread, few wavefronts to synchronize per row, partials summed while the later ones are still
-    // arriving) win on long rows and wherever eight partials meet full wavefronts, two in the longest launches of
-    // mid-length rows; elsewhere one vector per thread is as fast or faster.
-    int vpt = 1;
-    if (nvec >= 896) {
-        // Few rows are latency-bound and the widest row groups have the shortest dependent chain; from 256 rows
-        // up four vectors per thread are 4-13 % faster than one (8 partials, hidden 8192).  With two partials
-        // and up to 2048 rows two vectors per thread are another 2-7 % faster.
-        vpt = p->tokens >= 256 ? 4 : (p->tokens >= 128 ? 2 : 1);
-        if (p->nranks == 2 && p->tokens >= 256 && p->tokens <= 2048) vpt = 2;
-    } else if (nvec == 512 && p->nranks >= 8 && p->tokens >= 1024) {
-        vpt = p->tokens >= 16384 ? 2 : 4; // four: 3-4 % over one; from 16384 rows two are another 4-7 % ahead
-    } else if (nvec == 256 && p->nranks >= 8 && p->tokens >= 2048) {
-        // four: 3-6 % over one (with fewer partials or rows one is 3-16 % faster); from 32768 rows two: another 4-6 %
-        vpt = p->tokens >= 32768 ? 2 : 4;
-    } else if (nvec == 256 && p->nranks == 4 && p->tokens >= 32768) {
-        vpt = 2; // 3-4 % over one
-    } else if (nvec == 768 && p->nranks >= 8 && p->tokens >= 2048) {
-        // rows of 6144 2-byte elements: twelve wavefronts with one vector each lose to three with four vectors
-        // (2048 to 5600 rows: 1.5-2.3 %) and, in long launches, to six with two (3-6 % from 8192 rows)
-        if (p->tokens >= 8192) vpt = 2;
-        else if (p->tokens < 5632) vpt = 4;
-    } else if (nvec == 768 && p->nranks == 4 && p->tokens >= 1024 && p->tokens < 2048) {
-        vpt = 4; // 1-5 %
-    } else if (nvec == 384 && p->nranks >= 8 && p->tokens >= 8192 && p->quant != TDE_QUANT_NONE) {
-        vpt = p->tokens >= 32768 ? 2 : 4; // 4-5 % over one with quantized output; with T-typed output one is 2 % ahead
-    } else if (nvec == 128 && p->nranks >= 8 && p->tokens >= 4096 && p->tokens < 8192) {
-        vpt = 2; // 1-3 % over one
-    } else if (nvec == 640) {
-        // Ten wavefronts per row leave the compute units unevenly filled: from 640 rows up five wavefronts with two
-        // vectors each are 10-21 % faster until there are enough rows to even that out (2048 with eight partials,
-        // 16384 with four; with two partials one vector per thread stays 16 % behind at any size).  With four partials
-        // and 16384+ rows all three choices are within 1 %; four vectors per thread is the one whose launches take the
-        // same time from the first on (with one, launches 5 to 50 of a cold run took up to 30 % longer).
-        const int64_t even_from = p->nranks >= 8 ? 2048 : (p->nranks == 4 ? 16384 : INT64_MAX);
-        if (p->tokens >= 640 && p->tokens < even_from) vpt = 2;
-        else if (p->nranks == 4 && p->tokens >= even_from) vpt = 4;
-        else if (p->nranks >= 8 && p->tokens >= 16384) vpt = 2; // eight partials, long launches: 2 % over one
-    }
-    if (p->dtype == TDE_F64) vpt = vecs_per_thread_f64(p, nvec);
+    int vpt = p->dtype == TDE_F64 ? vecs_per_thread_f64(p, nvec) : vecs_per_thread(p, nvec);
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
