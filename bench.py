@@ -53,6 +53,22 @@ BENCH_CONFIGS = {
 }
 
 
+def moved_bytes(fused_bytes, nranks, tokens, hidden, elem, algo):
+    """(read, written) bytes of one launch, each input read once and each output written once.  `fused_bytes` is what tde_plan
+    counts for the fused launch.  The staged algorithms write the sums to the stage as well; with owned rows rank 0 sums
+    ceil(T / N) rows and reads the others' sums from the stage in the partials' place."""
+    row = hidden * elem
+    read = (nranks + 1) * tokens * row + row
+    written = fused_bytes - read
+    if algo == "staged":
+        written += tokens * row
+    elif algo == "staged_owned":
+        owned = -(-tokens // nranks)
+        read = owned * nranks * row + (tokens - owned) * row + tokens * row + row
+        written += owned * row
+    return read, written
+
+
 def kernel_sources_sha256():
     """One hash over the kernel sources, so that figures measured with other kernels are not reported for these."""
     h = hashlib.sha256()
@@ -262,6 +278,7 @@ def main():
     prob = problem(T)
     plan = _capi.plan(prob)
     bytes_per_launch = plan.algorithmic_bytes
+    read_bytes, written_bytes = moved_bytes(plan.algorithmic_bytes, N, T, H, e, args.algo)
     # Enough distinct sets that a buffer is touched again only after > 4 GiB of other inputs AND > 1 GiB of other
     # outputs have passed: the 256 MB memory-side cache then neither serves reads nor absorbs the writes
     # (c3 on one reused set measures 4 % faster than with this rotation, on three sets or more within 1 % of it).
@@ -271,15 +288,9 @@ def main():
     sets = make_sets(torch, cfg, nsets, dev, first)
     gamma = first[2].to(dev)
     staged = algo in (_capi.ALGO_STAGED, _capi.ALGO_STAGED_OWNED)
-    # One stage buffer per input set, so that stage B reads it from HBM like everything else.
+    # One stage buffer per input set, written (owned rows: the other ranks' rows, zeros here, read) from HBM like everything else.
     stages = [torch.zeros((T, H), dtype=dtype, device=dev) for _ in range(nsets)] if staged else None
-    if algo == _capi.ALGO_STAGED_OWNED:
-        # One rank's local share of the two-shot: stage A touches T/N rows of the N partials, stage B all T rows
-        # of the stage (the rows of the other ranks are taken as already delivered; they are zeros here).
-        owned = -(-T // N)
-        bytes_per_launch = (N + 1) * owned * H * e + 2 * T * H * e + H * e + T * H * e + out_bytes
-    elif staged:
-        bytes_per_launch += 2 * T * H * e      # the stage is written once and read once on top of the fused job
+    bytes_per_launch = read_bytes + written_bytes
     stream = torch.cuda.current_stream(dev)
     lib = _capi.load()
     hip_stream = ctypes.c_void_p(stream.cuda_stream)
@@ -434,7 +445,6 @@ def main():
             both_at_once(args.warmup)
         pattern["reads_and_writes_as_two_concurrent_kernels_us"] = both_at_once(args.steps)
     floor_us = pattern.get("traffic_only_us")
-    read_bytes = (N + 1) * T * H * e
     launch_floor_us = timed(lambda i: lib.tde_probe_launch(hip_stream), 500, 50)
 
     ms_per_step = wall * 1e3 / args.steps
@@ -458,8 +468,8 @@ def main():
         "pct_of_hbm_peak": 100.0 * gbs_job / HBM_PEAK_GBS,
         "config": {"workload": "%s: N=%d partials [%d,%d] %s, residual add + RMSNorm + %s%s" % (
                        args.config, N, T, H, dt, quant,
-                       {"staged": " (two launches through a stage buffer)",
-                        "staged_owned": " (two launches; stage A over this rank's T/N rows only)"}.get(args.algo, "")),
+                       {"staged": " (one launch that also stores the sums to a stage buffer)",
+                        "staged_owned": " (one launch; sums of this rank's T/N rows only, the others' read from the stage)"}.get(args.algo, "")),
                    "storage_dtype": dt, "output": quant, "algo": args.algo, "input_sets": nsets, "block_threads": plan.block_threads,
                    "workgroups_per_cu": plan.workgroups_per_cu, "grid_blocks": plan.grid_blocks, "algorithmic_bytes": bytes_per_launch,
                    "settle_steps": settle_steps},
@@ -476,7 +486,7 @@ def main():
                      "traffic_only_frac": (bytes_per_launch / (floor_us * 1e-6) / 1e9 / HBM_PEAK_GBS) if floor_us else None,
                      # the pattern's input streams alone and output streams alone (same workgroups, no arithmetic)
                      "reads_only_us": pattern.get("reads_only_us"),
-                     "reads_only_GBs": (read_bytes / (pattern["reads_only_us"] * 1e-6) / 1e9) if pattern.get("reads_only_us") else None,
+                     "reads_only_GBs": ((N + 1) * T * H * e / (pattern["reads_only_us"] * 1e-6) / 1e9) if pattern.get("reads_only_us") else None,
                      "writes_only_us": pattern.get("writes_only_us"),
                      "writes_only_GBs": (out_bytes / (pattern["writes_only_us"] * 1e-6) / 1e9) if pattern.get("writes_only_us") else None,
                      "reads_and_writes_as_two_concurrent_kernels_us": pattern.get("reads_and_writes_as_two_concurrent_kernels_us"),
@@ -501,7 +511,7 @@ def main():
     # at the write-only rate, times what the plain copy pays for moving both together, plus one dispatch.  No kernel with
     # this traffic goes below it on this box; the skeleton (traffic_only_us) is the same thing measured on the real pattern.
     mixing = (2.0 / rates["copy_GBs"]) / (1.0 / rates["read_only_GBs"] + 1.0 / rates["write_only_GBs"])
-    rates_us = (read_bytes / rates["read_only_GBs"] + max(out_bytes, 0) / rates["write_only_GBs"]) * 1e-3 * mixing + launch_floor_us
+    rates_us = (read_bytes / rates["read_only_GBs"] + written_bytes / rates["write_only_GBs"]) * 1e-3 * mixing + launch_floor_us
     out["roofline"]["device_rates_floor"] = {
         "us": rates_us, "frac": bytes_per_launch / (rates_us * 1e-6) / 1e9 / HBM_PEAK_GBS, "copy_mixing_factor": mixing,
         "what": "reads at device.read_only_GBs + writes at device.write_only_GBs, times the plain copy's cost of moving both together, plus launch_floor_us"}
