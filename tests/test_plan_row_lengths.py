@@ -7,7 +7,7 @@ from torch_dist_ext_amd import _capi
 
 def vecs(dtype, n, nvec, tokens, **kw):
     if torch.cuda.is_available() and _capi.device_info().compute_units != 256:
-        pytest.skip("expectations are for 256 compute units")
+        pytest.skip("the row counts are for 256 compute units; another number of units scales them")
     size = {_capi.F64: 8, _capi.F32: 4}.get(dtype, 2)
     return _capi.plan(_capi.make_problem(dtype, n, tokens, nvec * 16 // size, 1e-5, **kw)).vecs_per_thread
 

@@ -87,20 +87,29 @@ int compute_units() {
     return cached_cu;
 }
 
+// The row counts in the rules for vectors per thread below were swept on 256 compute units.  What they mark is how many rows
+// each unit gets -- a launch's time rises in steps, with every further workgroup on the fullest unit, and the steps lie at
+// different counts for workgroups of different sizes -- so a device (or partition) with another number of units is asked for
+// the same rows per unit.
+int64_t rows_as_on_256_units(int64_t tokens) {
+    const int64_t cus = compute_units();
+    return cus == 256 ? tokens : tokens / cus * 256 + tokens % cus * 256 / cus;
+}
+
 // Vectors per thread for rows of doubles (4 partials x 2048 rows of 2048: 39.9 -> 38.4 us, 8 x 2048 rows 62.4 -> 58.8, 8 x 300
 // rows 14.7 -> 12.9, 2 x 900 rows of 1700 15.3 -> 13.2).  From a sweep over 2/4/8 partials x rows of 128 to 1024 vectors x 300 to
 // 16000 rows: four vectors per thread are 1-15 % faster than one until there are enough rows to fill the compute units
 // evenly with the wide workgroups as well; beyond, one is 1-12 % faster (more wavefronts in flight).  Rows that fill their
 // lanes or need 13 wavefronts and more gain the longest.
-int vecs_per_thread_f64(const tde_problem *p, int64_t nvec) {
+int vecs_per_thread_f64(const tde_problem *p, int64_t nvec, int64_t t) {
     const bool many = p->nranks >= 8;
     // short rows, eight partials: 3-4 % at any length (300 vectors); 128 vectors 2-4 % from 8192 rows
-    if (many && p->algo != TDE_ALGO_STAGED_OWNED && nvec >= 128 && nvec <= 320 && p->tokens >= (nvec < 256 ? 8192 : 256)) return 4;
-    if (nvec < 256 || p->tokens < 256) return 1;
+    if (many && p->algo != TDE_ALGO_STAGED_OWNED && nvec >= 128 && nvec <= 320 && t >= (nvec < 256 ? 8192 : 256)) return 4;
+    if (nvec < 256 || t < 256) return 1;
     if (p->nranks == 2 && nvec > 576 && nvec <= 640) return 4; // ten wavefronts per row: 3-13 % at any length
     if (many && p->algo == TDE_ALGO_STAGED_OWNED && nvec > 640 && nvec <= 768) return 4; // 700 vectors: 3-6 % at any length
     const bool longest = nvec % 256 == 0 || nvec > 768;
-    return p->tokens < (longest ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
+    return t < (longest ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
 }
 
 // TDE_ALGO_STAGED_OWNED in one launch, per-token scales: most rows read two buffers only, so a row of one vector per thread has
@@ -108,15 +117,15 @@ int vecs_per_thread_f64(const tde_problem *p, int64_t nvec) {
 // against one vector per thread: two are 2-19 % faster with six wavefronts per row, 5-18 % with seven (two partials of a
 // 2-byte type: nothing), 4-24 % with nine, 8-21 % with ten; with eleven and twelve four are 3-24 % faster with four and
 // eight partials, two 4-17 % with two.
-int vecs_per_thread_owned(const tde_problem *p, int64_t nvec, int vpt) {
+int vecs_per_thread_owned(const tde_problem *p, int64_t nvec, int64_t t, int vpt) {
     const bool few = p->nranks == 2;
     switch ((nvec + 63) / 64) {
-    case 6: return p->tokens >= 1024 && (!few || nvec <= 352) ? 2 : vpt; // two partials, 371 vectors: +3 %
-    case 7: return p->tokens >= 1024 && (!few || p->dtype == TDE_F32) ? 2 : vpt;
-    case 9: return p->tokens >= (few ? 4096 : 2048) ? 2 : vpt;
-    case 10: return p->tokens >= 640 ? 2 : vpt;
+    case 6: return t >= 1024 && (!few || nvec <= 352) ? 2 : vpt; // two partials, 371 vectors: +3 %
+    case 7: return t >= 1024 && (!few || p->dtype == TDE_F32) ? 2 : vpt;
+    case 9: return t >= (few ? 4096 : 2048) ? 2 : vpt;
+    case 10: return t >= 640 ? 2 : vpt;
     case 11:
-    case 12: return p->tokens >= (few ? 4096 : 2048) ? (few ? 2 : 4) : vpt;
+    case 12: return t >= (few ? 4096 : 2048) ? (few ? 2 : 4) : vpt;
     }
     return vpt;
 }
@@ -124,9 +133,8 @@ int vecs_per_thread_owned(const tde_problem *p, int64_t nvec, int vpt) {
 // Two and four partials in one launch, rows of up to 768 vectors: a row has few loads per wavefront to cover its reduction, so
 // fewer wavefronts with more vectors each can be faster.  From sweeps over rows of 100 to 768 vectors x 300 to 25000 rows,
 // bf16, fp16 and fp32, every output mode; each line holds where all of its measured points agree.
-int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec) {
+int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) {
     const int waves = (int)((nvec + 63) / 64); // of a row, with one vector per thread
-    const int64_t t = p->tokens;
     const bool two = p->nranks == 2, f32 = p->dtype == TDE_F32;
     if (p->quant == TDE_QUANT_NONE) {
         // T-typed output is bound by memory either way; what counts is whether the launch is a little more than the
@@ -151,7 +159,7 @@ int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec) {
     return 1;
 }
 
-int vecs_per_thread(const tde_problem *p, int64_t nvec) {
+int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
     // Vectors per thread, from sweeps on MI355X over hidden 1024..8192 in steps of 1024, 2/4/8 partials, 128..32768 rows
     // and three output modes (bf16 and fp16 agree); only differences that held on two devices and across the row
     // counts between the swept powers of two are in here.  Four vectors per thread (small workgroups, many loads in
@@ -164,8 +172,8 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec) {
         // Few rows are latency-bound and the widest row groups have the shortest dependent chain; from 256 rows
         // up four vectors per thread are 4-13 % faster than one (8 partials, hidden 8192).  With two partials
         // and up to 2048 rows two vectors per thread are another 2-7 % faster.
-        vpt = p->tokens >= 256 ? 4 : (p->tokens >= 128 ? 2 : 1);
-        if (p->nranks == 2 && p->tokens >= 256 && p->tokens <= 2048) vpt = 2;
+        vpt = t >= 256 ? 4 : (t >= 128 ? 2 : 1);
+        if (p->nranks == 2 && t >= 256 && t <= 2048) vpt = 2;
         // Rows of 13 and 14 wavefronts, 769 to 888 vectors against one per thread: quantized output up to -27 % with two
         // partials, -22 % with four, -15 % with eight, T-typed output -1 to -13 %; but +2 to +6 % in long launches of two
         // and four partials that move more per row (T-typed rows, the stage), and around 1300 staged rows of two partials.
@@ -173,25 +181,25 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec) {
             const bool t_typed = p->quant == TDE_QUANT_NONE;
             const int64_t until = t_typed ? (p->dtype == TDE_F32 ? 6144 : 2048 * p->nranks / 2)
                                           : (staged || (p->nranks == 4 && p->quant == TDE_QUANT_FP8_STATIC) ? 12288 : INT64_MAX);
-            if (p->tokens > until || (staged && p->nranks == 2 && p->tokens >= 1024 && p->tokens < 1792)) vpt = 1;
+            if (t > until || (staged && p->nranks == 2 && t >= 1024 && t < 1792)) vpt = 1;
         }
-    } else if (nvec == 512 && p->nranks >= 8 && p->tokens >= 1024) {
-        vpt = p->tokens >= 16384 ? 2 : 4; // four: 3-4 % over one; from 16384 rows two are another 4-7 % ahead
-    } else if (nvec == 256 && p->nranks >= 8 && p->tokens >= 2048) {
+    } else if (nvec == 512 && p->nranks >= 8 && t >= 1024) {
+        vpt = t >= 16384 ? 2 : 4; // four: 3-4 % over one; from 16384 rows two are another 4-7 % ahead
+    } else if (nvec == 256 && p->nranks >= 8 && t >= 2048) {
         // four: 3-6 % over one (with fewer partials or rows one is 3-16 % faster); from 32768 rows two: another 4-6 %
-        vpt = p->tokens >= 32768 ? 2 : 4;
-    } else if (nvec == 256 && p->nranks == 4 && p->tokens >= 32768) {
+        vpt = t >= 32768 ? 2 : 4;
+    } else if (nvec == 256 && p->nranks == 4 && t >= 32768) {
         vpt = 2; // 3-4 % over one
-    } else if (nvec == 768 && p->nranks >= 8 && p->tokens >= 2048) {
+    } else if (nvec == 768 && p->nranks >= 8 && t >= 2048) {
         // rows of 6144 2-byte elements: twelve wavefronts with one vector each lose to three with four vectors
         // (2048 to 5600 rows: 1.5-2.3 %) and, in long launches, to six with two (3-6 % from 8192 rows)
-        if (p->tokens >= 8192) vpt = 2;
-        else if (p->tokens < 5632) vpt = 4;
-    } else if (nvec == 768 && p->nranks == 4 && p->tokens >= 1024 && p->tokens < 2048) {
+        if (t >= 8192) vpt = 2;
+        else if (t < 5632) vpt = 4;
+    } else if (nvec == 768 && p->nranks == 4 && t >= 1024 && t < 2048) {
         vpt = 4; // 1-5 %
-    } else if (nvec == 384 && p->nranks >= 8 && p->tokens >= 8192 && p->quant != TDE_QUANT_NONE) {
-        vpt = p->tokens >= 32768 ? 2 : 4; // 4-5 % over one with quantized output; with T-typed output one is 2 % ahead
-    } else if (nvec == 128 && p->nranks >= 8 && p->tokens >= 4096 && p->tokens < 8192) {
+    } else if (nvec == 384 && p->nranks >= 8 && t >= 8192 && p->quant != TDE_QUANT_NONE) {
+        vpt = t >= 32768 ? 2 : 4; // 4-5 % over one with quantized output; with T-typed output one is 2 % ahead
+    } else if (nvec == 128 && p->nranks >= 8 && t >= 4096 && t < 8192) {
         vpt = 2; // 1-3 % over one
     } else if (nvec > 576 && nvec <= 640) {
         // Ten wavefronts per row leave the compute units unevenly filled: from 640 rows up five wavefronts with two
@@ -203,18 +211,18 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec) {
         // where a row moves more: four partials with T-typed or staged rows +3 to +6 % from 2800 rows, eight +3 % at 1300.
         const bool full = nvec == 640, heavy = !full && (staged || (p->nranks == 4 && p->quant == TDE_QUANT_NONE));
         const int64_t even_from = p->nranks >= 8 ? (full ? 2048 : 1152) : (p->nranks == 4 ? 16384 : INT64_MAX);
-        if (heavy) vpt = p->tokens >= 640 && p->tokens < (p->nranks == 2 ? 6144 : (p->nranks == 4 ? 1792 : 1152)) ? 2 : 1;
-        else if (p->tokens >= (full || p->nranks < 8 ? 640 : 768) && p->tokens < even_from) vpt = 2;
-        else if (p->nranks == 4 && p->tokens >= even_from) vpt = nvec == 640 ? 4 : 2;
-        else if (p->nranks >= 8 && p->tokens >= 16384 && nvec == 640) vpt = 2; // eight partials, long launches: 2 % over one
+        if (heavy) vpt = t >= 640 && t < (p->nranks == 2 ? 6144 : (p->nranks == 4 ? 1792 : 1152)) ? 2 : 1;
+        else if (t >= (full || p->nranks < 8 ? 640 : 768) && t < even_from) vpt = 2;
+        else if (p->nranks == 4 && t >= even_from) vpt = nvec == 640 ? 4 : 2;
+        else if (p->nranks >= 8 && t >= 16384 && nvec == 640) vpt = 2; // eight partials, long launches: 2 % over one
     }
     const bool per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
     const bool owned = p->algo == TDE_ALGO_STAGED_OWNED, fused = !staged && !owned;
     // TDE_ALGO_STAGED, up to four partials, T-typed rows or static and group scales: one vector per thread stays 2-6 % ahead of the
     // ranges above between the lengths they were first swept at.
     if (staged && !per_token && p->nranks <= 4 && nvec > 576 && nvec < 896 && nvec != 640) vpt = nvec == 768 ? vpt : 1;
-    if (owned && per_token) vpt = vecs_per_thread_owned(p, nvec, vpt);
-    else if (fused && vpt == 1 && p->nranks <= 4) vpt = vecs_per_thread_few_partials(p, nvec);
+    if (owned && per_token) vpt = vecs_per_thread_owned(p, nvec, t, vpt);
+    else if (fused && vpt == 1 && p->nranks <= 4) vpt = vecs_per_thread_few_partials(p, nvec, t);
     return vpt;
 }
 
@@ -238,7 +246,8 @@ int validate(const tde_problem *p, tde::Geometry *geo) {
     int64_t total_bytes = 0; // tokens * hidden * elem must be addressable with 64-bit signed offsets
     if (__builtin_mul_overflow(p->tokens, p->hidden * eb, &total_bytes)) return TDE_ESHAPE;
 
-    int vpt = p->dtype == TDE_F64 ? vecs_per_thread_f64(p, nvec) : vecs_per_thread(p, nvec);
+    const int64_t t = rows_as_on_256_units(p->tokens);
+    int vpt = p->dtype == TDE_F64 ? vecs_per_thread_f64(p, nvec, t) : vecs_per_thread(p, nvec, t);
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
