@@ -28,7 +28,7 @@ NONE, FP8, GROUP, INT8, STATIC = (_capi.QUANT_NONE, _capi.QUANT_FP8_TOKEN, _capi
 
 @pytest.mark.parametrize("dtype,n,nvec,tokens,quant,vpt", [
     # 13 wavefronts per row and more
-    (_capi.BF16, 8, 768, 1000, FP8, 1), (_capi.BF16, 8, 769, 1000, FP8, 4), (_capi.BF16, 4, 830, 256, NONE, 4),
+    (_capi.BF16, 8, 768, 1000, FP8, 1), (_capi.BF16, 8, 769, 1000, FP8, 4), (_capi.BF16, 4, 830, 256, NONE, 1), (_capi.BF16, 4, 830, 257, NONE, 4),
     (_capi.BF16, 4, 830, 255, NONE, 2), (_capi.BF16, 4, 830, 4096, NONE, 4), (_capi.BF16, 4, 830, 4097, NONE, 1), (_capi.F16, 2, 830, 2048, INT8, 2), (_capi.F16, 2, 830, 2049, INT8, 4),
     (_capi.F16, 2, 830, 2049, NONE, 1), (_capi.F32, 2, 830, 2049, NONE, 4), (_capi.F16, 2, 896, 2049, NONE, 4),
     # ten wavefronts
@@ -44,11 +44,44 @@ NONE, FP8, GROUP, INT8, STATIC = (_capi.QUANT_NONE, _capi.QUANT_FP8_TOKEN, _capi
     # T-typed output: the windows of row counts
     (_capi.BF16, 2, 641, 575, NONE, 1), (_capi.BF16, 2, 641, 576, NONE, 4), (_capi.BF16, 2, 768, 1280, NONE, 1),
     (_capi.BF16, 2, 512, 1536, NONE, 4), (_capi.BF16, 2, 512, 1537, NONE, 1), (_capi.BF16, 4, 512, 1023, NONE, 4), (_capi.BF16, 4, 512, 1024, NONE, 1),
-    (_capi.F32, 2, 257, 1344, NONE, 4), (_capi.F32, 2, 256, 3071, NONE, 4), (_capi.F32, 4, 193, 2079, NONE, 4),
+    (_capi.F32, 2, 257, 1344, NONE, 4), (_capi.F32, 2, 256, 3071, NONE, 4), (_capi.F32, 4, 193, 2048, NONE, 4), (_capi.F32, 4, 193, 2049, NONE, 1),
     (_capi.F32, 4, 192, 2000, NONE, 1),
 ])
 def test_row_lengths(dtype, n, nvec, tokens, quant, vpt):
     assert vecs(dtype, n, nvec, tokens, quant=quant, static_scale=0.5 if quant == STATIC else 0.0) == vpt
+
+
+# Launches in which several vectors per thread measured slower than one: on both sides of each range, rows of whole 128-byte
+# lines (a multiple of eight vectors) and others, with and without T-typed rows beside the codes.
+@pytest.mark.parametrize("dtype,n,nvec,tokens,quant,wn,vpt", [
+    # T-typed rows beside the codes, two partials
+    (_capi.BF16, 2, 300, 20000, FP8, 0, 2), (_capi.BF16, 2, 300, 20000, FP8, 1, 1), (_capi.BF16, 2, 350, 3071, INT8, 1, 2),
+    (_capi.BF16, 2, 350, 3072, INT8, 1, 1), (_capi.BF16, 2, 430, 1791, FP8, 1, 2), (_capi.BF16, 2, 430, 1792, FP8, 1, 1),
+    (_capi.BF16, 2, 432, 8191, FP8, 1, 2), (_capi.BF16, 2, 432, 8192, FP8, 1, 1), (_capi.F32, 2, 430, 8191, FP8, 1, 2),
+    (_capi.F32, 2, 430, 8192, FP8, 1, 1), (_capi.BF16, 2, 550, 1343, FP8, 1, 2), (_capi.BF16, 2, 550, 1600, FP8, 1, 1),
+    (_capi.BF16, 2, 552, 1600, FP8, 1, 2), (_capi.BF16, 2, 550, 4096, STATIC, 0, 2), (_capi.BF16, 2, 550, 4096, STATIC, 1, 1),
+    (_capi.F32, 2, 550, 4096, STATIC, 1, 2), (_capi.BF16, 2, 690, 1536, FP8, 1, 2), (_capi.BF16, 2, 690, 1537, FP8, 1, 1),
+    (_capi.BF16, 2, 768, 1407, FP8, 1, 2), (_capi.BF16, 2, 768, 1408, FP8, 1, 1), (_capi.BF16, 2, 768, 20000, STATIC, 1, 1),
+    (_capi.F32, 2, 740, 20000, STATIC, 1, 1), (_capi.F32, 2, 744, 20000, STATIC, 1, 2), (_capi.BF16, 2, 768, 1280, STATIC, 1, 2),
+    (_capi.BF16, 2, 768, 1281, STATIC, 1, 1), (_capi.BF16, 2, 750, 1025, STATIC, 1, 1),
+    # ten wavefronts
+    (_capi.BF16, 2, 621, 8191, NONE, 0, 2), (_capi.BF16, 2, 621, 8192, NONE, 0, 1), (_capi.BF16, 2, 624, 8192, NONE, 0, 2),
+    (_capi.F32, 2, 621, 12288, NONE, 0, 1), (_capi.BF16, 4, 621, 4095, STATIC, 0, 2), (_capi.BF16, 4, 621, 4096, STATIC, 0, 1),
+    (_capi.BF16, 4, 621, 8191, FP8, 0, 1), (_capi.BF16, 4, 621, 8192, FP8, 0, 2), (_capi.BF16, 4, 624, 4096, FP8, 0, 2),
+    (_capi.BF16, 4, 621, 1280, STATIC, 1, 2), (_capi.BF16, 4, 621, 1281, STATIC, 1, 1), (_capi.BF16, 4, 621, 1792, FP8, 1, 1),
+    (_capi.BF16, 8, 600, 775, FP8, 0, 2), (_capi.BF16, 8, 600, 776, FP8, 0, 1), (_capi.BF16, 8, 600, 832, FP8, 0, 2),
+    # 13 and 14 wavefronts
+    (_capi.BF16, 8, 771, 768, STATIC, 0, 1), (_capi.BF16, 8, 771, 769, STATIC, 0, 4), (_capi.BF16, 8, 776, 641, STATIC, 0, 4),
+    (_capi.BF16, 8, 801, 650, NONE, 0, 1), (_capi.BF16, 8, 801, 650, FP8, 0, 4), (_capi.F32, 4, 867, 640, NONE, 0, 4),
+    (_capi.F32, 4, 867, 641, NONE, 0, 1), (_capi.F32, 4, 867, 769, NONE, 0, 4), (_capi.BF16, 4, 850, 448, STATIC, 0, 4),
+    (_capi.BF16, 4, 850, 449, STATIC, 0, 1), (_capi.BF16, 4, 850, 800, STATIC, 1, 1), (_capi.BF16, 4, 850, 3072, STATIC, 1, 1),
+    (_capi.BF16, 4, 848, 3072, STATIC, 1, 4), (_capi.F32, 4, 800, 383, GROUP, 0, 1), (_capi.F32, 4, 800, 384, GROUP, 0, 4),
+    # one partial step of the launch
+    (_capi.BF16, 2, 256, 2048, NONE, 0, 4), (_capi.BF16, 2, 256, 2049, NONE, 0, 1), (_capi.BF16, 2, 256, 2240, NONE, 0, 4),
+    (_capi.BF16, 2, 576, 1343, FP8, 0, 2), (_capi.BF16, 2, 576, 1344, FP8, 0, 1), (_capi.BF16, 2, 576, 1537, FP8, 0, 2),
+])
+def test_rows_that_lost(dtype, n, nvec, tokens, quant, wn, vpt):
+    assert vecs(dtype, n, nvec, tokens, quant=quant, write_norm=wn, static_scale=0.5 if quant == STATIC else 0.0) == vpt
 
 
 @pytest.mark.parametrize("n,nvec,tokens,quant,vpt", [

@@ -96,6 +96,12 @@ int64_t rows_as_on_256_units(int64_t tokens) {
     return cus == 256 ? tokens : tokens / cus * 256 + tokens % cus * 256 / cus;
 }
 
+// Whether every row starts and ends on a 128-byte line.  Where a row's wavefronts store at different times, the rows of a
+// launch that do not share their first and last line with a neighbour: several vectors per thread (fewer wavefronts, each
+// further behind the row's others) lose 2-6 % of a long launch of the others (2 x 16384 rows of 608 vectors, T-typed output
+// +3.1 % over one vector per thread, of 609 -3.1 %).
+bool rows_of_whole_lines(int64_t nvec) { return nvec % 8 == 0; }
+
 // Vectors per thread for rows of doubles (4 partials x 2048 rows of 2048: 39.9 -> 38.4 us, 8 x 2048 rows 62.4 -> 58.8, 8 x 300
 // rows 14.7 -> 12.9, 2 x 900 rows of 1700 15.3 -> 13.2).  From a sweep over 2/4/8 partials x rows of 128 to 1024 vectors x 300 to
 // 16000 rows: four vectors per thread are 1-15 % faster than one until there are enough rows to fill the compute units
@@ -131,32 +137,76 @@ int vecs_per_thread_owned(const tde_problem *p, int64_t nvec, int64_t t, int vpt
 }
 
 // Two and four partials in one launch, rows of up to 768 vectors: a row has few loads per wavefront to cover its reduction, so
-// fewer wavefronts with more vectors each can be faster.  From sweeps over rows of 100 to 768 vectors x 300 to 25000 rows,
-// bf16, fp16 and fp32, every output mode; each line holds where all of its measured points agree.
+// fewer wavefronts with more vectors each can be faster.  From sweeps over rows of 64 to 768 vectors x 256 to 32768 rows in
+// bf16, fp16 and fp32, every output mode, with and without T-typed rows beside the codes, against one vector per thread (some
+// 8000 launches of other sizes, and rows in steps of 32 to 64 where a range ends).  A launch's time rises in steps, with
+// every further workgroup on the fullest compute unit; the two geometries' steps lie apart, which is why a range can end at
+// a multiple of 256 rows and why the gain inside one goes from a few percent to twenty.
 int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) {
     const int waves = (int)((nvec + 63) / 64); // of a row, with one vector per thread
     const bool two = p->nranks == 2, f32 = p->dtype == TDE_F32;
     if (p->quant == TDE_QUANT_NONE) {
-        // T-typed output is bound by memory either way; what counts is whether the launch is a little more than the
-        // workgroups the compute units hold at once.  There four vectors per thread fit all rows in one go: two partials
-        // 700 to 900 rows of 656 and 768 vectors -14 %, 1400 and 1536 rows of 400 and 512 -10 to -20 %, of 304 -9 to -15 %, 2000 and
-        // 2700 rows of 200 to 256 -3 to -19 %; four partials 700 rows of 400 and 512 -4 to -11 %, 1536 and 2000 rows of 200 to 256
-        // -6 to -12 %.  1570 rows, a little more than six workgroups per compute unit, lose 2-4 % again.
+        // T-typed output is bound by memory either way, and the gain ends with the first steps: two partials 576 to 1279 rows
+        // of 656 and 768 vectors -4 to -20 %, 832 to 1536 rows of 400 and 512 -5 to -18 %, 1344 to 1536 of 260 to 384 -10 to -16 %,
+        // of 200 to 256 up to -18 % (2048 and 3072 rows), but of 256 +3 to +5 % from 2049 to 2239 rows, all +3 % beyond 3072; four partials
+        // 640 to 1023 rows of 400 and 512 -2 to -8 %, 1472 to 1536 and 1900 to 2048 of 200 to 256 -3 to -12 %, with +2 to +4 % from
+        // 1600 to 1800 rows and +5 to +14 % beyond 2048.
         if (two && waves >= 11) return t >= 576 && t < 1280 ? 4 : 1;
         if (waves == 7 || waves == 8) return two ? (t >= 832 && t <= 1536 ? 4 : 1) : (t >= 640 && t < 1024 ? 4 : 1);
         if (two && (waves == 5 || waves == 6)) return t >= 1344 && t <= 1536 ? 4 : 1;
-        if (waves == 4) return two ? (t >= 1536 && t < 3072 ? 4 : 1) : ((t >= 1472 && t <= 1536) || (t >= 1900 && t < 2080) ? 4 : 1);
+        if (waves == 4)
+            return two ? (t >= 1536 && t <= 3072 && !(nvec > 240 && t > 2048 && t < 2240) ? 4 : 1)
+                       : ((t >= 1472 && t <= 1536) || (t >= 1900 && t <= 2048) ? 4 : 1);
         return 1;
     }
     const bool per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
     if (!two) return f32 && per_token && waves == 9 && t >= 1536 ? 2 : 1; // 3-5 %
-    if (!per_token) return ((waves == 9 || waves >= 11) && t >= 4096) || (waves >= 11 && t >= 768 && t < 1400) ? 2 : 1; // 1-14 %, 0-6 %
-    if (waves >= 11) // 2-18 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
+    // With T-typed rows beside the codes a row moves more, and what several vectors gain without them ends sooner or is left
+    // to rows of whole lines; the rules say where two vectors were still no slower than one.
+    const bool t_rows = p->write_norm != 0, lines = rows_of_whole_lines(nvec);
+    if (!per_token) {
+        // Long launches 1-14 % (with T-typed rows fp32 1-5 %, a 2-byte type at best nothing).  768 to 1280 rows of eleven and twelve
+        // wavefronts -3 to +11 %, up to 1400 rows of them 0 to +3 %, fp32 2-12 %.
+        if (waves >= 11 && t >= 768 && t < (f32 || !t_rows ? 1400 : (lines ? 1281 : 1025))) return 2;
+        if (t < 4096 || !(waves == 9 || waves >= 11)) return 1;
+        return !t_rows || (f32 && (waves < 12 || lines)) || (waves == 11 && lines) ? 2 : 1;
+    }
+    if (waves >= 11) { // 2-18 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
+        if (t_rows && !f32 && (waves >= 12 ? t >= 1408 : !lines && t >= 1537)) return 1;
         return t >= 768 && (f32 || waves == 11 || t < 1536 || t >= 2304) ? 2 : 1;
-    if (waves == 9) return t >= 1024 ? 2 : 1;                           // 1-19 %
-    if (waves == 6 || waves == 7) return t >= 1536 ? 2 : 1;             // 1-14 %
-    if (waves == 5) return t >= (f32 ? 1536 : 16384) ? 2 : 1;           // fp32 3-13 %, others 0-10 %
+    }
+    if (waves == 9) { // 1-20 %; 2-byte types 1-6 % behind from 1344 to 1536 rows
+        if (t_rows && !f32 && !lines && t >= 1344) return 1;
+        return t >= 1024 && (f32 || t < 1344 || t > 1536) ? 2 : 1;
+    }
+    if (waves == 6) return t >= 1536 && (!t_rows || t < 3072) ? 2 : 1; // 1-14 %
+    if (waves == 7) return t >= 1536 && (!t_rows || t < (f32 || lines ? (f32 && lines ? INT64_MAX : 8192) : 1792)) ? 2 : 1; // 1-14 %
+    if (waves == 5) // fp32 3-13 %, others 0-10 %
+        return f32 ? (t >= 1536 && (!t_rows || t < (lines ? 16384 : 6144)) ? 2 : 1) : (t >= 16384 && !t_rows ? 2 : 1);
     return 1;
+}
+
+// Fused rows of 13 and 14 wavefronts: where several vectors per thread are no slower than one.  Per-token codes gain from 256 rows
+// on (1-5 %, from 800 rows 8-20 %).  Several against one elsewhere: eight partials of a 2-byte type with static or group
+// scales up to 768 rows +1 to +4 % (rows of whole lines up to 640), with T-typed output and other rows 0 to +3 %; four partials with
+// static or group scales 449 to 768 rows +1 to +2 %, with T-typed rows as well +2 to +5 % (and from 3072 rows of a 2-byte type that are
+// not whole lines +2 to +5 %); four partials 641 to 768 rows of T-typed output, or of fp32 per-token codes beside T-typed rows, +2 to +5 %;
+// fp32 with static or group scales, rows of whole lines up to 384, +1 to +2 %; up to four partials, exactly one row per compute
+// unit, T-typed output (four partials of a 2-byte type: static and group scales too) +2 to +6 %.
+bool several_vecs_pay(const tde_problem *p, int64_t nvec, int64_t t) {
+    if (t < 256) return true;
+    const bool f32 = p->dtype == TDE_F32, four = p->nranks == 4, many = p->nranks >= 8, lines = rows_of_whole_lines(nvec);
+    const bool none = p->quant == TDE_QUANT_NONE, fixed = p->quant == TDE_QUANT_FP8_GROUP || p->quant == TDE_QUANT_FP8_STATIC;
+    if (t == 256 && ((p->nranks <= 4 && none) || (four && fixed && !f32))) return false;
+    if (fixed && p->nranks >= 4) {
+        if (f32 && lines && !p->write_norm && t < 384) return false;
+        if (many) return f32 || t > (lines ? 640 : 768);
+        if (!p->write_norm) return f32 || !(t > 448 && t <= 768);
+        return f32 ? !(t > 576 && t <= 768) : !(t > 448 && t <= 800) && (lines || t < 3072);
+    }
+    if (none && many) return f32 || lines || t > 768;
+    if (four && (none || (f32 && p->write_norm))) return !(t > (lines ? 680 : 640) && t <= 768);
+    return true;
 }
 
 int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
@@ -183,6 +233,7 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
                                           : (staged || (p->nranks == 4 && p->quant == TDE_QUANT_FP8_STATIC) ? 12288 : INT64_MAX);
             if (t > until || (staged && p->nranks == 2 && t >= 1024 && t < 1792)) vpt = 1;
         }
+        if (nvec < 896 && p->algo <= TDE_ALGO_FUSED && !several_vecs_pay(p, nvec, t)) vpt = 1;
     } else if (nvec == 512 && p->nranks >= 8 && t >= 1024) {
         vpt = t >= 16384 ? 2 : 4; // four: 3-4 % over one; from 16384 rows two are another 4-7 % ahead
     } else if (nvec == 256 && p->nranks >= 8 && t >= 2048) {
@@ -203,18 +254,36 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
         vpt = 2; // 1-3 % over one
     } else if (nvec > 576 && nvec <= 640) {
         // Ten wavefronts per row leave the compute units unevenly filled: from 640 rows up five wavefronts with two
-        // vectors each are 10-21 % faster until there are enough rows to even that out (2048 with eight partials,
-        // 16384 with four; with two partials one vector per thread stays 16 % behind at any size).  With four partials
+        // vectors each are 5-30 % faster until there are enough rows to even that out (2048 with eight partials,
+        // 16384 with four; rows of 640 vectors of two partials 1-4 % at any length).  With four partials
         // and 16384+ rows all three choices are within 1 %; four vectors per thread is the one whose launches take the
-        // same time from the first on (with one, launches 5 to 50 of a cold run took up to 30 % longer); rows that do not
-        // fill four vectors per thread (592 vectors: -5 % with two, -1 % with four) keep two.  They also stop gaining sooner
-        // where a row moves more: four partials with T-typed or staged rows +3 to +6 % from 2800 rows, eight +3 % at 1300.
-        const bool full = nvec == 640, heavy = !full && (staged || (p->nranks == 4 && p->quant == TDE_QUANT_NONE));
+        // same time from the first on (with one, launches 5 to 50 of a cold run took up to 30 % longer).  Rows that do not
+        // fill two vectors per thread stop gaining sooner: eight partials at 1152 rows (+3 % at 1300); where a row moves more (the stage,
+        // T-typed output of four partials) at 1152 to 6144.
+        const bool full = nvec == 640, f32 = p->dtype == TDE_F32;
+        const bool heavy = !full && (staged || (p->nranks == 4 && p->quant == TDE_QUANT_NONE));
         const int64_t even_from = p->nranks >= 8 ? (full ? 2048 : 1152) : (p->nranks == 4 ? 16384 : INT64_MAX);
         if (heavy) vpt = t >= 640 && t < (p->nranks == 2 ? 6144 : (p->nranks == 4 ? 1792 : 1152)) ? 2 : 1;
         else if (t >= (full || p->nranks < 8 ? 640 : 768) && t < even_from) vpt = 2;
         else if (p->nranks == 4 && t >= even_from) vpt = nvec == 640 ? 4 : 2;
         else if (p->nranks >= 8 && t >= 16384 && nvec == 640) vpt = 2; // eight partials, long launches: 2 % over one
+        if (!full && p->algo <= TDE_ALGO_FUSED) {
+            // One vector against two: eight partials 776 to 831 rows -1 to -5 % (768 rows +8 to +12 %; fp32 T-typed output +1 to +6 %); four partials, rows that
+            // are not whole lines, from 4096 rows on -1 to -4 %, until the limit on workgroups per compute unit (below) makes two
+            // 1-5 % faster again, and with T-typed rows beside the codes from 1281 (static and group scales) or 1792 rows on -1 to -7 %
+            // (fp32 per-token codes as without them); two partials, T-typed rows, not whole lines: from 8192 rows of output -1 to -6 %
+            // (fp32 from 12288), beside static and group scales of a 2-byte type from 2304, beside per-token codes from 6144.
+            const bool fixed = p->quant == TDE_QUANT_FP8_GROUP || p->quant == TDE_QUANT_FP8_STATIC, none = p->quant == TDE_QUANT_NONE;
+            const bool beside = !none && p->write_norm != 0, lines = rows_of_whole_lines(nvec);
+            if (p->nranks >= 8 && !(f32 && none) && t >= 776 && t < 832) vpt = 1;
+            if (p->nranks == 4 && !lines && !none) {
+                if (beside && (fixed || !f32) && t >= (fixed && !f32 ? 1281 : 1792)) vpt = 1;
+                if ((beside || !f32) && t >= 4096 && t < kLimitFromWorkgroupsPerCu4 * 256) vpt = 1;
+            }
+            if (p->nranks == 2 && !lines && (none || (beside && !f32)) &&
+                t >= (none ? (f32 ? 12288 : 8192) : (fixed ? 2304 : 6144)))
+                vpt = 1;
+        }
     }
     const bool per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
     const bool owned = p->algo == TDE_ALGO_STAGED_OWNED, fused = !staged && !owned;
