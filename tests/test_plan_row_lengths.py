@@ -14,9 +14,17 @@ def vecs(dtype, n, nvec, tokens, **kw):
 
 @pytest.mark.parametrize("n,nvec,tokens,vpt", [
     (4, 1024, 255, 1), (4, 1024, 256, 4), (4, 1024, 3071, 4), (4, 1024, 3072, 1), (8, 1024, 6143, 4), (8, 1024, 6144, 1),
-    (4, 768, 1536, 4), (4, 767, 1535, 4), (4, 767, 1536, 1), (4, 769, 1536, 4), (4, 256, 256, 4), (4, 255, 256, 1),
-    (2, 576, 1536, 1), (2, 577, 30000, 4), (2, 640, 30000, 4), (2, 641, 1536, 1),
-    (8, 320, 30000, 4), (8, 321, 1536, 1), (8, 128, 8191, 1), (8, 128, 8192, 4), (8, 127, 8192, 1),
+    (4, 768, 575, 4), (4, 768, 576, 1), (4, 767, 1535, 1), (8, 768, 6143, 4), (8, 768, 6144, 1), (8, 744, 1535, 4), (8, 745, 448, 1),
+    (2, 768, 2303, 4), (2, 768, 2304, 1), (2, 767, 1024, 4), (2, 767, 1025, 1), (4, 769, 1536, 4), (4, 256, 256, 4), (4, 255, 256, 1),
+    (2, 576, 1280, 4), (2, 576, 1281, 1), (4, 576, 1024, 4), (4, 576, 1025, 1), (8, 576, 1535, 4), (8, 575, 768, 1),
+    (2, 577, 2303, 4), (2, 577, 2304, 1), (2, 584, 30000, 4), (2, 640, 30000, 4), (2, 641, 1024, 4), (2, 641, 1025, 1),
+    (4, 648, 1535, 4), (4, 641, 576, 1), (2, 641, 1536, 1), (4, 830, 639, 4), (4, 830, 640, 1), (4, 830, 768, 4), (4, 832, 700, 4),
+    (8, 320, 30000, 4), (8, 320, 1025, 1), (8, 321, 1536, 1), (2, 300, 640, 4), (2, 300, 641, 1), (2, 304, 1024, 4), (4, 300, 1280, 1),
+    (4, 300, 1281, 4), (4, 300, 1537, 1), (4, 350, 1024, 4), (4, 350, 1216, 1), (4, 350, 1217, 4), (4, 352, 1280, 1),
+    (4, 512, 1024, 4), (4, 512, 1280, 1), (4, 512, 1535, 4), (4, 512, 1536, 1), (2, 512, 1792, 1), (8, 512, 6143, 4),
+    (2, 256, 2048, 4), (2, 256, 2049, 1), (8, 256, 1024, 4), (8, 256, 1025, 1), (8, 256, 2304, 4), (8, 256, 6144, 1),
+    (2, 1000, 3071, 4), (2, 1001, 1280, 4), (2, 1001, 1281, 1), (4, 1001, 1152, 1), (4, 1017, 3071, 4), (8, 1001, 6143, 4),
+    (8, 128, 8191, 1), (8, 128, 8192, 4), (8, 127, 8192, 1),
 ])
 def test_doubles(n, nvec, tokens, vpt):
     assert vecs(_capi.F64, n, nvec, tokens) == vpt

@@ -102,20 +102,46 @@ int64_t rows_as_on_256_units(int64_t tokens) {
 // +3.1 % over one vector per thread, of 609 -3.1 %).
 bool rows_of_whole_lines(int64_t nvec) { return nvec % 8 == 0; }
 
-// Vectors per thread for rows of doubles (4 partials x 2048 rows of 2048: 39.9 -> 38.4 us, 8 x 2048 rows 62.4 -> 58.8, 8 x 300
-// rows 14.7 -> 12.9, 2 x 900 rows of 1700 15.3 -> 13.2).  From a sweep over 2/4/8 partials x rows of 128 to 1024 vectors x 300 to
-// 16000 rows: four vectors per thread are 1-15 % faster than one until there are enough rows to fill the compute units
-// evenly with the wide workgroups as well; beyond, one is 1-12 % faster (more wavefronts in flight).  Rows that fill their
-// lanes or need 13 wavefronts and more gain the longest.
+// Vectors per thread for rows of doubles in one launch (4 partials x 2048 rows of 2048 in all: 38.5 -> 38.0 us; 2 x 900 rows of
+// 1700: 15.3 -> 13.2).  Four against one, swept over 2/4/8 partials x rows of 128 to 1024 vectors x 256 to 32768 rows (some 5000
+// launches of other sizes): 1-20 % faster while the launch's steps (one workgroup more on the fullest compute unit) favour
+// the narrow workgroups, which ends at the row counts below; beyond them 1-9 % slower.  By wavefronts of a row with one
+// vector per thread; rows that fill their lanes, or nearly (13 and 14 wavefronts), gain the longest.
 int vecs_per_thread_f64(const tde_problem *p, int64_t nvec, int64_t t) {
-    const bool many = p->nranks >= 8;
-    // short rows, eight partials: 3-4 % at any length (300 vectors); 128 vectors 2-4 % from 8192 rows
-    if (many && p->algo != TDE_ALGO_STAGED_OWNED && nvec >= 128 && nvec <= 320 && t >= (nvec < 256 ? 8192 : 256)) return 4;
+    const bool two = p->nranks == 2, four = p->nranks == 4, many = p->nranks >= 8, full = nvec % 256 == 0;
+    const bool staged = p->algo == TDE_ALGO_STAGED, owned = p->algo == TDE_ALGO_STAGED_OWNED;
+    if (staged || owned) { // swept with the stage: the one launch moves a stream more, or its rows read two streams only
+        if (many && !owned && nvec >= 128 && nvec <= 320 && t >= (nvec < 256 ? 8192 : 256)) return 4; // 3-4 %
+        if (nvec < 256 || t < 256) return 1;
+        if (two && nvec > 576 && nvec <= 640) return 4;            // ten wavefronts per row: 3-13 % at any length
+        if (many && owned && nvec > 640 && nvec <= 768) return 4; // 700 vectors: 3-6 % at any length
+        return t < (full || nvec > 768 ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
+    }
+    if (many && nvec >= 128 && nvec < 256) return t >= 8192 ? 4 : 1; // 2-6 %
     if (nvec < 256 || t < 256) return 1;
-    if (p->nranks == 2 && nvec > 576 && nvec <= 640) return 4; // ten wavefronts per row: 3-13 % at any length
-    if (many && p->algo == TDE_ALGO_STAGED_OWNED && nvec > 640 && nvec <= 768) return 4; // 700 vectors: 3-6 % at any length
-    const bool longest = nvec % 256 == 0 || nvec > 768;
-    return t < (longest ? (many ? 6144 : 3072) : 1536) ? 4 : 1;
+    const bool lines = rows_of_whole_lines(nvec);
+    // the fifth workgroup per unit: four vectors 1-8 % behind in rows of up to eight wavefronts
+    const bool fifth = t > 1024 && t <= 1216, fifth_long = t > 1024 && t <= 1280;
+    int64_t until = 0;
+    switch ((nvec + 63) / 64) {
+    case 4: return two ? (t <= 2048 ? 4 : 1) : (many ? (t <= 1024 || (t >= 2304 && t < 6144) ? 4 : 1) : (t <= 2048 && !fifth_long ? 4 : 1));
+    case 5: return t <= (two && !lines ? 640 : 1024) || (t > 1280 && t <= 1536) || (many && t >= 1728) ? 4 : 1;
+    case 6: until = (lines || two ? fifth_long : fifth) ? 0 : 1536; break;
+    case 7: until = !two && fifth ? 0 : (four ? 1408 : 1536); break;
+    case 8:
+        if (full && t >= 1792) until = many ? 6144 : (four ? 2049 : 0);
+        else until = (many && fifth) || (four && fifth_long) ? 0 : 1536;
+        break;
+    case 9: until = two ? 1281 : (four ? 1025 : (lines ? 1536 : 768)); break;
+    case 10: until = two ? (lines ? INT64_MAX : 2304) : 1536; break;
+    case 11: until = lines || many ? 1536 : (two ? 1025 : 576); break;
+    case 12: until = four ? 576 : (lines ? (full ? (two ? 2304 : 6144) : 1536) : (two ? 1025 : 448)); break;
+    case 13:
+    case 14: until = four && !lines && t >= 640 && t < 768 ? 0 : (many ? 6144 : 3072); break;
+    case 15: until = many ? 6144 : 3072; break;
+    default: until = many ? 6144 : (lines || nvec > 1016 ? 3072 : (two ? 1281 : 1152)); break;
+    }
+    return t < until ? 4 : 1;
 }
 
 // TDE_ALGO_STAGED_OWNED in one launch, per-token scales: most rows read two buffers only, so a row of one vector per thread has
