@@ -144,6 +144,28 @@ int vecs_per_thread_f64(const tde_problem *p, int64_t nvec, int64_t t) {
     return t < until ? 4 : 1;
 }
 
+// The same for the norm phase alone (tde_stage_norm, or the second of two launches), which reads two streams whatever the
+// number of partials.  Four against one: up to 37 % faster below 1536 rows (ten to twelve wavefronts), 1-6 % slower beyond the
+// ends below.
+int vecs_per_thread_f64_norm(int64_t nvec, int64_t t) {
+    if (nvec < 256 || t < 256) return 1;
+    switch ((nvec + 63) / 64) {
+    case 4: return t >= 1344 && t <= 3072 ? 4 : 1;
+    case 5: return t >= 1344 && t < 1792 ? 4 : 1;
+    case 6: return t <= 896 || (t > 1280 && t < 1536) ? 4 : 1;
+    case 7:
+    case 8:
+    case 9:
+    case 11:
+    case 12: return t < 1536 ? 4 : 1;
+    case 10: return rows_of_whole_lines(nvec) || t < 8192 ? 4 : 1;
+    case 13:
+    case 14: return 4;
+    case 15: return t < 4096 ? 4 : 1;
+    }
+    return t < 1152 ? 4 : 1;
+}
+
 // TDE_ALGO_STAGED_OWNED in one launch, per-token scales: most rows read two buffers only, so a row of one vector per thread has
 // little in flight for its many wavefronts.  Swept over 2/4/8 partials x rows of 240 to 832 vectors x 300 to 16000 rows
 // against one vector per thread: two are 2-19 % faster with six wavefronts per row, 5-18 % with seven (two partials of a
@@ -321,7 +343,8 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
     return vpt;
 }
 
-int validate(const tde_problem *p, tde::Geometry *geo) {
+// `norm_alone`: the geometry of a launch that only norms the rows of the stage.
+int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) {
     if (p == nullptr) return TDE_EINVAL;
     const int eb = elem_bytes(p->dtype);
     if (eb == 0) return TDE_EDTYPE;
@@ -342,7 +365,7 @@ int validate(const tde_problem *p, tde::Geometry *geo) {
     if (__builtin_mul_overflow(p->tokens, p->hidden * eb, &total_bytes)) return TDE_ESHAPE;
 
     const int64_t t = rows_as_on_256_units(p->tokens);
-    int vpt = p->dtype == TDE_F64 ? vecs_per_thread_f64(p, nvec, t) : vecs_per_thread(p, nvec, t);
+    int vpt = p->dtype != TDE_F64 ? vecs_per_thread(p, nvec, t) : (norm_alone ? vecs_per_thread_f64_norm(nvec, t) : vecs_per_thread_f64(p, nvec, t));
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
@@ -632,6 +655,21 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     if (quant && ((reinterpret_cast<uintptr_t>(b->q_out) & 7u) || (reinterpret_cast<uintptr_t>(b->scale_out) & 3u)))
         return TDE_EALIGN;
 
+    bool from_table = false;
+    for (int r = 0; reads_partials && r < p->nranks; ++r) from_table = from_table || b->partial[r] == nullptr;
+    // The staged algorithms as a whole are one launch of the row kernel that also stores the sums to the stage (owned
+    // rows: reads the other rows' sums from it), which saves reading the sums back, a launch and the gap before it.  Both
+    // are bound by memory: 8 x [2048, 8192] bf16 -> fp8 takes 63.2 us (6.11 TB/s of what must be moved) against 70.3 us in
+    // two launches, with owned rows 28.2 us (5.35 TB/s) against 31.2; 8 x [64, 5120] 5.9 against 9.7 and 5.8 against 7.8,
+    // 4 x [13721, 532] fp32 38.5 against 47.3 and 27.3 against 36.3.  A stage that overlaps a buffer the norm reads or
+    // writes, or a partial that overlaps an output, keeps the two launches, whose second only starts when every sum has
+    // been stored; so do partials that only a device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
+    const bool one_launch = staged && both && !from_table && !phases_overlap(p, b);
+    if (staged && !one_launch) {
+        const int alone = validate(p, &g, true);
+        if (alone != TDE_OK) return alone;
+    }
+
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);
     tde::RowArgs a{};
     if (reads_partials) {
@@ -666,15 +704,6 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
         e = tde::launch_traffic(n, g.vpt, code_bytes, wn, a, g, (uint32_t)g.nvec * 16u, (uint32_t)probe_parts, stream);
         return e == hipSuccess ? TDE_OK : hip_fail(e);
     }
-    // The staged algorithms as a whole are one launch of the row kernel that also stores the sums to the stage (owned
-    // rows: reads the other rows' sums from it), which saves reading the sums back, a launch and the gap before it.  Both
-    // are bound by memory: 8 x [2048, 8192] bf16 -> fp8 takes 63.2 us (6.11 TB/s of what must be moved) against 70.3 us in
-    // two launches, with owned rows 28.2 us (5.35 TB/s) against 31.2; 8 x [64, 5120] 5.9 against 9.7 and 5.8 against 7.8,
-    // 4 x [13721, 532] fp32 38.5 against 47.3 and 27.3 against 36.3.  A stage that overlaps a buffer the norm reads or
-    // writes, or a partial that overlaps an output, keeps the two launches, whose second only starts when every sum has
-    // been stored; so do partials that only a
-    // device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
-    const bool one_launch = staged && both && a.table_mask == 0 && !phases_overlap(p, b);
     if (one_launch) {
         a.set(tde::kPtrStage, b->stage);
         g.form = p->algo == TDE_ALGO_STAGED_OWNED ? tde::kFormOwned : tde::kFormStaged;
