@@ -186,6 +186,13 @@ def test_torch_schemas_match_reference():
     assert inspect.signature(tde.setup_env).parameters["max_size_in_bytes"].default == 8192 * 16384
 
 
+def test_operator_that_returns_its_outputs_names_the_stage_it_writes():
+    import torch_dist_ext_amd  # noqa: F401
+    written = [a.name for a in torch.ops.torch_dist_ext.reduce_rms_partials.default._schema.arguments
+               if a.alias_info is not None and a.alias_info.is_write]
+    assert written == ["stage"]
+
+
 def test_reference_package_name_resolves_to_this_build():
     """A caller written against the reference does `import torch_dist_ext` (test/test_all_reduce_fusion.py:8) and
     the reference loads `<parent of the package>/libtorch_dist_ext.so` (torch_dist_ext/__init__.py:8-12)."""

@@ -515,7 +515,7 @@ TORCH_LIBRARY(torch_dist_ext, m) {
           "Tensor? norm_out, Tensor? q_out, Tensor? scale_out, float eps, int quant_mode, int algo, Tensor? stage, "
           "float static_scale=0.0) -> ()");
     m.def("reduce_rms_partials(Tensor[] partials, Tensor residual_in, Tensor rms_gamma, float eps, int quant_mode, bool write_norm, "
-          "int algo, Tensor? stage, float static_scale) -> (Tensor, Tensor?, Tensor?, Tensor?)");
+          "int algo, Tensor(a!)? stage, float static_scale) -> (Tensor, Tensor?, Tensor?, Tensor?)");
 }
 
 TORCH_LIBRARY_IMPL(torch_dist_ext, CUDA, m) {
