@@ -127,7 +127,8 @@ typedef struct tde_plan_out {
                                 2 = two-shot (impl.h:491) */
     int32_t vec_elems;       /* elements per 16-byte access: 8 (bf16/f16), 4 (f32); impl.h:478 */
     int32_t block_threads;   /* threads per workgroup (multiple of 64) */
-    int32_t vecs_per_thread; /* 16-byte vectors each thread owns per row */
+    int32_t vecs_per_thread; /* 16-byte vectors each thread owns per row, in the launch of tde_reduce_rms (the norm phase
+                                of doubles alone, tde_stage_norm, has a choice of its own) */
     int32_t rows_per_block;  /* rows a workgroup processes side by side (one wave group per row) */
     int32_t grid_blocks;     /* workgroups launched for the row kernel */
     int32_t xcd_chunk;       /* row groups each XCD takes in a row: workgroup b of every 8*xcd_chunk takes row group
@@ -175,7 +176,7 @@ int tde_reduce_rms(const tde_problem *problem, const tde_buffers *buffers, void 
    buffers->stage; partial[] and partial_table are ignored.
    tde_reduce_rms with the same problem computes and stores exactly what tde_stage_reduce followed by tde_stage_norm
    does, in one launch (in those two where `stage` overlaps another output, the residual or gamma, or a partial an
-   output). */
+   output, and where a partial's address comes from partial_table). */
 int tde_stage_reduce(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 int tde_stage_norm(const tde_problem *problem, const tde_buffers *buffers, void *hip_stream);
 

@@ -53,6 +53,44 @@ def test_stage_that_overlaps_another_buffer(cuda_device, where):
     assert bits_equal(buf["norm_out"].cpu(), want["norm_out"])
 
 
+@pytest.mark.parametrize("where", ["residual_ahead", "residual_behind", "gamma"])
+@pytest.mark.parametrize("algo", [_capi.ALGO_STAGED, _capi.ALGO_STAGED_OWNED])
+def test_stage_over_an_input_of_the_norm(cuda_device, where, algo):
+    """What the norm reads through an overlap are sums of other rows, all of them stored before: the residual of row t is the stage's
+    row t + 40 or t - 40, or gamma is the stage's last row.  A single launch would read most of them before they are there."""
+    import torch_dist_ext_amd as tde
+    print("case", where, algo, flush=True)
+    shift, tokens, hidden, n = 40, 3000, 1024, 4
+    p, r, g = eager.make_inputs(n, tokens, hidden, torch.bfloat16, 0.25, seed=11)
+    sums = torch.zeros((tokens, hidden))
+    for k in range(n):
+        sums = sums + p[k].float()
+    sums = sums.to(p.dtype)
+    memory = torch.cat([r, r[:shift]]).to(cuda_device)
+    before = memory.cpu()
+    stage = memory[shift:] if where == "residual_behind" else memory[:tokens]
+    if algo == _capi.ALGO_STAGED_OWNED:   # what the peers delivered, and nothing yet in this rank's rows (0, 4, 8, ...)
+        owned = torch.arange(tokens) % n == 0
+        stage.copy_(torch.where(owned[:, None], stage.cpu(), sums))
+        before = memory.cpu()
+    at = shift if where == "residual_behind" else 0
+    before[at: at + tokens] = sums        # the memory once every sum has been stored
+    res, gamma = r.to(cuda_device), g.to(cuda_device)
+    if where == "gamma":
+        gamma = stage[tokens - 4]         # an owned row
+        want = eager.reduce_rms(p, r, sums[tokens - 4], 1e-6, "none")
+    else:
+        first = 0 if where == "residual_behind" else shift
+        res = memory[first: first + tokens]
+        want = eager.reduce_rms(p, before[first: first + tokens], g, 1e-6, "none")
+    res_out, norm_out = torch.empty_like(r, device=cuda_device), torch.empty_like(r, device=cuda_device)
+    tde.reduce_rms_local_impl([p[k].to(cuda_device) for k in range(n)], res, gamma, res_out, norm_out, None, None, 1e-6,
+                              tde.QUANT_NONE, algo, stage, 0.0)
+    torch.cuda.synchronize()
+    assert bits_equal(res_out.cpu(), want["residual_out"])
+    assert bits_equal(norm_out.cpu(), want["norm_out"])
+
+
 @pytest.mark.parametrize("out", ["norm_out", "residual_out", "q_out"])
 @pytest.mark.parametrize("algo", [_capi.ALGO_STAGED, _capi.ALGO_STAGED_OWNED])
 def test_output_that_overlaps_a_partial(cuda_device, out, algo):

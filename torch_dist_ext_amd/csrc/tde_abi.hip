@@ -393,7 +393,12 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     // threshold itself the gain is small: 4 x [8192, 7168] with per-group scales 0.4 % on a device that has been under
     // load for 20 ms (0.9 % slower in the first milliseconds after idling).
     int wgs_per_cu = 0;
-    const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED; // its row kernel reads 2 streams
+    // The staged algorithms are limited only on request.  With owned rows, and in the norm phase alone, most rows read two streams.
+    // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more; two workgroups per CU against
+    // none planned: 8 x [16384, 8192] bf16 -> fp8 513.7 -> 497.8 us, 4 x [32768, 8192] 688.2 -> 628.3, 4 x [16384, 5120] 203.6 ->
+    // 200.2 (three: 200.1), 8 x [8192, 8192] 251.2 -> 246.4; at 2048 rows +0.4 to -0.4 %; rows of 256 vectors of four partials +11 to
+    // +14 % with two, -4 % with four at 16384 rows.
+    const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED;
     if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
         const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
         const int waves = tpr * rpb / 64;

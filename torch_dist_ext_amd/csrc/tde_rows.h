@@ -1044,7 +1044,7 @@ hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t r
 hipError_t launch_reduce_f16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 
-// Rows of doubles (tde_rows_f64.hip): one vector per thread, no quantized output.
+// Rows of doubles (tde_rows_f64.hip): no quantized output.
 hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 

@@ -4,11 +4,13 @@
 //   x   = ((0 + p_0) + ... + p_{N-1}) + residual_in        all in double, rank order          -> residual_out
 //   rs  = 1 / sqrt( sum(float(x)^2) / H + eps )             fp32: RMSNorm.forward squares x.float()
 //   y   = gamma * (x * double(rs))                          double                              -> norm_out
-// No quantized output for this type.  One, two or four 16-byte vectors per thread (the plan's vecs_per_thread_f64 says which and
-// what it measured), the row kernel's geometry and XCD-aware row mapping.  Bound by memory: 4 x [2048, 2048] moves 235 MB.  As
-// in the row kernel the partials are added as they arrive, gamma of several vectors is requested once the row's registers
-// are free, and residual_out is stored with the row's other output (one write burst per row).  N == 0: the sum was staged (part[0] holds it), as in the row kernel; reduce_kernel_f64 is that stage A.
-// With a stage the sums are stored to it; OWNED sums rows == owner (mod N) only and reads the others' sums from the stage.
+// No quantized output for this type.  One or four 16-byte vectors per thread as planned (vecs_per_thread_f64 says which and what
+// it measured), two only on request (tune_vecs_per_thread); the row kernel's geometry and XCD-aware row mapping.  Bound by
+// memory: 4 x [2048, 2048] moves 235 MB.  As in the row kernel the partials are added as they arrive and gamma of several
+// vectors is requested once the row's registers are free; residual_out is stored as soon as it is known, or with the row's
+// other output in launches of few bytes (kEarlyStoreBytes).  N == 0: the sum was staged (part[0] holds it), as in the row
+// kernel; reduce_kernel_f64 is that stage A.  With a stage the sums are stored to it; OWNED sums rows == owner (mod N) only
+// and reads the others' sums from the stage.
 #include <hip/hip_runtime.h>
 
 #include "tde_rows.h"

@@ -231,7 +231,8 @@ Tensor get_workspace_op(const Tensor &ref) {
 }
 
 // A new output tensor, straight from the allocator: at::empty and at::empty_like go through the dispatcher once and twice
-// more, 0.3-0.45 us of host time for each output (allreduce_rms 6.7 -> 5.8 us a call, allreduce_rms_quant 8.2 -> 7.0).
+// more, 0.2-0.3 us of host time for each output (with the kernel arguments in 120 bytes, the other change between the two
+// figures: allreduce_rms 8 x [128, 4096] 5.97 -> 5.37 us a call, allreduce_rms_quant 4 x [64, 5120] int8 7.18 -> 6.24).
 Tensor new_output(at::IntArrayRef sizes, at::ScalarType dtype, const Tensor &on) {
     return Tensor(at::detail::empty_cuda(sizes, dtype, on.device(), c10::nullopt));
 }
