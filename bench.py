@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "55bb90777cf227977d0f7689232b58b52ca6a471a27da75b4f630d2904ba9706",
-    "bytes": {"c2": 11693631, "c3": 352653693, "c4": 765467842, "c5": 2181249484},
+    "sources_sha256": "4c4a18b67df58f2822f1746bb6caee21b910851249a42340734706522f1fa447",
+    "bytes": {"c2": 11696152, "c3": 352657666, "c4": 765446713, "c5": 2181258557},
 }
 
 BENCH_CONFIGS = {
