@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "4c4a18b67df58f2822f1746bb6caee21b910851249a42340734706522f1fa447",
-    "bytes": {"c2": 11696152, "c3": 352657666, "c4": 765446713, "c5": 2181258557},
+    "sources_sha256": "6a4798ea29fbce3f54c56a8f086b3ecfa49e575636a6a0f94c2b9659af1880c7",
+    "bytes": {"c2": 1232695758, "c3": 1521613313, "c4": 1033206196, "c5": 1162374479},
 }
 
 BENCH_CONFIGS = {

@@ -128,7 +128,7 @@ typedef struct tde_plan_out {
     int32_t vec_elems;       /* elements per 16-byte access: 8 (bf16/f16), 4 (f32); impl.h:478 */
     int32_t block_threads;   /* threads per workgroup (multiple of 64) */
     int32_t vecs_per_thread; /* 16-byte vectors each thread owns per row, in the launch of tde_reduce_rms (the norm phase
-                                of doubles alone, tde_stage_norm, has a choice of its own) */
+                                alone, tde_stage_norm, may take another choice) */
     int32_t rows_per_block;  /* rows a workgroup processes side by side (one wave group per row) */
     int32_t grid_blocks;     /* workgroups launched for the row kernel */
     int32_t xcd_chunk;       /* row groups each XCD takes in a row: workgroup b of every 8*xcd_chunk takes row group

@@ -19,8 +19,10 @@ pytestmark = pytest.mark.gpu
     (8, 7, 8191, 32, torch.float32, "fp8_static", 4, 0), (8, 3, 8200, 8, torch.bfloat16, "int8_token", 0, 0),
     (8, 6, 5, 1000, torch.float16, "int8_token", 4, 1), (8, 1, 300, 8192, torch.bfloat16, "fp8_token", 0, 0),
     (4, 2, 4097, 6, torch.float64, "none", 0, 0), (2, 1, 130, 2048, torch.float64, "none", 0, 0),
-    # doubles whose norm phase alone takes other vectors per thread than the one launch: one against four, four against one
+    # the norm phase alone takes other vectors per thread than the one launch: doubles one against four, four against one
     (2, 0, 300, 512, torch.float64, "none", 0, 0), (2, 1, 1400, 1960, torch.float64, "none", 0, 0), (4, 1, 3100, 1602, torch.float64, "none", 0, 0),
+    # rows that are not whole 128-byte lines, T-typed rows beside the codes: owned rows four, their norm phase alone one
+    (4, 1, 2100, 2820, torch.float32, "fp8_token", 0, 0),
 ])
 def test_one_launch_equals_its_phases(cuda_device, n, rank, tokens, hidden, dtype, quant, vpt, rpb):
     print("case", n, rank, tokens, hidden, dtype, quant, vpt, rpb, flush=True)

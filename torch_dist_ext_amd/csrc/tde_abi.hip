@@ -257,7 +257,7 @@ bool several_vecs_pay(const tde_problem *p, int64_t nvec, int64_t t) {
     return true;
 }
 
-int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
+int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alone) {
     // Vectors per thread, from sweeps on MI355X over hidden 1024..8192 in steps of 1024, 2/4/8 partials, 128..32768 rows
     // and three output modes (bf16 and fp16 agree); only differences that held on two devices and across the row
     // counts between the swept powers of two are in here.  Four vectors per thread (small workgroups, many loads in
@@ -338,7 +338,12 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t) {
     // TDE_ALGO_STAGED, up to four partials, T-typed rows or static and group scales: one vector per thread stays 2-6 % ahead of the
     // ranges above between the lengths they were first swept at.
     if (staged && !per_token && p->nranks <= 4 && nvec > 576 && nvec < 896 && nvec != 640) vpt = nvec == 768 ? vpt : 1;
-    if (owned && per_token) vpt = vecs_per_thread_owned(p, nvec, t, vpt);
+    // The norm phase alone keeps one vector per thread where it stores T-typed rows beside the codes and the rows are not whole
+    // lines: several are 2-7 % slower there with six and seven wavefronts per row from 4096 rows on, 2-10 % with eleven and twelve.
+    const int waves = (int)((nvec + 63) / 64);
+    const bool alone_loses = norm_alone && p->write_norm != 0 && !rows_of_whole_lines(nvec) &&
+                             (waves == 11 || waves == 12 || ((waves == 6 || waves == 7) && t >= 4096));
+    if (owned && per_token && !alone_loses) vpt = vecs_per_thread_owned(p, nvec, t, vpt);
     else if (fused && vpt == 1 && p->nranks <= 4) vpt = vecs_per_thread_few_partials(p, nvec, t);
     return vpt;
 }
@@ -365,7 +370,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     if (__builtin_mul_overflow(p->tokens, p->hidden * eb, &total_bytes)) return TDE_ESHAPE;
 
     const int64_t t = rows_as_on_256_units(p->tokens);
-    int vpt = p->dtype != TDE_F64 ? vecs_per_thread(p, nvec, t) : (norm_alone ? vecs_per_thread_f64_norm(nvec, t) : vecs_per_thread_f64(p, nvec, t));
+    int vpt = p->dtype != TDE_F64 ? vecs_per_thread(p, nvec, t, norm_alone) : (norm_alone ? vecs_per_thread_f64_norm(nvec, t) : vecs_per_thread_f64(p, nvec, t));
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
