@@ -41,7 +41,7 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # traffic as null.
 TRAFFIC = {
     "sources_sha256": "6a4798ea29fbce3f54c56a8f086b3ecfa49e575636a6a0f94c2b9659af1880c7",
-    "bytes": {"c2": 1232695758, "c3": 1521613313, "c4": 1033206196, "c5": 1162374479},
+    "bytes": {"c2": 11696301, "c3": 352656556, "c4": 765446898, "c5": 2181261437},
 }
 
 BENCH_CONFIGS = {
