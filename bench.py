@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "6a4798ea29fbce3f54c56a8f086b3ecfa49e575636a6a0f94c2b9659af1880c7",
-    "bytes": {"c2": 11696301, "c3": 352656556, "c4": 765446898, "c5": 2181261437},
+    "sources_sha256": "3756b1420ecc4e48b4c134d3c7c1b02b5e110584f9e509568f6debfd56cb92a5",
+    "bytes": {"c2": 11696277, "c3": 352658057, "c4": 765445425, "c5": 2181259183},
 }
 
 BENCH_CONFIGS = {

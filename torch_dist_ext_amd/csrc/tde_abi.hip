@@ -96,10 +96,9 @@ int64_t rows_as_on_256_units(int64_t tokens) {
     return cus == 256 ? tokens : tokens / cus * 256 + tokens % cus * 256 / cus;
 }
 
-// Whether every row starts and ends on a 128-byte line.  Where a row's wavefronts store at different times, the rows of a
-// launch that do not share their first and last line with a neighbour: several vectors per thread (fewer wavefronts, each
-// further behind the row's others) lose 2-6 % of a long launch of the others (2 x 16384 rows of 608 vectors, T-typed output
-// +3.1 % over one vector per thread, of 609 -3.1 %).
+// Whether every row starts and ends on a 128-byte line.  Other rows share their first and last line with their neighbours, and
+// several vectors per thread (fewer wavefronts, whose stores lie further apart in time) then lose 2-6 % of a long launch that stores
+// much: 2 x 16384 rows of 608 vectors, T-typed output, +3.1 % over one vector per thread, of 609 -3.1 %.
 bool rows_of_whole_lines(int64_t nvec) { return nvec % 8 == 0; }
 
 // Vectors per thread for rows of doubles in one launch (4 partials x 2048 rows of 2048 in all: 38.5 -> 38.0 us; 2 x 900 rows of
@@ -228,7 +227,10 @@ int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) 
         return t >= 1024 && (f32 || t < 1344 || t > 1536) ? 2 : 1;
     }
     if (waves == 6) return t >= 1536 && (!t_rows || t < 3072) ? 2 : 1; // 1-14 %
-    if (waves == 7) return t >= 1536 && (!t_rows || t < (f32 || lines ? (f32 && lines ? INT64_MAX : 8192) : 1792)) ? 2 : 1; // 1-14 %
+    if (waves == 7) { // 1-14 %
+        const int64_t until = !t_rows || (f32 && lines) ? INT64_MAX : (f32 || lines ? 8192 : 1792);
+        return t >= 1536 && t < until ? 2 : 1;
+    }
     if (waves == 5) // fp32 3-13 %, others 0-10 %
         return f32 ? (t >= 1536 && (!t_rows || t < (lines ? 16384 : 6144)) ? 2 : 1) : (t >= 16384 && !t_rows ? 2 : 1);
     return 1;
@@ -316,11 +318,12 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alo
         else if (p->nranks == 4 && t >= even_from) vpt = nvec == 640 ? 4 : 2;
         else if (p->nranks >= 8 && t >= 16384 && nvec == 640) vpt = 2; // eight partials, long launches: 2 % over one
         if (!full && p->algo <= TDE_ALGO_FUSED) {
-            // One vector against two: eight partials 776 to 831 rows -1 to -5 % (768 rows +8 to +12 %; fp32 T-typed output +1 to +6 %); four partials, rows that
-            // are not whole lines, from 4096 rows on -1 to -4 %, until the limit on workgroups per compute unit (below) makes two
-            // 1-5 % faster again, and with T-typed rows beside the codes from 1281 (static and group scales) or 1792 rows on -1 to -7 %
-            // (fp32 per-token codes as without them); two partials, T-typed rows, not whole lines: from 8192 rows of output -1 to -6 %
-            // (fp32 from 12288), beside static and group scales of a 2-byte type from 2304, beside per-token codes from 6144.
+            // One vector against two: eight partials 776 to 831 rows -1 to -5 % (768 rows +8 to +12 %; fp32 T-typed output +1 to
+            // +6 %).  Rows that are not whole lines: four partials from 4096 rows on -1 to -4 %, until the limit on workgroups per
+            // compute unit (below) makes two 1-5 % faster again, and with T-typed rows beside the codes from 1281 (static and group
+            // scales) or 1792 rows on -1 to -7 % (fp32 per-token codes as without them); two partials, T-typed output from 8192 rows
+            // on -1 to -6 % (fp32 from 12288), T-typed rows beside static and group scales of a 2-byte type from 2304, beside
+            // per-token codes from 6144.
             const bool fixed = p->quant == TDE_QUANT_FP8_GROUP || p->quant == TDE_QUANT_FP8_STATIC, none = p->quant == TDE_QUANT_NONE;
             const bool beside = !none && p->write_norm != 0, lines = rows_of_whole_lines(nvec);
             if (p->nranks >= 8 && !(f32 && none) && t >= 776 && t < 832) vpt = 1;
