@@ -260,6 +260,15 @@ __device__ __forceinline__ uint32_t row_max(uint32_t v, uint32_t *slots, int wav
 // (16 reads 32 floats apart), the block sums go through LDS (`bs`), and lanes 4m+k of every wavefront finish chain
 // (m, k).  With 8 floats per 16-byte vector (2-byte element types) a block of 64 vectors is exactly what one
 // wavefront loaded with one load instruction, so the first step needs no workgroup barrier (WAVE_BLOCKS).
+//
+// This stands between a row's last load and its first store, where a wavefront pays at least four cycles for every
+// instruction of any kind, so nothing in it is guarded element by element: what the chains do not take (V % 4 vectors and n % 8
+// scalars) goes to a place of its own (`left`) with zeros in the image, lanes past the row's end hold zeros, and a row's block sums
+// are filled up with zeros to a number that has straight-line code (sum_slots).  Adding +0 to a sum of squares changes
+// nothing, and neither does leaving out the +0 a sum starts from: a square is never -0.  8 x [1, 4096] bf16: from a
+// wavefront's last partial to the reciprocal RMS 2416 -> 1992 cycles with guarded and with straight code, the wait for the
+// slowest wavefront in both; launches 2 x [16, 1024] 2.35 -> 2.13 us, 8 x [128, 4096] 4.79 -> 4.53, 4 x [512, 5120] fp16 -> int8
+// 8.72 -> 8.27, 2 x [20000, 200] bf16 -> fp8 13.6 -> 11.8.
 // ---------------------------------------------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ float quad_bcast(float v) {
@@ -308,37 +317,47 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Block `b` of chain `cl` (= 4m + k): the first `terms` (0..16) of 16 elements 32 floats apart, summed left to
-// right.  GUARD: never read past the last term (rows whose LDS image ends inside the block).
-template <bool GUARD>
-__device__ __forceinline__ float chain_block_sum(const float *img, int b, int cl, int terms) {
-    const float *src = img + 512 * b + 8 * (cl & 3) + (cl >> 2);
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = src[(!GUARD || i < terms) ? 32 * i : 0];
-    float acc = 0.0f;
-    if (__builtin_amdgcn_ballot_w64(terms != 16) == 0) { // every lane of the wavefront has a full block
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += v[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc += (i < terms) ? v[i] : 0.0f;
+// Block sums per row as the last step reads them: the number rounded up to one that has straight-line code.  A workgroup's
+// slots and its rows' `left` floats (32 each) fit the 1024 floats behind the image: it holds at most 16 blocks in all, so at
+// most 16 rows of one slot, 8 of two, 5 of four, 3 of eight or one of more.
+__device__ __forceinline__ int sum_slots(int blocks) {
+    return blocks <= 1 ? 1 : (blocks <= 2 ? 2 : (blocks <= 4 ? 4 : (blocks <= 8 ? 8 : (blocks <= 12 ? 12 : 16))));
+}
+
+// Where a row group's floats lie in LDS; wavefront-uniform, from the row's length and the launch geometry.
+//   img  one float per element the group holds (threads * VPT * VECF)
+//   bs   32 * slots block sums
+//   left the floats from `chained` to n
+template <int VPT, int VECF, bool WAVE_BLOCKS>
+struct SumLayout {
+    float *img, *bs, *left;
+    int n, chained; // floats of the row, and how many of them the chains take
+    int blocks;     // 512-float blocks that are summed: with WAVE_BLOCKS all that the group holds, else those of the chains
+    int slots;
+
+    __device__ __forceinline__ SumLayout(float *lds_img, float *lds_bs, int n_, int tpr, int rows_per_block, int group) {
+        n = n_;
+        chained = n & ~31;
+        blocks = WAVE_BLOCKS ? (tpr >> 6) * VPT : (chained + 511) >> 9;
+        slots = sum_slots(blocks);
+        img = lds_img + group * (tpr * VPT * VECF);
+        bs = lds_bs + group * (slots * 32);
+        left = lds_bs + rows_per_block * (slots * 32) + group * 32;
     }
-    return acc;
+};
+
+// Zeros for the block sums that the last step reads and no thread writes.  Anywhere before the squares are complete: under
+// the row's loads.  At most three slots: fewer floats than the group has threads (one slot takes three blocks or none, more
+// take five blocks, i.e. 192 threads).
+template <int VPT, int VECF, bool WAVE_BLOCKS>
+__device__ __forceinline__ void sumsq_clear(const SumLayout<VPT, VECF, WAVE_BLOCKS> &s, int t) {
+    if (s.slots != s.blocks && t < (s.slots - s.blocks) * 32) s.bs[s.blocks * 32 + t] = 0.0f;
 }
 
-// Wavefront-uniform variant of not_before (the value comes back in a scalar register).
-__device__ __forceinline__ int uniform_not_before(int v, uint32_t after) {
-    return __builtin_amdgcn_readfirstlane(not_before(v, after));
-}
-
-// The squares of this thread's vector j (vector index j * tpr + t of the row) go to their place in the row group's
-// image, which holds the row's squares in element order.  `after`: a word of the data the squares were computed from.
-template <int VPT, int VECF>
-__device__ __forceinline__ void sumsq_put(float *lds_img, int j, int tpr, int group, int t, const float (&sq)[VECF], uint32_t after) {
+// The squares of one vector (number `vec` of the row) go to their place in the image ...
+template <int VECF>
+__device__ __forceinline__ void put_squares(float *dst, const float (&sq)[VECF]) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const int vec = not_before(group * (tpr * VPT) + j * tpr + t, after);
-    float *dst = lds_img + vec * VECF;
     if constexpr (VECF % 4 == 0) {
 #pragma unroll
         for (int c = 0; c < VECF; c += 4) *reinterpret_cast<f32x4 *>(dst + c) = f32x4{sq[c], sq[c + 1], sq[c + 2], sq[c + 3]};
@@ -348,111 +367,160 @@ __device__ __forceinline__ void sumsq_put(float *lds_img, int j, int tpr, int gr
     }
 }
 
-// After every thread of the row group has put its squares: the sum, the same value in every thread.
-// lds_img: one float per element the workgroup holds (threads * VPT * VECF), lds_bs: 1024 floats (32 per block),
-// both shared by the workgroup's row groups (sumsq_lds_bytes gives the total).
-// Contains workgroup barriers when a row spans several wavefronts: all threads of the workgroup must call it together.
+// ... and from there to the floats that the chains do not take, zeros in their place.  A step of its own behind all of a
+// thread's puts: a branch between them keeps the arithmetic of several vectors from overlapping (8 x [2048, 8192] +1.5 %).
 template <int VPT, int VECF, bool WAVE_BLOCKS>
-__device__ __forceinline__ float sumsq_torch_order(float *lds_img, float *lds_bs, int n, int t, int tpr, int group, int lane,
-                                                   uint32_t after) {
-    n = uniform_not_before(n, after);
-    tpr = uniform_not_before(tpr, after);
-    group = uniform_not_before(group, after);
-    t = not_before(t, after);
-    lane = not_before(lane, after);
-    const int waves_per_row = tpr >> 6;
-    const int cap = tpr * VPT * VECF;        // floats this row group can hold
-    const int cap_blocks = (cap + 511) >> 9; // 64-vector blocks this row group can hold (<= 16)
-    float *img = lds_img + group * cap;
-    float *bs = lds_bs + group * (cap_blocks * 32);
-    const int V = n >> 3, tail = n & 7, I = V >> 2, L = V & 3, NB = (I + 15) >> 4;
+__device__ __forceinline__ void split_left(const SumLayout<VPT, VECF, WAVE_BLOCKS> &s, int vec, const float (&sq)[VECF]) {
+    const uint32_t behind = (uint32_t)(vec * VECF - s.chained);
+    if (behind < (uint32_t)(s.n - s.chained)) {
+        const float zeros[VECF] = {};
+        put_squares(s.img + vec * VECF, zeros);
+        put_squares(s.left + behind, sq);
+    }
+}
 
+// Sixteen elements of chain `cl` (= 4m + k) 32 floats apart, summed left to right.  GUARD: only the first `terms` (4, 8 or
+// 12, or more than that: all) are inside the image.
+template <bool GUARD>
+__device__ __forceinline__ float chain_block_sum(const float *block, int cl, int terms) {
+    const float *src = block + 8 * (cl & 3) + (cl >> 2);
+    float v[16];
+#pragma unroll
+    for (int g = 0; g < 16; g += 4) {
+        const bool inside = !GUARD || g == 0 || g < terms;
+        const float *from = src + (inside ? 32 * g : 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[g + i] = from[32 * i];
+        if (GUARD && g != 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[g + i] = inside ? v[g + i] : 0.0f;
+        }
+    }
+    float acc = v[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) acc += v[i];
+    return acc;
+}
+
+template <int SLOTS>
+__device__ __forceinline__ float chain_sum(const float *bs, int cl) {
+    float v[SLOTS];
+#pragma unroll
+    for (int b = 0; b < SLOTS; ++b) v[b] = bs[b * 32 + cl];
+    float chain = v[0];
+#pragma unroll
+    for (int b = 1; b < SLOTS; ++b) chain += v[b];
+    return chain;
+}
+
+// After every thread of the row group has put its squares: the sum, the same value in every thread.
+// Contains workgroup barriers when a row spans several wavefronts: all threads of the workgroup must call it together.
+// wave: the wavefront's number in its row group.
+template <int VPT, int VECF, bool WAVE_BLOCKS>
+__device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WAVE_BLOCKS> &s, int t, int tpr, int wave, int lane) {
+    const int waves_per_row = tpr >> 6;
     const int cl = lane & 31;
-    int blocks = NB; // block sums that exist in `bs`
     if constexpr (WAVE_BLOCKS) {
         static_assert(VECF == 8, "one wavefront load = one block of 64 eight-float vectors");
-        // Block j * waves_per_row + w is what wavefront w wrote for its vector j: no other wavefront is involved.
-        // Blocks past the row's end sum to zero, and adding zero to a sum of squares changes nothing.
+        // Block j * waves_per_row + wave is what this wavefront wrote for its vector j: no other wavefront is involved.
         wave_lds_fence();
-        const int w = t >> 6;
         if constexpr (VPT == 1) {
-            if (lane < 32) { // one block per wavefront: half of its lanes have a chain
-                int terms = I - 16 * w;
-                terms = terms < 0 ? 0 : (terms > 16 ? 16 : terms);
-                bs[w * 32 + cl] = chain_block_sum<false>(img, w, cl, terms);
-            }
+            // one block per wavefront: both of its halves sum it
+            s.bs[wave * 32 + cl] = chain_block_sum<false>(s.img + 512 * wave, cl, 16);
         } else {
             // two blocks at a time, one per half of the wavefront; their reads and sums interleave
             float sum[VPT / 2];
             int b[VPT / 2];
 #pragma unroll
-            for (int s = 0; s < VPT / 2; ++s) {
-                b[s] = ((lane >> 5) + 2 * s) * waves_per_row + w;
-                int terms = I - 16 * b[s];
-                terms = terms < 0 ? 0 : (terms > 16 ? 16 : terms);
-                sum[s] = chain_block_sum<false>(img, b[s], cl, terms);
+            for (int k = 0; k < VPT / 2; ++k) {
+                b[k] = ((lane >> 5) + 2 * k) * waves_per_row + wave;
+                sum[k] = chain_block_sum<false>(s.img + 512 * b[k], cl, 16);
             }
 #pragma unroll
-            for (int s = 0; s < VPT / 2; ++s) bs[b[s] * 32 + cl] = sum[s];
+            for (int k = 0; k < VPT / 2; ++k) s.bs[b[k] * 32 + cl] = sum[k];
         }
-        blocks = cap_blocks;
     } else {
         if (waves_per_row > 1) __syncthreads(); else wave_lds_fence();
-        for (int c = t; c < 32 * NB; c += tpr) {
-            const int b = c >> 5;
-            int terms = I - 16 * b;
-            terms = terms > 16 ? 16 : terms;
-            bs[c] = chain_block_sum<true>(img, b, c & 31, terms);
+        // one thread per chain and block: the group has at least 32 threads per block of its chains
+        if (t < 32 * s.blocks) {
+            const int b = t >> 5;
+            const int terms = (tpr * VPT * VECF - 512 * b) >> 5;
+            float sum;
+            if (((tpr * VPT * VECF) & 511) == 0) sum = chain_block_sum<false>(s.img + 512 * b, cl, 16);
+            else sum = chain_block_sum<true>(s.img + 512 * b, cl, terms);
+            s.bs[t] = sum;
         }
     }
     if (waves_per_row > 1) __syncthreads(); else wave_lds_fence();
 
     // Lane 4m + k of every wavefront sums the blocks of chain (m, k); the quad then holds the four chains of m.
-    float chain = 0.0f;
-    if (blocks == 16) {
-        float v[16];
-#pragma unroll
-        for (int b2 = 0; b2 < 16; ++b2) v[b2] = bs[b2 * 32 + cl];
-#pragma unroll
-        for (int b2 = 0; b2 < 16; ++b2) chain += v[b2];
-    } else if (blocks <= 8) {
-        float v[8];
-#pragma unroll
-        for (int b2 = 0; b2 < 8; ++b2) v[b2] = bs[(b2 < blocks ? b2 : 0) * 32 + cl];
-#pragma unroll
-        for (int b2 = 0; b2 < 8; ++b2) chain += (b2 < blocks) ? v[b2] : 0.0f;
-    } else {
-        float v[16];
-#pragma unroll
-        for (int b2 = 0; b2 < 16; ++b2) v[b2] = bs[(b2 < blocks ? b2 : 0) * 32 + cl];
-#pragma unroll
-        for (int b2 = 0; b2 < 16; ++b2) chain += (b2 < blocks) ? v[b2] : 0.0f;
+    float chain;
+    switch (s.slots) {
+    case 1: chain = chain_sum<1>(s.bs, cl); break;
+    case 2: chain = chain_sum<2>(s.bs, cl); break;
+    case 4: chain = chain_sum<4>(s.bs, cl); break;
+    case 8: chain = chain_sum<8>(s.bs, cl); break;
+    case 12: chain = chain_sum<12>(s.bs, cl); break;
+    default: chain = chain_sum<16>(s.bs, cl); break;
     }
-    const int m = cl >> 2;
     float p = quad_bcast<0x00>(chain);
-    for (int l = 0; l < L; ++l) p += img[8 * (4 * I + l) + m];
+    float sum = 0.0f; // the scalars left over
+    if (s.n != s.chained) {
+        const int m = cl >> 2, L = (s.n >> 3) & 3;
+        for (int l = 0; l < L; ++l) p += s.left[8 * l + m];
+        if (s.n < 8) {
+            // four interleaved scalars, the first of them also takes what is left over
+            sum = s.left[0];
+            if (s.n < 4) {
+                for (int e = 1; e < s.n; ++e) sum += s.left[e];
+            } else {
+                for (int e = 4; e < s.n; ++e) sum += s.left[e];
+                sum += s.left[1];
+                sum += s.left[2];
+                sum += s.left[3];
+            }
+        } else if constexpr (VECF != 8) {
+            for (int e = s.n & ~7; e < s.n; ++e) sum += s.left[e - s.chained];
+        }
+    }
     p += quad_bcast<0x55>(chain);
     p += quad_bcast<0xAA>(chain);
     p += quad_bcast<0xFF>(chain);
-
-    float sum = 0.0f;
-    if (V == 0) {
-        // fewer than 8 floats: four interleaved scalars, the first of them also takes what is left over
-        if (n < 4) {
-            for (int e = 0; e < n; ++e) sum += img[e];
-        } else {
-            sum = img[0];
-            for (int e = 4; e < n; ++e) sum += img[e];
-            sum += img[1];
-            sum += img[2];
-            sum += img[3];
-        }
+    if constexpr (VECF == 8) { // 2-byte types: whole vectors of eight floats, no scalars left over
+        sum = read_lane(p, 0);
     } else {
-        for (int e = 0; e < tail; ++e) sum += img[8 * V + e];
+        sum += read_lane(p, 0);
     }
 #pragma unroll
-    for (int mm = 0; mm < 8; ++mm) sum += read_lane(p, 4 * mm);
+    for (int mm = 1; mm < 8; ++mm) sum += read_lane(p, 4 * mm);
     return sum;
+}
+
+// 1/h, correctly rounded for every row length.
+__device__ __forceinline__ float reciprocal_of_length(float h) {
+    const float r = __builtin_amdgcn_rcpf(h);
+    return __builtin_fmaf(__builtin_fmaf(-h, r, 1.0f), r, r);
+}
+
+// 1 / sqrt(sumsq / h + eps) with every step rounded as the IEEE operation (rcp_h: the correctly rounded 1/h).
+// The quotient by Markstein's correction (see div_shared), the root by his iteration on g ~ sqrt(m) and y ~ 1 / (2 sqrt(m))
+// ("Computation of elementary functions on the IBM RISC System/6000 processor", 1990), which leaves 1/sqrt(m) in 2y
+// for the reciprocal: 15 instructions where two divisions and a square root are 45.  Checked on gfx950 against
+// the plain operations for every m in [1, 4) -- powers of four only shift it -- and every h.  Outside [2^-60, 2^100], and
+// for NaN, the plain operations.  (Inside it no step underflows: a mean small enough for that leaves m == eps.)
+__device__ __forceinline__ float reciprocal_rms(float sumsq, float h, float rcp_h, float eps) {
+    const float q0 = sumsq * rcp_h;
+    const float m = __builtin_fmaf(-__builtin_fmaf(q0, h, -sumsq), rcp_h, q0) + eps;
+    if (!(m >= 0x1p-60f && m <= 0x1p100f)) return 1.0f / __builtin_sqrtf(sumsq / h + eps);
+    float y = __builtin_amdgcn_rsqf(m);
+    float g = m * y;
+    y *= 0.5f;
+    const float e = __builtin_fmaf(-y, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    y = __builtin_fmaf(y, e, y);
+    g = __builtin_fmaf(__builtin_fmaf(-g, g, m), y, g); // sqrt(m)
+    const float r = y + y;
+    return __builtin_fmaf(__builtin_fmaf(-g, r, 1.0f), r, r);
 }
 
 // Every buffer is device (global) memory: the few accesses that do not go through a buffer resource
@@ -627,6 +695,8 @@ __global__ void __launch_bounds__(1024 / VPT)
 // Thread index inside the row group and lane index, rebuilt from the first load offset where they are needed:
 // the thread id itself does not stay in a register through the load phase, which has none to spare.
 #define TDE_T ((int)(lane0 >> 4))
+// The same, not before `after` is there: with several vectors per thread the row loads leave no registers for LDS addresses.
+#define TDE_T_BEHIND(after) (VPT == 1 ? TDE_T : not_before(TDE_T, after))
 #define TDE_LANE ((int)(lane0 >> 4) & (kWave - 1))
 
     auto issue_loads = [&](RowLoads<NP, VPT> &d, int64_t row) {
@@ -690,6 +760,9 @@ __global__ void __launch_bounds__(1024 / VPT)
     uint32_t lane0 = lane_off[0];
     asm volatile("" : "+v"(lane0));
     const uint32_t vec_stride = (uint32_t)tpr * 16u;
+    const SumLayout<VPT, VEC, E::BYTES == 2> sums(lds_img, lds_bs, a.hidden(), tpr, a.rows_per_block, group);
+    sumsq_clear(sums, TDE_T);
+    const float rcp_h = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, reciprocal_of_length((float)a.hidden()))));
 #define TDE_OFF(j) (lane0 + (uint32_t)(j) * vec_stride)
 
     {
@@ -811,7 +884,17 @@ __global__ void __launch_bounds__(1024 / VPT)
             float sq[VEC];
 #pragma unroll
             for (int i = 0; i < VEC; ++i) sq[i] = x[i] * x[i];
-            sumsq_put<VPT, VEC>(lds_img, j, tpr, group, TDE_T, sq, xraw[j][0]);
+            put_squares(sums.img + (j * tpr + TDE_T_BEHIND(xraw[j][0])) * VEC, sq);
+        }
+        if (sums.n != sums.chained) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {
+                float x[VEC], sq[VEC];
+                E::unpack(xraw[j], x);
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) sq[i] = x[i] * x[i];
+                split_left(sums, j * tpr + TDE_T_BEHIND(xraw[j][0]), sq);
+            }
         }
         // gamma (shared by all rows, served from L2).  With several vectors per thread it is requested
         // only now (unless it went out first, see GAMMA_FIRST): the registers of the row loads are free
@@ -837,8 +920,9 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
             for (int j = 0; j < VPT; ++j) rsrc_store16(stage, TDE_OFF(j), sraw[j]);
         }
-        const float sumsq = sumsq_torch_order<VPT, VEC, E::BYTES == 2>(lds_img, lds_bs, a.hidden(), TDE_T, tpr, group, TDE_LANE, xraw[VPT - 1][0]);
-        const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
+        const int t_behind = TDE_T_BEHIND(xraw[VPT - 1][0]);
+        const float sumsq = sumsq_torch_order(sums, t_behind, tpr, wave - first_wave, t_behind & (kWave - 1));
+        const float rs = reciprocal_rms(sumsq, (float)a.hidden(), rcp_h, a.eps);
 
         // ---- normalize ------------------------------------------------------------------------------
         u32x4 yraw[VPT];
@@ -960,6 +1044,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     }
 }
 #undef TDE_T
+#undef TDE_T_BEHIND
 #undef TDE_LANE
 #undef TDE_OFF
 

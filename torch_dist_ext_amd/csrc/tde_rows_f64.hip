@@ -50,7 +50,6 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     float *const lds_img = lds_dyn;
     float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * (VPT * 2);
     const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
     const int tpr = a.threads_per_row;
     const int group = __builtin_amdgcn_readfirstlane(tid / tpr);
     const int t = tid - group * tpr;
@@ -89,6 +88,10 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     };
     if constexpr (VPT == 1) load_gamma();
     else __builtin_amdgcn_sched_barrier(0);
+
+    const SumLayout<VPT, 2, false> sums(lds_img, lds_bs, a.hidden(), tpr, a.rows_per_block, group);
+    sumsq_clear(sums, t);
+    const float rcp_h = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, reciprocal_of_length((float)a.hidden()))));
 
     // The partials are summed rank by rank, as they arrive.
     double acc[VPT][2];
@@ -134,15 +137,24 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
         const float f0 = (float)x[j][0], f1 = (float)x[j][1];
         const float sq[2] = {f0 * f0, f1 * f1};
         landed = __builtin_bit_cast(uint32_t, sq[0]);
-        sumsq_put<VPT, 2>(lds_img, j, tpr, group, t, sq, landed);
+        put_squares(sums.img + (j * tpr + (VPT == 1 ? t : not_before(t, landed))) * 2, sq);
+    }
+    if (sums.n != sums.chained) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const float f0 = (float)x[j][0], f1 = (float)x[j][1];
+            const float sq[2] = {f0 * f0, f1 * f1};
+            split_left(sums, j * tpr + t, sq);
+        }
     }
     if constexpr (VPT > 1) {
         __builtin_amdgcn_sched_barrier(0);
         load_gamma();
         store_sums();
     }
-    const float sumsq = sumsq_torch_order<VPT, 2, false>(lds_img, lds_bs, a.hidden(), t, tpr, group, lane, landed);
-    const float rs = 1.0f / __builtin_sqrtf(sumsq / (float)a.hidden() + a.eps);
+    const int t_behind = VPT == 1 ? t : not_before(t, landed);
+    const float sumsq = sumsq_torch_order(sums, t_behind, tpr, 0, t_behind & (kWave - 1));
+    const float rs = reciprocal_rms(sumsq, (float)a.hidden(), rcp_h, a.eps);
 
     const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
 #pragma unroll
