@@ -701,6 +701,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     a.set(tde::kPtrScale, b->scale_out);
     a.set_hidden(p->hidden);
     a.threads_per_row = (uint16_t)g.threads_per_row;
+    a.wave_step = (uint16_t)(32768 / (g.threads_per_row / tde::kWave) + 1);
     a.rows_per_block = (uint8_t)g.rows_per_block;
     a.xcd_chunk = (uint8_t)g.xcd_chunk;
     a.tokens = p->tokens;

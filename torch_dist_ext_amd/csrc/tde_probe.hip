@@ -17,7 +17,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     constexpr int NP = (N == 0) ? 1 : N;
     const int tid = threadIdx.x;
     const int tpr = a.threads_per_row;
-    const int group = __builtin_amdgcn_readfirstlane(tid / tpr);
+    const int group = a.row_group(__builtin_amdgcn_readfirstlane(tid >> 6));
     const int t = tid - group * tpr;
     const void *part[NP];
     partial_addresses(a, a.address(kPtrStage), part);

@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * (VPT * 2);
     const int tid = threadIdx.x;
     const int tpr = a.threads_per_row;
-    const int group = __builtin_amdgcn_readfirstlane(tid / tpr);
+    const int group = a.row_group(__builtin_amdgcn_readfirstlane(tid >> 6));
     const int t = tid - group * tpr;
     const uint32_t row_bytes = (uint32_t)a.hidden() * 8u;
     uint32_t off[VPT];
