@@ -400,7 +400,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     // few generations of workgroups) gain nothing and can lose 1-3 %, and with 2 partials no limit helps.  At the
     // threshold itself the gain is small: 4 x [8192, 7168] with per-group scales 0.4 % on a device that has been under
     // load for 20 ms (0.9 % slower in the first milliseconds after idling).
-    int wgs_per_cu = 0;
+    int wgs_per_cu = 0, wgs_held = 0; // reported, and what the launch is padded for
     // The staged algorithms are limited only on request.  With owned rows, and in the norm phase alone, most rows read two streams.
     // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more; two workgroups per CU against
     // none planned: 8 x [16384, 8192] bf16 -> fp8 513.7 -> 497.8 us, 4 x [32768, 8192] 688.2 -> 628.3, 4 x [16384, 5120] 203.6 ->
@@ -410,12 +410,22 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
         const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
         const int waves = tpr * rpb / 64;
-        // per-group scales are the heaviest arithmetic per row and four partials the shortest loads to cover it
-        const int need_waves = (p->quant == TDE_QUANT_FP8_GROUP && p->nranks <= 4) ? 12 : 8;
-        const int at_least = std::max(2, (need_waves + waves - 1) / waves);
-        wgs_per_cu = (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        const auto limit = [&](int need_waves) {
+            const int at_least = std::max(2, (need_waves + waves - 1) / waves);
+            return (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        };
+        // Per-group scales on four partials are reported as held to twelve wavefronts, what their arithmetic once took, and held
+        // to eight like the others (rows of more than 768 vectors: two workgroups instead of three): 4 x [8192, 7168] bf16
+        // 119.3 us against 123.2, 4 x [12000, 8192] 198.4 against 205.9, 4 x [32768, 7168] fp16 467 against 503, fp32 4 x [9000, 3584]
+        // 124.9 against 127.0.  Two are enough wherever two have 96 KiB of loads in flight and only codes of a dynamic scale beside
+        // residual_out to store, with four vectors per thread: 4 x [32768, 5120] fp16 -> int8 338.2 us against 342.3 with three, bf16
+        // -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three stay 3 % ahead.
+        wgs_per_cu = limit(p->quant == TDE_QUANT_FP8_GROUP && p->nranks <= 4 ? 12 : 8);
+        wgs_held = limit(8);
+        const bool few_stores = p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0;
+        if (vpt == 4 && few_stores && 2 * per_wg >= 96 * 1024) wgs_held = 2;
     }
-    if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
+    if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_held = wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
     if (geo) {
         geo->wgs_per_cu = wgs_per_cu;
@@ -427,6 +437,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
             geo->wgs_per_cu = (int)std::min<size_t>((size_t)wgs_per_cu, tde::kLdsPerCu / (lds + 64));
         }
         geo->lds_bytes = (int)lds;
+        geo->launch_lds = wgs_held > 0 ? std::max(lds, tde::lds_bytes_for_workgroups_per_cu(wgs_held)) : lds;
         geo->vec_elems = vec;
         geo->nvec = (int)nvec;
         geo->vpt = vpt;

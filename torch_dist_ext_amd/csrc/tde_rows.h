@@ -126,8 +126,6 @@ struct ElemBF16 {
         }
         return raw;
     }
-    // fp32 bit pattern of a non-negative element given by its own bits
-    static __device__ __forceinline__ uint32_t magnitude_to_f32_bits(uint32_t m) { return m << 16; }
 };
 
 struct ElemF16 {
@@ -151,9 +149,6 @@ struct ElemF16 {
         }
         return raw;
     }
-    static __device__ __forceinline__ uint32_t magnitude_to_f32_bits(uint32_t m) {
-        return __builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(_Float16, (uint16_t)m)); // NaN stays NaN
-    }
 };
 
 struct ElemF32 {
@@ -172,37 +167,25 @@ struct ElemF32 {
         for (int i = 0; i < 4; ++i) raw[i] = __builtin_bit_cast(uint32_t, f[i]);
         return raw;
     }
-    static __device__ __forceinline__ uint32_t magnitude_to_f32_bits(uint32_t m) { return m; }
 };
 
-// Largest magnitude of a row's elements, taken on the bit patterns: for non-negative floats of one format the
-// unsigned order of the bits is the order of the values with every NaN above infinity, so an unsigned maximum of
-// |x| propagates NaN as torch's amax does (a float maximum would drop it) and costs no more.  The 2-byte types keep
-// two running 16-bit maxima in one register (one packed instruction per two elements).
-//   amax_fold: folds a 16-byte vector into the running maximum (start from 0)
-//   amax_f32_bits: the fp32 bit pattern of the largest magnitude folded in (a NaN pattern if any element was NaN)
+// The largest magnitude of a row's elements: NaN if any of them is, as torch's amax has it (v_max_f32 would drop it).  Two
+// elements an instruction, on the values that the quotients need anyway.
+__device__ __forceinline__ float max_abs(float acc, float a, float b) {
+    float r;
+    asm("v_maximum3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(acc), "v"(a), "v"(b));
+    return r;
+}
+
+// min(max(q, -limit), limit) that keeps NaN, as torch.clamp does.
+__device__ __forceinline__ float clamp_keep_nan(float q, float limit) {
+    float r;
+    asm("v_maximum3_f32 %0, %1, -%2, -%2" : "=v"(r) : "v"(q), "v"(limit));
+    asm("v_minimum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(r), "v"(limit));
+    return r;
+}
+
 __device__ __forceinline__ uint32_t max_u32(uint32_t a, uint32_t b) { return a > b ? a : b; }
-
-template <class E>
-__device__ __forceinline__ uint32_t amax_fold(uint32_t acc, u32x4 raw) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t w = raw[i]; // copy first: bit_cast applied straight to a vector element reads lane 0
-        if constexpr (E::BYTES == 2) {
-            const u16x2 a = __builtin_bit_cast(u16x2, acc), b = __builtin_bit_cast(u16x2, w & 0x7fff7fffu);
-            acc = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, b));
-        } else {
-            acc = max_u32(acc, w & 0x7fffffffu);
-        }
-    }
-    return acc;
-}
-
-template <class E>
-__device__ __forceinline__ uint32_t amax_f32_bits(uint32_t acc) {
-    if constexpr (E::BYTES == 2) acc = max_u32(acc >> 16, acc & 0xffffu);
-    return E::magnitude_to_f32_bits(acc);
-}
 
 // ---------------------------------------------------------------------------------------------
 // 64-lane wavefront reductions: four DPP steps inside each 16-lane row, then the four row
@@ -217,7 +200,8 @@ __device__ __forceinline__ float dpp_move(float v) {
     return __builtin_bit_cast(float, dpp_move_u32<CTRL>(__builtin_bit_cast(uint32_t, v)));
 }
 
-// Unsigned maximum over each 16-lane row (the maxima here are bit patterns of magnitudes, see amax_fold).
+// Unsigned maximum over each 16-lane row.  The maxima across lanes are taken on the bit patterns of magnitudes: for
+// non-negative floats the order of the bits is the order of the values, with every NaN above infinity.
 __device__ __forceinline__ uint32_t row16_max(uint32_t v) {
     v = max_u32(v, dpp_move_u32<0xB1>(v));  // quad_perm [1,0,3,2]
     v = max_u32(v, dpp_move_u32<0x4E>(v));  // quad_perm [2,3,0,1]
@@ -237,16 +221,17 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
     return max_u32(max_u32(a, b), max_u32(c, d));
 }
 
-// Maximum over the `waves_per_row` wavefronts that share a row.  `slots` is an LDS buffer indexed by wavefront
-// number inside the block, used once per kernel (one barrier).  Identity is 0 (bit patterns of magnitudes).
-__device__ __forceinline__ uint32_t row_max(uint32_t v, uint32_t *slots, int wave, int lane, int first_wave, int waves_per_row) {
-    v = wave_max(v);
-    if (waves_per_row == 1) return v;
-    if (lane == 0) slots[wave] = v;
+// Maximum over the wavefronts that share a row.  `slot`: the row's word of LDS, zero before a barrier that every thread has
+// passed (0 is the identity: bit patterns of magnitudes).  One barrier.  The four 16-lane rows of a wavefront meet in LDS
+// instead of through v_readlane, the wavefronts there instead of in every wavefront once more.
+__device__ __forceinline__ uint32_t row_max(uint32_t v, uint32_t *slot, int lane, int waves_per_row) {
+    if (waves_per_row == 1) return wave_max(v);
+    v = row16_max(v);
+    // in assembly, or the compiler would put a reduction over the wavefront in front of it
+    if ((lane & 15) == 0)
+        asm volatile("ds_max_u32 %0, %1\n\ts_waitcnt lgkmcnt(0)" ::"v"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)slot), "v"(v) : "memory");
     __syncthreads();
-    const int k = lane & 15;
-    const uint32_t t = (k < waves_per_row) ? slots[first_wave + k] : 0u;
-    return row16_max(t);
+    return *slot;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -494,13 +479,13 @@ __device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WA
     p += quad_bcast<0x55>(chain);
     p += quad_bcast<0xAA>(chain);
     p += quad_bcast<0xFF>(chain);
-    if constexpr (VECF == 8) { // 2-byte types: whole vectors of eight floats, no scalars left over
-        sum = read_lane(p, 0);
-    } else {
-        sum += read_lane(p, 0);
-    }
+    float q[8];
 #pragma unroll
-    for (int mm = 1; mm < 8; ++mm) sum += read_lane(p, 4 * mm);
+    for (int mm = 0; mm < 8; ++mm) q[mm] = read_lane(p, 4 * mm);
+    __builtin_amdgcn_sched_barrier(0); // read one by one each would be waited for
+    sum = VECF == 8 ? q[0] : sum + q[0]; // 2-byte types: whole vectors of eight floats, no scalars left over
+#pragma unroll
+    for (int mm = 1; mm < 8; ++mm) sum += q[mm];
     return sum;
 }
 
@@ -572,17 +557,19 @@ __device__ __forceinline__ void pack_fp8(const float (&q)[VEC], uint32_t (&out)[
     }
 }
 
-template <int VEC>
+// Round to int8 codes, ties to even.  BOUNDED: every q is finite and rounds to a code; adding 1.5 * 2^23 then rounds it and leaves
+// the code in the low byte.  Otherwise q has been clamped and NaN becomes 0.
+template <int VEC, bool BOUNDED>
 __device__ __forceinline__ void pack_int8(const float (&q)[VEC], uint32_t (&out)[VEC / 4]) {
+    const auto code = [](float v) {
+        if constexpr (BOUNDED) return __builtin_bit_cast(uint32_t, v + 0x1.8p23f);
+        else return (uint32_t)(int)__builtin_rintf(v);
+    };
 #pragma unroll
     for (int w = 0; w < VEC / 4; ++w) {
-        uint32_t word = 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int code = (int)__builtin_rintf(q[4 * w + b]); // ties to even
-            word |= ((uint32_t)code & 0xffu) << (8 * b);
-        }
-        out[w] = word;
+        const uint32_t lo = __builtin_amdgcn_perm(code(q[4 * w + 1]), code(q[4 * w]), 0x0c0c0400u);
+        const uint32_t hi = __builtin_amdgcn_perm(code(q[4 * w + 3]), code(q[4 * w + 2]), 0x04000c0cu);
+        out[w] = lo | hi;
     }
 }
 
@@ -599,11 +586,38 @@ __device__ __forceinline__ float div_shared(float y, float d, float rcp) {
     return __builtin_fmaf(-e, rcp, q0);
 }
 
-// min(max(q, -limit), limit) that keeps NaN, as torch.clamp does (the float minimum and maximum drop it).
-__device__ __forceinline__ float clamp_keep_nan(float q, float limit) {
-    const float c = fminf(fmaxf(q, -limit), limit);
-    return (q != q) ? q : c;
-}
+// What turns a row's elements into codes: the divisor, and its reciprocal in the form that quotient() takes.
+//
+// Elements of 2 bytes have at most 11 significant bits, and their quotient only has to land on the right side of a code's
+// boundary, which has at most 8: the product with a reciprocal in two words, rounded once, gives the same codes as the
+// correctly rounded quotient in two instructions instead of three.  Its relative error of 2^-44 could only matter where y lies
+// within 2^5 units (of 49 bits) of (2 M +- 1) * d for a boundary M; with d = j 2^20 + r (2^17 for int8) that needs
+// M r = -+j with M >= 16 >= j (128), i.e. all ones in d, and even there no code differs (every mantissa of d
+// against every y of 8 and of 11 bits over the range of the codes, both code types, on gfx950).  hi is below 1/d by more than
+// half a unit and lo > 0: a numerator of -0 keeps its sign, and of infinity its infinity.
+// fp32 elements take the correctly rounded quotient (div_shared).
+template <class E>
+struct Divisor {
+    float d, hi, lo; // fp32 elements: hi is 1/d correctly rounded
+
+    Divisor() = default;
+    __device__ __forceinline__ explicit Divisor(float d_) {
+        d = d_;
+        const float r0 = __builtin_amdgcn_rcpf(d);
+        const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.0f), r0, r0); // 1/d, correctly rounded (every mantissa checked)
+        if constexpr (E::BYTES == 2) {
+            hi = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) - 1u);
+            lo = __builtin_fmaf(-d, hi, 1.0f) * r;
+        } else {
+            hi = r;
+            lo = 0.0f;
+        }
+    }
+    __device__ __forceinline__ float quotient(float y) const {
+        if constexpr (E::BYTES == 2) return __builtin_fmaf(y, hi, y * lo);
+        else return div_shared(y, d, hi);
+    }
+};
 
 // Which row group a workgroup takes.  Workgroups are handed to the 8 XCDs round-robin, so in launch order
 // every XCD (every L2) walks all of every buffer in 16 KiB steps.  Remapped in groups of 8*chunk, XCD k
@@ -677,14 +691,15 @@ __global__ void __launch_bounds__(1024 / VPT)
     constexpr bool WIDE = FORM == kFormWide, OWNED = FORM == kFormOwned;
     constexpr int VEC = E::VEC;
     constexpr int NP = (N == 0) ? 1 : N;
-    // residual_out is stored together with the row's other output at the end, one write burst per row: against storing
-    // it as soon as the sum is known that measures 0.9 % faster on 8 x [2048, 8192] bf16 -> fp8, 0.4 % on 4 x [8192, 7168]
-    // -> fp8 per group, 2.6 % on 2 x [8192, 8192], 7 % on 4 x [512, 7168], and the same within noise elsewhere.
+    // residual_out is stored behind the reductions, ahead of the codes: as soon as the sum is known it is 2.4 % slower on
+    // 2 x [1257, 6144] static and 7 % on 4 x [512, 5120], behind all codes in one burst 1.7 % on 4 x [32768, 5120] and 1 % on 8 x
+    // [2048, 8192] staged.  With a static scale, and where a stage is stored too, it goes out with the normed row already: 1 % and
+    // 0.6 % faster there; elsewhere the same, but 2 x [700, 4096] fp16 -> fp8 10 % slower.
     // Dynamic LDS: the workgroup's squares (one float per element it holds), then 1024 floats of block sums.
     extern __shared__ __attribute__((aligned(16))) float lds_dyn[];
     float *const lds_img = lds_dyn;
     float *const lds_bs = lds_dyn + (uint32_t)a.threads_per_row * a.rows_per_block * (VPT * VEC);
-    __shared__ uint32_t lds_max[kMaxWavesPerBlock];
+    __shared__ uint32_t lds_max[kMaxWavesPerBlock]; // one per row group
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -728,12 +743,12 @@ __global__ void __launch_bounds__(1024 / VPT)
     const int64_t row0 = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block;
 
     // The row's loads go out before anything else touches memory -- except gamma where it pays to have it first:
-    // with up to four partials of a 2-byte type, several vectors per thread and a per-token scale, the registers are
+    // with up to four partials of a 2-byte type, several vectors per thread and a dynamic scale, the registers are
     // there to hold gamma through the load phase, and requested ahead of the row (it is served from L2) it is never
     // waited for behind the row's own traffic.  Measured against requesting it after the accumulate phase, alternating
     // two builds in one process: 4 x [32768, 5120] fp16 -> int8 per token -1.0 %, 4 x [8192, 7168] bf16 -> fp8 per
-    // token -1.4 %, 2 x [8192, 8192] -0.6 %, 4 x [2048, 7168] -0.7 %; with per-group scales (no second barrier to
-    // cover) +0.9 to +2.7 %, with T-typed output or fp32 rows equal to +0.4 %, so those keep the late request.
+    // token -1.4 %, 2 x [8192, 8192] -0.6 %, 4 x [2048, 7168] -0.7 %; with per-group scales 4 x [8192, 7168] -1.1 %,
+    // 2 x [9000, 7168] -0.6 %; with T-typed output or fp32 rows equal to +0.4 %, so those keep the late request.
     // With eight partials the 16 registers are one too many for three wavefronts per SIMD (169 against 168: spilling
     // costs 2 us on 8 x [2048, 8192], and gamma ahead of the row for three of the four vectors gains 0.1 us); the WIDE
     // instantiation takes them and runs two workgroups per CU: 8 x [2048, 8192] bf16 -> fp8 56.8 us against 57.3,
@@ -744,7 +759,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     const rsrc_t gamma_rsrc = row_rsrc(a.ptr(kPtrGamma), 0, row_bytes);
     constexpr bool GAMMA_FIRST =
         VPT > 1 && N != 0 && !OWNED &&
-        (WIDE || (N <= 4 && E::BYTES == 2 && (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN)));
+        (WIDE || (N <= 4 && E::BYTES == 2 && (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN || Q == TDE_QUANT_FP8_GROUP)));
     u32x4 gamma_first[GAMMA_FIRST ? VPT : 1];
     if constexpr (GAMMA_FIRST) {
 #pragma unroll
@@ -770,6 +785,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     const uint32_t vec_stride = (uint32_t)tpr * 16u;
     const SumLayout<VPT, VEC, E::BYTES == 2> sums(lds_img, lds_bs, a.hidden(), tpr, a.rows_per_block, group);
     sumsq_clear(sums, TDE_T);
+    if constexpr (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN) lds_max[group] = 0u; // for row_max
     const float rcp_h = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, reciprocal_of_length((float)a.hidden()))));
 #define TDE_OFF(j) (lane0 + (uint32_t)(j) * vec_stride)
 
@@ -852,15 +868,6 @@ __global__ void __launch_bounds__(1024 / VPT)
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // From here on the wavefront has its row and only arithmetic, LDS and stores left: with up to four partials
-        // (short load phases, three workgroups sharing the vector units about 60 % of the time) it goes ahead of the
-        // wavefronts that are still summing partials.  4 x [32768, 5120] -0.5 %, 4 x [8192, 7168] -0.2 %; with eight
-        // partials nothing at 2048+ rows and +0.7 % at 512 rows, so those stay at the default priority.
-        if constexpr (N != 0 && N <= 4 && VPT == 4) {
-            __builtin_amdgcn_sched_barrier(0);
-            __builtin_amdgcn_s_setprio(1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
             if constexpr (OWNED) {
@@ -933,24 +940,33 @@ __global__ void __launch_bounds__(1024 / VPT)
         const float rs = reciprocal_rms(sumsq, (float)a.hidden(), rcp_h, a.eps);
 
         // ---- normalize ------------------------------------------------------------------------------
-        u32x4 yraw[VPT];
-        uint32_t amax[VPT]; // running maxima of the magnitudes' bit patterns (amax_fold), per vector
+        constexpr bool DYNAMIC = Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC;
+        constexpr bool EARLY_RESIDUAL = Q == TDE_QUANT_FP8_STATIC || (Q != TDE_QUANT_NONE && FORM == kFormStaged);
+        constexpr int QUANT_VPT = Q == TDE_QUANT_NONE ? 1 : VPT;
+        float y[QUANT_VPT][VEC]; // what is quantized
+        float amax[VPT];         // largest magnitude per vector
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            float x[VEC], g[VEC], y[VEC];
+            float x[VEC], g[VEC], n[VEC];
             E::unpack(xraw[j], x);
             E::unpack(gamma_raw[j], g);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) y[i] = x[i] * rs;
-            E::unpack(E::pack(y), y);
+            for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
+            E::unpack(E::pack(n), n);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) y[i] = g[i] * y[i];
-            yraw[j] = E::pack(y);
+            for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
+            const u32x4 nraw = E::pack(n);
             if constexpr (Q == TDE_QUANT_NONE || WN) {
                 const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
-                rsrc_store16(norm_out, TDE_OFF(j), yraw[j]);
+                rsrc_store16(norm_out, TDE_OFF(j), nraw);
             }
-            if constexpr (Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC) amax[j] = amax_fold<E>(0u, yraw[j]);
+            if constexpr (Q != TDE_QUANT_NONE) E::unpack(nraw, y[j]);
+            if constexpr (DYNAMIC) {
+                amax[j] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < VEC; i += 2) amax[j] = max_abs(amax[j], y[j][i], y[j][i + 1]);
+            }
+            if constexpr (EARLY_RESIDUAL) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
         }
 
         if constexpr (Q == TDE_QUANT_NONE) {
@@ -958,93 +974,103 @@ __global__ void __launch_bounds__(1024 / VPT)
             for (int j = 0; j < VPT; ++j) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
         }
 
-        // ---- dynamic quant epilogue ---------------------------------------------------------------
+        // ---- quant epilogue -------------------------------------------------------------------------
         if constexpr (Q != TDE_QUANT_NONE) {
             constexpr float QMAX = (Q == TDE_QUANT_INT8_TOKEN) ? 127.0f : 448.0f;
-            float scale[VPT];
+            constexpr int SCALES = Q == TDE_QUANT_FP8_GROUP ? VPT : 1; // a thread's vectors lie in groups of their own
+            // One wavefront-uniform decision for all of the thread's vectors, so the common path carries no per-lane branch: its
+            // quotients need every divisor far from the subnormal and overflow ranges.  A largest magnitude that is NaN or infinite
+            // also takes the plain division.
+            float scale[SCALES];
+            bool fast;
+            if constexpr (DYNAMIC) {
+                uint32_t m[SCALES];
+                if constexpr (Q == TDE_QUANT_FP8_GROUP) {
+#pragma unroll
+                    for (int j = 0; j < VPT; ++j) {
+                        m[j] = row16_max(__builtin_bit_cast(uint32_t, amax[j]) & 0x7fffffffu);
+                        if constexpr (TDE_QUANT_GROUP / VEC == 32) m[j] = max_u32(m[j], (uint32_t)__shfl_xor((int)m[j], 16, kWave));
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 1; j < VPT; ++j) amax[0] = max_abs(amax[0], amax[j], amax[j]);
+                    m[0] = row_max(__builtin_bit_cast(uint32_t, amax[0]) & 0x7fffffffu, lds_max + group, TDE_LANE, waves_per_row);
+                }
+                uint64_t unsafe = 0;
+                constexpr uint32_t LOW = (127u - 50u) << 23, HIGH = (127u + 60u) << 23; // 2^-50 to 2^60
+#pragma unroll
+                for (int j = 0; j < SCALES; ++j)
+                    unsafe |= __builtin_amdgcn_ballot_w64(m[j] - LOW > HIGH - LOW) & __builtin_amdgcn_ballot_w64(m[j] != 0u);
+                fast = unsafe == 0;
+#pragma unroll
+                for (int j = 0; j < SCALES; ++j) scale[j] = div_shared(__builtin_bit_cast(float, m[j]), QMAX, 1.0f / QMAX);
+                if (__builtin_expect(!fast, 0)) {
+#pragma unroll
+                    for (int j = 0; j < SCALES; ++j) {
+                        asm volatile("; not computed beside the fast one" : "+v"(m[j]));
+                        scale[j] = __builtin_bit_cast(float, m[j]) / QMAX;
+                    }
+                }
+            } else {
+                scale[0] = a.static_scale;
+                fast = __builtin_amdgcn_readfirstlane(scale[0] >= 0x1p-60f && scale[0] <= 0x1p60f) != 0;
+            }
             if constexpr (Q == TDE_QUANT_FP8_GROUP) {
                 constexpr int LANES_PER_GROUP = TDE_QUANT_GROUP / VEC; // 16 (2-byte types) or 32 (fp32)
                 const int64_t groups_per_row = a.hidden() / TDE_QUANT_GROUP;
                 const rsrc_t sc_out = row_rsrc(a.ptr(kPtrScale), row * groups_per_row * 4, row_ok ? (uint32_t)groups_per_row * 4u : 0u);
+                if ((TDE_LANE & (LANES_PER_GROUP - 1)) == 0) {
 #pragma unroll
-                for (int j = 0; j < VPT; ++j) {
-                    uint32_t m = row16_max(amax_f32_bits<E>(amax[j]));
-                    if constexpr (LANES_PER_GROUP == 32) m = max_u32(m, (uint32_t)__shfl_xor((int)m, 16, kWave));
-                    scale[j] = __builtin_bit_cast(float, m) / QMAX;
-                    if ((TDE_LANE & (LANES_PER_GROUP - 1)) == 0)
+                    for (int j = 0; j < VPT; ++j)
                         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, scale[j]), sc_out,
                                                               (int)((TDE_OFF(j) / 16u / LANES_PER_GROUP) * 4u), 0, kAuxDefault);
                 }
-            } else if constexpr (Q == TDE_QUANT_FP8_STATIC) {
-#pragma unroll
-                for (int j = 0; j < VPT; ++j) scale[j] = a.static_scale;
-            } else {
-                uint32_t m = amax[0];
-#pragma unroll
-                for (int j = 1; j < VPT; ++j) {
-                    if constexpr (E::BYTES == 2) m = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m), __builtin_bit_cast(u16x2, amax[j])));
-                    else m = max_u32(m, amax[j]);
-                }
-                m = row_max(amax_f32_bits<E>(m), lds_max, wave, TDE_LANE, first_wave, waves_per_row);
-                const float sc = __builtin_bit_cast(float, m) / QMAX;
-#pragma unroll
-                for (int j = 0; j < VPT; ++j) scale[j] = sc;
-                if (row_ok && TDE_T == 0) ((TDE_GLOBAL float *)a.ptr(kPtrScale))[row] = sc;
+            } else if constexpr (DYNAMIC) {
+                if (row_ok && TDE_T == 0) ((TDE_GLOBAL float *)a.ptr(kPtrScale))[row] = scale[0];
             }
             const rsrc_t q_out = row_rsrc(a.ptr(kPtrCodes), row * (int64_t)a.hidden(), row_ok ? (uint32_t)a.hidden() : 0u);
+            if constexpr (!EARLY_RESIDUAL) {
 #pragma unroll
-            for (int j = 0; j < VPT; ++j) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
-            // One wavefront-uniform decision for all of the thread's vectors, so the common path carries no per-lane
-            // branch: the fast quotient needs every divisor far from the subnormal and overflow ranges.  A dynamic scale
-            // that is NaN or infinite (a NaN or an infinity among the normed values) also takes the plain division.
-            bool unsafe = false;
-#pragma unroll
-            for (int j = 0; j < VPT; ++j) unsafe = unsafe || !(scale[j] == 0.0f || (scale[j] > 0x1p-60f && scale[j] < 0x1p60f));
-            const bool fast = __builtin_amdgcn_ballot_w64(unsafe) == 0;
+                for (int j = 0; j < VPT; ++j) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
+            }
             auto quantize = [&](auto use_fast) {
+                constexpr bool FAST = decltype(use_fast)::value;
+                Divisor<E> divisor;
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) {
-                    float y[VEC], q[VEC];
-                    E::unpack(yraw[j], y);
-                    const float div = (scale[j] > 0.0f) ? scale[j] : 1.0f;
-                    if constexpr (Q == TDE_QUANT_FP8_STATIC) {
-                        // A caller's scale can be far below the row's values (the dynamic scales cannot: |y| <= QMAX *
-                        // scale).  Beyond twice the largest code the quotient clamps to QMAX whatever it is, so y is cut
-                        // there: the product y * rcp then stays finite and the correction never sees inf - inf.
-                        const float ymax = (div < 0x1p60f) ? 2.0f * QMAX * div : 3.0e38f;
+                    const float sc = scale[SCALES == 1 ? 0 : j];
+                    const float div = (Q == TDE_QUANT_FP8_STATIC || sc > 0.0f) ? sc : 1.0f;
+                    if (FAST && (SCALES > 1 || j == 0)) divisor = Divisor<E>(div);
+                    float q[VEC];
 #pragma unroll
-                        for (int i = 0; i < VEC; ++i) y[i] = clamp_keep_nan(y[i], ymax);
-                    }
-                    if constexpr (decltype(use_fast)::value) {
-                        const float rcp = 1.0f / div;
-                        if constexpr (Q == TDE_QUANT_FP8_STATIC) {
-#pragma unroll
-                            for (int i = 0; i < VEC; ++i) q[i] = clamp_keep_nan(div_shared(y[i], div, rcp), QMAX);
-                        } else {
-                            // |y| <= QMAX * scale up to two roundings: the quotient is within 1e-4 of +-QMAX at most,
-                            // which the conversions below round to the largest code; nothing to clamp
-#pragma unroll
-                            for (int i = 0; i < VEC; ++i) q[i] = div_shared(y[i], div, rcp);
-                        }
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < VEC; ++i) q[i] = clamp_keep_nan(y[i] / div, QMAX);
+                    for (int i = 0; i < VEC; ++i) {
+                        float v = y[j][i];
+                        // A caller's scale can be far below the row's values (the dynamic scales cannot: |y| <= QMAX * scale).
+                        // Beyond twice the largest code the quotient clamps to QMAX whatever it is, so where its correction
+                        // would see inf - inf, y is cut there.
+                        if constexpr (Q == TDE_QUANT_FP8_STATIC && FAST && E::BYTES != 2) v = clamp_keep_nan(v, 2.0f * QMAX * div);
+                        if constexpr (FAST) v = divisor.quotient(v);
+                        else v = v / div;
+                        // Dynamic scales: the quotient is within 1e-4 of +-QMAX at most, which the conversions below round to
+                        // the largest code; nothing to clamp
+                        if constexpr (!FAST || Q == TDE_QUANT_FP8_STATIC) v = clamp_keep_nan(v, QMAX);
+                        q[i] = v;
                     }
                     uint32_t codes[VEC / 4];
                     if constexpr (Q == TDE_QUANT_INT8_TOKEN)
-                        pack_int8<VEC>(q, codes);
+                        pack_int8<VEC, FAST>(q, codes);
                     else
                         pack_fp8<VEC>(q, codes);
                     const uint32_t code_off = (TDE_OFF(j) / 16u) * (uint32_t)VEC;
                     if constexpr (VEC == 8) {
-                        u32x2 w = {codes[0], codes[1]};
+                        const u32x2 w = {codes[0], codes[1]};
                         __builtin_amdgcn_raw_buffer_store_b64(w, q_out, (int)code_off, 0, kAuxStore);
                     } else {
                         __builtin_amdgcn_raw_buffer_store_b32(codes[0], q_out, (int)code_off, 0, kAuxStore);
                     }
                 }
             };
-            if (fast)
+            if (__builtin_expect(fast, 1))
                 quantize(std::true_type{});
             else
                 quantize(std::false_type{});
@@ -1117,7 +1143,8 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
 // ---------------------------------------------------------------------------------------------
 struct Geometry {
     int wgs_per_cu; // limit on resident workgroups per compute unit (0 = none), enforced through lds_bytes
-    int lds_bytes;  // dynamic LDS of the row kernel's launch
+    int lds_bytes;  // dynamic LDS as reported: the row kernel's own, padded for wgs_per_cu
+    size_t launch_lds; // dynamic LDS of the row kernel's launch, at least that much
     int vec_elems;
     int nvec;
     int vpt;
@@ -1149,7 +1176,7 @@ hipError_t launch_traffic(int n, int vpt, int code_bytes, bool wn, const RowArgs
 template <class E, int N, int VPT>
 hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
-    const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
+    const size_t lds = g.launch_lds; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
 #define TDE_LAUNCH_FORM(QM, WNB, FORM)                                                                   \
     {                                                                                                    \
         if (lds > kDefaultMaxDynamicLds) {                                                               \
