@@ -91,8 +91,7 @@ int compute_units() {
 // each unit gets -- a launch's time rises in steps, with every further workgroup on the fullest unit, and the steps lie at
 // different counts for workgroups of different sizes -- so a device (or partition) with another number of units is asked for
 // the same rows per unit.
-int64_t rows_as_on_256_units(int64_t tokens) {
-    const int64_t cus = compute_units();
+int64_t rows_as_on_256_units(int64_t tokens, int64_t cus) {
     return cus == 256 ? tokens : tokens / cus * 256 + tokens % cus * 256 / cus;
 }
 
@@ -372,7 +371,8 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     int64_t total_bytes = 0; // tokens * hidden * elem must be addressable with 64-bit signed offsets
     if (__builtin_mul_overflow(p->tokens, p->hidden * eb, &total_bytes)) return TDE_ESHAPE;
 
-    const int64_t t = rows_as_on_256_units(p->tokens);
+    const int cus = compute_units(); // once a call: asking the runtime for the device takes it 50 ns
+    const int64_t t = rows_as_on_256_units(p->tokens, cus);
     int vpt = p->dtype != TDE_F64 ? vecs_per_thread(p, nvec, t, norm_alone) : (norm_alone ? vecs_per_thread_f64_norm(nvec, t) : vecs_per_thread_f64(p, nvec, t));
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
@@ -384,7 +384,6 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     const int tpr = (int)((lanes + 63) / 64 * 64);
     int rpb = 256 / tpr; // pack short rows so a workgroup has at least four wavefronts
     if (rpb * tpr > kMaxBlock / vpt) rpb = (kMaxBlock / vpt) / tpr; // never beyond the kernel's launch bound
-    const int cus = compute_units();
     while (rpb > 1 && (p->tokens + rpb - 1) / rpb < 2 * cus) rpb /= 2; // keep every CU busy first
     if (rpb < 1) rpb = 1;
     if (p->tune_rows_per_block > 0 && p->tune_rows_per_block * tpr <= kMaxBlock / vpt) rpb = p->tune_rows_per_block;

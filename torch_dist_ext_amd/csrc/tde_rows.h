@@ -297,6 +297,16 @@ hipError_t allow_large_lds() {
     return e;
 }
 
+// One launch.  hipLaunchKernel itself: the <<<>>> form goes through a pushed and popped call configuration and leaves its
+// status to hipGetLastError, 0.15 us of host time a launch (2.42 against 2.27 us for an empty kernel).
+template <auto KERNEL, class... Args>
+hipError_t launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t s, const Args &...args) {
+    void *ptrs[] = {const_cast<void *>(static_cast<const void *>(&args))...};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(KERNEL), grid, block, ptrs, lds, s);
+    if (e != hipSuccess) (void)hipGetLastError(); // reported through the return value, not left behind for the next call
+    return e;
+}
+
 // Returns `v`, but only once `after` exists: index arithmetic built on the result cannot be hoisted above the
 // row loads, whose registers leave no room for it.
 __device__ __forceinline__ int not_before(int v, uint32_t after) {
@@ -1183,8 +1193,7 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
             const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB, FORM>>();                \
             if (e != hipSuccess) return e;                                                               \
         }                                                                                                \
-        hipLaunchKernelGGL((row_kernel<E, N, VPT, QM, WNB, FORM>), grid, block, lds, s, a);            \
-        return hipGetLastError();                                                                        \
+        return launch_kernel<row_kernel<E, N, VPT, QM, WNB, FORM>>(grid, block, lds, s, a);              \
     }
 #define TDE_LAUNCH(QM, WNB)                                                                              \
     if constexpr (N == 8 && VPT == 4) {                                                                  \
@@ -1239,8 +1248,7 @@ hipError_t launch_reduce_nu(const RowArgs &a, uint64_t table, int64_t row_bytes,
     if (blocks <= 0) return hipSuccess;
     if (blocks > 0x7fffffff) return hipErrorInvalidValue; // grid dimension limit
     sp.chunked_blocks = chunked_blocks(blocks, sp.xcd_chunk);
-    hipLaunchKernelGGL((reduce_kernel<E, N, U>), dim3((unsigned)blocks), dim3(256), 0, s, a, sp);
-    return hipGetLastError();
+    return launch_kernel<reduce_kernel<E, N, U>>(dim3((unsigned)blocks), dim3(256), 0, s, a, sp);
 }
 
 template <class E, int N>

@@ -213,25 +213,22 @@ hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t ro
     sp.chunked_blocks = chunked_blocks(blocks, sp.xcd_chunk);
     const dim3 grid((unsigned)blocks), block(256);
     switch (n) {
-    case 2: hipLaunchKernelGGL((reduce_kernel_f64<2, U>), grid, block, 0, s, a, sp); break;
-    case 4: hipLaunchKernelGGL((reduce_kernel_f64<4, U>), grid, block, 0, s, a, sp); break;
-    case 8: hipLaunchKernelGGL((reduce_kernel_f64<8, U>), grid, block, 0, s, a, sp); break;
-    default: return hipErrorInvalidValue;
+    case 2: return launch_kernel<reduce_kernel_f64<2, U>>(grid, block, 0, s, a, sp);
+    case 4: return launch_kernel<reduce_kernel_f64<4, U>>(grid, block, 0, s, a, sp);
+    case 8: return launch_kernel<reduce_kernel_f64<8, U>>(grid, block, 0, s, a, sp);
     }
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 template <int N, int VPT>
 hipError_t launch_rows_f64_nv(const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, VPT, 2): doubles are never limited per CU
-    if constexpr (N == 0)
-        hipLaunchKernelGGL((row_kernel_f64<0, VPT>), grid, block, lds, s, a);
-    else
-        hipLaunchKernelGGL((g.form == kFormOwned    ? row_kernel_f64<N, VPT, kFormOwned>
-                            : g.form == kFormStaged ? row_kernel_f64<N, VPT, kFormStaged>
-                                                    : row_kernel_f64<N, VPT>), grid, block, lds, s, a);
-    return hipGetLastError();
+    if constexpr (N != 0) {
+        if (g.form == kFormOwned) return launch_kernel<row_kernel_f64<N, VPT, kFormOwned>>(grid, block, lds, s, a);
+        if (g.form == kFormStaged) return launch_kernel<row_kernel_f64<N, VPT, kFormStaged>>(grid, block, lds, s, a);
+    }
+    return launch_kernel<row_kernel_f64<N, VPT>>(grid, block, lds, s, a);
 }
 
 template <int N>
