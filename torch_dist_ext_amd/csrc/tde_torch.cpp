@@ -5,7 +5,8 @@
 // One GPU plays every rank: CommWorkspace owns N local allocations ("slots") where the reference
 // maps N peers' comm buffers through HIP IPC (src/ops/all_reduce_fusion.cpp:107-141).
 #include <ATen/ATen.h>
-#include <ATen/hip/EmptyTensor.h>
+#include <ATen/EmptyTensor.h>
+#include <ATen/hip/HIPContextLight.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/custom_class.h>
@@ -230,14 +231,29 @@ Tensor get_workspace_op(const Tensor &ref) {
     return cur->get_workspace(ref);
 }
 
-// A new output tensor, straight from the allocator: at::empty and at::empty_like go through the dispatcher once and twice
-// more, 0.2-0.3 us of host time for each output (with the kernel arguments in 120 bytes, the other change between the two
-// figures: allreduce_rms 8 x [128, 4096] 5.97 -> 5.37 us a call, allreduce_rms_quant 4 x [64, 5120] int8 7.18 -> 6.24).
-Tensor new_output(at::IntArrayRef sizes, at::ScalarType dtype, const Tensor &on) {
-    return Tensor(at::detail::empty_cuda(sizes, dtype, on.device(), c10::nullopt));
-}
+// The device of a call's tensors, made the current one for the call's duration.
+class CallDevice {
+public:
+    explicit CallDevice(const Tensor &on) : index_(on.device().index()) {
+        if (index_ != c10::hip::current_device()) guard_.set_index(index_);
+    }
 
-Tensor new_like(const Tensor &t) { return new_output(t.sizes(), t.scalar_type(), t); }
+    // A new output tensor, straight from the allocator.  at::empty and at::empty_like go through the dispatcher once and twice
+    // more, at::detail::empty_cuda asks for the device and the global context each time.  A call's host time without its launch,
+    // through both, empty_cuda and this: allreduce_rms 2.14 -> 1.78 us from the second to the third, allreduce_rms_quant 3.15 -> 2.49
+    // (from the first to the second 0.2-0.3 us an output).
+    Tensor new_output(at::IntArrayRef sizes, at::ScalarType dtype) const {
+        return Tensor(at::detail::empty_generic(sizes, allocator_, c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype, c10::nullopt));
+    }
+    Tensor new_like(const Tensor &t) const { return new_output(t.sizes(), t.scalar_type()); }
+
+    hipStream_t stream() const { return c10::hip::getCurrentHIPStream(index_).stream(); }
+
+private:
+    c10::DeviceIndex index_;
+    c10::hip::OptionalHIPGuard guard_;
+    c10::Allocator *allocator_ = at::cuda::getCUDADeviceAllocator();
+};
 
 struct Call {
     tde_problem p{};
@@ -297,12 +313,7 @@ void fill_quant(Call &c, int64_t quant_mode, const Tensor &like, const Tensor *n
 
 const Tensor *given(const c10::optional<Tensor> &t) { return t.has_value() ? &*t : nullptr; }
 
-void run(Call &c, const Tensor &on) {
-    c10::hip::OptionalHIPGuard guard;
-    if (on.device().index() != c10::hip::current_device()) guard.set_index(on.device().index());
-    hipStream_t stream = c10::hip::getCurrentHIPStream(on.device().index()).stream();
-    check_status(tde_reduce_rms(&c.p, &c.b, stream), "torch_dist_ext");
-}
+void run(Call &c, const CallDevice &device) { check_status(tde_reduce_rms(&c.p, &c.b, device.stream()), "torch_dist_ext"); }
 
 // Points the call at the workspace's slots, with the caller's own partial read straight from allreduce_in.
 void use_table(Call &c, int64_t rank, int64_t nranks, const Tensor &allreduce_in, const Tensor &workspace) {
@@ -334,7 +345,7 @@ void allreduce_rms_fusion(int64_t rank, int64_t nranks, Tensor &allreduce_in, Te
     fill_common(c, rank, nranks, allreduce_in, residual_in, rms_gamma, residual_out, eps);
     fill_quant(c, TDE_QUANT_NONE, allreduce_in, &norm_out, nullptr, nullptr);
     use_table(c, rank, nranks, allreduce_in, workspace);
-    run(c, allreduce_in);
+    run(c, CallDevice(allreduce_in));
 }
 
 // Quantizing variant behind the same workspace protocol.
@@ -346,7 +357,7 @@ void allreduce_rms_quant_fusion(int64_t rank, int64_t nranks, Tensor &allreduce_
     fill_common(c, rank, nranks, allreduce_in, residual_in, rms_gamma, residual_out, eps);
     fill_quant(c, quant_mode, allreduce_in, given(norm_out), &q_out, given(scale_out), static_scale);
     use_table(c, rank, nranks, allreduce_in, workspace);
-    run(c, allreduce_in);
+    run(c, CallDevice(allreduce_in));
 }
 
 // Before outputs shaped like these two are allocated.
@@ -363,15 +374,16 @@ std::tuple<Tensor, Tensor> allreduce_rms(int64_t rank, int64_t nranks, const Ten
                                          const Tensor &rms_gamma, double eps, const Tensor &workspace) {
     TORCH_CHECK(allreduce_in.dim() >= 1 && allreduce_in.size(-1) <= 8192, "allreduce_rms: hidden_dim <= 8192 expected");
     check_outputs_like(allreduce_in, residual_in);
-    Tensor norm_out = new_like(allreduce_in);
-    Tensor residual_out = new_like(residual_in);
+    const CallDevice device(allreduce_in);
+    Tensor norm_out = device.new_like(allreduce_in);
+    Tensor residual_out = device.new_like(residual_in);
     Call c;
     fill_common(c, rank, nranks, allreduce_in, residual_in, rms_gamma, residual_out, eps);
     c.p.quant = TDE_QUANT_NONE;
     c.b.norm_out = norm_out.data_ptr();
     c.p.write_norm = 1;
     use_table(c, rank, nranks, allreduce_in, workspace);
-    run(c, allreduce_in);
+    run(c, device);
     return {norm_out, residual_out};
 }
 
@@ -411,14 +423,15 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> allreduce_rms_quant(int64_t rank, int
                                                                const Tensor &workspace, int64_t quant_mode, bool write_norm,
                                                                double static_scale) {
     check_outputs_like(allreduce_in, residual_in);
+    const CallDevice device(allreduce_in);
     QuantOutputs o = quant_outputs(allreduce_in, residual_in, quant_mode, write_norm,
-                                   [&](at::IntArrayRef sizes, at::ScalarType dtype) { return new_output(sizes, dtype, allreduce_in); });
+                                   [&](at::IntArrayRef sizes, at::ScalarType dtype) { return device.new_output(sizes, dtype); });
     Call c;
     fill_common(c, rank, nranks, allreduce_in, residual_in, rms_gamma, o.residual_out, eps);
     fill_quant(c, quant_mode, allreduce_in, write_norm ? &o.norm_out : nullptr, &o.q,
                quant_mode == TDE_QUANT_FP8_STATIC ? nullptr : &o.scale, static_scale);
     use_table(c, rank, nranks, allreduce_in, workspace);
-    run(c, allreduce_in);
+    run(c, device);
     return {std::move(o.q), std::move(o.scale), std::move(o.residual_out), std::move(o.norm_out)};
 }
 
@@ -434,7 +447,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> allreduce_rms_quant_meta(int64_t, int
 // The same stage with the N partials given directly as N tensors (no workspace object), into the given outputs.
 void run_local(const std::vector<Tensor> &partials, const Tensor &residual_in, const Tensor &rms_gamma, const Tensor &residual_out,
                const Tensor *norm_out, const Tensor *q_out, const Tensor *scale_out, double eps, int64_t quant_mode, int64_t algo,
-               const Tensor *stage, double static_scale) {
+               const Tensor *stage, double static_scale, const CallDevice *device = nullptr) {
     TORCH_CHECK(!partials.empty() && partials.size() <= TDE_MAX_RANKS, "reduce_rms_local: 2, 4 or 8 partials expected");
     Call c;
     fill_common(c, 0, (int64_t)partials.size(), partials[0], residual_in, rms_gamma, residual_out, eps);
@@ -448,7 +461,8 @@ void run_local(const std::vector<Tensor> &partials, const Tensor &residual_in, c
         check_row_tensor(*stage, partials[0], "stage");
         c.b.stage = stage->data_ptr();
     }
-    run(c, partials[0]);
+    if (device != nullptr) run(c, *device);
+    else run(c, CallDevice(partials[0]));
 }
 
 void reduce_rms_local(std::vector<Tensor> partials, Tensor &residual_in, Tensor &rms_gamma, Tensor &residual_out,
@@ -467,23 +481,24 @@ reduce_rms_partials(std::vector<Tensor> partials, const Tensor &residual_in, con
     const Tensor &ref = partials[0];
     TORCH_CHECK(ref.dim() >= 1, "reduce_rms: partials must have at least one dimension");
     check_outputs_like(ref, residual_in);
-    const Tensor residual_out = new_like(residual_in);
+    const CallDevice device(ref);
+    const Tensor residual_out = device.new_like(residual_in);
     c10::optional<Tensor> norm_out, q, scale;
     if (quant_mode == TDE_QUANT_NONE) {
-        norm_out = new_like(ref);
+        norm_out = device.new_like(ref);
     } else {
-        if (write_norm) norm_out = new_like(ref);
-        q = new_output(ref.sizes(), quant_mode == TDE_QUANT_INT8_TOKEN ? at::kChar : at::kFloat8_e4m3fn, ref);
+        if (write_norm) norm_out = device.new_like(ref);
+        q = device.new_output(ref.sizes(), quant_mode == TDE_QUANT_INT8_TOKEN ? at::kChar : at::kFloat8_e4m3fn);
         if (quant_mode != TDE_QUANT_FP8_STATIC) {
             c10::SmallVector<int64_t, 5> shape(ref.sizes().begin(), ref.sizes().end() - 1);
             if (quant_mode == TDE_QUANT_FP8_GROUP) shape.push_back(ref.size(-1) / TDE_QUANT_GROUP);
-            scale = new_output(shape, at::kFloat, ref);
+            scale = device.new_output(shape, at::kFloat);
         }
     }
     const bool staged = algo == TDE_ALGO_STAGED || algo == TDE_ALGO_STAGED_OWNED;
-    const Tensor own_stage = staged && !stage.has_value() ? new_like(ref) : Tensor();
+    const Tensor own_stage = staged && !stage.has_value() ? device.new_like(ref) : Tensor();
     run_local(partials, residual_in, rms_gamma, residual_out, given(norm_out), given(q), given(scale), eps, quant_mode, algo,
-              stage.has_value() ? &*stage : &own_stage, static_scale);
+              stage.has_value() ? &*stage : &own_stage, static_scale, &device);
     return {residual_out, norm_out, q, scale};
 }
 
