@@ -405,15 +405,41 @@ __device__ __forceinline__ float chain_block_sum(const float *block, int cl, int
     return acc;
 }
 
-template <int SLOTS>
-__device__ __forceinline__ float chain_sum(const float *bs, int cl) {
-    float v[SLOTS];
+// A chain's block sums, left to right.  All that could be there are requested before the first is added; what lies in slots that
+// are not used is the next row's or nobody's, and inside the 1024 floats for every row (the last of several rows starts at slot
+// 16 at most).  Up to eight and up to sixteen have code of their own: always sixteen costs 8 x [1, 4096] 2 %, a switch over every
+// number, which the compiler turns into a tree of branches and flags, 4 x [64, 5120] fp16 -> int8 3 % and 4 x [300, 2048] 2 %.
+template <int MOST>
+__device__ __forceinline__ float chain_sum_of(const float *bs, int cl, int slots) {
+    float v[MOST];
 #pragma unroll
-    for (int b = 0; b < SLOTS; ++b) v[b] = bs[b * 32 + cl];
-    float chain = v[0];
+    for (int b = 0; b < MOST; ++b) v[b] = bs[b * 32 + cl];
+    float chain = v[0] + v[1];
+    if (slots > 2) chain = (chain + v[2]) + v[3];
+    if (slots > 4) {
 #pragma unroll
-    for (int b = 1; b < SLOTS; ++b) chain += v[b];
+        for (int b = 4; b < 8; ++b) chain += v[b];
+    }
+    if constexpr (MOST == 16) {
+#pragma unroll
+        for (int b = 8; b < 12; ++b) chain += v[b];
+        if (slots > 12) {
+#pragma unroll
+            for (int b = 12; b < 16; ++b) chain += v[b];
+        }
+    }
     return chain;
+}
+__device__ __forceinline__ float chain_sum(const float *bs, int cl, int slots) {
+    if (slots == 1) return bs[cl];
+    return slots > 8 ? chain_sum_of<16>(bs, cl, slots) : chain_sum_of<8>(bs, cl, slots);
+}
+
+// Waits for the wavefronts that share a row; one wavefront alone only for its own LDS traffic.
+__device__ __forceinline__ void row_barrier(int waves_per_row) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    if (waves_per_row > 1) __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // After every thread of the row group has put its squares: the sum, the same value in every thread.
@@ -443,7 +469,7 @@ __device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WA
             for (int k = 0; k < VPT / 2; ++k) s.bs[b[k] * 32 + cl] = sum[k];
         }
     } else {
-        if (waves_per_row > 1) __syncthreads(); else wave_lds_fence();
+        row_barrier(waves_per_row);
         // one thread per chain and block: the group has at least 32 threads per block of its chains
         if (t < 32 * s.blocks) {
             const int b = t >> 5;
@@ -454,18 +480,10 @@ __device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WA
             s.bs[t] = sum;
         }
     }
-    if (waves_per_row > 1) __syncthreads(); else wave_lds_fence();
+    row_barrier(waves_per_row);
 
     // Lane 4m + k of every wavefront sums the blocks of chain (m, k); the quad then holds the four chains of m.
-    float chain;
-    switch (s.slots) {
-    case 1: chain = chain_sum<1>(s.bs, cl); break;
-    case 2: chain = chain_sum<2>(s.bs, cl); break;
-    case 4: chain = chain_sum<4>(s.bs, cl); break;
-    case 8: chain = chain_sum<8>(s.bs, cl); break;
-    case 12: chain = chain_sum<12>(s.bs, cl); break;
-    default: chain = chain_sum<16>(s.bs, cl); break;
-    }
+    const float chain = chain_sum(s.bs, cl, s.slots);
     float p = quad_bcast<0x00>(chain);
     float sum = 0.0f; // the scalars left over
     if (s.n != s.chained) {
@@ -514,7 +532,9 @@ __device__ __forceinline__ float reciprocal_of_length(float h) {
 __device__ __forceinline__ float reciprocal_rms(float sumsq, float h, float rcp_h, float eps) {
     const float q0 = sumsq * rcp_h;
     const float m = __builtin_fmaf(-__builtin_fmaf(q0, h, -sumsq), rcp_h, q0) + eps;
-    if (!(m >= 0x1p-60f && m <= 0x1p100f)) return 1.0f / __builtin_sqrtf(sumsq / h + eps);
+    constexpr uint32_t LOW = (127u - 60u) << 23, HIGH = (127u + 100u) << 23;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, m) - LOW > HIGH - LOW) != 0, 0))
+        return 1.0f / __builtin_sqrtf(sumsq / h + eps); // the same value in every lane
     float y = __builtin_amdgcn_rsqf(m);
     float g = m * y;
     y *= 0.5f;
