@@ -138,9 +138,10 @@ typedef struct tde_plan_out {
                                   already admits fewer.  Also 2, without LDS padding, where the plan picks the row
                                   kernel built for two wavefronts per SIMD (eight partials, four vectors per thread,
                                   4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its registers admit two.
-                                  The staged algorithms are never limited unless asked to.  Long launches of four
-                                  partials whose dynamic-scale codes are all they store beside residual_out may be held
-                                  to two where this says three */
+                                  0 for the staged algorithms unless asked for, though long launches of
+                                  TDE_ALGO_STAGED are held to two to four.  Long launches of four partials whose
+                                  dynamic-scale codes are all they store beside residual_out may be held to two where
+                                  this says three */
     int32_t lds_bytes;         /* dynamic LDS per workgroup of the row kernel, padded for that limit */
     int64_t algorithmic_bytes; /* (N+1)*T*H*e + H*e + T*H*e + OUT, OUT as documented for the quant mode */
     int64_t scale_elems;       /* number of fp32 scales written */

@@ -400,11 +400,14 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     // threshold itself the gain is small: 4 x [8192, 7168] with per-group scales 0.4 % on a device that has been under
     // load for 20 ms (0.9 % slower in the first milliseconds after idling).
     int wgs_per_cu = 0, wgs_held = 0; // reported, and what the launch is padded for
-    // The staged algorithms are limited only on request.  With owned rows, and in the norm phase alone, most rows read two streams.
-    // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more; two workgroups per CU against
-    // none planned: 8 x [16384, 8192] bf16 -> fp8 513.7 -> 497.8 us, 4 x [32768, 8192] 688.2 -> 628.3, 4 x [16384, 5120] 203.6 ->
-    // 200.2 (three: 200.1), 8 x [8192, 8192] 251.2 -> 246.4; at 2048 rows +0.4 to -0.4 %; rows of 256 vectors of four partials +11 to
-    // +14 % with two, -4 % with four at 16384 rows.
+    // Reported for fused launches only.  With owned rows, and in the norm phase alone, most rows read two streams, and a limit
+    // only costs (25 launches of four and eight partials: up to 50 %).
+    // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more.  From 16 workgroups per CU
+    // on four and eight partials gain from the same 128 KiB, counted with the stage's stores, but never more than four workgroups
+    // (56 launches of 4096 to 40188 rows: 2.0 % faster on average, none more than 0.4 % slower; without a limit against with): 8 x [32005, 2512] bf16 -> fp8 322.8 -> 304.2
+    // us (three), 8 x [32012, 1032] fp16 137.1 -> 126.0 (four), 8 x [4096, 3000] 51.8 -> 50.0 (two), 8 x [12091, 8192] 396 -> 381 (two),
+    // 4 x [30550, 748] fp32 114.5 -> 106.9 (four), 4 x [16384, 8192] 318.1 -> 313.4 (two).  Rows packed more than two to a workgroup
+    // lose up to 2 %, two partials with one vector per thread up to 19 % with two and gain nothing with four.
     const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED;
     if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
         const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
@@ -423,6 +426,10 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
         wgs_held = limit(8);
         const bool few_stores = p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0;
         if (vpt == 4 && few_stores && 2 * per_wg >= 96 * 1024) wgs_held = 2;
+    }
+    if (p->dtype != TDE_F64 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks >= 4 && rpb <= 2 && grid >= 16 * (int64_t)cus) {
+        const int64_t per_wg = (int64_t)rpb * (p->nranks + 2) * nvec * 16;
+        wgs_held = (int)std::min<int64_t>(4, std::max<int64_t>(2, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
     }
     if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_held = wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
