@@ -99,3 +99,14 @@ def test_rows_that_lost(dtype, n, nvec, tokens, quant, wn, vpt):
 ])
 def test_owned_row_lengths(n, nvec, tokens, quant, vpt):
     assert vecs(_capi.BF16, n, nvec, tokens, quant=quant, algo=_capi.ALGO_STAGED_OWNED) == vpt
+
+
+# Rows of eleven and twelve wavefronts on two partials: two of them fit a compute unit, so from a little beyond two rows per unit
+# several vectors per thread pay.
+@pytest.mark.parametrize("dtype,nvec,tokens,quant,wn,vpt", [
+    (_capi.BF16, 768, 543, FP8, 0, 1), (_capi.BF16, 768, 544, FP8, 0, 2), (_capi.F32, 641, 767, INT8, 1, 2), (_capi.BF16, 640, 544, FP8, 0, 1),
+    (_capi.BF16, 768, 543, STATIC, 1, 1), (_capi.BF16, 768, 544, STATIC, 1, 4), (_capi.BF16, 768, 1279, STATIC, 1, 4), (_capi.BF16, 650, 1024, STATIC, 1, 4),
+    (_capi.BF16, 650, 1025, STATIC, 1, 1), (_capi.BF16, 704, 767, GROUP, 1, 2), (_capi.F32, 704, 1200, GROUP, 1, 4), (_capi.BF16, 768, 600, STATIC, 0, 1),
+])
+def test_just_beyond_two_rows_per_unit(dtype, nvec, tokens, quant, wn, vpt):
+    assert vecs(dtype, 2, nvec, tokens, quant=quant, write_norm=wn, static_scale=0.5 if quant == STATIC else 0.0) == vpt

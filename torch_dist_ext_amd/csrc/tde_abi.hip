@@ -211,15 +211,23 @@ int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) 
     // to rows of whole lines; the rules say where two vectors were still no slower than one.
     const bool t_rows = p->write_norm != 0, lines = rows_of_whole_lines(nvec);
     if (!per_token) {
+        // Just beyond two rows per unit the wide workgroups of rows of eleven and twelve wavefronts no longer fit at once (two to a
+        // unit), and with T-typed rows beside the codes more vectors pay at once: 543 to 767 rows 5-16 %.  Four stay ahead of two
+        // up to 1279 rows, except per group in a 2-byte type: static -1 to +12 % (1257 rows of 768 vectors +3 %), fp32 per group
+        // 1-5 %; other row lengths lose 7 % from 1154 rows on.
+        if (waves >= 11 && t_rows && t >= 544 && t < 1280) {
+            if ((f32 || p->quant == TDE_QUANT_FP8_STATIC) && (lines || t < 1025)) return 4;
+            if (t < 768) return 2;
+        }
         // Long launches 1-14 % (with T-typed rows fp32 1-5 %, a 2-byte type at best nothing).  768 to 1280 rows of eleven and twelve
         // wavefronts -3 to +11 %, up to 1400 rows of them 0 to +3 %, fp32 2-12 %.
         if (waves >= 11 && t >= 768 && t < (f32 || !t_rows ? 1400 : (lines ? 1281 : 1025))) return 2;
         if (t < 4096 || !(waves == 9 || waves >= 11)) return 1;
         return !t_rows || (f32 && (waves < 12 || lines)) || (waves == 11 && lines) ? 2 : 1;
     }
-    if (waves >= 11) { // 2-18 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
+    if (waves >= 11) { // 2-18 %, 544 to 767 rows 3-27 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
         if (t_rows && !f32 && (waves >= 12 ? t >= 1408 : !lines && t >= 1537)) return 1;
-        return t >= 768 && (f32 || waves == 11 || t < 1536 || t >= 2304) ? 2 : 1;
+        return t >= 544 && (f32 || waves == 11 || t < 1536 || t >= 2304) ? 2 : 1;
     }
     if (waves == 9) { // 1-20 %; 2-byte types 1-6 % behind from 1344 to 1536 rows
         if (t_rows && !f32 && !lines && t >= 1344) return 1;
