@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "3756b1420ecc4e48b4c134d3c7c1b02b5e110584f9e509568f6debfd56cb92a5",
-    "bytes": {"c2": 11696277, "c3": 352658057, "c4": 765445425, "c5": 2181259183},
+    "sources_sha256": "8805655cb393b05ce0068af1470053bc277869830dcae0fe0fdd144142fd7bd8",
+    "bytes": {"c2": 11670521, "c3": 352603868, "c4": 765402984, "c5": 2181212142},
 }
 
 BENCH_CONFIGS = {
