@@ -517,33 +517,53 @@ __device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WA
     return sum;
 }
 
-// 1/h, correctly rounded for every row length.
-__device__ __forceinline__ float reciprocal_of_length(float h) {
-    const float r = __builtin_amdgcn_rcpf(h);
-    return __builtin_fmaf(__builtin_fmaf(-h, r, 1.0f), r, r);
+// 1/d from an approximation within one unit in the last place: correctly rounded unless d is all ones and the approximation
+// half a unit low (2^23 mantissas of d and both neighbours of 1/d, on the host: unit_test_rounding.cpp).
+__host__ __device__ __forceinline__ float refined_reciprocal(float d, float approx) {
+    return __builtin_fmaf(__builtin_fmaf(-d, approx, 1.0f), approx, approx);
 }
 
-// 1 / sqrt(sumsq / h + eps) with every step rounded as the IEEE operation (rcp_h: the correctly rounded 1/h).
-// The quotient by Markstein's correction (see div_shared), the root by his iteration on g ~ sqrt(m) and y ~ 1 / (2 sqrt(m))
-// ("Computation of elementary functions on the IBM RISC System/6000 processor", 1990), which leaves 1/sqrt(m) in 2y
-// for the reciprocal: 15 instructions where two divisions and a square root are 45.  Checked on gfx950 against
-// the plain operations for every m in [1, 4) -- powers of four only shift it -- and every h.  Outside [2^-60, 2^100], and
-// for NaN, the plain operations.  (Inside it no step underflows: a mean small enough for that leaves m == eps.)
-__device__ __forceinline__ float reciprocal_rms(float sumsq, float h, float rcp_h, float eps) {
-    const float q0 = sumsq * rcp_h;
-    const float m = __builtin_fmaf(-__builtin_fmaf(q0, h, -sumsq), rcp_h, q0) + eps;
-    constexpr uint32_t LOW = (127u - 60u) << 23, HIGH = (127u + 100u) << 23;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, m) - LOW > HIGH - LOW) != 0, 0))
-        return 1.0f / __builtin_sqrtf(sumsq / h + eps); // the same value in every lane
-    float y = __builtin_amdgcn_rsqf(m);
+// y / d, correctly rounded, for a divisor shared by many elements.  `rcp` must be the correctly
+// rounded 1/d.  q0 = RN(y*rcp) is within one ulp of the quotient; the residual y - q0*d is exact
+// in one fma; adding residual*rcp back in a second fma rounds to the correctly rounded quotient
+// (Markstein's division theorem) as long as nothing underflows.  Callers take this path only when
+// d is far from the subnormal and overflow ranges and use a plain division otherwise.
+// The residual is taken as q0*d - y and subtracted, not as y - q0*d and added: the same value for every non-zero y,
+// and for y = -0 the result is then -0 like the quotient's (the other form ends in (+0) + (-0) = +0).
+__host__ __device__ __forceinline__ float div_shared(float y, float d, float rcp) {
+    const float q0 = y * rcp;
+    const float e = __builtin_fmaf(q0, d, -y);
+    return __builtin_fmaf(-e, rcp, q0);
+}
+
+// 1/h, correctly rounded: no row length is all ones in 24 bits.
+__device__ __forceinline__ float reciprocal_of_length(float h) { return refined_reciprocal(h, __builtin_amdgcn_rcpf(h)); }
+
+// 1 / sqrt(m) with the root and its reciprocal each rounded as the IEEE operation, from y, an approximation of 1 / sqrt(m).
+// The root by Markstein's iteration on g ~ sqrt(m) and y ~ 1 / (2 sqrt(m)) ("Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990), which leaves 1/sqrt(m) in 2y.  That is not yet 1/g, which g's own rounding has moved by
+// up to half a unit: two steps of Newton's, or the reciprocal is a unit off for three of 2^24 mantissas.  They start a unit high:
+// below 1/g the last step ends in a tie for g all ones and rounds it down.  Right for every mantissa and every y up to three
+// units off (on the host, unit_test_rounding.cpp).
+__host__ __device__ __forceinline__ float reciprocal_of_root(float m, float y) {
     float g = m * y;
     y *= 0.5f;
     const float e = __builtin_fmaf(-y, g, 0.5f);
     g = __builtin_fmaf(g, e, g);
     y = __builtin_fmaf(y, e, y);
     g = __builtin_fmaf(__builtin_fmaf(-g, g, m), y, g); // sqrt(m)
-    const float r = y + y;
-    return __builtin_fmaf(__builtin_fmaf(-g, r, 1.0f), r, r);
+    return refined_reciprocal(g, refined_reciprocal(g, y * (2.0f + 0x1p-22f)));
+}
+
+// 1 / sqrt(sumsq / h + eps) with every step rounded as the IEEE operation (rcp_h: the correctly rounded 1/h).  17 instructions
+// where two divisions and a square root are 45.  Outside [2^-60, 2^100], and for NaN, the plain operations.  (Inside it no step
+// underflows: a mean small enough for that leaves m == eps.)
+__device__ __forceinline__ float reciprocal_rms(float sumsq, float h, float rcp_h, float eps) {
+    const float m = div_shared(sumsq, h, rcp_h) + eps;
+    constexpr uint32_t LOW = (127u - 60u) << 23, HIGH = (127u + 100u) << 23;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, m) - LOW > HIGH - LOW) != 0, 0))
+        return 1.0f / __builtin_sqrtf(sumsq / h + eps); // the same value in every lane
+    return reciprocal_of_root(m, __builtin_amdgcn_rsqf(m));
 }
 
 // Every buffer is device (global) memory: the few accesses that do not go through a buffer resource
@@ -601,19 +621,6 @@ __device__ __forceinline__ void pack_int8(const float (&q)[VEC], uint32_t (&out)
         const uint32_t hi = __builtin_amdgcn_perm(code(q[4 * w + 3]), code(q[4 * w + 2]), 0x04000c0cu);
         out[w] = lo | hi;
     }
-}
-
-// y / d, correctly rounded, for a divisor shared by many elements.  `rcp` must be the correctly
-// rounded 1/d.  q0 = RN(y*rcp) is within one ulp of the quotient; the residual y - q0*d is exact
-// in one fma; adding residual*rcp back in a second fma rounds to the correctly rounded quotient
-// (Markstein's division theorem) as long as nothing underflows.  Callers take this path only when
-// d is far from the subnormal and overflow ranges and use a plain division otherwise.
-// The residual is taken as q0*d - y and subtracted, not as y - q0*d and added: the same value for every non-zero y,
-// and for y = -0 the result is then -0 like the quotient's (the other form ends in (+0) + (-0) = +0).
-__device__ __forceinline__ float div_shared(float y, float d, float rcp) {
-    const float q0 = y * rcp;
-    const float e = __builtin_fmaf(q0, d, -y);
-    return __builtin_fmaf(-e, rcp, q0);
 }
 
 // What turns a row's elements into codes: the divisor, and its reciprocal in the form that quotient() takes.
