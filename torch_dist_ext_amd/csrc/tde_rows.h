@@ -214,6 +214,14 @@ __device__ __forceinline__ float read_lane(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 
+// A value that is the same in every lane.  SCALAR: in a scalar register (the compiler drops __builtin_amdgcn_readfirstlane of what it
+// knows to be uniform, and leaves that in a vector register).
+template <bool SCALAR>
+__device__ __forceinline__ float uniform_value(float v) {
+    if constexpr (SCALAR) asm("" : "+v"(v));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
     v = row16_max(v);
     const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
@@ -536,8 +544,16 @@ __host__ __device__ __forceinline__ float div_shared(float y, float d, float rcp
     return __builtin_fmaf(-e, rcp, q0);
 }
 
-// 1/h, correctly rounded: no row length is all ones in 24 bits.
-__device__ __forceinline__ float reciprocal_of_length(float h) { return refined_reciprocal(h, __builtin_amdgcn_rcpf(h)); }
+// A row's length and its reciprocal, correctly rounded (no row length is all ones in 24 bits), for reciprocal_rms.  They live
+// through the load phase.  SCALAR: in scalar registers, where the vector registers are all taken there.
+template <bool SCALAR = false>
+struct RowLength {
+    float h, rcp;
+    __device__ __forceinline__ explicit RowLength(int hidden) {
+        h = uniform_value<SCALAR>((float)hidden);
+        rcp = uniform_value<SCALAR>(refined_reciprocal(h, __builtin_amdgcn_rcpf(h)));
+    }
+};
 
 // 1 / sqrt(m) with the root and its reciprocal each rounded as the IEEE operation, from y, an approximation of 1 / sqrt(m).
 // The root by Markstein's iteration on g ~ sqrt(m) and y ~ 1 / (2 sqrt(m)) ("Computation of elementary functions on the IBM
@@ -555,14 +571,15 @@ __host__ __device__ __forceinline__ float reciprocal_of_root(float m, float y) {
     return refined_reciprocal(g, refined_reciprocal(g, y * (2.0f + 0x1p-22f)));
 }
 
-// 1 / sqrt(sumsq / h + eps) with every step rounded as the IEEE operation (rcp_h: the correctly rounded 1/h).  17 instructions
-// where two divisions and a square root are 45.  Outside [2^-60, 2^100], and for NaN, the plain operations.  (Inside it no step
+// 1 / sqrt(sumsq / length + eps) with every step rounded as the IEEE operation: 17 instructions where two divisions and a square
+// root are 45.  Outside [2^-60, 2^100], and for NaN, the plain operations.  (Inside it no step
 // underflows: a mean small enough for that leaves m == eps.)
-__device__ __forceinline__ float reciprocal_rms(float sumsq, float h, float rcp_h, float eps) {
-    const float m = div_shared(sumsq, h, rcp_h) + eps;
+template <class Length>
+__device__ __forceinline__ float reciprocal_rms(float sumsq, Length length, float eps) {
+    const float m = div_shared(sumsq, length.h, length.rcp) + eps;
     constexpr uint32_t LOW = (127u - 60u) << 23, HIGH = (127u + 100u) << 23;
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, m) - LOW > HIGH - LOW) != 0, 0))
-        return 1.0f / __builtin_sqrtf(sumsq / h + eps); // the same value in every lane
+        return 1.0f / __builtin_sqrtf(sumsq / length.h + eps); // the same value in every lane
     return reciprocal_of_root(m, __builtin_amdgcn_rsqf(m));
 }
 
@@ -823,7 +840,9 @@ __global__ void __launch_bounds__(1024 / VPT)
     const SumLayout<VPT, VEC, E::BYTES == 2> sums(lds_img, lds_bs, a.hidden(), tpr, a.rows_per_block, group);
     sumsq_clear(sums, TDE_T);
     if constexpr (Q == TDE_QUANT_FP8_TOKEN || Q == TDE_QUANT_INT8_TOKEN) lds_max[group] = 0u; // for row_max
-    const float rcp_h = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, reciprocal_of_length((float)a.hidden()))));
+    // Scalar registers for owned rows: with eight partials and four vectors per thread their 128 vector registers spilled one
+    // otherwise (4 bytes a lane to scratch and back; 8 x [2048, 8192] 27.32 -> 27.24 us).
+    const RowLength<OWNED> length(a.hidden());
 #define TDE_OFF(j) (lane0 + (uint32_t)(j) * vec_stride)
 
     {
@@ -974,7 +993,7 @@ __global__ void __launch_bounds__(1024 / VPT)
         }
         const int t_behind = TDE_T_BEHIND(xraw[VPT - 1][0]);
         const float sumsq = sumsq_torch_order(sums, t_behind, tpr, wave - first_wave, t_behind & (kWave - 1));
-        const float rs = reciprocal_rms(sumsq, (float)a.hidden(), rcp_h, a.eps);
+        const float rs = reciprocal_rms(sumsq, length, a.eps);
 
         // ---- normalize ------------------------------------------------------------------------------
         constexpr bool DYNAMIC = Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC;

@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
 
     const SumLayout<VPT, 2, false> sums(lds_img, lds_bs, a.hidden(), tpr, a.rows_per_block, group);
     sumsq_clear(sums, t);
-    const float rcp_h = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, reciprocal_of_length((float)a.hidden()))));
+    const RowLength<> length(a.hidden());
 
     // The partials are summed rank by rank, as they arrive.
     double acc[VPT][2];
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     }
     const int t_behind = VPT == 1 ? t : not_before(t, landed);
     const float sumsq = sumsq_torch_order(sums, t_behind, tpr, 0, t_behind & (kWave - 1));
-    const float rs = reciprocal_rms(sumsq, (float)a.hidden(), rcp_h, a.eps);
+    const float rs = reciprocal_rms(sumsq, length, a.eps);
 
     const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
 #pragma unroll
