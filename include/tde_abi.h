@@ -133,16 +133,15 @@ typedef struct tde_plan_out {
     int32_t grid_blocks;     /* workgroups launched for the row kernel */
     int32_t xcd_chunk;       /* row groups each XCD takes in a row: workgroup b of every 8*xcd_chunk takes row group
                                 (b % 8) * xcd_chunk + b / 8 of that span (1 = launch order) */
-    int32_t workgroups_per_cu; /* limit on resident workgroups per compute unit the launch enforces through its LDS
-                                  (0 = none); below a requested tune_workgroups_per_cu where the geometry's own LDS
-                                  already admits fewer.  Also 2, without LDS padding, where the plan picks the row
-                                  kernel built for two wavefronts per SIMD (eight partials, four vectors per thread,
-                                  4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its registers admit two.
-                                  0 for the staged algorithms unless asked for, though long launches of
-                                  TDE_ALGO_STAGED are held to two to four.  Long launches of four partials whose
-                                  dynamic-scale codes are all they store beside residual_out may be held to two where
-                                  this says three */
-    int32_t lds_bytes;         /* dynamic LDS per workgroup of the row kernel, padded for that limit */
+    int32_t workgroups_per_cu; /* limit on resident workgroups per compute unit that the launch of tde_reduce_rms enforces
+                                  through its LDS (0 = none); below a requested tune_workgroups_per_cu where the
+                                  geometry's own LDS already admits fewer.  Also 2, without LDS padding, where the
+                                  plan picks the row kernel built for two wavefronts per SIMD (eight partials, four
+                                  vectors per thread, 4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its
+                                  registers admit two.  For TDE_ALGO_STAGED it belongs to the one launch that stores the
+                                  stage; where that call needs two launches, neither is limited unless asked to, and
+                                  TDE_ALGO_STAGED_OWNED only if asked to */
+    int32_t lds_bytes;         /* dynamic LDS per workgroup of that launch, padded for that limit */
     int64_t algorithmic_bytes; /* (N+1)*T*H*e + H*e + T*H*e + OUT, OUT as documented for the quant mode */
     int64_t scale_elems;       /* number of fp32 scales written */
 } tde_plan_out;

@@ -307,22 +307,38 @@ def test_plan_vectors_per_thread(kw, vpt, threads):
 
 
 @pytest.mark.parametrize("kw,limit,lds", [
-    # fewer than 6144 workgroups, two partials, the staged algorithms and doubles: no limit, LDS = what the reduction needs
+    # fewer than 6144 workgroups, two partials, owned rows and doubles: no limit, LDS = what the reduction needs
     # (eight partials at 1024 to 6143 workgroups: the kernel for two wavefronts per SIMD, reported as 2, no LDS padding)
     (dict(nranks=8, tokens=1023, hidden=8192), 0, (256 * 4 * 8 + 1024) * 4),
     (dict(nranks=4, tokens=6143, hidden=8192), 0, (256 * 4 * 8 + 1024) * 4),
     (dict(nranks=2, tokens=32768, hidden=8192), 0, (256 * 4 * 8 + 1024) * 4),
-    (dict(nranks=8, tokens=32768, hidden=8192, algo=_capi.ALGO_STAGED), 0, (256 * 4 * 8 + 1024) * 4),
-    # long launches: about 128 KiB of loads in flight per CU, never fewer than two workgroups or eight wavefronts
+    (dict(nranks=8, tokens=32768, hidden=8192, algo=_capi.ALGO_STAGED_OWNED), 0, (256 * 4 * 8 + 1024) * 4),
+    # long launches: about 128 KiB of loads in flight per CU, never fewer than two workgroups, nor than eight wavefronts with
+    # T-typed rows to store (two workgroups with 96 KiB of loads where dynamic-scale codes are all beside residual_out)
     (dict(nranks=8, tokens=6144, hidden=8192), 2, 80896),                                    # 144 KiB per workgroup
     (dict(nranks=4, tokens=32768, hidden=8192), 2, 80896),                                   # 80 KiB per workgroup
-    (dict(nranks=4, tokens=32768, hidden=5120, dtype=_capi.F16, quant=_capi.QUANT_INT8_TOKEN), 3, 53504),  # 3 wavefronts each
-    (dict(nranks=4, tokens=8192, hidden=7168, quant=_capi.QUANT_FP8_GROUP), 3, 53504),      # twelve wavefronts for group scales
+    (dict(nranks=4, tokens=32768, hidden=5120, dtype=_capi.F16, quant=_capi.QUANT_INT8_TOKEN), 2, 80896),  # 3 wavefronts each
+    (dict(nranks=4, tokens=32768, hidden=5120, dtype=_capi.F16, quant=_capi.QUANT_INT8_TOKEN, write_norm=1), 3, 53504),
+    (dict(nranks=4, tokens=32768, hidden=4904, quant=_capi.QUANT_FP8_TOKEN, vecs_per_thread=4), 3, 53504),      # rows of 613 vectors: 95.8 KiB
+    (dict(nranks=4, tokens=32768, hidden=4920, quant=_capi.QUANT_FP8_TOKEN, vecs_per_thread=4), 2, 80896),      # 615 vectors: 96.1 KiB
+    (dict(nranks=4, tokens=8192, hidden=7168, quant=_capi.QUANT_FP8_GROUP), 2, 80896),
+    (dict(nranks=4, tokens=8192, hidden=7168, quant=_capi.QUANT_FP8_GROUP, write_norm=1), 2, 80896),
     (dict(nranks=4, tokens=8192, hidden=7168, quant=_capi.QUANT_FP8_TOKEN), 2, 80896),
     (dict(nranks=4, tokens=8191, hidden=7168, quant=_capi.QUANT_FP8_TOKEN), 0, (256 * 4 * 8 + 1024) * 4),   # four partials: from 8192
     (dict(nranks=8, tokens=32768, hidden=1024), 4, 39936),                                   # 2 rows x 18 KiB per workgroup
     (dict(nranks=4, tokens=16384, hidden=2048), 6, 26112),
     (dict(nranks=8, tokens=32768, hidden=2048, dtype=_capi.F64), 0, (1024 * 2 + 1024) * 4),   # doubles: 2 per vector, 1024 threads
+    # the stage stored by the same launch: from 16 workgroups per CU, at most four of them, rows packed at most two to a workgroup
+    (dict(nranks=8, tokens=32768, hidden=8192, algo=_capi.ALGO_STAGED), 2, 80896),
+    (dict(nranks=8, tokens=4096, hidden=8192, algo=_capi.ALGO_STAGED), 2, 80896),
+    (dict(nranks=8, tokens=4095, hidden=8192, algo=_capi.ALGO_STAGED), 0, (256 * 4 * 8 + 1024) * 4),
+    (dict(nranks=8, tokens=32005, hidden=2512, quant=_capi.QUANT_FP8_TOKEN, algo=_capi.ALGO_STAGED), 3, 53504),
+    (dict(nranks=8, tokens=32012, hidden=1032, dtype=_capi.F16, algo=_capi.ALGO_STAGED), 4, 39936),
+    (dict(nranks=4, tokens=8197, hidden=520, algo=_capi.ALGO_STAGED), 4, 39936),              # two rows to a workgroup
+    (dict(nranks=4, tokens=8190, hidden=520, algo=_capi.ALGO_STAGED), 0, (256 * 8 + 1024) * 4),
+    (dict(nranks=4, tokens=65536, hidden=512, algo=_capi.ALGO_STAGED), 0, (256 * 8 + 1024) * 4),   # four rows to a workgroup
+    (dict(nranks=2, tokens=32768, hidden=8192, algo=_capi.ALGO_STAGED), 0, (256 * 4 * 8 + 1024) * 4),
+    (dict(nranks=8, tokens=32768, hidden=8192, algo=_capi.ALGO_STAGED, workgroups_per_cu=-1), 0, (256 * 4 * 8 + 1024) * 4),
     # the per-call override
     (dict(nranks=8, tokens=16, hidden=1024, workgroups_per_cu=1), 1, 162816),
     (dict(nranks=8, tokens=16, hidden=1024, workgroups_per_cu=8), 8, 19456),

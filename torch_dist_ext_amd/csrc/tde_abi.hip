@@ -402,44 +402,40 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     // Resident workgroups per compute unit.  Left alone, a CU takes as many workgroups as its registers and LDS hold
     // (3-6 here), each with all of its rows' loads in flight.  On MI355X long launches run fastest with 120-160 KiB
     // of loads in flight per CU: more costs 1-8 % from 8192 rows up with 4 or 8 partials (32768 x 8192: 7.5 % with
-    // 4 partials, 4.5 % with 8; 16384 rows: 1-3 %; 8192 rows with 8 partials: 1 %), fewer than two workgroups or
-    // eight wavefronts per CU leave the arithmetic of one row uncovered by the loads of another.  Short launches (a
-    // few generations of workgroups) gain nothing and can lose 1-3 %, and with 2 partials no limit helps.  At the
-    // threshold itself the gain is small: 4 x [8192, 7168] with per-group scales 0.4 % on a device that has been under
-    // load for 20 ms (0.9 % slower in the first milliseconds after idling).
-    int wgs_per_cu = 0, wgs_held = 0; // reported, and what the launch is padded for
-    // Reported for fused launches only.  With owned rows, and in the norm phase alone, most rows read two streams, and a limit
-    // only costs (25 launches of four and eight partials: up to 50 %).
+    // 4 partials, 4.5 % with 8; 16384 rows: 1-3 %; 8192 rows with 8 partials: 1 %), fewer than two workgroups, or than
+    // eight wavefronts that have T-typed rows to store, leave the arithmetic of one row uncovered by the loads of another.
+    // Short launches (a few generations of workgroups) gain nothing and can lose 1-3 %, and with 2 partials no limit helps.
+    // Eight wavefronts are enough for per-group scales on four partials too (two workgroups against three): 4 x [8192, 7168]
+    // bf16 119.3 us against 123.2, 4 x [12000, 8192] 198.4 against 205.9, 4 x [32768, 7168] fp16 467 against 503, fp32
+    // 4 x [9000, 3584] 124.9 against 127.0.
+    const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED;
+    int wgs_per_cu = 0;
+    if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
+        const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
+        const int waves = tpr * rpb / 64;
+        const int at_least = std::max(2, (8 + waves - 1) / waves);
+        wgs_per_cu = (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        // Two workgroups are enough, six wavefronts among them, wherever two have 96 KiB of loads in flight and only codes of a
+        // dynamic scale beside residual_out to store, with four vectors per thread: 4 x [32768, 5120] fp16 -> int8 338.2 us against
+        // 342.3 with three, bf16 -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three
+        // stay 3 % ahead.  Among the plan's own choices that is rows of 640 vectors on four partials; longer rows, and eight
+        // partials, have two already.
+        const bool few_stores = p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0;
+        if (vpt == 4 && few_stores && 2 * per_wg >= 96 * 1024) wgs_per_cu = 2;
+    }
     // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more.  From 16 workgroups per CU
     // on four and eight partials gain from the same 128 KiB, counted with the stage's stores, but never more than four workgroups
     // (56 launches of 4096 to 40188 rows: 2.0 % faster on average, none more than 0.4 % slower; without a limit against with): 8 x [32005, 2512] bf16 -> fp8 322.8 -> 304.2
     // us (three), 8 x [32012, 1032] fp16 137.1 -> 126.0 (four), 8 x [4096, 3000] 51.8 -> 50.0 (two), 8 x [12091, 8192] 396 -> 381 (two),
     // 4 x [30550, 748] fp32 114.5 -> 106.9 (four), 4 x [16384, 8192] 318.1 -> 313.4 (two).  Rows packed more than two to a workgroup
     // lose up to 2 %, two partials with one vector per thread up to 19 % with two and gain nothing with four.
-    const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED;
-    if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
-        const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
-        const int waves = tpr * rpb / 64;
-        const auto limit = [&](int need_waves) {
-            const int at_least = std::max(2, (need_waves + waves - 1) / waves);
-            return (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
-        };
-        // Per-group scales on four partials are reported as held to twelve wavefronts, what their arithmetic once took, and held
-        // to eight like the others (rows of more than 768 vectors: two workgroups instead of three): 4 x [8192, 7168] bf16
-        // 119.3 us against 123.2, 4 x [12000, 8192] 198.4 against 205.9, 4 x [32768, 7168] fp16 467 against 503, fp32 4 x [9000, 3584]
-        // 124.9 against 127.0.  Two are enough wherever two have 96 KiB of loads in flight and only codes of a dynamic scale beside
-        // residual_out to store, with four vectors per thread: 4 x [32768, 5120] fp16 -> int8 338.2 us against 342.3 with three, bf16
-        // -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three stay 3 % ahead.
-        wgs_per_cu = limit(p->quant == TDE_QUANT_FP8_GROUP && p->nranks <= 4 ? 12 : 8);
-        wgs_held = limit(8);
-        const bool few_stores = p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0;
-        if (vpt == 4 && few_stores && 2 * per_wg >= 96 * 1024) wgs_held = 2;
-    }
+    // With owned rows, and in the norm phase alone, most rows read two streams, and a limit only costs (25 launches of four and
+    // eight partials: up to 50 %).
     if (p->dtype != TDE_F64 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks >= 4 && rpb <= 2 && grid >= 16 * (int64_t)cus) {
         const int64_t per_wg = (int64_t)rpb * (p->nranks + 2) * nvec * 16;
-        wgs_held = (int)std::min<int64_t>(4, std::max<int64_t>(2, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        wgs_per_cu = (int)std::min<int64_t>(4, std::max<int64_t>(2, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
     }
-    if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_held = wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
+    if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
     if (geo) {
         geo->wgs_per_cu = wgs_per_cu;
@@ -451,7 +447,6 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
             geo->wgs_per_cu = (int)std::min<size_t>((size_t)wgs_per_cu, tde::kLdsPerCu / (lds + 64));
         }
         geo->lds_bytes = (int)lds;
-        geo->launch_lds = wgs_held > 0 ? std::max(lds, tde::lds_bytes_for_workgroups_per_cu(wgs_held)) : lds;
         geo->vec_elems = vec;
         geo->nvec = (int)nvec;
         geo->vpt = vpt;

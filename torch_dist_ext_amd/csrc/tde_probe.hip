@@ -81,7 +81,7 @@ hipError_t launch_traffic_nv(int code_bytes, bool wn, const RowArgs &a, const Ge
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     // The LDS the row kernel of this geometry allocates (never touched here), padding included, and its
     // wavefronts-per-SIMD bound: the skeleton then fills a compute unit with as many workgroups as the kernel does.
-    const size_t lds = g.launch_lds;
+    const size_t lds = (size_t)g.lds_bytes;
 #define TDE_TRAFFIC(CB, WNB)                                                                   \
     if (lds > kDefaultMaxDynamicLds) {                                                         \
         const hipError_t e = allow_large_lds<traffic_kernel<N, VPT, CB, WNB>>();               \

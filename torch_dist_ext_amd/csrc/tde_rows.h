@@ -1199,8 +1199,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
 // ---------------------------------------------------------------------------------------------
 struct Geometry {
     int wgs_per_cu; // limit on resident workgroups per compute unit (0 = none), enforced through lds_bytes
-    int lds_bytes;  // dynamic LDS as reported: the row kernel's own, padded for wgs_per_cu
-    size_t launch_lds; // dynamic LDS of the row kernel's launch, at least that much
+    int lds_bytes;  // dynamic LDS of the row kernel's launch: its own, padded for wgs_per_cu
     int vec_elems;
     int nvec;
     int vpt;
@@ -1232,7 +1231,7 @@ hipError_t launch_traffic(int n, int vpt, int code_bytes, bool wn, const RowArgs
 template <class E, int N, int VPT>
 hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
-    const size_t lds = g.launch_lds; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
+    const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
 #define TDE_LAUNCH_FORM(QM, WNB, FORM)                                                                   \
     {                                                                                                    \
         if (lds > kDefaultMaxDynamicLds) {                                                               \
