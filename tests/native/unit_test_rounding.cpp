@@ -99,5 +99,32 @@ int main() {
         }
         return false;
     });
+    // Codes of 2-byte elements: the elements of 11 bits on both sides of every boundary (those of 8 bits are among these, and the
+    // quotient grows with y).  The boundaries of fp8 codes are those of int8 codes times powers of two, which only shift it; the
+    // divisors are taken at the ends of the fast range too.  All ones in d: from 1/d as it is correctly rounded, which is what the
+    // instruction gives (test_codes_of_every_element_gpu.py has that divisor); from the float below, 2^k / d would be a tie.
+    const auto side = [](float q, float b) { return q < b ? -1 : (q > b ? 1 : 0); };
+    for (int shift : {0, -60, 59}) {
+        const uint32_t step = shift == 0 ? 1 : 61;
+        sweep("codes of 2-byte elements", (1u << 23) / step + 1, [&, shift, step](uint32_t i) {
+            const uint32_t mantissa = i * step < 0x7fffffu ? i * step : 0x7fffffu;
+            const float d = std::ldexp(value(0x3f800000u + mantissa), shift);
+            float approx[2];
+            around_reciprocal(d, approx);
+            if (mantissa == 0x7fffffu) approx[0] = approx[1] = 1.0f / d;
+            for (float start : approx) {
+                const tde::Divisor<tde::ElemF16> divisor(d, start);
+                for (float b : boundaries) {
+                    const uint32_t below = bits(b * d) & ~0x1fffu; // 10 bits behind the leading one
+                    for (uint32_t off : {0u, 0x2000u}) {
+                        const float y = value(below + off);
+                        if (side(divisor.quotient(y), b) != side(y / d, b)) return true;
+                    }
+                }
+                if (bits(divisor.quotient(-0.0f)) != 0x80000000u || divisor.quotient(-INFINITY) != -INFINITY || divisor.quotient(INFINITY) != INFINITY) return true;
+            }
+            return false;
+        });
+    }
     return failed;
 }

@@ -29,7 +29,6 @@ namespace tde {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -646,19 +645,20 @@ __device__ __forceinline__ void pack_int8(const float (&q)[VEC], uint32_t (&out)
 // boundary, which has at most 8: the product with a reciprocal in two words, rounded once, gives the same codes as the
 // correctly rounded quotient in two instructions instead of three.  Its relative error of 2^-44 could only matter where y lies
 // within 2^5 units (of 49 bits) of (2 M +- 1) * d for a boundary M; with d = j 2^20 + r (2^17 for int8) that needs
-// M r = -+j with M >= 16 >= j (128), i.e. all ones in d, and even there no code differs (every mantissa of d
-// against every y of 8 and of 11 bits over the range of the codes, both code types, on gfx950).  hi is below 1/d by more than
-// half a unit and lo > 0: a numerator of -0 keeps its sign, and of infinity its infinity.
+// M r = -+j with M >= 16 >= j (128), i.e. all ones in d, and even there no code differs as long as the approximation is 1/d
+// correctly rounded, which gfx950's is (test_codes_of_every_element_gpu.py).  hi is below 1/d by more than half a unit and lo > 0:
+// a numerator of -0 keeps its sign, and of infinity its infinity.  (On the host, for every other mantissa of d, both neighbours
+// of 1/d as the approximation and the elements beside every boundary: unit_test_rounding.cpp.)
 // fp32 elements take the correctly rounded quotient (div_shared).
 template <class E>
 struct Divisor {
     float d, hi, lo; // fp32 elements: hi is 1/d correctly rounded
 
     Divisor() = default;
-    __device__ __forceinline__ explicit Divisor(float d_) {
+    __device__ __forceinline__ explicit Divisor(float d_) : Divisor(d_, __builtin_amdgcn_rcpf(d_)) {}
+    __host__ __device__ __forceinline__ Divisor(float d_, float approx) {
         d = d_;
-        const float r0 = __builtin_amdgcn_rcpf(d);
-        const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.0f), r0, r0); // 1/d, correctly rounded (every mantissa checked)
+        const float r = refined_reciprocal(d, approx);
         if constexpr (E::BYTES == 2) {
             hi = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) - 1u);
             lo = __builtin_fmaf(-d, hi, 1.0f) * r;
@@ -667,7 +667,7 @@ struct Divisor {
             lo = 0.0f;
         }
     }
-    __device__ __forceinline__ float quotient(float y) const {
+    __host__ __device__ __forceinline__ float quotient(float y) const {
         if constexpr (E::BYTES == 2) return __builtin_fmaf(y, hi, y * lo);
         else return div_shared(y, d, hi);
     }
