@@ -110,3 +110,12 @@ def test_owned_row_lengths(n, nvec, tokens, quant, vpt):
 ])
 def test_just_beyond_two_rows_per_unit(dtype, nvec, tokens, quant, wn, vpt):
     assert vecs(dtype, 2, nvec, tokens, quant=quant, write_norm=wn, static_scale=0.5 if quant == STATIC else 0.0) == vpt
+
+
+# Beside T-typed rows of fp32, two vectors per thread with twelve wavefronts were slower than one at 590 to 700 rows; four are not.
+@pytest.mark.parametrize("nvec,tokens,quant,wn,vpt", [
+    (768, 543, FP8, 1, 1), (768, 544, FP8, 1, 4), (768, 640, INT8, 1, 4), (705, 640, FP8, 1, 4), (704, 640, FP8, 1, 2), (768, 767, FP8, 1, 4),
+    (768, 768, FP8, 1, 2), (768, 640, FP8, 0, 2),
+])
+def test_twelve_wavefronts_beside_rows_of_fp32(nvec, tokens, quant, wn, vpt):
+    assert vecs(_capi.F32, 2, nvec, tokens, quant=quant, write_norm=wn) == vpt

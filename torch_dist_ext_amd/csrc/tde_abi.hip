@@ -225,7 +225,11 @@ int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) 
         if (t < 4096 || !(waves == 9 || waves >= 11)) return 1;
         return !t_rows || (f32 && (waves < 12 || lines)) || (waves == 11 && lines) ? 2 : 1;
     }
-    if (waves >= 11) { // 2-18 %, 544 to 767 rows 3-27 %; 768 vectors of a 2-byte type +1 to +2 % around 2000 rows
+    if (waves >= 11) { // two 2-18 % faster, 544 to 767 rows up to 22 %; 768 vectors of a 2-byte type 1-2 % slower around 2000 rows
+        // fp32 beside T-typed rows: with twelve wavefronts two are up to 6 % slower than one from 590 to 700 rows (768 vectors, 640
+        // rows: 9.06 us with one, 9.54 with two, 8.19 with four), four 7-21 % faster over the whole band; with eleven two lose nowhere
+        // (704 vectors, 640 rows -7 %).  From 768 rows on two are 17 % faster to 4 % slower than one.
+        if (t_rows && f32 && waves >= 12 && t >= 544 && t < 768) return 4;
         if (t_rows && !f32 && (waves >= 12 ? t >= 1408 : !lines && t >= 1537)) return 1;
         return t >= 544 && (f32 || waves == 11 || t < 1536 || t >= 2304) ? 2 : 1;
     }
