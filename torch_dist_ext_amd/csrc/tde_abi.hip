@@ -212,15 +212,22 @@ int vecs_per_thread_few_partials(const tde_problem *p, int64_t nvec, int64_t t) 
     const bool t_rows = p->write_norm != 0, lines = rows_of_whole_lines(nvec);
     if (!per_token) {
         // Just beyond two rows per unit the wide workgroups of rows of eleven and twelve wavefronts no longer fit at once (two to a
-        // unit), and with T-typed rows beside the codes more vectors pay at once: 543 to 767 rows 5-16 %.  Four stay ahead of two
-        // up to 1279 rows, except per group in a 2-byte type: static -1 to +12 % (1257 rows of 768 vectors +3 %), fp32 per group
-        // 1-5 %; other row lengths lose 7 % from 1154 rows on.
+        // unit), and with T-typed rows beside the codes more vectors pay at once.  Time against one vector per thread, two | four,
+        // rows of 650, 704 and 768 vectors:
+        //   static, 2-byte    544 rows -2 to -6 % | +1 to -8 %, 704 -13 % | -11 %, 767 -14 to -18 % | -12 to -17 %, 896 +3 % | -10 %,
+        //                     1024 -1 to -7 % | -13 to -18 %, 1154 +4 % | +4 %, 1257 and 1280 rows of whole lines -1 to -5 % | -5 to -7 %,
+        //                     others +2 % | +1 %
+        //   static, fp32      544 to 704 rows -5 to +8 % | -5 to -14 %, 767 -3 to -8 % | -15 to -22 %, 1024 -3 % | -3 to -12 %, 1154 +4 % | +4 %,
+        //                     1257 and 1280 -1 to -3 % | -1 to -5 %
+        //   group, fp32       544 to 704 rows +7 to -14 % | -7 to -16 %, 767 -7 to -20 % | -20 %, 1024 -4 % | -12 %, 1154 +2 % | +3 %, 1280 -4 % | -7 %
+        //   group, 2-byte     544 to 704 rows 0 to -15 % | -2 to -11 %, 767 -14 % | -14 %, 1024 -6 % | -11 %, 1280 -4 % | -5 %
         if (waves >= 11 && t_rows && t >= 544 && t < 1280) {
             if ((f32 || p->quant == TDE_QUANT_FP8_STATIC) && (lines || t < 1025)) return 4;
             if (t < 768) return 2;
         }
-        // Long launches 1-14 % (with T-typed rows fp32 1-5 %, a 2-byte type at best nothing).  768 to 1280 rows of eleven and twelve
-        // wavefronts -3 to +11 %, up to 1400 rows of them 0 to +3 %, fp32 2-12 %.
+        // Long launches 1-14 % faster with two (with T-typed rows fp32 1-5 %, a 2-byte type at best nothing).  Rows of eleven and
+        // twelve wavefronts: 768 rows 10-15 % faster with two (fp32 up to 9 %), 1024 3-5 %, 1280 2-5 %, around 900 and 1100 rows up to 2 %
+        // slower, 1344 to 1400 -1 to +2 %, fp32 0 to -4 %.
         if (waves >= 11 && t >= 768 && t < (f32 || !t_rows ? 1400 : (lines ? 1281 : 1025))) return 2;
         if (t < 4096 || !(waves == 9 || waves >= 11)) return 1;
         return !t_rows || (f32 && (waves < 12 || lines)) || (waves == 11 && lines) ? 2 : 1;

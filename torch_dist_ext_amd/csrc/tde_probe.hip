@@ -87,8 +87,7 @@ hipError_t launch_traffic_nv(int code_bytes, bool wn, const RowArgs &a, const Ge
         const hipError_t e = allow_large_lds<traffic_kernel<N, VPT, CB, WNB>>();               \
         if (e != hipSuccess) return e;                                                         \
     }                                                                                          \
-    hipLaunchKernelGGL((traffic_kernel<N, VPT, CB, WNB>), grid, block, lds, s, a, row_bytes, parts); \
-    return hipGetLastError();
+    return launch_kernel<traffic_kernel<N, VPT, CB, WNB>>(grid, block, lds, s, a, row_bytes, parts);
     if (code_bytes == 0) { TDE_TRAFFIC(0, true) }
     if (code_bytes == 8) { if (wn) { TDE_TRAFFIC(8, true) } else { TDE_TRAFFIC(8, false) } }
     if (code_bytes == 4) { if (wn) { TDE_TRAFFIC(4, true) } else { TDE_TRAFFIC(4, false) } }
