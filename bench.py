@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "8805655cb393b05ce0068af1470053bc277869830dcae0fe0fdd144142fd7bd8",
-    "bytes": {"c2": 11670521, "c3": 352603868, "c4": 765402984, "c5": 2181212142},
+    "sources_sha256": "8d4c2f12e440286f073e14373880d5f201b28c1b14b11f0103bd937051b29b45",
+    "bytes": {"c2": 11670827, "c3": 352602770, "c4": 765406431, "c5": 2181214650},
 }
 
 BENCH_CONFIGS = {
