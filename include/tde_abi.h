@@ -129,7 +129,8 @@ typedef struct tde_plan_out {
     int32_t block_threads;   /* threads per workgroup (multiple of 64) */
     int32_t vecs_per_thread; /* 16-byte vectors each thread owns per row, in the launch of tde_reduce_rms (the norm phase
                                 alone, tde_stage_norm, may take another choice) */
-    int32_t rows_per_block;  /* rows a workgroup processes side by side (one wave group per row) */
+    int32_t rows_per_block;  /* rows a workgroup processes side by side: one wave group per row, or two or four rows to a
+                                wavefront (rows of up to 32 vectors) */
     int32_t grid_blocks;     /* workgroups launched for the row kernel */
     int32_t xcd_chunk;       /* row groups each XCD takes in a row: workgroup b of every 8*xcd_chunk takes row group
                                 (b % 8) * xcd_chunk + b / 8 of that span (1 = launch order) */

@@ -369,8 +369,21 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alo
     return vpt;
 }
 
-// `norm_alone`: the geometry of a launch that only norms the rows of the stage.
-int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) {
+// Rows that share a wavefront (tde_short_rows.hip) against one wavefront each (row_kernel), 1400 launches of 1 to 60000 rows: up to 16
+// vectors 4-15 % faster below 4096 rows, 30 % from there and 35-55 % from 16384 rows on (2 x [30046, 152] bf16 -> fp8 15.2 -> 9.3 us); 17
+// to 32 vectors 3-8 % faster below 8192 rows and there, where memory begins to bind, 20 % faster to 3 % slower with two and four
+// partials (2 x [40459, 192] 18.2 -> 13.5, 4 x [28759, 192] 14.5 -> 14.8).  Eight partials keep memory busy either way: from 8192
+// rows of more than 20 vectors on one row to a wavefront is up to 5 % faster (up to 20 vectors 2-8 % slower).  Owned rows, and the norm
+// phase alone, read two buffers for most rows and gain at any length (8 x [45945, 144] 23.4 -> 17.2).
+bool share_a_wavefront(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alone) {
+    if (p->dtype == TDE_F64 || nvec > tde::kShortRowVecs) return false;
+    return nvec <= 20 || p->nranks < 8 || t < 8192 || p->algo == TDE_ALGO_STAGED_OWNED || norm_alone;
+}
+
+// `launch`: what the geometry is for.
+enum Launch { kWhole, kNormAlone /* norms the rows of the stage */, kSkeleton /* the traffic probe: row_kernel's geometry */ };
+int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
+    const bool norm_alone = launch == kNormAlone;
     if (p == nullptr) return TDE_EINVAL;
     const int eb = elem_bytes(p->dtype);
     if (eb == 0) return TDE_EDTYPE;
@@ -399,14 +412,17 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
     }
     if (p->tune_rows_per_block < 0) return TDE_EINVAL;
     if (p->tune_workgroups_per_cu < -1 || p->tune_workgroups_per_cu > 8 || p->reserved != 0) return TDE_EINVAL;
+    const bool short_rows = launch != kSkeleton && p->tune_vecs_per_thread == 0 && p->tune_rows_per_block == 0 && share_a_wavefront(p, nvec, t, norm_alone);
     const int64_t lanes = (nvec + vpt - 1) / vpt;
-    const int tpr = (int)((lanes + 63) / 64 * 64);
-    int rpb = 256 / tpr; // pack short rows so a workgroup has at least four wavefronts
+    const int tpr = short_rows ? (nvec <= 16 ? 16 : 32) : (int)((lanes + 63) / 64 * 64);
+    // pack short rows so a workgroup has at least four wavefronts (two of two rows each: 1 % faster than four)
+    int rpb = (tpr == 32 ? 128 : 256) / tpr;
     if (rpb * tpr > kMaxBlock / vpt) rpb = (kMaxBlock / vpt) / tpr; // never beyond the kernel's launch bound
-    while (rpb > 1 && (p->tokens + rpb - 1) / rpb < 2 * cus) rpb /= 2; // keep every CU busy first
-    if (rpb < 1) rpb = 1;
+    const int least = std::max(1, tde::kWave / tpr); // whole wavefronts
+    while (rpb > least && (p->tokens + rpb - 1) / rpb < 2 * cus) rpb /= 2; // keep every CU busy first
+    if (rpb < least) rpb = least;
     if (p->tune_rows_per_block > 0 && p->tune_rows_per_block * tpr <= kMaxBlock / vpt) rpb = p->tune_rows_per_block;
-    if (p->tokens > 0 && rpb > p->tokens) rpb = (int)p->tokens;
+    if (p->tokens > 0 && rpb > p->tokens && !short_rows) rpb = (int)p->tokens;
     const int64_t grid = (p->tokens + rpb - 1) / rpb; // one workgroup per group of rows, no loop
     if (grid > 0x7fffffff) return TDE_ESHAPE;
 
@@ -450,7 +466,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) 
 
     if (geo) {
         geo->wgs_per_cu = wgs_per_cu;
-        size_t lds = tde::sumsq_lds_bytes(tpr * rpb, vpt, vec);
+        size_t lds = short_rows ? tde::short_rows_lds_bytes(tpr * rpb, rpb, vec) : tde::sumsq_lds_bytes(tpr * rpb, vpt, vec);
         if (wgs_per_cu > 0) {
             lds = std::max(lds, tde::lds_bytes_for_workgroups_per_cu(wgs_per_cu)); // never with doubles
             // what the launch enforces: a geometry whose own LDS is larger than the padding admits fewer still
@@ -666,7 +682,7 @@ bool phases_overlap(const tde_problem *p, const tde_buffers *b) {
 
 int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int phases, int probe_parts = 7) {
     tde::Geometry g{};
-    const int st = validate(p, &g);
+    const int st = validate(p, &g, phases == kTrafficOnly ? kSkeleton : kWhole);
     if (st != TDE_OK) return st;
     if (b == nullptr) return TDE_EINVAL;
     if (p->tokens == 0) return TDE_OK; // nothing to do; empty buffers may be null
@@ -710,7 +726,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     // been stored; so do partials that only a device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
     const bool one_launch = staged && both && !from_table && !phases_overlap(p, b);
     if (staged && !one_launch) {
-        const int alone = validate(p, &g, true);
+        const int alone = validate(p, &g, kNormAlone);
         if (alone != TDE_OK) return alone;
     }
 
@@ -726,13 +742,13 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     const uint64_t table = reinterpret_cast<uint64_t>(b->partial_table);
     a.set(tde::kPtrResidualIn, b->residual_in);
     a.set(tde::kPtrResidualOut, b->residual_out);
-    a.set(tde::kPtrNorm, b->norm_out);
+    a.set(tde::kPtrNorm, wn ? b->norm_out : nullptr);
     a.set(tde::kPtrGamma, b->gamma);
     a.set(tde::kPtrCodes, b->q_out);
     a.set(tde::kPtrScale, b->scale_out);
     a.set_hidden(p->hidden);
     a.threads_per_row = (uint16_t)g.threads_per_row;
-    a.wave_step = (uint16_t)(32768 / (g.threads_per_row / tde::kWave) + 1);
+    a.wave_step = (uint16_t)(32768 / std::max(1, g.threads_per_row / tde::kWave) + 1);
     a.rows_per_block = (uint8_t)g.rows_per_block;
     a.xcd_chunk = (uint8_t)g.xcd_chunk;
     a.tokens = p->tokens;
@@ -776,6 +792,10 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
         a.table_mask = 0;
         a.set(tde::kPtrPart, b->stage);
         n = 0;
+    }
+    if (g.threads_per_row < tde::kWave) {
+        e = tde::launch_short_rows(p->dtype, n, p->quant, a, g, stream);
+        return e == hipSuccess ? TDE_OK : hip_fail(e);
     }
     switch (p->dtype) {
     case TDE_BF16: e = tde::launch_rows_bf16(n, g.vpt, p->quant, wn, a, g, stream); break;

@@ -47,7 +47,7 @@ enum : int { kPtrPart = 0, kPtrResidualIn = kMaxKernelRanks, kPtrResidualOut, kP
 struct RowArgs {
     uint32_t lo[kPtrs];
     uint32_t hi[(kPtrs + 1) / 2]; // two per word; the last half word is `hidden`
-    uint16_t threads_per_row;     // multiple of 64
+    uint16_t threads_per_row;     // multiple of 64; short rows (tde_short_rows.hip): 16 or 32 lanes of a wavefront
     uint8_t rows_per_block;       // at most 16
     uint8_t xcd_chunk;            // workgroups per XCD chunk of the row mapping (power of two; 0 or 1 = rows in launch order)
     int64_t tokens;
@@ -673,6 +673,78 @@ struct Divisor {
     }
 };
 
+// T(gamma * T(x * rs)) of one vector.
+template <class E>
+__device__ __forceinline__ u32x4 normed(u32x4 xraw, u32x4 gamma_raw, float rs) {
+    constexpr int VEC = E::VEC;
+    float x[VEC], g[VEC], n[VEC];
+    E::unpack(xraw, x);
+    E::unpack(gamma_raw, g);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
+    E::unpack(E::pack(n), n);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
+    return E::pack(n);
+}
+
+// The largest code of a mode.
+template <int Q>
+constexpr float kQuantMax = Q == TDE_QUANT_INT8_TOKEN ? 127.0f : 448.0f;
+
+// The dynamic scales of a thread's vectors from the bit patterns of their largest magnitudes.  Returns one wavefront-uniform decision
+// for all of them, so the common path carries no per-lane branch: whether every divisor is far from the subnormal and overflow
+// ranges, as its quotients need.  A largest magnitude that is NaN or infinite takes the plain division too.
+template <int Q, int SCALES>
+__device__ __forceinline__ bool scales_of_largest(uint32_t (&m)[SCALES], float (&scale)[SCALES]) {
+    constexpr float QMAX = kQuantMax<Q>;
+    uint64_t unsafe = 0;
+    constexpr uint32_t LOW = (127u - 50u) << 23, HIGH = (127u + 60u) << 23; // 2^-50 to 2^60
+#pragma unroll
+    for (int j = 0; j < SCALES; ++j)
+        unsafe |= __builtin_amdgcn_ballot_w64(m[j] - LOW > HIGH - LOW) & __builtin_amdgcn_ballot_w64(m[j] != 0u);
+    const bool fast = unsafe == 0;
+#pragma unroll
+    for (int j = 0; j < SCALES; ++j) scale[j] = div_shared(__builtin_bit_cast(float, m[j]), QMAX, 1.0f / QMAX);
+    if (__builtin_expect(!fast, 0)) {
+#pragma unroll
+        for (int j = 0; j < SCALES; ++j) {
+            asm volatile("; not computed beside the fast one" : "+v"(m[j]));
+            scale[j] = __builtin_bit_cast(float, m[j]) / QMAX;
+        }
+    }
+    return fast;
+}
+__device__ __forceinline__ bool static_scale_is_fast(float scale) {
+    return __builtin_amdgcn_readfirstlane(scale >= 0x1p-60f && scale <= 0x1p60f) != 0;
+}
+
+// The codes of one vector's elements.  FAST: `divisor` is div's; otherwise the plain division.
+template <class E, int Q, bool FAST>
+__device__ __forceinline__ void codes_of(const float (&y)[E::VEC], const Divisor<E> &divisor, float div, uint32_t (&codes)[E::VEC / 4]) {
+    constexpr int VEC = E::VEC;
+    constexpr float QMAX = kQuantMax<Q>;
+    float q[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        float v = y[i];
+        // A caller's scale can be far below the row's values (the dynamic scales cannot: |y| <= QMAX * scale).
+        // Beyond twice the largest code the quotient clamps to QMAX whatever it is, so where its correction
+        // would see inf - inf, y is cut there.
+        if constexpr (Q == TDE_QUANT_FP8_STATIC && FAST && E::BYTES != 2) v = clamp_keep_nan(v, 2.0f * QMAX * div);
+        if constexpr (FAST) v = divisor.quotient(v);
+        else v = v / div;
+        // Dynamic scales: the quotient is within 1e-4 of +-QMAX at most, which the conversions below round to
+        // the largest code; nothing to clamp
+        if constexpr (!FAST || Q == TDE_QUANT_FP8_STATIC) v = clamp_keep_nan(v, QMAX);
+        q[i] = v;
+    }
+    if constexpr (Q == TDE_QUANT_INT8_TOKEN)
+        pack_int8<VEC, FAST>(q, codes);
+    else
+        pack_fp8<VEC>(q, codes);
+}
+
 // Which row group a workgroup takes.  Workgroups are handed to the 8 XCDs round-robin, so in launch order
 // every XCD (every L2) walks all of every buffer in 16 KiB steps.  Remapped in groups of 8*chunk, XCD k
 // instead takes `chunk` consecutive row groups of each group, i.e. a contiguous piece of every buffer:
@@ -1032,11 +1104,7 @@ __global__ void __launch_bounds__(1024 / VPT)
 
         // ---- quant epilogue -------------------------------------------------------------------------
         if constexpr (Q != TDE_QUANT_NONE) {
-            constexpr float QMAX = (Q == TDE_QUANT_INT8_TOKEN) ? 127.0f : 448.0f;
             constexpr int SCALES = Q == TDE_QUANT_FP8_GROUP ? VPT : 1; // a thread's vectors lie in groups of their own
-            // One wavefront-uniform decision for all of the thread's vectors, so the common path carries no per-lane branch: its
-            // quotients need every divisor far from the subnormal and overflow ranges.  A largest magnitude that is NaN or infinite
-            // also takes the plain division.
             float scale[SCALES];
             bool fast;
             if constexpr (DYNAMIC) {
@@ -1052,24 +1120,10 @@ __global__ void __launch_bounds__(1024 / VPT)
                     for (int j = 1; j < VPT; ++j) amax[0] = max_abs(amax[0], amax[j], amax[j]);
                     m[0] = row_max(__builtin_bit_cast(uint32_t, amax[0]) & 0x7fffffffu, lds_max + group, TDE_LANE, waves_per_row);
                 }
-                uint64_t unsafe = 0;
-                constexpr uint32_t LOW = (127u - 50u) << 23, HIGH = (127u + 60u) << 23; // 2^-50 to 2^60
-#pragma unroll
-                for (int j = 0; j < SCALES; ++j)
-                    unsafe |= __builtin_amdgcn_ballot_w64(m[j] - LOW > HIGH - LOW) & __builtin_amdgcn_ballot_w64(m[j] != 0u);
-                fast = unsafe == 0;
-#pragma unroll
-                for (int j = 0; j < SCALES; ++j) scale[j] = div_shared(__builtin_bit_cast(float, m[j]), QMAX, 1.0f / QMAX);
-                if (__builtin_expect(!fast, 0)) {
-#pragma unroll
-                    for (int j = 0; j < SCALES; ++j) {
-                        asm volatile("; not computed beside the fast one" : "+v"(m[j]));
-                        scale[j] = __builtin_bit_cast(float, m[j]) / QMAX;
-                    }
-                }
+                fast = scales_of_largest<Q>(m, scale);
             } else {
                 scale[0] = a.static_scale;
-                fast = __builtin_amdgcn_readfirstlane(scale[0] >= 0x1p-60f && scale[0] <= 0x1p60f) != 0;
+                fast = static_scale_is_fast(a.static_scale);
             }
             if constexpr (Q == TDE_QUANT_FP8_GROUP) {
                 constexpr int LANES_PER_GROUP = TDE_QUANT_GROUP / VEC; // 16 (2-byte types) or 32 (fp32)
@@ -1097,26 +1151,8 @@ __global__ void __launch_bounds__(1024 / VPT)
                     const float sc = scale[SCALES == 1 ? 0 : j];
                     const float div = (Q == TDE_QUANT_FP8_STATIC || sc > 0.0f) ? sc : 1.0f;
                     if (FAST && (SCALES > 1 || j == 0)) divisor = Divisor<E>(div);
-                    float q[VEC];
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) {
-                        float v = y[j][i];
-                        // A caller's scale can be far below the row's values (the dynamic scales cannot: |y| <= QMAX * scale).
-                        // Beyond twice the largest code the quotient clamps to QMAX whatever it is, so where its correction
-                        // would see inf - inf, y is cut there.
-                        if constexpr (Q == TDE_QUANT_FP8_STATIC && FAST && E::BYTES != 2) v = clamp_keep_nan(v, 2.0f * QMAX * div);
-                        if constexpr (FAST) v = divisor.quotient(v);
-                        else v = v / div;
-                        // Dynamic scales: the quotient is within 1e-4 of +-QMAX at most, which the conversions below round to
-                        // the largest code; nothing to clamp
-                        if constexpr (!FAST || Q == TDE_QUANT_FP8_STATIC) v = clamp_keep_nan(v, QMAX);
-                        q[i] = v;
-                    }
                     uint32_t codes[VEC / 4];
-                    if constexpr (Q == TDE_QUANT_INT8_TOKEN)
-                        pack_int8<VEC, FAST>(q, codes);
-                    else
-                        pack_fp8<VEC>(q, codes);
+                    codes_of<E, Q, FAST>(y[j], divisor, div, codes);
                     const uint32_t code_off = (TDE_OFF(j) / 16u) * (uint32_t)VEC;
                     if constexpr (VEC == 8) {
                         const u32x2 w = {codes[0], codes[1]};
@@ -1203,7 +1239,7 @@ struct Geometry {
     int vec_elems;
     int nvec;
     int vpt;
-    int threads_per_row;
+    int threads_per_row; // below 64: short rows, several to a wavefront
     int rows_per_block;
     int block_threads;
     int64_t grid;
@@ -1218,6 +1254,14 @@ hipError_t launch_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, con
 hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
+
+// Rows of up to 32 vectors, several to a wavefront (tde_short_rows.hip; not doubles).  The normed rows go where the arguments have a
+// buffer for them.
+constexpr int kShortRowVecs = 32;
+inline size_t short_rows_lds_bytes(int block_threads, int rows_per_block, int vec_floats) {
+    return ((size_t)block_threads * vec_floats + (size_t)rows_per_block * 32) * sizeof(float);
+}
+hipError_t launch_short_rows(int dtype, int n, int q, const RowArgs &a, const Geometry &g, hipStream_t s);
 
 // Rows of doubles (tde_rows_f64.hip): no quantized output.
 hipError_t launch_rows_f64(int n, const RowArgs &a, const Geometry &g, hipStream_t s);
