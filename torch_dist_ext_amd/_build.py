@@ -23,7 +23,8 @@ HIP_LIB = os.path.join(PKG_DIR, "libtde_hip.so")
 TORCH_LIB = os.path.join(ROOT, "libtorch_dist_ext.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["tde_abi.hip", "tde_rows_bf16.hip", "tde_rows_f16.hip", "tde_rows_f32.hip", "tde_rows_f64.hip", "tde_short_rows.hip", "tde_probe.hip"]
+HIP_SOURCES = ["tde_abi.hip", "tde_rows_bf16.hip", "tde_rows_f16.hip", "tde_rows_f32.hip", "tde_rows_f64.hip", "tde_shifted_rows_bf16.hip", "tde_shifted_rows_f16.hip",
+               "tde_shifted_rows_f32.hip", "tde_short_rows.hip", "tde_probe.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     # keep fp32 arithmetic scalar: packed fp32 forms are not used on this hardware pool
@@ -60,7 +61,7 @@ def build_hip(verbose=False):
             print(out)
         return obj
 
-    with ThreadPoolExecutor(max_workers=7) as pool:
+    with ThreadPoolExecutor(max_workers=8) as pool:
         objs = list(pool.map(compile_one, HIP_SOURCES))
     # only the C ABI is exported: a second copy of this library in the process (another version, a build under test)
     # then runs its own launchers and kernels, not the first one's

@@ -380,6 +380,53 @@ bool share_a_wavefront(const tde_problem *p, int64_t nvec, int64_t t, bool norm_
     return nvec <= 20 || p->nranks < 8 || t < 8192 || p->algo == TDE_ALGO_STAGED_OWNED || norm_alone;
 }
 
+// Megabytes that a launch moves in T-typed rows, roughly: what the rules for shifted rows go by.
+int64_t row_megabytes(const tde_problem *p, int64_t nvec) {
+    const int64_t streams = p->algo == TDE_ALGO_STAGED_OWNED ? 4 : p->nranks + 2; // an owned launch reads two streams for most rows
+    return (streams * p->tokens * nvec) >> 16;
+}
+
+// Vectors of a line of the narrowest buffer that counts.
+int line_vectors(const tde_problem *p) { return p->quant == TDE_QUANT_NONE ? 8 : (p->dtype == TDE_F32 ? 32 : 16); }
+
+// Whether rows that start inside a line are moved along their threads (tde_rows.h: SHIFTED).  A launch pays 0.07 us for it (the row
+// is known before its addresses are) and, with 2-byte types, another barrier ahead of the sums; what it gains is 2-8 % of its
+// time in memory.  From 3000 launches of 5 to 2200 MB in place and shifted, the same vectors per thread: 10 MB +1.5 %, 20 MB
+// 0 to +0.5 %, 40 MB -1.5 % (single ones up to +3.5 % with two and four partials of one vector per thread), 100 MB -2.2 %,
+// from 300 MB on -3.3 % (2 x [31779, 3256] bf16 -> static fp8 and T-typed rows 198.4 -> 183.3 us, 4 x [26096, 962] doubles staged
+// 285 -> 255, 2 x [30413, 4008] fp32 -> int8 375 -> 323).  Two wavefronts a row: 0 to -0.5 %, 2-byte types nothing.  Eight partials of a 2-byte type, one
+// vector per thread: owned rows +0.2 %, up to four wavefronts a row with workgroups limited per unit +0.3 %.
+// Rows of whole T-typed lines whose codes start inside lines: two partials -1 to -3 %, others nothing.
+bool rows_are_shifted(const tde_problem *p, int64_t nvec, int64_t t, int vpt) {
+    const bool owned = p->algo == TDE_ALGO_STAGED_OWNED, staged = p->algo == TDE_ALGO_STAGED, few = p->nranks <= 4;
+    const int line = p->nranks == 2 && !staged && !owned ? line_vectors(p) : 8;
+    if (nvec % line == 0 || nvec <= tde::kWave) return false;
+    const int64_t mb = row_megabytes(p, nvec);
+    if (elem_bytes(p->dtype) > 2) return mb >= (nvec <= 128 ? 56 : 32);
+    if (nvec <= 128) return false;
+    if (!few && vpt == 1 && (owned || (nvec <= 256 && t >= kLimitFromWorkgroupsPerCu8 * 256))) return false;
+    return mb >= (owned || (vpt == 1 && few) ? 56 : 28);
+}
+
+// Vectors per thread where rows are shifted and the lengths that vecs_per_thread was swept at do not speak for them (same launches; against
+// its choice).
+int vecs_per_thread_shifted(const tde_problem *p, int64_t nvec, int64_t t, int vpt) {
+    const int waves = (int)((nvec + 63) / 64);
+    const bool none = p->quant == TDE_QUANT_NONE;
+    if (p->dtype == TDE_F64 || p->algo == TDE_ALGO_STAGED) return vpt;
+    if (p->algo == TDE_ALGO_STAGED_OWNED) return p->nranks >= 8 && vpt == 1 && waves >= 5 && waves <= 10 && t >= 1200 ? 2 : vpt; // 1-12 %
+    if (p->nranks == 2) {
+        if (!none && waves >= 13 && t >= 2560) return 2; // 2 % over four
+        if (none && waves >= 15 && t >= 8192) return 1; // 2-3 % over four
+    } else if (p->nranks == 4) {
+        if (waves == 15 && vpt == 4 && t <= 2048) return 2; // 2 %
+    } else if (vpt == 1) {
+        if (waves == 9 || (waves == 6 && !none)) return t >= 8192 ? 2 : 1; // 2-5 %
+        if (nvec >= 600) return t >= 2048 ? 4 : 1;                          // 1-3 %; shorter rows leave four's lanes too empty
+    }
+    return vpt;
+}
+
 // `launch`: what the geometry is for.
 enum Launch { kWhole, kNormAlone /* norms the rows of the stage */, kSkeleton /* the traffic probe: row_kernel's geometry */ };
 int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
@@ -406,6 +453,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     const int cus = compute_units(); // once a call: asking the runtime for the device takes it 50 ns
     const int64_t t = rows_as_on_256_units(p->tokens, cus);
     int vpt = p->dtype != TDE_F64 ? vecs_per_thread(p, nvec, t, norm_alone) : (norm_alone ? vecs_per_thread_f64_norm(nvec, t) : vecs_per_thread_f64(p, nvec, t));
+    if (!norm_alone && rows_are_shifted(p, nvec, t, 4)) vpt = vecs_per_thread_shifted(p, nvec, t, vpt);
     if (p->tune_vecs_per_thread != 0) {
         if (p->tune_vecs_per_thread != 1 && p->tune_vecs_per_thread != 2 && p->tune_vecs_per_thread != 4) return TDE_EINVAL;
         vpt = p->tune_vecs_per_thread;
@@ -481,6 +529,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         geo->rows_per_block = rpb;
         geo->block_threads = tpr * rpb;
         geo->grid = grid;
+        geo->line_mask = !short_rows && !norm_alone && rows_are_shifted(p, nvec, t, vpt) ? line_vectors(p) - 1 : 0;
         // Row groups per XCD chunk of the row mapping (tde_rows.h: xcd_chunked_block); 16 measured best with 8
         // partials, 8 with 4.
         geo->xcd_chunk = p->nranks >= 8 ? 16 : 8;
@@ -756,6 +805,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     a.static_scale = p->static_scale;
     a.chunked_blocks = tde::chunked_blocks(g.grid, (uint32_t)g.xcd_chunk);
     a.owner = (uint8_t)p->rank;
+    a.line_mask = (uint8_t)(traffic ? 0 : g.line_mask);
 
     int n = p->nranks;
     hipError_t e = hipSuccess;
@@ -797,10 +847,11 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
         e = tde::launch_short_rows(p->dtype, n, p->quant, a, g, stream);
         return e == hipSuccess ? TDE_OK : hip_fail(e);
     }
+    const bool shifted = a.line_mask != 0;
     switch (p->dtype) {
-    case TDE_BF16: e = tde::launch_rows_bf16(n, g.vpt, p->quant, wn, a, g, stream); break;
-    case TDE_F16: e = tde::launch_rows_f16(n, g.vpt, p->quant, wn, a, g, stream); break;
-    case TDE_F32: e = tde::launch_rows_f32(n, g.vpt, p->quant, wn, a, g, stream); break;
+    case TDE_BF16: e = (shifted ? tde::launch_shifted_rows_bf16 : tde::launch_rows_bf16)(n, g.vpt, p->quant, wn, a, g, stream); break;
+    case TDE_F16: e = (shifted ? tde::launch_shifted_rows_f16 : tde::launch_rows_f16)(n, g.vpt, p->quant, wn, a, g, stream); break;
+    case TDE_F32: e = (shifted ? tde::launch_shifted_rows_f32 : tde::launch_rows_f32)(n, g.vpt, p->quant, wn, a, g, stream); break;
     case TDE_F64: e = tde::launch_rows_f64(n, a, g, stream); break;
     }
     if (e != hipSuccess) return hip_fail(e);

@@ -54,7 +54,8 @@ struct RowArgs {
     float eps;
     float static_scale;
     uint32_t chunked_blocks; // workgroups the XCD mapping permutes: the whole groups of 8 * xcd_chunk of the grid
-    uint8_t owner;           // OWNED row kernels: rows == owner (mod N) are summed here, the others are read from the stage
+    uint8_t owner : 3;       // OWNED row kernels: rows == owner (mod N) are summed here, the others are read from the stage
+    uint8_t line_mask : 5;   // row_shift()
     uint8_t table_mask;      // bit r: partial r's address is entry r of a device pointer table.  The table's own address
                              // stands in the stage's place: a launch has one or the other
     uint16_t wave_step; // 32768 / wavefronts per row + 1: row_group()
@@ -67,6 +68,10 @@ struct RowArgs {
     // first load)
     __host__ __device__ int row_group(int wave) const { return wave * wave_step >> 15; }
     __host__ __device__ int hidden() const { return (int)(hi[kPtrs >> 1] >> 16); }
+    // By how many vectors the row that starts at byte `row_byte` is moved along its threads (SHIFTED row kernels): thread t of the
+    // row group takes vectors (t - shift) mod threads_per_row first.  line_mask: how many vectors a 128-byte line of the
+    // narrowest buffer holds, less one (7 of T-typed rows, 15 or 31 of codes); 0: rows stay in place.
+    __host__ __device__ int row_shift(int64_t row_byte) const { return (int)((uint32_t)row_byte >> 4 & line_mask); }
     void set(int i, const void *p) {
         const uint64_t v = reinterpret_cast<uint64_t>(p);
         lo[i] = (uint32_t)v;
@@ -452,14 +457,17 @@ __device__ __forceinline__ void row_barrier(int waves_per_row) {
 // After every thread of the row group has put its squares: the sum, the same value in every thread.
 // Contains workgroup barriers when a row spans several wavefronts: all threads of the workgroup must call it together.
 // wave: the wavefront's number in its row group.
-template <int VPT, int VECF, bool WAVE_BLOCKS>
+// t, lane: the thread's place in its row group and wavefront.  SHIFTED: the row may be moved along its threads (RowArgs::row_shift).
+template <bool SHIFTED, int VPT, int VECF, bool WAVE_BLOCKS>
 __device__ __forceinline__ float sumsq_torch_order(const SumLayout<VPT, VECF, WAVE_BLOCKS> &s, int t, int tpr, int wave, int lane) {
     const int waves_per_row = tpr >> 6;
     const int cl = lane & 31;
     if constexpr (WAVE_BLOCKS) {
         static_assert(VECF == 8, "one wavefront load = one block of 64 eight-float vectors");
-        // Block j * waves_per_row + wave is what this wavefront wrote for its vector j: no other wavefront is involved.
-        wave_lds_fence();
+        // Block j * waves_per_row + wave is what this wavefront wrote for its vector j: no other wavefront is involved, unless
+        // the row has been moved.
+        if constexpr (SHIFTED) row_barrier(waves_per_row);
+        else wave_lds_fence();
         if constexpr (VPT == 1) {
             // one block per wavefront: both of its halves sum it
             s.bs[wave * 32 + cl] = chain_block_sum<false>(s.img + 512 * wave, cl, 16);
@@ -791,6 +799,27 @@ struct RowLoads {
     u32x4 r[VPT];
 };
 
+// SHIFTED kernels, rows of which start anywhere in a line of memory.  In place, thread t takes vectors t, t + tpr, ... of its row, and what
+// each of the row's wavefronts loads and stores begins inside a line whose other part is a neighbour's: nine lines of memory for
+// eight lines' worth of data, and stores that are merged, or not, with another wavefront's.  So the row is moved along its threads
+// until its wavefronts begin on lines (RowArgs::row_shift), the vectors that fall off the end on the first threads; the row's
+// own first and last line are all it still shares.
+// Rates in memory, in place -> moved -> the next longer row of whole lines, 12000 rows of 511 vectors: 2 x doubles 5.88 -> 6.26 -> 6.30 TB/s,
+// 2 x bf16 5.79 -> 6.14 -> 6.23, 2 x bf16 -> fp8 5.82 -> 6.22 -> 6.27, 4 x fp32 6.10 -> 6.37 -> 6.40, 4 x bf16 -> fp8 staged 5.95 -> 6.25 -> 6.30.
+// As a template parameter: the same code without it, a shift of zero, costs launches of whole lines 0.07 us.
+template <bool SHIFTED>
+__device__ __forceinline__ int first_vector_of(int thread, int shift, int tpr) {
+    if constexpr (!SHIFTED) return thread;
+    const int v = thread - shift;
+    return v < 0 ? v + tpr : v;
+}
+template <bool SHIFTED>
+__device__ __forceinline__ int thread_of(int first_vector, int shift, int tpr) {
+    if constexpr (!SHIFTED) return first_vector;
+    const int t = first_vector + shift;
+    return t >= tpr ? t - tpr : t;
+}
+
 // ---------------------------------------------------------------------------------------------
 // The row kernel.
 //   E      element traits
@@ -805,12 +834,14 @@ struct RowLoads {
 //          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
 //          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
 //          partials and their sums stored to the stage, every other row's sum is read from the stage
+//   SHIFTED rows that are not whole lines of memory, in launches long enough to gain from it (rows_are_shifted)
 // Block layout: rows_per_block row groups of threads_per_row threads; thread t of a row group
-// owns vectors t, t + threads_per_row, ... (coalesced 1 KiB per wavefront per load).
+// owns vectors t, t + threads_per_row, ... (coalesced 1 KiB per wavefront per load) of its row,
+// moved along the threads by row_shift() vectors where the row does not start on a line of memory.
 // ---------------------------------------------------------------------------------------------
 enum : int { kFormPlain = 0, kFormWide = 1, kFormStaged = 2, kFormOwned = 3 };
 
-template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain>
+template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain, bool SHIFTED = false>
 __global__ void __launch_bounds__(1024 / VPT)
     __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))))))
     row_kernel(const RowArgs a) {
@@ -838,15 +869,24 @@ __global__ void __launch_bounds__(1024 / VPT)
     const void *part[NP];
     partial_addresses(a, a.address(kPtrStage), part);
 
+    // One workgroup, one group of rows: the grid covers every row (no loop; a looping wavefront waits for its
+    // own stores, a fresh workgroup does not).
+    int64_t row = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block + group;
+    bool sum_is_new = FORM == kFormStaged; // the row's sums go to the stage as well
+    if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
+
+    // Thread t of the row group owns vectors t, t + tpr, ... of the row, which is first moved along the threads.
+    const int shift = SHIFTED ? a.row_shift(row * (int64_t)row_bytes) : 0;
+    const int t_row = first_vector_of<SHIFTED>(tid - group * tpr, shift, tpr);
     uint32_t lane_off[VPT]; // byte offset of this thread's vector j inside a row
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) lane_off[j] = (uint32_t)(j * tpr + tid - group * tpr) * 16u;
-// Thread index inside the row group and lane index, rebuilt from the first load offset where they are needed:
+    for (int j = 0; j < VPT; ++j) lane_off[j] = (uint32_t)(j * tpr + t_row) * 16u;
+// The row's first vector of this thread and the lane index, rebuilt from the first load offset where they are needed:
 // the thread id itself does not stay in a register through the load phase, which has none to spare.
 #define TDE_T ((int)(lane0 >> 4))
 // The same, not before `after` is there: with several vectors per thread the row loads leave no registers for LDS addresses.
 #define TDE_T_BEHIND(after) (VPT == 1 ? TDE_T : not_before(TDE_T, after))
-#define TDE_LANE ((int)(lane0 >> 4) & (kWave - 1))
+#define TDE_LANE (((int)(lane0 >> 4) + shift) & (kWave - 1))
 
     auto issue_loads = [&](RowLoads<NP, VPT> &d, int64_t row) {
         const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
@@ -863,10 +903,6 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
         for (int j = 0; j < VPT; ++j) d.r[j] = rsrc_load16(rr, lane_off[j]);
     };
-
-    // One workgroup, one group of rows: the grid covers every row (no loop; a looping wavefront waits for its
-    // own stores, a fresh workgroup does not).
-    const int64_t row0 = (int64_t)xcd_chunked_block(blockIdx.x, a.chunked_blocks, a.xcd_chunk) * a.rows_per_block;
 
     // The row's loads go out before anything else touches memory -- except gamma where it pays to have it first:
     // with up to four partials of a 2-byte type, several vectors per thread and a dynamic scale, the registers are
@@ -894,9 +930,6 @@ __global__ void __launch_bounds__(1024 / VPT)
         __builtin_amdgcn_sched_barrier(0);
     }
     RowLoads<NP, VPT> cur;
-    int64_t row = row0 + group;
-    bool sum_is_new = FORM == kFormStaged; // the row's sums go to the stage as well
-    if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
     issue_loads(cur, row);
     u32x4 gamma_early = u32x4{0, 0, 0, 0};
     if constexpr (VPT == 1) {
@@ -1063,8 +1096,8 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
             for (int j = 0; j < VPT; ++j) rsrc_store16(stage, TDE_OFF(j), sraw[j]);
         }
-        const int t_behind = TDE_T_BEHIND(xraw[VPT - 1][0]);
-        const float sumsq = sumsq_torch_order(sums, t_behind, tpr, wave - first_wave, t_behind & (kWave - 1));
+        const int t_behind = thread_of<SHIFTED>(TDE_T_BEHIND(xraw[VPT - 1][0]), shift, tpr);
+        const float sumsq = sumsq_torch_order<SHIFTED>(sums, t_behind, tpr, wave - first_wave, t_behind & (kWave - 1));
         const float rs = reciprocal_rms(sumsq, length, a.eps);
 
         // ---- normalize ------------------------------------------------------------------------------
@@ -1244,6 +1277,7 @@ struct Geometry {
     int block_threads;
     int64_t grid;
     int xcd_chunk;
+    int line_mask; // RowArgs::line_mask
     int form;  // which instantiation of the row kernel (kFormPlain, kFormWide, kFormStaged, kFormOwned)
 };
 
@@ -1251,6 +1285,10 @@ struct Geometry {
 hipError_t launch_rows_bf16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_rows_f16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
+// The same for rows that are moved along their threads (a.line_mask), in tde_shifted_rows_<dtype>.hip; n != 0, no per-group scales.
+hipError_t launch_shifted_rows_bf16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
+hipError_t launch_shifted_rows_f16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
+hipError_t launch_shifted_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
@@ -1272,17 +1310,17 @@ hipError_t launch_traffic(int n, int vpt, int code_bytes, bool wn, const RowArgs
                           hipStream_t s);
 
 // Instantiation + dispatch body used by the three per-dtype translation units.
-template <class E, int N, int VPT>
+template <class E, bool SHIFTED, int N, int VPT>
 hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes of this geometry, padded where the launch limits workgroups per CU
 #define TDE_LAUNCH_FORM(QM, WNB, FORM)                                                                   \
     {                                                                                                    \
         if (lds > kDefaultMaxDynamicLds) {                                                               \
-            const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB, FORM>>();                \
+            const hipError_t e = allow_large_lds<row_kernel<E, N, VPT, QM, WNB, FORM, SHIFTED>>();       \
             if (e != hipSuccess) return e;                                                               \
         }                                                                                                \
-        return launch_kernel<row_kernel<E, N, VPT, QM, WNB, FORM>>(grid, block, lds, s, a);              \
+        return launch_kernel<row_kernel<E, N, VPT, QM, WNB, FORM, SHIFTED>>(grid, block, lds, s, a);     \
     }
 #define TDE_LAUNCH(QM, WNB)                                                                              \
     if constexpr (N == 8 && VPT == 4) {                                                                  \
@@ -1298,7 +1336,10 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
     case TDE_QUANT_FP8_TOKEN:
         if (wn) { TDE_LAUNCH(TDE_QUANT_FP8_TOKEN, true) } else { TDE_LAUNCH(TDE_QUANT_FP8_TOKEN, false) }
     case TDE_QUANT_FP8_GROUP:
-        if (wn) { TDE_LAUNCH(TDE_QUANT_FP8_GROUP, true) } else { TDE_LAUNCH(TDE_QUANT_FP8_GROUP, false) }
+        if constexpr (!SHIFTED) { // rows of whole groups are whole lines
+            if (wn) { TDE_LAUNCH(TDE_QUANT_FP8_GROUP, true) } else { TDE_LAUNCH(TDE_QUANT_FP8_GROUP, false) }
+        }
+        break;
     case TDE_QUANT_INT8_TOKEN:
         if (wn) { TDE_LAUNCH(TDE_QUANT_INT8_TOKEN, true) } else { TDE_LAUNCH(TDE_QUANT_INT8_TOKEN, false) }
     case TDE_QUANT_FP8_STATIC:
@@ -1309,21 +1350,23 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
     return hipErrorInvalidValue;
 }
 
-template <class E, int N>
+template <class E, bool SHIFTED, int N>
 hipError_t launch_rows_n(int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
-    if (vpt == 1) return launch_rows_nv<E, N, 1>(q, wn, a, g, s);
-    if (vpt == 2) return launch_rows_nv<E, N, 2>(q, wn, a, g, s);
-    if (vpt == 4) return launch_rows_nv<E, N, 4>(q, wn, a, g, s);
+    if (vpt == 1) return launch_rows_nv<E, SHIFTED, N, 1>(q, wn, a, g, s);
+    if (vpt == 2) return launch_rows_nv<E, SHIFTED, N, 2>(q, wn, a, g, s);
+    if (vpt == 4) return launch_rows_nv<E, SHIFTED, N, 4>(q, wn, a, g, s);
     return hipErrorInvalidValue;
 }
 
-template <class E>
+template <class E, bool SHIFTED>
 hipError_t launch_rows_e(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
     switch (n) {
-    case 0: return launch_rows_n<E, 0>(vpt, q, wn, a, g, s);
-    case 2: return launch_rows_n<E, 2>(vpt, q, wn, a, g, s);
-    case 4: return launch_rows_n<E, 4>(vpt, q, wn, a, g, s);
-    case 8: return launch_rows_n<E, 8>(vpt, q, wn, a, g, s);
+    case 0:
+        if constexpr (!SHIFTED) return launch_rows_n<E, false, 0>(vpt, q, wn, a, g, s);
+        break;
+    case 2: return launch_rows_n<E, SHIFTED, 2>(vpt, q, wn, a, g, s);
+    case 4: return launch_rows_n<E, SHIFTED, 4>(vpt, q, wn, a, g, s);
+    case 8: return launch_rows_n<E, SHIFTED, 8>(vpt, q, wn, a, g, s);
     }
     return hipErrorInvalidValue;
 }

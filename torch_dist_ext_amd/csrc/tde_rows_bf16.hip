@@ -4,7 +4,7 @@
 namespace tde {
 
 hipError_t launch_rows_bf16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s) {
-    return launch_rows_e<ElemBF16>(n, vpt, q, wn, a, g, s);
+    return launch_rows_e<ElemBF16, false>(n, vpt, q, wn, a, g, s);
 }
 
 hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows,

@@ -42,7 +42,7 @@ __device__ __forceinline__ u32x4 pack_f64(const double (&d)[2]) {
 // per thread: 2 x 300 rows of 2048 -10 %, 2 x 900 of 1024 -11 %, 4 x 900 of 600 -10 %; 4 x 2048 rows of 2048 +3.3 %, 8 x 2048 of 600 +2.8 %.
 constexpr int64_t kEarlyStoreBytes = 9 << 20;
 
-template <int N, int VPT, int FORM = kFormPlain>
+template <int N, int VPT, int FORM = kFormPlain, bool SHIFTED = false>
 __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     constexpr bool OWNED = FORM == kFormOwned, STAGED = FORM == kFormStaged;
     constexpr int NP = (N == 0) ? 1 : N;
@@ -52,11 +52,7 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     const int tid = threadIdx.x;
     const int tpr = a.threads_per_row;
     const int group = a.row_group(__builtin_amdgcn_readfirstlane(tid >> 6));
-    const int t = tid - group * tpr;
     const uint32_t row_bytes = (uint32_t)a.hidden() * 8u;
-    uint32_t off[VPT];
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
 
     const void *part[NP];
     partial_addresses(a, a.address(kPtrStage), part);
@@ -69,6 +65,11 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     if constexpr (OWNED) row = owned_first_row<N>(row, a.tokens, a.owner, sum_is_new);
     const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
     const int64_t row_byte = row * (int64_t)row_bytes;
+    const int shift = SHIFTED ? a.row_shift(row_byte) : 0;
+    const int t = first_vector_of<SHIFTED>(tid - group * tpr, shift, tpr);
+    uint32_t off[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
     const auto load_row = [&](const void *base, u32x4(&v)[VPT]) {
         const rsrc_t rs = row_rsrc(base, row_byte, bytes);
 #pragma unroll
@@ -152,8 +153,8 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
         load_gamma();
         store_sums();
     }
-    const int t_behind = VPT == 1 ? t : not_before(t, landed);
-    const float sumsq = sumsq_torch_order(sums, t_behind, tpr, 0, t_behind & (kWave - 1));
+    const int t_behind = thread_of<SHIFTED>(VPT == 1 ? t : not_before(t, landed), shift, tpr);
+    const float sumsq = sumsq_torch_order<SHIFTED>(sums, t_behind, tpr, 0, t_behind & (kWave - 1));
     const float rs = reciprocal_rms(sumsq, length, a.eps);
 
     const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
@@ -220,15 +221,16 @@ hipError_t launch_reduce_f64(int n, const RowArgs &a, uint64_t table, int64_t ro
     return hipErrorInvalidValue;
 }
 
-template <int N, int VPT>
+template <int N, int VPT, bool SHIFTED = false>
 hipError_t launch_rows_f64_nv(const RowArgs &a, const Geometry &g, hipStream_t s) {
     const dim3 grid((unsigned)g.grid), block((unsigned)g.block_threads);
     const size_t lds = (size_t)g.lds_bytes; // sumsq_lds_bytes(g.block_threads, VPT, 2): doubles are never limited per CU
     if constexpr (N != 0) {
-        if (g.form == kFormOwned) return launch_kernel<row_kernel_f64<N, VPT, kFormOwned>>(grid, block, lds, s, a);
-        if (g.form == kFormStaged) return launch_kernel<row_kernel_f64<N, VPT, kFormStaged>>(grid, block, lds, s, a);
+        if (!SHIFTED && a.line_mask != 0) return launch_rows_f64_nv<N, VPT, true>(a, g, s);
+        if (g.form == kFormOwned) return launch_kernel<row_kernel_f64<N, VPT, kFormOwned, SHIFTED>>(grid, block, lds, s, a);
+        if (g.form == kFormStaged) return launch_kernel<row_kernel_f64<N, VPT, kFormStaged, SHIFTED>>(grid, block, lds, s, a);
     }
-    return launch_kernel<row_kernel_f64<N, VPT>>(grid, block, lds, s, a);
+    return launch_kernel<row_kernel_f64<N, VPT, kFormPlain, SHIFTED>>(grid, block, lds, s, a);
 }
 
 template <int N>
