@@ -114,6 +114,7 @@ __device__ __forceinline__ void partial_addresses(const RowArgs &a, uint64_t tab
 struct ElemBF16 {
     static constexpr int VEC = 8;
     static constexpr int BYTES = 2;
+    static constexpr bool MIXED = false;
     static __device__ __forceinline__ void unpack(u32x4 raw, float (&f)[VEC]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -135,6 +136,7 @@ struct ElemBF16 {
 struct ElemF16 {
     static constexpr int VEC = 8;
     static constexpr int BYTES = 2;
+    static constexpr bool MIXED = true; // see fma_mix
     static __device__ __forceinline__ void unpack(u32x4 raw, float (&f)[VEC]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -148,8 +150,11 @@ struct ElemF16 {
         u32x4 raw;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            f16x2 h = {(_Float16)f[2 * i], (_Float16)f[2 * i + 1]};
-            raw[i] = __builtin_bit_cast(uint32_t, h);
+            float lo = f[2 * i], hi = f[2 * i + 1];
+            // one rounding here and one in the operation before it: never one instruction that rounds its exact result once
+            asm("" : "+v"(lo), "+v"(hi));
+            f32x2 v = {lo, hi};
+            raw[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
         }
         return raw;
     }
@@ -158,6 +163,7 @@ struct ElemF16 {
 struct ElemF32 {
     static constexpr int VEC = 4;
     static constexpr int BYTES = 4;
+    static constexpr bool MIXED = false;
     static __device__ __forceinline__ void unpack(u32x4 raw, float (&f)[VEC]) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -173,6 +179,139 @@ struct ElemF32 {
     }
 };
 
+// fp16 rows (E::MIXED) never unpack.  v_fma_mix_f32 takes a half of a packed pair as an fp32 operand, so that a conversion costs
+// nothing beside the operation it is for; and where two fp16 numbers are added or multiplied and the result is rounded to fp16,
+// the packed instructions, which round once, give the bits of the two roundings of the fp32 operation: a product of two
+// has 22 bits and is exact in fp32, and a sum rounded to 24 bits, no fewer than 2 * 11 + 1, never lands on a different side of a
+// boundary between two fp16 numbers (Figueroa, "When is double rounding innocuous?", 1995).
+// The mixed forms issue at half the rate, so a launch that is bound by instructions of many wavefronts gains from the packed ones
+// only; one that waits for a row's chain gains from every instruction left out.  With conversions against this: 2 x [79, 8096] 4.28 -> 4.16 us,
+// 4 x [89, 4256] 3.83 -> 3.70, 2 x [1162, 1152] -> int8 4.44 -> 4.33, 2 x [1651, 6328] -> int8 19.85 -> 18.5; 2-3 % up to 40 MB, from 200 MB on nothing.
+// HALF: which one of `pair`, 0 or 1.  fma(pair, b, c).
+template <int HALF>
+__device__ __forceinline__ float fma_mix(uint32_t pair, float b, float c) {
+    float r;
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(b), "v"(c));
+    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(b), "v"(c));
+    return r;
+}
+// pair + 0, which turns -0 into +0 as the sums that start from 0 do
+template <int HALF>
+__device__ __forceinline__ float widen_mix(uint32_t pair) {
+    float r;
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, 1.0, 0 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair));
+    else asm("v_fma_mix_f32 %0, %1, 1.0, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair));
+    return r;
+}
+// c + pair, in c's register
+template <int HALF>
+__device__ __forceinline__ float add_mix(uint32_t pair, float c) {
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(c) : "v"(pair));
+    else asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(c) : "v"(pair));
+    return c;
+}
+// pair * b, -0 kept
+template <int HALF>
+__device__ __forceinline__ float mul_mix(uint32_t pair, float b) {
+    float r;
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(b));
+    else asm("v_fma_mix_f32 %0, %1, %2, neg(0) op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(b));
+    return r;
+}
+template <int HALF>
+__device__ __forceinline__ float square_mix(uint32_t pair) {
+    float r;
+    if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, %1, 0 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(pair));
+    else asm("v_fma_mix_f32 %0, %1, %1, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(pair));
+    return r;
+}
+
+// acc = (first ? 0 : acc) + one vector of a partial
+template <class E>
+__device__ __forceinline__ void accumulate(u32x4 raw, float (&acc)[E::VEC], bool first) {
+    if constexpr (E::MIXED) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[2 * i] = first ? widen_mix<0>(raw[i]) : add_mix<0>(raw[i], acc[2 * i]);
+            acc[2 * i + 1] = first ? widen_mix<1>(raw[i]) : add_mix<1>(raw[i], acc[2 * i + 1]);
+        }
+    } else {
+        float p[E::VEC];
+        E::unpack(raw, p);
+#pragma unroll
+        for (int i = 0; i < E::VEC; ++i) acc[i] = first ? 0.0f + p[i] : acc[i] + p[i];
+    }
+}
+
+// T(a + b)
+template <class E>
+__device__ __forceinline__ u32x4 added(u32x4 a, u32x4 b) {
+    if constexpr (E::MIXED) {
+        u32x4 sum;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t u = a[i], v = b[i];
+            sum[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, u) + __builtin_bit_cast(f16x2, v));
+        }
+        return sum;
+    } else {
+        float x[E::VEC], y[E::VEC];
+        E::unpack(a, x);
+        E::unpack(b, y);
+#pragma unroll
+        for (int i = 0; i < E::VEC; ++i) x[i] = x[i] + y[i];
+        return E::pack(x);
+    }
+}
+
+template <class E>
+__device__ __forceinline__ void squares_of(u32x4 raw, float (&sq)[E::VEC]) {
+    if constexpr (E::MIXED) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sq[2 * i] = square_mix<0>(raw[i]);
+            sq[2 * i + 1] = square_mix<1>(raw[i]);
+        }
+    } else {
+        float x[E::VEC];
+        E::unpack(raw, x);
+#pragma unroll
+        for (int i = 0; i < E::VEC; ++i) sq[i] = x[i] * x[i];
+    }
+}
+
+// T(gamma * T(x * rs)) of one vector.
+template <class E>
+__device__ __forceinline__ u32x4 normed(u32x4 xraw, u32x4 gamma_raw, float rs) {
+    constexpr int VEC = E::VEC;
+    float n[VEC];
+    if constexpr (E::MIXED) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            n[2 * i] = mul_mix<0>(xraw[i], rs);
+            n[2 * i + 1] = mul_mix<1>(xraw[i], rs);
+        }
+        const u32x4 first = E::pack(n);
+        u32x4 y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t u = first[i], v = gamma_raw[i];
+            y[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, v) * __builtin_bit_cast(f16x2, u));
+        }
+        return y;
+    } else {
+        float x[VEC], g[VEC];
+        E::unpack(xraw, x);
+        E::unpack(gamma_raw, g);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
+        E::unpack(E::pack(n), n);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
+        return E::pack(n);
+    }
+}
+
 // The largest magnitude of a row's elements: NaN if any of them is, as torch's amax has it (v_max_f32 would drop it).  Two
 // elements an instruction, on the values that the quotients need anyway.
 __device__ __forceinline__ float max_abs(float acc, float a, float b) {
@@ -180,6 +319,40 @@ __device__ __forceinline__ float max_abs(float acc, float a, float b) {
     asm("v_maximum3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(acc), "v"(a), "v"(b));
     return r;
 }
+
+// A vector of normed elements on its way to codes: fp32, or as it is where E is MIXED.
+template <class E, bool MIXED = E::MIXED>
+struct Normed {
+    float y[E::VEC];
+    Normed() = default;
+    __device__ __forceinline__ explicit Normed(u32x4 raw) { E::unpack(raw, y); }
+    __device__ __forceinline__ void values(float (&v)[E::VEC]) const {
+#pragma unroll
+        for (int i = 0; i < E::VEC; ++i) v[i] = y[i];
+    }
+    __device__ __forceinline__ float largest() const {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < E::VEC; i += 2) m = max_abs(m, y[i], y[i + 1]);
+        return m;
+    }
+};
+template <class E>
+struct Normed<E, true> {
+    u32x4 raw;
+    Normed() = default;
+    __device__ __forceinline__ explicit Normed(u32x4 raw_) : raw(raw_) {}
+    __device__ __forceinline__ void values(float (&v)[E::VEC]) const { E::unpack(raw, v); }
+    __device__ __forceinline__ float largest() const { // of even and odd elements side by side, then of the two
+        uint32_t m;
+        asm("v_pk_maximum3_f16 %0, %1, %1, %1 neg_lo:[0,0,1] neg_hi:[0,0,1]" : "=v"(m) : "v"(raw[0]));
+#pragma unroll
+        for (int i = 1; i < 4; ++i) asm("v_pk_maximum3_f16 %0, %0, %1, %1 neg_lo:[0,0,1] neg_hi:[0,0,1]" : "+v"(m) : "v"(raw[i]));
+        const f16x2 h = __builtin_bit_cast(f16x2, m);
+        const float lo = (float)h[0], hi = (float)h[1];
+        return max_abs(lo, hi, hi);
+    }
+};
 
 // min(max(q, -limit), limit) that keeps NaN, as torch.clamp does.
 __device__ __forceinline__ float clamp_keep_nan(float q, float limit) {
@@ -679,22 +852,19 @@ struct Divisor {
         if constexpr (E::BYTES == 2) return __builtin_fmaf(y, hi, y * lo);
         else return div_shared(y, d, hi);
     }
+    __device__ __forceinline__ void quotients(const Normed<E> &y, float (&q)[E::VEC]) const {
+        if constexpr (E::MIXED) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                q[2 * i] = fma_mix<0>(y.raw[i], hi, mul_mix<0>(y.raw[i], lo));
+                q[2 * i + 1] = fma_mix<1>(y.raw[i], hi, mul_mix<1>(y.raw[i], lo));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < E::VEC; ++i) q[i] = quotient(y.y[i]);
+        }
+    }
 };
-
-// T(gamma * T(x * rs)) of one vector.
-template <class E>
-__device__ __forceinline__ u32x4 normed(u32x4 xraw, u32x4 gamma_raw, float rs) {
-    constexpr int VEC = E::VEC;
-    float x[VEC], g[VEC], n[VEC];
-    E::unpack(xraw, x);
-    E::unpack(gamma_raw, g);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
-    E::unpack(E::pack(n), n);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
-    return E::pack(n);
-}
 
 // The largest code of a mode.
 template <int Q>
@@ -729,23 +899,28 @@ __device__ __forceinline__ bool static_scale_is_fast(float scale) {
 
 // The codes of one vector's elements.  FAST: `divisor` is div's; otherwise the plain division.
 template <class E, int Q, bool FAST>
-__device__ __forceinline__ void codes_of(const float (&y)[E::VEC], const Divisor<E> &divisor, float div, uint32_t (&codes)[E::VEC / 4]) {
+__device__ __forceinline__ void codes_of(const Normed<E> &y, const Divisor<E> &divisor, float div, uint32_t (&codes)[E::VEC / 4]) {
     constexpr int VEC = E::VEC;
     constexpr float QMAX = kQuantMax<Q>;
     float q[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        float v = y[i];
+    if constexpr (FAST && Q == TDE_QUANT_FP8_STATIC && E::BYTES != 2) {
         // A caller's scale can be far below the row's values (the dynamic scales cannot: |y| <= QMAX * scale).
         // Beyond twice the largest code the quotient clamps to QMAX whatever it is, so where its correction
         // would see inf - inf, y is cut there.
-        if constexpr (Q == TDE_QUANT_FP8_STATIC && FAST && E::BYTES != 2) v = clamp_keep_nan(v, 2.0f * QMAX * div);
-        if constexpr (FAST) v = divisor.quotient(v);
-        else v = v / div;
-        // Dynamic scales: the quotient is within 1e-4 of +-QMAX at most, which the conversions below round to
-        // the largest code; nothing to clamp
-        if constexpr (!FAST || Q == TDE_QUANT_FP8_STATIC) v = clamp_keep_nan(v, QMAX);
-        q[i] = v;
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) q[i] = divisor.quotient(clamp_keep_nan(y.y[i], 2.0f * QMAX * div));
+    } else if constexpr (FAST) {
+        divisor.quotients(y, q);
+    } else {
+        y.values(q);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) q[i] = q[i] / div;
+    }
+    // Dynamic scales: the quotient is within 1e-4 of +-QMAX at most, which the conversions below round to
+    // the largest code; nothing to clamp
+    if constexpr (!FAST || Q == TDE_QUANT_FP8_STATIC) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) q[i] = clamp_keep_nan(q[i], QMAX);
     }
     if constexpr (Q == TDE_QUANT_INT8_TOKEN)
         pack_int8<VEC, FAST>(q, codes);
@@ -986,12 +1161,7 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
                 for (int r = 0; r < N; ++r) {
 #pragma unroll
-                    for (int j = 0; j < VPT; ++j) {
-                        float v[VEC];
-                        E::unpack(p[j][r % B], v);
-#pragma unroll
-                        for (int i = 0; i < VEC; ++i) acc[j][i] = (r == 0 ? 0.0f : acc[j][i]) + v[i];
-                    }
+                    for (int j = 0; j < VPT; ++j) accumulate<E>(p[j][r % B], acc[j], r == 0);
                     if (r + B < N) request(r + B);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -1010,22 +1180,14 @@ __global__ void __launch_bounds__(1024 / VPT)
             // two vectors arrived in, so the accumulators cost no registers while all other loads are in flight.
 #pragma unroll
             for (int j = 0; j < VPT; ++j) {
-                float p0[VEC], p1[VEC];
-                E::unpack(cur.p[j][0], p0);
-                E::unpack(cur.p[j][1], p1);
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) racc[j][i] = (0.0f + p0[i]) + p1[i];
+                accumulate<E>(cur.p[j][0], racc[j], true);
+                accumulate<E>(cur.p[j][1], racc[j], false);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int r = 2; r < NP; ++r) {
 #pragma unroll
-                for (int j = 0; j < VPT; ++j) {
-                    float p[VEC];
-                    E::unpack(cur.p[j][r], p);
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) racc[j][i] += p[i];
-                }
+                for (int j = 0; j < VPT; ++j) accumulate<E>(cur.p[j][r], racc[j], false);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -1040,35 +1202,19 @@ __global__ void __launch_bounds__(1024 / VPT)
             } else {
                 float acc[VEC];
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
-#pragma unroll
-                for (int r = 0; r < NP; ++r) {
-                    float p[VEC];
-                    E::unpack(cur.p[j][r], p);
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) acc[i] += p[i];
-                }
+                for (int r = 0; r < NP; ++r) accumulate<E>(cur.p[j][r], acc, r == 0);
                 sraw[j] = E::pack(acc);
             }
-            float s[VEC], res[VEC], x[VEC];
-            E::unpack(sraw[j], s);
-            E::unpack(cur.r[j], res);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) x[i] = s[i] + res[i];
-            xraw[j] = E::pack(x);
-            E::unpack(xraw[j], x);
+            xraw[j] = added<E>(sraw[j], cur.r[j]);
             float sq[VEC];
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) sq[i] = x[i] * x[i];
+            squares_of<E>(xraw[j], sq);
             put_squares(sums.img + (j * tpr + TDE_T_BEHIND(xraw[j][0])) * VEC, sq);
         }
         if (sums.n != sums.chained) {
 #pragma unroll
             for (int j = 0; j < VPT; ++j) {
-                float x[VEC], sq[VEC];
-                E::unpack(xraw[j], x);
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) sq[i] = x[i] * x[i];
+                float sq[VEC];
+                squares_of<E>(xraw[j], sq);
                 split_left(sums, j * tpr + TDE_T_BEHIND(xraw[j][0]), sq);
             }
         }
@@ -1104,29 +1250,17 @@ __global__ void __launch_bounds__(1024 / VPT)
         constexpr bool DYNAMIC = Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC;
         constexpr bool EARLY_RESIDUAL = Q == TDE_QUANT_FP8_STATIC || (Q != TDE_QUANT_NONE && FORM == kFormStaged);
         constexpr int QUANT_VPT = Q == TDE_QUANT_NONE ? 1 : VPT;
-        float y[QUANT_VPT][VEC]; // what is quantized
+        Normed<E> y[QUANT_VPT]; // what is quantized
         float amax[VPT];         // largest magnitude per vector
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            float x[VEC], g[VEC], n[VEC];
-            E::unpack(xraw[j], x);
-            E::unpack(gamma_raw[j], g);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
-            E::unpack(E::pack(n), n);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
-            const u32x4 nraw = E::pack(n);
+            const u32x4 nraw = normed<E>(xraw[j], gamma_raw[j], rs);
             if constexpr (Q == TDE_QUANT_NONE || WN) {
                 const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
                 rsrc_store16(norm_out, TDE_OFF(j), nraw);
             }
-            if constexpr (Q != TDE_QUANT_NONE) E::unpack(nraw, y[j]);
-            if constexpr (DYNAMIC) {
-                amax[j] = 0.0f;
-#pragma unroll
-                for (int i = 0; i < VEC; i += 2) amax[j] = max_abs(amax[j], y[j][i], y[j][i + 1]);
-            }
+            if constexpr (Q != TDE_QUANT_NONE) y[j] = Normed<E>(nraw);
+            if constexpr (DYNAMIC) amax[j] = y[j].largest();
             if constexpr (EARLY_RESIDUAL) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
         }
 
@@ -1250,14 +1384,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(const RowArgs a, const Redu
     for (int u = 0; u < U; ++u) {
         float acc[VEC];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
-#pragma unroll
-        for (int r = 0; r < N; ++r) {
-            float p[VEC];
-            E::unpack(raw[u][r], p);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] += p[i];
-        }
+        for (int r = 0; r < N; ++r) accumulate<E>(raw[u][r], acc, r == 0);
         // The staged sum is re-read by stage B right away: default (cacheable) store.
         __builtin_amdgcn_raw_buffer_store_b128(E::pack(acc), out, (int)((u * 256 + threadIdx.x) * 16), 0, kAuxDefault);
     }

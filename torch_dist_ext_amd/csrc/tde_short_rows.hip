@@ -154,32 +154,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) s
     } else {
         float acc[VEC];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[i] = 0.0f;
-#pragma unroll
-        for (int r = 0; r < NP; ++r) {
-            float v[VEC];
-            E::unpack(p[r], v);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] += v[i];
-        }
+        for (int r = 0; r < NP; ++r) accumulate<E>(p[r], acc, r == 0);
         sraw = E::pack(acc);
         if constexpr (OWNED) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) sraw[i] = sum_is_new ? sraw[i] : staged[i];
         }
     }
-    float s[VEC], res[VEC], x[VEC];
-    E::unpack(sraw, s);
-    E::unpack(residual, res);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) x[i] = s[i] + res[i];
-    const u32x4 xraw = E::pack(x);
-    E::unpack(xraw, x);
+    const u32x4 xraw = added<E>(sraw, residual);
     float *const img = lds_dyn + wave * (kWave * VEC);
     float *const left = lds_dyn + (uint32_t)slot * a.rows_per_block * VEC + (wave * rows + nth) * 32;
     float sq[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) sq[i] = x[i] * x[i];
+    squares_of<E>(xraw, sq);
     put_squares(img + lane * VEC, sq);
     const int chained = hidden & ~31;
     if (hidden != chained) {
@@ -194,14 +180,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) s
     const float rs = reciprocal_rms(slot_sum<VEC>(img + nth * slot * VEC, left, hidden, chained, slot, lane), length, a.eps);
 
     // ---- normalize, outputs --------------------------------------------------------------------------
-    float g[VEC], n[VEC];
-    E::unpack(gamma_raw, g);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) n[i] = x[i] * rs;
-    E::unpack(E::pack(n), n);
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) n[i] = g[i] * n[i];
-    const u32x4 nraw = E::pack(n);
+    const u32x4 nraw = normed<E>(xraw, gamma_raw, rs);
     if (FORM == kFormStaged || (OWNED && any_new))
         rsrc_store16(row_rsrc(a.ptr(kPtrStage), base_byte, bytes), sum_is_new ? off : kPastEnd, sraw);
     if (Q == TDE_QUANT_NONE || a.address(kPtrNorm) != 0) rsrc_store16(row_rsrc(a.ptr(kPtrNorm), base_byte, bytes), off, nraw);
@@ -209,15 +188,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) s
 
     if constexpr (Q != TDE_QUANT_NONE) {
         constexpr bool DYNAMIC = Q != TDE_QUANT_FP8_STATIC;
-        float y[VEC], scale[1];
-        E::unpack(nraw, y);
+        const Normed<E> y(nraw);
+        float scale[1];
         bool fast;
         if constexpr (DYNAMIC) {
             constexpr bool GROUP = Q == TDE_QUANT_FP8_GROUP;
             constexpr int LANES_PER_GROUP = TDE_QUANT_GROUP / VEC; // 16 (2-byte types) or 32 (fp32: whole rows)
-            float amax = 0.0f;
-#pragma unroll
-            for (int i = 0; i < VEC; i += 2) amax = max_abs(amax, y[i], y[i + 1]);
+            const float amax = y.largest();
             uint32_t m[1] = {lanes_max(__builtin_bit_cast(uint32_t, amax) & 0x7fffffffu, GROUP ? LANES_PER_GROUP : slot)};
             fast = scales_of_largest<Q>(m, scale);
             const uint32_t scales = GROUP ? (uint32_t)hidden / TDE_QUANT_GROUP : 1u; // of a row
