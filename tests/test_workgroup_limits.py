@@ -1,0 +1,41 @@
+"""Limits on resident workgroups per compute unit where launches are shorter, or their rows, than those of test_abi_host.py: on both sides
+of each range, and what such launches leave."""
+import pytest
+import torch
+
+from helpers import bits_equal, run_hip
+from oracle import eager
+from torch_dist_ext_amd import _capi
+
+BF16, F16, F32 = _capi.BF16, _capi.F16, _capi.F32
+FP8, GROUP, INT8, STATIC, NONE = _capi.QUANT_FP8_TOKEN, _capi.QUANT_FP8_GROUP, _capi.QUANT_INT8_TOKEN, _capi.QUANT_FP8_STATIC, _capi.QUANT_NONE
+
+
+@pytest.mark.parametrize("dtype,n,tokens,hidden,quant,wn,algo,limit", [
+    # four partials, four vectors per thread, only codes of a dynamic scale to store: 16 to 30 workgroups per unit
+    (BF16, 4, 4095, 7168, FP8, 0, _capi.ALGO_AUTO, 0), (BF16, 4, 4096, 7168, FP8, 0, _capi.ALGO_AUTO, 2), (F16, 4, 7679, 8192, INT8, 0, _capi.ALGO_AUTO, 2),
+    (F16, 4, 7680, 8192, INT8, 0, _capi.ALGO_AUTO, 0), (F32, 4, 5000, 4096, GROUP, 0, _capi.ALGO_AUTO, 2), (BF16, 4, 5000, 7168, FP8, 1, _capi.ALGO_AUTO, 0),
+    (BF16, 4, 5000, 7168, STATIC, 0, _capi.ALGO_AUTO, 0), (BF16, 4, 5000, 7168, NONE, 0, _capi.ALGO_AUTO, 0), (BF16, 2, 5000, 7168, FP8, 0, _capi.ALGO_AUTO, 0),
+    (BF16, 4, 5000, 4096, FP8, 0, _capi.ALGO_AUTO, 0),
+    # short rows with a stage: six workgroups, of rows up to 181 vectors, in launches of 56 MB on
+    (F16, 4, 26425, 1144, INT8, 0, _capi.ALGO_STAGED, 6), (F32, 4, 27056, 316, INT8, 0, _capi.ALGO_STAGED, 6), (BF16, 4, 9000, 1440, FP8, 0, _capi.ALGO_STAGED, 6),
+    (BF16, 4, 9000, 1456, FP8, 0, _capi.ALGO_STAGED, 4), (BF16, 4, 9000, 1440, NONE, 0, _capi.ALGO_STAGED, 4), (BF16, 4, 8600, 520, FP8, 0, _capi.ALGO_STAGED, 4),
+    (BF16, 8, 9000, 1440, FP8, 0, _capi.ALGO_STAGED, 4),
+])
+def test_limits(dtype, n, tokens, hidden, quant, wn, algo, limit):
+    if torch.cuda.is_available() and _capi.device_info().compute_units != 256:
+        pytest.skip("the row counts are for 256 compute units")
+    p = _capi.make_problem(dtype, n, tokens, hidden, 1e-5, quant=quant, algo=algo, write_norm=wn, static_scale=0.5 if quant == STATIC else 0.0)
+    assert _capi.plan(p).workgroups_per_cu == limit
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,n,tokens,hidden,quant,algo", [(torch.float16, 4, 4099, 6152, "int8_token", _capi.ALGO_AUTO), (torch.float32, 4, 8003, 400, "fp8_token", _capi.ALGO_STAGED),
+                                                              (torch.float16, 8, 1027, 6200, "fp8_token", _capi.ALGO_AUTO)])
+def test_limited_launch_equals_the_unlimited(cuda_device, dtype, n, tokens, hidden, quant, algo):
+    print("case", dtype, n, tokens, hidden, quant, algo, flush=True)
+    p, r, g = eager.make_inputs(n, tokens, hidden, dtype, 1.0, seed=hidden)
+    want = run_hip(p, r, g, 1e-6, quant, algo=algo, workgroups_per_cu=-1)
+    got = run_hip(p, r, g, 1e-6, quant, algo=algo)
+    for k in want:
+        assert bits_equal(got[k], want[k]), k

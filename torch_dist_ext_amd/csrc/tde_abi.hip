@@ -63,8 +63,9 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 constexpr int kMaxBlock = 1024;
 constexpr int64_t kLoadsInFlightPerCu = 128 * 1024; // target for the limit on resident workgroups (see validate)
 // launches with fewer workgroups per compute unit are not limited: 24 with 8 partials, 32 with 4 (whose launches are
-// shorter), i.e. 6144 and 8192 workgroups on the 256 CUs of an unpartitioned MI355X
+// shorter), i.e. 6144 and 8192 workgroups on the 256 CUs of an unpartitioned MI355X; launches of 4 that store little also from 16 to 30
 constexpr int64_t kLimitFromWorkgroupsPerCu8 = 24, kLimitFromWorkgroupsPerCu4 = 32;
+constexpr int64_t kFewStoresFrom = 16, kFewStoresUntil = 30;
 constexpr int kDefaultComputeUnits = 256; // MI355X; used when no device can be asked (planning on a host without one)
 
 // Compute units of the current device, asked once per device and thread (no lock on the launch path).
@@ -485,32 +486,44 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     // 4 x [9000, 3584] 124.9 against 127.0.
     const bool staged = p->algo == TDE_ALGO_STAGED || p->algo == TDE_ALGO_STAGED_OWNED;
     int wgs_per_cu = 0;
-    if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus) {
-        const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
+    const int64_t per_wg = (int64_t)rpb * (p->nranks + 1) * nvec * 16; // bytes of loads one workgroup keeps in flight
+    // Only codes of a dynamic scale beside residual_out to store, four vectors per thread and 96 KiB of loads in two workgroups.
+    const bool few_stores = vpt == 4 && p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0 && 2 * per_wg >= 96 * 1024;
+    const bool many_workgroups = grid >= (p->nranks >= 8 ? kLimitFromWorkgroupsPerCu8 : kLimitFromWorkgroupsPerCu4) * cus ||
+                                 (few_stores && grid >= kFewStoresFrom * cus && grid < kFewStoresUntil * cus);
+    if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && many_workgroups) {
         const int waves = tpr * rpb / 64;
         const int at_least = std::max(2, (8 + waves - 1) / waves);
         wgs_per_cu = (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
-        // Two workgroups are enough, six wavefronts among them, wherever two have 96 KiB of loads in flight and only codes of a
-        // dynamic scale beside residual_out to store, with four vectors per thread: 4 x [32768, 5120] fp16 -> int8 338.2 us against
+        // Two workgroups are enough for few_stores, six wavefronts among them: 4 x [32768, 5120] fp16 -> int8 338.2 us against
         // 342.3 with three, bf16 -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three
-        // stay 3 % ahead.  Among the plan's own choices that is rows of 640 vectors on four partials; longer rows, and eight
-        // partials, have two already.
-        const bool few_stores = p->quant != TDE_QUANT_NONE && p->quant != TDE_QUANT_FP8_STATIC && p->write_norm == 0;
-        if (vpt == 4 && few_stores && 2 * per_wg >= 96 * 1024) wgs_per_cu = 2;
+        // stay 3 % ahead.  For them the limit pays from 16 workgroups per unit on: 4 x rows of 770 to 1024 vectors, 4096 to 6143 of them -1.3 % (bf16),
+        // -2.3 (fp16) and 0 (fp32), 6144 to 8191 -2.5 to -2.9, per group -2 (below 4096 +0.5; static scales +0.5, T-typed output -0.5).
+        if (few_stores) wgs_per_cu = 2;
     }
     // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more.  From 16 workgroups per CU
     // on four and eight partials gain from the same 128 KiB, counted with the stage's stores, but never more than four workgroups
     // (56 launches of 4096 to 40188 rows: 2.0 % faster on average, none more than 0.4 % slower; without a limit against with): 8 x [32005, 2512] bf16 -> fp8 322.8 -> 304.2
     // us (three), 8 x [32012, 1032] fp16 137.1 -> 126.0 (four), 8 x [4096, 3000] 51.8 -> 50.0 (two), 8 x [12091, 8192] 396 -> 381 (two),
     // 4 x [30550, 748] fp32 114.5 -> 106.9 (four), 4 x [16384, 8192] 318.1 -> 313.4 (two).  Rows packed more than two to a workgroup
-    // lose up to 2 %, two partials with one vector per thread up to 19 % with two and gain nothing with four.
+    // lose up to 2 %, two partials with one vector per thread up to 19 % with two and gain nothing with four.  Four workgroups of short
+    // rows hold too little: below 68 KiB of loads and stores in four (four partials, rows of up to 180 vectors) six take 0.96 of the
+    // time of four with quantized output, single ones 0.86 (70 launches; 4 x [26425, 1144] fp16 -> int8 84.8 -> 74.0 us, 4 x [27056, 316] fp32
+    // 46.8 -> 41.6), and more nothing on top; T-typed output alone is 1 % slower with six.
     // With owned rows, and in the norm phase alone, most rows read two streams, and a limit only costs (25 launches of four and
     // eight partials: up to 50 %).
     if (p->dtype != TDE_F64 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks >= 4 && rpb <= 2 && grid >= 16 * (int64_t)cus) {
-        const int64_t per_wg = (int64_t)rpb * (p->nranks + 2) * nvec * 16;
-        wgs_per_cu = (int)std::min<int64_t>(4, std::max<int64_t>(2, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        const int64_t moved = (int64_t)rpb * (p->nranks + 2) * nvec * 16;
+        const int64_t most = p->quant != TDE_QUANT_NONE && 4 * moved < 68 * 1024 && row_megabytes(p, nvec) >= 56 ? 6 : 4;
+        wgs_per_cu = (int)std::min<int64_t>(most, std::max<int64_t>(2, (kLoadsInFlightPerCu + moved / 2) / moved));
     }
     if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
+
+    // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
+    // row kernel's two-wavefronts-per-SIMD instantiation (tde_rows.h: WIDE) is 0.2-2.2 % faster there; it is
+    // reported as the limit of two workgroups per CU that its registers amount to.
+    const bool wide = p->nranks == 8 && vpt == 4 && p->dtype != TDE_F64 && !staged && wgs_per_cu == 0 &&
+                p->tune_workgroups_per_cu == 0 && grid >= 4 * (int64_t)cus;
 
     if (geo) {
         geo->wgs_per_cu = wgs_per_cu;
@@ -533,11 +546,6 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         // Row groups per XCD chunk of the row mapping (tde_rows.h: xcd_chunked_block); 16 measured best with 8
         // partials, 8 with 4.
         geo->xcd_chunk = p->nranks >= 8 ? 16 : 8;
-        // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
-        // row kernel's two-wavefronts-per-SIMD instantiation (tde_rows.h: WIDE) is 0.2-2.2 % faster there; it is
-        // reported as the limit of two workgroups per CU that its registers amount to.
-        const bool wide = p->nranks == 8 && vpt == 4 && p->dtype != TDE_F64 && !staged && wgs_per_cu == 0 &&
-                    p->tune_workgroups_per_cu == 0 && grid >= 4 * (int64_t)cus;
         geo->form = wide ? tde::kFormWide : tde::kFormPlain;
         if (wide) geo->wgs_per_cu = 2;
     }

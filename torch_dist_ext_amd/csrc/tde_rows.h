@@ -1004,7 +1004,9 @@ __device__ __forceinline__ int thread_of(int first_vector, int shift, int tpr) {
 //   Q      tde_quant
 //   WN     write the T-typed normed row (always true for Q == NONE)
 //   FORM   kFormWide: compiled for two wavefronts per SIMD (256 registers) instead of three, with gamma requested ahead
-//          of the row also for eight partials: two workgroups per CU whose gamma never waits.  Launched for eight
+//          of the row also for eight partials: two workgroups per CU whose gamma never waits.  Never more than two wavefronts,
+//          also where the registers would hold three (fp16 and fp32, 168 and 166 of them: 8 x rows of 600 to 1024 vectors, 1024 to
+//          6200 of them, 0.983 of the time, single ones 0.953).  Launched for eight
 //          partials with four vectors per thread at 4 to 24 workgroups per CU (launch_rows_nv, Geometry::form).
 //          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
 //          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
@@ -1018,7 +1020,7 @@ enum : int { kFormPlain = 0, kFormWide = 1, kFormStaged = 2, kFormOwned = 3 };
 
 template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain, bool SHIFTED = false>
 __global__ void __launch_bounds__(1024 / VPT)
-    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))))))
+    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))), FORM == kFormWide ? 2 : 8)))
     row_kernel(const RowArgs a) {
     constexpr bool WIDE = FORM == kFormWide, OWNED = FORM == kFormOwned;
     constexpr int VEC = E::VEC;
