@@ -21,6 +21,10 @@ FP8, GROUP, INT8, STATIC, NONE = _capi.QUANT_FP8_TOKEN, _capi.QUANT_FP8_GROUP, _
     (F16, 4, 26425, 1144, INT8, 0, _capi.ALGO_STAGED, 6), (F32, 4, 27056, 316, INT8, 0, _capi.ALGO_STAGED, 6), (BF16, 4, 9000, 1440, FP8, 0, _capi.ALGO_STAGED, 6),
     (BF16, 4, 9000, 1456, FP8, 0, _capi.ALGO_STAGED, 4), (BF16, 4, 9000, 1440, NONE, 0, _capi.ALGO_STAGED, 4), (BF16, 4, 8600, 520, FP8, 0, _capi.ALGO_STAGED, 4),
     (BF16, 8, 9000, 1440, FP8, 0, _capi.ALGO_STAGED, 4),
+    # eight partials, rows of three wavefronts, and of four with T-typed output: 96 KiB from 48 workgroups per unit on
+    (BF16, 8, 12287, 1280, FP8, 0, _capi.ALGO_AUTO, 6), (BF16, 8, 12288, 1280, FP8, 0, _capi.ALGO_AUTO, 4), (BF16, 8, 12288, 1544, FP8, 0, _capi.ALGO_AUTO, 5),
+    (F32, 8, 12288, 772, NONE, 0, _capi.ALGO_AUTO, 4), (F16, 8, 12288, 1920, NONE, 0, _capi.ALGO_AUTO, 3), (F16, 8, 12287, 1920, NONE, 0, _capi.ALGO_AUTO, 4),
+    (F16, 8, 12288, 2056, NONE, 0, _capi.ALGO_AUTO, 4), (F16, 8, 12288, 1024, NONE, 0, _capi.ALGO_AUTO, 4),
 ])
 def test_limits(dtype, n, tokens, hidden, quant, wn, algo, limit):
     if torch.cuda.is_available() and _capi.device_info().compute_units != 256:
@@ -31,7 +35,8 @@ def test_limits(dtype, n, tokens, hidden, quant, wn, algo, limit):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,n,tokens,hidden,quant,algo", [(torch.float16, 4, 4099, 6152, "int8_token", _capi.ALGO_AUTO), (torch.float32, 4, 8003, 400, "fp8_token", _capi.ALGO_STAGED),
-                                                              (torch.float16, 8, 1027, 6200, "fp8_token", _capi.ALGO_AUTO)])
+                                                              (torch.float16, 8, 1027, 6200, "fp8_token", _capi.ALGO_AUTO),
+                                                              (torch.bfloat16, 8, 12290, 1032, "none", _capi.ALGO_AUTO)])
 def test_limited_launch_equals_the_unlimited(cuda_device, dtype, n, tokens, hidden, quant, algo):
     print("case", dtype, n, tokens, hidden, quant, algo, flush=True)
     p, r, g = eager.make_inputs(n, tokens, hidden, dtype, 1.0, seed=hidden)

@@ -494,7 +494,12 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     if (p->dtype != TDE_F64 && !staged && p->nranks >= 4 && many_workgroups) {
         const int waves = tpr * rpb / 64;
         const int at_least = std::max(2, (8 + waves - 1) / waves);
-        wgs_per_cu = (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (kLoadsInFlightPerCu + per_wg / 2) / per_wg));
+        // Eight partials, rows of three wavefronts with one vector per thread, and of four with T-typed output: 96 KiB from 48 workgroups
+        // per unit on, 2 to 2.8 % ahead with T-typed output, 1.3 % with codes (of four wavefronts 1 % ahead to 1.6 % behind, shorter
+        // launches 2 % ahead to 1 % behind).
+        const bool short_many = p->nranks >= 8 && vpt == 1 && nvec > 128 && nvec <= (p->quant == TDE_QUANT_NONE ? 256 : 192) && grid >= 48 * (int64_t)cus;
+        const int64_t in_flight = short_many ? 96 * 1024 : kLoadsInFlightPerCu;
+        wgs_per_cu = (int)std::min<int64_t>(8, std::max<int64_t>(at_least, (in_flight + per_wg / 2) / per_wg));
         // Two workgroups are enough for few_stores, six wavefronts among them: 4 x [32768, 5120] fp16 -> int8 338.2 us against
         // 342.3 with three, bf16 -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three
         // stay 3 % ahead.  For them the limit pays from 16 workgroups per unit on: 4 x rows of 770 to 1024 vectors, 4096 to 6143 of them -1.3 % (bf16),
