@@ -54,3 +54,19 @@ def test_products_and_codes(cuda_device, hidden, geometry, quant):
         for k in want:
             undefined = ~want["norm_out"].isfinite().all(-1, keepdim=True) if k == "q" and quant == "int8_token" else None # infinity / infinity
             assert equal_where_not_nan(got[k], want[k], nan_codes=k == "q" and quant != "int8_token", ignore=undefined), k
+
+
+@pytest.mark.parametrize("quant", ["none", "fp8_token", "fp8_group", "int8_token", "fp8_static"])
+@pytest.mark.parametrize("hidden", [640, 1032])
+def test_long_launches_keep_conversions(cuda_device, hidden, quant):
+    """Four partials, four vectors per thread, 48 workgroups per compute unit: the kernels with conversions, rows in place and moved."""
+    if quant == "fp8_group" and hidden % 128:
+        pytest.skip("whole groups only")
+    print("case", hidden, quant, flush=True)
+    p, r, g = eager.make_inputs(4, 12290, hidden, torch.float16, 1.0, seed=hidden)
+    kw = dict(quant=quant, static_scale=0.03 if quant == "fp8_static" else 0.0)
+    want = run_hip(p, r, g, 1e-6, vecs_per_thread=1, **kw)
+    for write_norm in (False, True):
+        got = run_hip(p, r, g, 1e-6, vecs_per_thread=4, rows_per_block=1, write_norm=write_norm, **kw)
+        for k in got:
+            assert equal_where_not_nan(got[k], want[k]), k

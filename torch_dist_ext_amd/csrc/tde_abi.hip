@@ -361,6 +361,8 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alo
     // TDE_ALGO_STAGED, up to four partials, T-typed rows or static and group scales: one vector per thread stays 2-6 % ahead of the
     // ranges above between the lengths they were first swept at.
     if (staged && !per_token && p->nranks <= 4 && nvec > 576 && nvec < 896 && nvec != 640) vpt = nvec == 768 ? vpt : 1;
+    // Of fp16, whose arithmetic is shorter, two are 0.6 to 2.7 % ahead in long launches of four partials (5632 to 7080 elements, 9000 to 24000 rows).
+    if (staged && p->dtype == TDE_F16 && p->quant == TDE_QUANT_NONE && p->nranks == 4 && nvec > 640 && nvec < 896 && t >= 8192) vpt = 2;
     // The norm phase alone keeps one vector per thread where it stores T-typed rows beside the codes and the rows are not whole
     // lines: several are 2-7 % slower there with six and seven wavefronts per row from 4096 rows on, 2-10 % with eleven and twelve.
     const int waves = (int)((nvec + 63) / 64);
@@ -516,6 +518,8 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     // rows hold too little: below 68 KiB of loads and stores in four (four partials, rows of up to 180 vectors) six take 0.96 of the
     // time of four with quantized output, single ones 0.86 (70 launches; 4 x [26425, 1144] fp16 -> int8 84.8 -> 74.0 us, 4 x [27056, 316] fp32
     // 46.8 -> 41.6), and more nothing on top; T-typed output alone is 1 % slower with six.
+    // Two partials of fp16 with two vectors per thread, whose arithmetic is short: three workgroups 1.5 to 2 % ahead of no limit
+    // (2 x [7341 to 24000, 5120], [16000, 4960]).
     // With owned rows, and in the norm phase alone, most rows read two streams, and a limit only costs (25 launches of four and
     // eight partials: up to 50 %).
     if (p->dtype != TDE_F64 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks >= 4 && rpb <= 2 && grid >= 16 * (int64_t)cus) {
@@ -523,6 +527,8 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         const int64_t most = p->quant != TDE_QUANT_NONE && 4 * moved < 68 * 1024 && row_megabytes(p, nvec) >= 56 ? 6 : 4;
         wgs_per_cu = (int)std::min<int64_t>(most, std::max<int64_t>(2, (kLoadsInFlightPerCu + moved / 2) / moved));
     }
+    if (p->dtype == TDE_F16 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks == 2 && vpt == 2 && nvec > 576 && nvec <= 640 && grid >= 24 * (int64_t)cus)
+        wgs_per_cu = 3;
     if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
     // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
@@ -552,7 +558,8 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         // Row groups per XCD chunk of the row mapping (tde_rows.h: xcd_chunked_block); 16 measured best with 8
         // partials, 8 with 4.
         geo->xcd_chunk = p->nranks >= 8 ? 16 : 8;
-        geo->form = wide ? tde::kFormWide : tde::kFormPlain;
+        const bool f16_long = p->dtype == TDE_F16 && p->nranks == 4 && vpt == 4 && !staged && grid >= 48 * (int64_t)cus; // below it the shorter arithmetic is level or ahead
+        geo->form = wide ? tde::kFormWide : (f16_long ? tde::kFormLong : tde::kFormPlain);
         if (wide) geo->wgs_per_cu = 2;
     }
     return TDE_OK;

@@ -160,6 +160,11 @@ struct ElemF16 {
     }
 };
 
+// The same rows with conversions in place of the mixed instructions: longer arithmetic (kFormLong).
+struct ElemF16Unmixed : ElemF16 {
+    static constexpr bool MIXED = false;
+};
+
 struct ElemF32 {
     static constexpr int VEC = 4;
     static constexpr int BYTES = 4;
@@ -1011,12 +1016,19 @@ __device__ __forceinline__ int thread_of(int first_vector, int shift, int tpr) {
 //          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
 //          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
 //          partials and their sums stored to the stage, every other row's sum is read from the stage
+//          kFormLong: fp16 with conversions instead of mixed-precision instructions, for long launches of four partials with four
+//          vectors per thread.  What bounds those is memory, and it is served best when the arithmetic holds a row's
+//          stores back from the next rows' loads: with the mixed instructions 4 x [32768, 5120] -> int8 takes 341.8 us, 4 x [20000, 8192]
+//          370 and 4 x [24000, 5120] per group 252, with conversions 335, 360 and 246
 //   SHIFTED rows that are not whole lines of memory, in launches long enough to gain from it (rows_are_shifted)
 // Block layout: rows_per_block row groups of threads_per_row threads; thread t of a row group
 // owns vectors t, t + threads_per_row, ... (coalesced 1 KiB per wavefront per load) of its row,
 // moved along the threads by row_shift() vectors where the row does not start on a line of memory.
 // ---------------------------------------------------------------------------------------------
-enum : int { kFormPlain = 0, kFormWide = 1, kFormStaged = 2, kFormOwned = 3 };
+enum : int { kFormPlain = 0, kFormWide = 1, kFormStaged = 2, kFormOwned = 3, kFormLong = 4 };
+
+template <class E, int FORM> struct Arithmetic { typedef E type; };
+template <> struct Arithmetic<ElemF16, kFormLong> { typedef ElemF16Unmixed type; };
 
 template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain, bool SHIFTED = false>
 __global__ void __launch_bounds__(1024 / VPT)
@@ -1024,6 +1036,7 @@ __global__ void __launch_bounds__(1024 / VPT)
     row_kernel(const RowArgs a) {
     constexpr bool WIDE = FORM == kFormWide, OWNED = FORM == kFormOwned;
     constexpr int VEC = E::VEC;
+    typedef typename Arithmetic<E, FORM>::type A;
     constexpr int NP = (N == 0) ? 1 : N;
     // residual_out is stored behind the reductions, ahead of the codes: as soon as the sum is known it is 2.4 % slower on
     // 2 x [1257, 6144] static and 7 % on 4 x [512, 5120], behind all codes in one burst 1.7 % on 4 x [32768, 5120] and 1 % on 8 x
@@ -1163,7 +1176,7 @@ __global__ void __launch_bounds__(1024 / VPT)
 #pragma unroll
                 for (int r = 0; r < N; ++r) {
 #pragma unroll
-                    for (int j = 0; j < VPT; ++j) accumulate<E>(p[j][r % B], acc[j], r == 0);
+                    for (int j = 0; j < VPT; ++j) accumulate<A>(p[j][r % B], acc[j], r == 0);
                     if (r + B < N) request(r + B);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -1182,14 +1195,14 @@ __global__ void __launch_bounds__(1024 / VPT)
             // two vectors arrived in, so the accumulators cost no registers while all other loads are in flight.
 #pragma unroll
             for (int j = 0; j < VPT; ++j) {
-                accumulate<E>(cur.p[j][0], racc[j], true);
-                accumulate<E>(cur.p[j][1], racc[j], false);
+                accumulate<A>(cur.p[j][0], racc[j], true);
+                accumulate<A>(cur.p[j][1], racc[j], false);
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int r = 2; r < NP; ++r) {
 #pragma unroll
-                for (int j = 0; j < VPT; ++j) accumulate<E>(cur.p[j][r], racc[j], false);
+                for (int j = 0; j < VPT; ++j) accumulate<A>(cur.p[j][r], racc[j], false);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -1204,19 +1217,19 @@ __global__ void __launch_bounds__(1024 / VPT)
             } else {
                 float acc[VEC];
 #pragma unroll
-                for (int r = 0; r < NP; ++r) accumulate<E>(cur.p[j][r], acc, r == 0);
+                for (int r = 0; r < NP; ++r) accumulate<A>(cur.p[j][r], acc, r == 0);
                 sraw[j] = E::pack(acc);
             }
-            xraw[j] = added<E>(sraw[j], cur.r[j]);
+            xraw[j] = added<A>(sraw[j], cur.r[j]);
             float sq[VEC];
-            squares_of<E>(xraw[j], sq);
+            squares_of<A>(xraw[j], sq);
             put_squares(sums.img + (j * tpr + TDE_T_BEHIND(xraw[j][0])) * VEC, sq);
         }
         if (sums.n != sums.chained) {
 #pragma unroll
             for (int j = 0; j < VPT; ++j) {
                 float sq[VEC];
-                squares_of<E>(xraw[j], sq);
+                squares_of<A>(xraw[j], sq);
                 split_left(sums, j * tpr + TDE_T_BEHIND(xraw[j][0]), sq);
             }
         }
@@ -1252,16 +1265,16 @@ __global__ void __launch_bounds__(1024 / VPT)
         constexpr bool DYNAMIC = Q != TDE_QUANT_NONE && Q != TDE_QUANT_FP8_STATIC;
         constexpr bool EARLY_RESIDUAL = Q == TDE_QUANT_FP8_STATIC || (Q != TDE_QUANT_NONE && FORM == kFormStaged);
         constexpr int QUANT_VPT = Q == TDE_QUANT_NONE ? 1 : VPT;
-        Normed<E> y[QUANT_VPT]; // what is quantized
+        Normed<A> y[QUANT_VPT]; // what is quantized
         float amax[VPT];         // largest magnitude per vector
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-            const u32x4 nraw = normed<E>(xraw[j], gamma_raw[j], rs);
+            const u32x4 nraw = normed<A>(xraw[j], gamma_raw[j], rs);
             if constexpr (Q == TDE_QUANT_NONE || WN) {
                 const rsrc_t norm_out = row_rsrc(a.ptr(kPtrNorm), row_byte, bytes);
                 rsrc_store16(norm_out, TDE_OFF(j), nraw);
             }
-            if constexpr (Q != TDE_QUANT_NONE) y[j] = Normed<E>(nraw);
+            if constexpr (Q != TDE_QUANT_NONE) y[j] = Normed<A>(nraw);
             if constexpr (DYNAMIC) amax[j] = y[j].largest();
             if constexpr (EARLY_RESIDUAL) rsrc_store16(res_out, TDE_OFF(j), xraw[j]);
         }
@@ -1314,14 +1327,14 @@ __global__ void __launch_bounds__(1024 / VPT)
             }
             auto quantize = [&](auto use_fast) {
                 constexpr bool FAST = decltype(use_fast)::value;
-                Divisor<E> divisor;
+                Divisor<A> divisor;
 #pragma unroll
                 for (int j = 0; j < VPT; ++j) {
                     const float sc = scale[SCALES == 1 ? 0 : j];
                     const float div = (Q == TDE_QUANT_FP8_STATIC || sc > 0.0f) ? sc : 1.0f;
-                    if (FAST && (SCALES > 1 || j == 0)) divisor = Divisor<E>(div);
+                    if (FAST && (SCALES > 1 || j == 0)) divisor = Divisor<A>(div);
                     uint32_t codes[VEC / 4];
-                    codes_of<E, Q, FAST>(y[j], divisor, div, codes);
+                    codes_of<A, Q, FAST>(y[j], divisor, div, codes);
                     const uint32_t code_off = (TDE_OFF(j) / 16u) * (uint32_t)VEC;
                     if constexpr (VEC == 8) {
                         const u32x2 w = {codes[0], codes[1]};
@@ -1407,7 +1420,7 @@ struct Geometry {
     int64_t grid;
     int xcd_chunk;
     int line_mask; // RowArgs::line_mask
-    int form;  // which instantiation of the row kernel (kFormPlain, kFormWide, kFormStaged, kFormOwned)
+    int form;  // which instantiation of the row kernel (kFormPlain, kFormWide, kFormStaged, kFormOwned, kFormLong)
 };
 
 // Per-dtype launchers, defined in tde_rows_<dtype>.hip.
@@ -1454,6 +1467,9 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
 #define TDE_LAUNCH(QM, WNB)                                                                              \
     if constexpr (N == 8 && VPT == 4) {                                                                  \
         if (g.form == kFormWide) TDE_LAUNCH_FORM(QM, WNB, kFormWide)                                     \
+    }                                                                                                    \
+    if constexpr (N == 4 && VPT == 4 && E::MIXED) {                                                      \
+        if (g.form == kFormLong) TDE_LAUNCH_FORM(QM, WNB, kFormLong)                                     \
     }                                                                                                    \
     if constexpr (N != 0) {                                                                              \
         if (g.form == kFormStaged) TDE_LAUNCH_FORM(QM, WNB, kFormStaged)                                 \
