@@ -52,7 +52,11 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     const int tid = threadIdx.x;
     const int tpr = a.threads_per_row;
     const int group = a.row_group(__builtin_amdgcn_readfirstlane(tid >> 6));
+    int t = tid - group * tpr; // of the row group; of SHIFTED rows the row's first vector of this thread, as soon as the row is known
     const uint32_t row_bytes = (uint32_t)a.hidden() * 8u;
+    uint32_t off[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
 
     const void *part[NP];
     partial_addresses(a, a.address(kPtrStage), part);
@@ -66,10 +70,11 @@ __global__ void __launch_bounds__(1024 / VPT) row_kernel_f64(const RowArgs a) {
     const uint32_t bytes = (row < a.tokens) ? row_bytes : 0u;
     const int64_t row_byte = row * (int64_t)row_bytes;
     const int shift = SHIFTED ? a.row_shift(row_byte) : 0;
-    const int t = first_vector_of<SHIFTED>(tid - group * tpr, shift, tpr);
-    uint32_t off[VPT];
+    if constexpr (SHIFTED) {
+        t = first_vector_of<true>(t, shift, tpr);
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
+        for (int j = 0; j < VPT; ++j) off[j] = (uint32_t)(j * tpr + t) * 16u;
+    }
     const auto load_row = [&](const void *base, u32x4(&v)[VPT]) {
         const rsrc_t rs = row_rsrc(base, row_byte, bytes);
 #pragma unroll
