@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "8d4c2f12e440286f073e14373880d5f201b28c1b14b11f0103bd937051b29b45",
-    "bytes": {"c2": 11670827, "c3": 352602770, "c4": 765406431, "c5": 2181214650},
+    "sources_sha256": "e0d444b6d27db3d251b1636357d2d20598985d914095467479702250b6047b73",
+    "bytes": {"c2": 11670726, "c3": 352603386, "c4": 765409876, "c5": 2181210598},
 }
 
 BENCH_CONFIGS = {
