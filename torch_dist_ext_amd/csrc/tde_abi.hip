@@ -418,7 +418,15 @@ int vecs_per_thread_shifted(const tde_problem *p, int64_t nvec, int64_t t, int v
     const int waves = (int)((nvec + 63) / 64);
     const bool none = p->quant == TDE_QUANT_NONE;
     if (p->dtype == TDE_F64 || p->algo == TDE_ALGO_STAGED) return vpt;
-    if (p->algo == TDE_ALGO_STAGED_OWNED) return p->nranks >= 8 && vpt == 1 && waves >= 5 && waves <= 10 && t >= 1200 ? 2 : vpt; // 1-12 %
+    if (p->algo == TDE_ALGO_STAGED_OWNED) {
+        // Eight partials, rows of five to ten wavefronts: two vectors 2-20 % ahead of one where codes alone are stored (720 launches).  With
+        // T-typed rows to store nine and ten wavefronts keep that (1 to 5 %; T-typed output of fp32 rows of nine +-1 %), eight lose 0.5 to 4 %
+        // at any length, five to seven from 18 rows per unit on 0.5 to 5 % (T-typed output; of fp32 also beside codes: of
+        // 2-byte rows beside codes two stay 0.5 to 6 % ahead): 8 x [17457, 1476] fp32 90.7 us with two, 86.3 with one, [14836, 2144] bf16 54.0 and 53.2, [2123, 4040] fp16 -> int8 and rows 20.8 and 20.0.
+        const bool rows_out = none || p->write_norm != 0;
+        const bool one = rows_out && (waves == 8 || (waves < 8 && t >= 18 * 256 && (none || p->dtype == TDE_F32)));
+        return p->nranks >= 8 && vpt == 1 && waves >= 5 && waves <= 10 && t >= 1200 && !one ? 2 : vpt;
+    }
     if (p->nranks == 2) {
         if (!none && waves >= 13 && t >= 2560) return 2; // 2 % over four
         if (none && waves >= 15 && t >= 8192) return 1; // 2-3 % over four
