@@ -27,3 +27,18 @@ def plan(dtype, n, nvec, tokens, quant, write_norm=0):
 ])
 def test_vectors_per_thread_of_eight_partials(dtype, nvec, tokens, quant, write_norm, vpt):
     assert plan(dtype, 8, nvec, tokens, quant, write_norm).vecs_per_thread == vpt
+
+
+@pytest.mark.parametrize("dtype,n,nvec,tokens,quant,write_norm,shared", [
+    # up to four partials: few rows of a 2-byte type and more than 16 vectors have a wavefront each
+    (BF16, 4, 17, 255, NONE, 0, False), (BF16, 4, 17, 256, NONE, 0, True), (F16, 2, 32, 1, INT8, 1, False), (BF16, 4, 16, 3, FP8, 0, True),
+    (F32, 4, 30, 5, FP8, 0, True), (BF16, 8, 30, 5, FP8, 0, True),
+    # two partials, many rows of more than 24 vectors whose T-typed rows are stored: from 30 MB on, T-typed output of fp32 from 72
+    (BF16, 2, 25, 19660, NONE, 0, True), (BF16, 2, 25, 19661, NONE, 0, False), (F16, 2, 24, 40000, NONE, 0, True), (F16, 2, 32, 15360, STATIC, 1, False),
+    (F16, 2, 32, 30000, INT8, 1, True), (BF16, 2, 32, 30000, FP8, 0, True), (F32, 2, 32, 36863, NONE, 0, True), (F32, 2, 32, 36864, NONE, 0, False),
+    (F32, 2, 25, 19661, FP8, 1, False),
+    (BF16, 4, 32, 30000, NONE, 0, True), (BF16, 8, 32, 30000, NONE, 0, True),
+])
+def test_rows_that_share_a_wavefront(dtype, n, nvec, tokens, quant, write_norm, shared):
+    p = plan(dtype, n, nvec, tokens, quant, write_norm)
+    assert (p.block_threads // p.rows_per_block < 64) == shared

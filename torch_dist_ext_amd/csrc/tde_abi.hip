@@ -373,21 +373,32 @@ int vecs_per_thread(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alo
     return vpt;
 }
 
+// Megabytes that a launch moves in T-typed rows, roughly: what the rules for short and for shifted rows go by.
+int64_t row_megabytes(const tde_problem *p, int64_t nvec) {
+    const int64_t streams = p->algo == TDE_ALGO_STAGED_OWNED ? 4 : p->nranks + 2; // an owned launch reads two streams for most rows
+    return (streams * p->tokens * nvec) >> 16;
+}
+
 // Rows that share a wavefront (tde_short_rows.hip) against one wavefront each (row_kernel), 1400 launches of 1 to 60000 rows: up to 16
 // vectors 4-15 % faster below 4096 rows, 30 % from there and 35-55 % from 16384 rows on (2 x [30046, 152] bf16 -> fp8 15.2 -> 9.3 us); 17
 // to 32 vectors 3-8 % faster below 8192 rows and there, where memory begins to bind, 20 % faster to 3 % slower with two and four
 // partials (2 x [40459, 192] 18.2 -> 13.5, 4 x [28759, 192] 14.5 -> 14.8).  Eight partials keep memory busy either way: from 8192
 // rows of more than 20 vectors on one row to a wavefront is up to 5 % faster (up to 20 vectors 2-8 % slower).  Owned rows, and the norm
-// phase alone, read two buffers for most rows and gain at any length (8 x [45945, 144] 23.4 -> 17.2).
+// phase alone, read two buffers for most rows and gain more (8 x [45945, 144] 23.4 -> 17.2), but for two kinds of owned launches (2600
+// launches): up to four partials, few rows of a 2-byte type and more than 16 vectors, where the wait for the
+// partials behind the stage's is all that counts (below 256 rows 1 % slower, single ones 6 %; fp32 4 % faster), and two partials with
+// T-typed rows to store, more than 24 vectors long (from 30 MB on 1 to 14 % slower, T-typed output of fp32 from 72 MB; beside per-token
+// codes of a 2-byte type level): one row to a wavefront against two, 4 x [1, 240] bf16 -> fp8 2.42 us and 2.53, 2 x [50271, 248] fp16
+// 25.5 and 28.7, 2 x [59915, 124] fp32 -> static fp8 and rows 33.0 and 38.3.
 bool share_a_wavefront(const tde_problem *p, int64_t nvec, int64_t t, bool norm_alone) {
     if (p->dtype == TDE_F64 || nvec > tde::kShortRowVecs) return false;
+    if (p->algo == TDE_ALGO_STAGED_OWNED && !norm_alone && p->nranks <= 4) {
+        const bool f32 = p->dtype == TDE_F32, none = p->quant == TDE_QUANT_NONE;
+        if (!f32 && nvec > 16 && t < 256) return false;
+        const bool rows_out = none || (p->write_norm != 0 && (f32 || p->quant == TDE_QUANT_FP8_STATIC));
+        if (p->nranks == 2 && nvec > 24 && rows_out && row_megabytes(p, nvec) >= (f32 && none ? 72 : 30)) return false;
+    }
     return nvec <= 20 || p->nranks < 8 || t < 8192 || p->algo == TDE_ALGO_STAGED_OWNED || norm_alone;
-}
-
-// Megabytes that a launch moves in T-typed rows, roughly: what the rules for shifted rows go by.
-int64_t row_megabytes(const tde_problem *p, int64_t nvec) {
-    const int64_t streams = p->algo == TDE_ALGO_STAGED_OWNED ? 4 : p->nranks + 2; // an owned launch reads two streams for most rows
-    return (streams * p->tokens * nvec) >> 16;
 }
 
 // Vectors of a line of the narrowest buffer that counts.
