@@ -44,3 +44,17 @@ def test_limited_launch_equals_the_unlimited(cuda_device, dtype, n, tokens, hidd
     got = run_hip(p, r, g, 1e-6, quant, algo=algo)
     for k in want:
         assert bits_equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("dtype,n,tokens,hidden,quant,wn,limit", [
+    # fp16, two partials, codes beside the stage, four vectors per thread: two workgroups from 24 per unit on
+    (F16, 2, 6143, 8192, FP8, 0, 0), (F16, 2, 6144, 8192, FP8, 0, 2), (F16, 2, 20000, 7424, STATIC, 1, 2), (F16, 2, 9000, 7680, GROUP, 0, 2), (F16, 2, 9000, 8184, INT8, 1, 2),
+    (F16, 2, 9000, 8192, NONE, 0, 0), (BF16, 2, 9000, 8192, FP8, 0, 0), (F16, 2, 9000, 4096, FP8, 0, 0),
+])
+def test_staged_fp16_limits(dtype, n, tokens, hidden, quant, wn, limit):
+    test_limits(dtype, n, tokens, hidden, quant, wn, _capi.ALGO_STAGED, limit)
+
+
+@pytest.mark.gpu
+def test_staged_fp16_limited_launch_equals_the_unlimited(cuda_device):
+    test_limited_launch_equals_the_unlimited(cuda_device, torch.float16, 2, 6147, 7176, "int8_token", _capi.ALGO_STAGED)

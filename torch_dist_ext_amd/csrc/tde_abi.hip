@@ -538,7 +538,10 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     // time of four with quantized output, single ones 0.86 (70 launches; 4 x [26425, 1144] fp16 -> int8 84.8 -> 74.0 us, 4 x [27056, 316] fp32
     // 46.8 -> 41.6), and more nothing on top; T-typed output alone is 1 % slower with six.
     // Two partials of fp16 with two vectors per thread, whose arithmetic is short: three workgroups 1.5 to 2 % ahead of no limit
-    // (2 x [7341 to 24000, 5120], [16000, 4960]).
+    // (2 x [7341 to 24000, 5120], [16000, 4960]; 23 more of 592, 608, 624 and 640 vectors 0.5 to 3 %).  With four vectors per thread and
+    // codes to store no limit is up to 3 % behind what the same launch took with conversions in place of mixed instructions, two workgroups 0 to
+    // 4 % ahead of it, from 24 per unit on (120 launches; 2 x [22974, 8128] -> static fp8 340.9 -> 327.6 us, [8607, 6976] -> int8 and rows 133.2 ->
+    // 126.7); T-typed output loses 1 to 2 % with two.
     // With owned rows, and in the norm phase alone, most rows read two streams, and a limit only costs (25 launches of four and
     // eight partials: up to 50 %).
     if (p->dtype != TDE_F64 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks >= 4 && rpb <= 2 && grid >= 16 * (int64_t)cus) {
@@ -548,6 +551,8 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     }
     if (p->dtype == TDE_F16 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks == 2 && vpt == 2 && nvec > 576 && nvec <= 640 && grid >= 24 * (int64_t)cus)
         wgs_per_cu = 3;
+    if (p->dtype == TDE_F16 && p->algo == TDE_ALGO_STAGED && !norm_alone && p->nranks == 2 && vpt == 4 && p->quant != TDE_QUANT_NONE && grid >= 24 * (int64_t)cus)
+        wgs_per_cu = 2;
     if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
     // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
