@@ -24,7 +24,7 @@ TORCH_LIB = os.path.join(ROOT, "libtorch_dist_ext.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 HIP_SOURCES = ["tde_abi.hip", "tde_rows_bf16.hip", "tde_rows_f16.hip", "tde_rows_f32.hip", "tde_rows_f64.hip", "tde_shifted_rows_bf16.hip", "tde_shifted_rows_f16.hip",
-               "tde_shifted_rows_f32.hip", "tde_short_rows.hip", "tde_probe.hip"]
+               "tde_shifted_rows_f32.hip", "tde_converted_rows_f16.hip", "tde_short_rows.hip", "tde_probe.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     # keep fp32 arithmetic scalar: packed fp32 forms are not used on this hardware pool
@@ -34,6 +34,9 @@ HIP_FLAGS = [
     "-fno-slp-vectorize",
     "-Wno-unused-command-line-argument",
 ]
+# no v_fma_mix* where fp16 rows are converted: the compiler folds "multiply in fp32, then convert to fp16" into v_fma_mixlo_f16, which
+# rounds the exact product once; the operator's contract is the two roundings of the eager composition
+SOURCE_FLAGS = {"tde_converted_rows_f16.hip": ["-Xclang", "-target-feature", "-Xclang", "-fma-mix-insts"]}
 
 
 def _run(cmd, quiet_substr=None):
@@ -52,8 +55,8 @@ def build_hip(verbose=False):
 
     def compile_one(src):
         obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc] + HIP_FLAGS + ["-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]
-        out = _run(cmd, quiet_substr="packed-fp32-ops")
+        cmd = [hipcc] + HIP_FLAGS + SOURCE_FLAGS.get(src, []) + ["-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]
+        out = _run(cmd, quiet_substr="is not a recognized feature")
         if verbose and out.strip():
             print(out)
         return obj

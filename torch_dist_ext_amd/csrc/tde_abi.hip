@@ -582,8 +582,21 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         // Row groups per XCD chunk of the row mapping (tde_rows.h: xcd_chunked_block); 16 measured best with 8
         // partials, 8 with 4.
         geo->xcd_chunk = p->nranks >= 8 ? 16 : 8;
-        const bool f16_long = p->dtype == TDE_F16 && p->nranks == 4 && vpt == 4 && !staged && grid >= 48 * (int64_t)cus; // below it the shorter arithmetic is level or ahead
-        geo->form = wide ? tde::kFormWide : (f16_long ? tde::kFormLong : tde::kFormPlain);
+        geo->form = wide ? tde::kFormWide : tde::kFormPlain;
+        geo->converted = false;
+        if (p->dtype == TDE_F16 && p->nranks == 4 && vpt == 4) {
+            // Long fp16 launches with longer arithmetic (tde_converted_rows_f16.hip, tde_rows.h: kFormLong).  Mixed instructions against
+            // conversions, rows of 768 to 1024 vectors (250 launches): T-typed output from 32 workgroups per unit on (where its own limit
+            // begins) 0.3 to 2 % behind, below it level; static scales and rows beside codes from 48 on 0.3 to 1.7 % behind, below it 0.3 %
+            // ahead to level; dynamic codes alone, more than 832 vectors, 0.4 to 0.8 % behind; T-typed output beside a
+            // stage from 16 on (where that limit begins) 1 to 2 % behind.
+            const bool none = p->quant == TDE_QUANT_NONE, per_token = p->quant == TDE_QUANT_FP8_TOKEN || p->quant == TDE_QUANT_INT8_TOKEN;
+            const int from = staged ? 16 : (none ? 32 : 48);
+            if (grid >= from * (int64_t)cus && (!staged || (p->algo == TDE_ALGO_STAGED && none && !norm_alone))) {
+                geo->converted = !(per_token && p->write_norm == 0 && nvec <= 832);
+                if (!geo->converted) geo->form = tde::kFormLong;
+            }
+        }
         if (wide) geo->wgs_per_cu = 2;
     }
     return TDE_OK;
@@ -895,7 +908,10 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     const bool shifted = a.line_mask != 0;
     switch (p->dtype) {
     case TDE_BF16: e = (shifted ? tde::launch_shifted_rows_bf16 : tde::launch_rows_bf16)(n, g.vpt, p->quant, wn, a, g, stream); break;
-    case TDE_F16: e = (shifted ? tde::launch_shifted_rows_f16 : tde::launch_rows_f16)(n, g.vpt, p->quant, wn, a, g, stream); break;
+    case TDE_F16:
+        e = g.converted ? tde::launch_converted_rows_f16(p->quant, wn, a, g, stream)
+                        : (shifted ? tde::launch_shifted_rows_f16 : tde::launch_rows_f16)(n, g.vpt, p->quant, wn, a, g, stream);
+        break;
     case TDE_F32: e = (shifted ? tde::launch_shifted_rows_f32 : tde::launch_rows_f32)(n, g.vpt, p->quant, wn, a, g, stream); break;
     case TDE_F64: e = tde::launch_rows_f64(n, a, g, stream); break;
     }

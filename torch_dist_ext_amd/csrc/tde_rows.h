@@ -191,7 +191,9 @@ struct ElemF32 {
 // boundary between two fp16 numbers (Figueroa, "When is double rounding innocuous?", 1995).
 // The mixed forms issue at half the rate, so a launch that is bound by instructions of many wavefronts gains from the packed ones
 // only; one that waits for a row's chain gains from every instruction left out.  With conversions against this: 2 x [79, 8096] 4.28 -> 4.16 us,
-// 4 x [89, 4256] 3.83 -> 3.70, 2 x [1162, 1152] -> int8 4.44 -> 4.33, 2 x [1651, 6328] -> int8 19.85 -> 18.5; 2-3 % up to 40 MB, from 200 MB on nothing.
+// 4 x [89, 4256] 3.83 -> 3.70, 2 x [1162, 1152] -> int8 4.44 -> 4.33, 2 x [1651, 6328] -> int8 19.85 -> 18.5; 2-3 % up to 40 MB, 0.5 % and less from
+// 200 MB on, where four vectors per thread lose up to 2.5 %: four partials convert there (tde_converted_rows_f16.hip), two have a
+// limit on workgroups beside a stage (tde_abi.hip).
 // HALF: which one of `pair`, 0 or 1.  fma(pair, b, c).
 template <int HALF>
 __device__ __forceinline__ float fma_mix(uint32_t pair, float b, float c) {
@@ -1016,10 +1018,11 @@ __device__ __forceinline__ int thread_of(int first_vector, int shift, int tpr) {
 //          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
 //          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
 //          partials and their sums stored to the stage, every other row's sum is read from the stage
-//          kFormLong: fp16 with conversions instead of mixed-precision instructions, for long launches of four partials with four
-//          vectors per thread.  What bounds those is memory, and it is served best when the arithmetic holds a row's
-//          stores back from the next rows' loads: with the mixed instructions 4 x [32768, 5120] -> int8 takes 341.8 us, 4 x [20000, 8192]
-//          370 and 4 x [24000, 5120] per group 252, with conversions 335, 360 and 246
+//          kFormLong: fp16 with conversions instead of mixed-precision instructions and packed ones for the rest, for long launches of four partials with
+//          four vectors per thread that store codes of per-token scales alone, rows of up to 832 vectors.  What bounds those is memory, and it is served
+//          best when the arithmetic holds a row's stores back from the next rows' loads: launches alone, 4 x [32768, 5120] -> int8 takes 341.8 us
+//          with the mixed instructions, 339.3 all converted and 334.9 so (as a call of the operator 336.5 either way).  The other long launches of
+//          such rows are ahead all converted (tde_converted_rows_f16.hip)
 //   SHIFTED rows that are not whole lines of memory, in launches long enough to gain from it (rows_are_shifted)
 // Block layout: rows_per_block row groups of threads_per_row threads; thread t of a row group
 // owns vectors t, t + threads_per_row, ... (coalesced 1 KiB per wavefront per load) of its row,
@@ -1421,6 +1424,7 @@ struct Geometry {
     int xcd_chunk;
     int line_mask; // RowArgs::line_mask
     int form;  // which instantiation of the row kernel (kFormPlain, kFormWide, kFormStaged, kFormOwned, kFormLong)
+    bool converted; // fp16: tde_converted_rows_f16.hip
 };
 
 // Per-dtype launchers, defined in tde_rows_<dtype>.hip.
@@ -1431,6 +1435,8 @@ hipError_t launch_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, con
 hipError_t launch_shifted_rows_bf16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_shifted_rows_f16(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_shifted_rows_f32(int n, int vpt, int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
+// fp16, four partials, four vectors per thread, rows in place or moved: plain and, T-typed output only, staged.
+hipError_t launch_converted_rows_f16(int q, bool wn, const RowArgs &a, const Geometry &g, hipStream_t s);
 hipError_t launch_reduce_bf16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f16(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
 hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t row_bytes, int64_t first_row, int64_t row_step, int64_t rows, hipStream_t s);
@@ -1468,7 +1474,7 @@ hipError_t launch_rows_nv(int q, bool wn, const RowArgs &a, const Geometry &g, h
     if constexpr (N == 8 && VPT == 4) {                                                                  \
         if (g.form == kFormWide) TDE_LAUNCH_FORM(QM, WNB, kFormWide)                                     \
     }                                                                                                    \
-    if constexpr (N == 4 && VPT == 4 && E::MIXED) {                                                      \
+    if constexpr (N == 4 && VPT == 4 && E::MIXED && !WNB && (QM == TDE_QUANT_FP8_TOKEN || QM == TDE_QUANT_INT8_TOKEN)) { \
         if (g.form == kFormLong) TDE_LAUNCH_FORM(QM, WNB, kFormLong)                                     \
     }                                                                                                    \
     if constexpr (N != 0) {                                                                              \
