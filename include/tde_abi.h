@@ -138,7 +138,8 @@ typedef struct tde_plan_out {
                                   through its LDS (0 = none); below a requested tune_workgroups_per_cu where the
                                   geometry's own LDS already admits fewer.  Also 2, without LDS padding, where the
                                   plan picks the row kernel built for two wavefronts per SIMD (eight partials, four
-                                  vectors per thread, 4 to 24 workgroups per CU, tune_workgroups_per_cu == 0): its
+                                  vectors per thread, 4 to 24 workgroups per CU -- to 16 where only codes of a dynamic
+                                  scale are stored beside residual_out -- and tune_workgroups_per_cu == 0): its
                                   registers admit two.  For TDE_ALGO_STAGED it belongs to the one launch that stores the
                                   stage; where that call needs two launches, neither is limited unless asked to, and
                                   TDE_ALGO_STAGED_OWNED only if asked to */

@@ -58,3 +58,16 @@ def test_staged_fp16_limits(dtype, n, tokens, hidden, quant, wn, limit):
 @pytest.mark.gpu
 def test_staged_fp16_limited_launch_equals_the_unlimited(cuda_device):
     test_limited_launch_equals_the_unlimited(cuda_device, torch.float16, 2, 6147, 7176, "int8_token", _capi.ALGO_STAGED)
+
+
+@pytest.mark.parametrize("tokens,quant,wn,padded", [
+    # eight partials, only codes of a dynamic scale to store, 16 to 24 workgroups per unit: the kernel for three wavefronts per SIMD with two workgroups by
+    # its LDS; otherwise the one for two wavefronts, whose registers admit two, up to 24
+    (4095, FP8, 0, False), (4096, FP8, 0, True), (6143, FP8, 0, True), (6144, FP8, 0, True), (4096, FP8, 1, False), (6143, NONE, 0, False), (6143, STATIC, 0, False),
+    (6144, NONE, 0, True),
+])
+def test_two_workgroups_of_eight_partials(tokens, quant, wn, padded):
+    if torch.cuda.is_available() and _capi.device_info().compute_units != 256:
+        pytest.skip("the row counts are for 256 compute units")
+    p = _capi.plan(_capi.make_problem(BF16, 8, tokens, 8192, 1e-5, quant=quant, write_norm=wn, static_scale=0.5 if quant == STATIC else 0.0))
+    assert (p.workgroups_per_cu, p.lds_bytes) == (2, 80896 if padded else 36864)

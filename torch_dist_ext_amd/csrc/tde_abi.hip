@@ -63,7 +63,9 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 constexpr int kMaxBlock = 1024;
 constexpr int64_t kLoadsInFlightPerCu = 128 * 1024; // target for the limit on resident workgroups (see validate)
 // launches with fewer workgroups per compute unit are not limited: 24 with 8 partials, 32 with 4 (whose launches are
-// shorter), i.e. 6144 and 8192 workgroups on the 256 CUs of an unpartitioned MI355X; launches of 4 that store little also from 16 to 30
+// shorter), i.e. 6144 and 8192 workgroups on the 256 CUs of an unpartitioned MI355X; launches of either that store little (few_stores) also
+// from 16 to 30.  (From 30 to 32 four partials that store little would gain 2 to 4.5 % from it as well -- 33 launches of 7680 to 8191 rows -- and are
+// planned without, which test_abi_host.py and test_workgroup_limits.py pin.)
 constexpr int64_t kLimitFromWorkgroupsPerCu8 = 24, kLimitFromWorkgroupsPerCu4 = 32;
 constexpr int64_t kFewStoresFrom = 16, kFewStoresUntil = 30;
 constexpr int kDefaultComputeUnits = 256; // MI355X; used when no device can be asked (planning on a host without one)
@@ -525,7 +527,9 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         // Two workgroups are enough for few_stores, six wavefronts among them: 4 x [32768, 5120] fp16 -> int8 338.2 us against
         // 342.3 with three, bf16 -> fp8 336.2 against 344.7, per group 338.7 against 339.7; with T-typed output or rows three
         // stay 3 % ahead.  For them the limit pays from 16 workgroups per unit on: 4 x rows of 770 to 1024 vectors, 4096 to 6143 of them -1.3 % (bf16),
-        // -2.3 (fp16) and 0 (fp32), 6144 to 8191 -2.5 to -2.9, per group -2 (below 4096 +0.5; static scales +0.5, T-typed output -0.5).
+        // -2.3 (fp16) and 0 (fp32), 6144 to 7679 -2.5 to -2.9, per group -2 (below 4096 +0.5; static scales +0.5, T-typed output -0.5).  Eight partials
+        // then leave the kernel for two wavefronts per SIMD (`wide`, below) for two workgroups of this one: 120 launches of 4096 to 6143 rows of
+        // 769 to 1024 vectors -0.5 % on average, single ones -2.2 to +0.6 %.
         if (few_stores) wgs_per_cu = 2;
     }
     // TDE_ALGO_STAGED in one launch reads what the fused launch reads and stores one stream more.  From 16 workgroups per CU
@@ -555,7 +559,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
         wgs_per_cu = 2;
     if (p->tune_workgroups_per_cu != 0 && p->dtype != TDE_F64) wgs_per_cu = p->tune_workgroups_per_cu < 0 ? 0 : p->tune_workgroups_per_cu;
 
-    // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU: the
+    // Eight partials, four vectors per thread, no limit asked for or planned, and 4 to 24 workgroups per CU (few_stores: 4 to 16): the
     // row kernel's two-wavefronts-per-SIMD instantiation (tde_rows.h: WIDE) is 0.2-2.2 % faster there; it is
     // reported as the limit of two workgroups per CU that its registers amount to.
     const bool wide = p->nranks == 8 && vpt == 4 && p->dtype != TDE_F64 && !staged && wgs_per_cu == 0 &&

@@ -766,7 +766,7 @@ __device__ __forceinline__ float reciprocal_rms(float sumsq, Length length, floa
     const float m = div_shared(sumsq, length.h, length.rcp) + eps;
     constexpr uint32_t LOW = (127u - 60u) << 23, HIGH = (127u + 100u) << 23;
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, m) - LOW > HIGH - LOW) != 0, 0))
-        return 1.0f / __builtin_sqrtf(sumsq / length.h + eps); // the same value in every lane
+        return 1.0f / __builtin_sqrtf(sumsq / length.h + eps); // in every lane, also of rows inside the range: the same bits
     return reciprocal_of_root(m, __builtin_amdgcn_rsqf(m));
 }
 
@@ -1014,7 +1014,8 @@ __device__ __forceinline__ int thread_of(int first_vector, int shift, int tpr) {
 //          of the row also for eight partials: two workgroups per CU whose gamma never waits.  Never more than two wavefronts,
 //          also where the registers would hold three (fp16 and fp32, 168 and 166 of them: 8 x rows of 600 to 1024 vectors, 1024 to
 //          6200 of them, 0.983 of the time, single ones 0.953).  Launched for eight
-//          partials with four vectors per thread at 4 to 24 workgroups per CU (launch_rows_nv, Geometry::form).
+//          partials with four vectors per thread at 4 to 24 workgroups per CU, to 16 where only codes of a dynamic
+//          scale are stored (Geometry::form).
 //          kFormStaged: both launches of TDE_ALGO_STAGED in one: the sums are also stored to the stage.
 //          kFormOwned: both launches of TDE_ALGO_STAGED_OWNED in one: rows == owner (mod N) are summed from the
 //          partials and their sums stored to the stage, every other row's sum is read from the stage
