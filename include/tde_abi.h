@@ -148,6 +148,23 @@ typedef struct tde_plan_out {
     int64_t scale_elems;       /* number of fp32 scales written */
 } tde_plan_out;
 
+/* Which kernel tde_reduce_rms launches, beyond its geometry (tde_plan_route). */
+typedef enum tde_kernel {
+    TDE_KERNEL_ROWS = 0,      /* a row to one or more wavefronts; a staged algorithm's form of it where the algorithm is staged */
+    TDE_KERNEL_WIDE = 1,      /* the same for two wavefronts per SIMD */
+    TDE_KERNEL_LONG = 2,      /* the same with conversions instead of mixed-precision instructions, packed fp16 arithmetic elsewhere */
+    TDE_KERNEL_CONVERTED = 3, /* the same with conversions throughout */
+    TDE_KERNEL_SHORT = 4      /* two or four rows to a wavefront */
+} tde_kernel;
+
+typedef struct tde_route_out {
+    int32_t kernel;          /* tde_kernel */
+    int32_t lanes_per_row;   /* threads of a row: a multiple of 64, or 16 or 32 of a wavefront (TDE_KERNEL_SHORT) */
+    int32_t moved_to_lines;  /* rows are moved along their threads until their wavefronts begin on 128-byte lines: vectors of a
+                                line of the buffer whose lines count (8 T-typed, 16 or 32 of codes); 0: rows stay in place */
+    int32_t reserved;        /* 0 */
+} tde_route_out;
+
 /* ---- entry points --------------------------------------------------------------------------- */
 
 /* Library / ABI version (TDE_ABI_VERSION of the build). */
@@ -165,6 +182,10 @@ int tde_last_hip_error(void);
    shape/nranks asserts and the grid/block/algorithm selection of allreduce_fusion_kernel_launcher
    (impl.h:476-498, 526-534). */
 int tde_plan(const tde_problem *problem, tde_plan_out *plan);
+
+/* Pure host: which kernel tde_reduce_rms launches for the problem, validated as tde_plan validates it (for a staged
+   algorithm: in its one launch).  No counterpart in the reference, whose two kernels are told apart by tokens alone (impl.h:491). */
+int tde_plan_route(const tde_problem *problem, tde_route_out *route);
 
 /* Enqueue the row kernel(s) on `hip_stream` (a hipStream_t, null = default stream) of the current
    device and return without synchronizing.  Replaces allreduce_rms_fusion_impl<T>

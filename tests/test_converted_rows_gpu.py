@@ -12,11 +12,14 @@ from torch_dist_ext_amd import _capi
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,hidden,quant,algo", [
+CASES = [  # rows, elements of a row, quant, algorithm
     (12290, 640, "none", _capi.ALGO_AUTO), (8195, 1032, "none", _capi.ALGO_AUTO), (8191, 640, "none", _capi.ALGO_AUTO), (4098, 640, "none", _capi.ALGO_STAGED),
     (4097, 1032, "none", _capi.ALGO_STAGED), (12290, 640, "fp8_static", _capi.ALGO_AUTO), (12288, 1032, "int8_token", _capi.ALGO_AUTO),
     (12289, 1024, "fp8_group", _capi.ALGO_AUTO), (12288, 6664, "fp8_token", _capi.ALGO_AUTO), (12289, 6656, "int8_token", _capi.ALGO_AUTO),
-])
+]
+
+
+@pytest.mark.parametrize("tokens,hidden,quant,algo", CASES)
 def test_converted_rows(cuda_device, tokens, hidden, quant, algo):
     print("case", tokens, hidden, quant, algo, flush=True)
     p, r, g = eager.make_inputs(4, tokens, hidden, torch.float16, 1.0, seed=hidden)

@@ -20,7 +20,7 @@ ALGO_AUTO, ALGO_FUSED, ALGO_STAGED, ALGO_STAGED_OWNED = 0, 1, 2, 3
 ABI_VERSION = 4   # TDE_ABI_VERSION of include/tde_abi.h
 
 EXPORTS = (
-    "tde_abi_version", "tde_status_string", "tde_last_hip_error", "tde_plan", "tde_reduce_rms", "tde_stage_reduce", "tde_stage_norm",
+    "tde_abi_version", "tde_status_string", "tde_last_hip_error", "tde_plan", "tde_plan_route", "tde_reduce_rms", "tde_stage_reduce", "tde_stage_norm",
     "tde_reduce_rms_static_stage",
     "tde_probe_copy", "tde_probe_launch", "tde_probe_stream", "tde_probe_rows", "tde_probe_rows_parts", "tde_device_info",
     "tde_workspace_create", "tde_workspace_destroy", "tde_workspace_slot", "tde_workspace_stage",
@@ -56,6 +56,13 @@ class PlanOut(ctypes.Structure):
     ]
 
 
+KERNEL_ROWS, KERNEL_WIDE, KERNEL_LONG, KERNEL_CONVERTED, KERNEL_SHORT = 0, 1, 2, 3, 4
+
+
+class RouteOut(ctypes.Structure):
+    _fields_ = [("kernel", ctypes.c_int32), ("lanes_per_row", ctypes.c_int32), ("moved_to_lines", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+
+
 class DeviceInfo(ctypes.Structure):
     _fields_ = [
         ("compute_units", ctypes.c_int32), ("memory_clock_khz", ctypes.c_int32), ("memory_bus_bits", ctypes.c_int32),
@@ -89,6 +96,8 @@ def load():
     lib.tde_last_hip_error.restype = ctypes.c_int
     lib.tde_plan.restype = ctypes.c_int
     lib.tde_plan.argtypes = [ctypes.POINTER(Problem), ctypes.POINTER(PlanOut)]
+    lib.tde_plan_route.restype = ctypes.c_int
+    lib.tde_plan_route.argtypes = [ctypes.POINTER(Problem), ctypes.POINTER(RouteOut)]
     lib.tde_reduce_rms.restype = ctypes.c_int
     lib.tde_reduce_rms.argtypes = [ctypes.POINTER(Problem), ctypes.POINTER(Buffers), ctypes.c_void_p]
     for fn in (lib.tde_stage_reduce, lib.tde_stage_norm, lib.tde_probe_rows, lib.tde_reduce_rms_static_stage):
@@ -140,6 +149,13 @@ def make_problem(dtype, nranks, tokens, hidden, eps, quant=QUANT_NONE, algo=ALGO
                    tokens=tokens, hidden=hidden, eps=eps, static_scale=static_scale,
                    tune_vecs_per_thread=vecs_per_thread, tune_rows_per_block=rows_per_block,
                    tune_workgroups_per_cu=workgroups_per_cu)
+
+
+def route(problem):
+    """tde_plan_route -> RouteOut (raises TdeError on a rejected problem)."""
+    out = RouteOut()
+    check(load().tde_plan_route(ctypes.byref(problem), ctypes.byref(out)))
+    return out
 
 
 def plan(problem):

@@ -770,6 +770,22 @@ int tde_plan(const tde_problem *problem, tde_plan_out *plan) {
     return TDE_OK;
 }
 
+int tde_plan_route(const tde_problem *problem, tde_route_out *route) {
+    if (route == nullptr) return TDE_EINVAL;
+    tde::Geometry g{};
+    const int st = validate(problem, &g);
+    if (st != TDE_OK) return st;
+    std::memset(route, 0, sizeof(*route));
+    route->kernel = g.threads_per_row < tde::kWave ? TDE_KERNEL_SHORT
+                    : g.converted                  ? TDE_KERNEL_CONVERTED
+                    : g.form == tde::kFormWide     ? TDE_KERNEL_WIDE
+                    : g.form == tde::kFormLong     ? TDE_KERNEL_LONG
+                                                   : TDE_KERNEL_ROWS;
+    route->lanes_per_row = g.threads_per_row;
+    route->moved_to_lines = g.line_mask != 0 ? g.line_mask + 1 : 0;
+    return TDE_OK;
+}
+
 namespace {
 enum : int { kPhaseReduce = 1, kPhaseNorm = 2, kTrafficOnly = 4 };
 
