@@ -236,7 +236,7 @@ int tde_probe_launch(void *hip_stream);
 int tde_probe_stream(void *dst, const void *src, int64_t bytes, int32_t mode, void *hip_stream);
 
 /* Measurement aid: the memory traffic of tde_reduce_rms for the same problem and buffers with the arithmetic
-   removed -- same workgroups, lane mapping, load order and cache policies, every input byte read and every
+   removed -- same workgroups, lane mapping (short and moved rows included), load order and cache policies, every input byte read and every
    output byte (scales excepted) written once, contents meaningless.  OVERWRITES residual_out, norm_out and
    q_out.  Fused algorithm only (TDE_EALGO for the staged ones).  Timing it next to tde_reduce_rms shows how
    far the kernel is from what its access pattern alone achieves.  No counterpart in the reference. */

@@ -90,3 +90,31 @@ def test_partials_from_a_table(cuda_device, n, tokens, hidden, dtype, quant, mov
             assert bits_equal(got[k], want[k]), (rank, k)
     rows = list(range(0, tokens, max(1, tokens // 200)))
     check_against_oracle({k: v[rows] for k, v in want.items()}, eager.reduce_rms(p[:, rows], res[rows], g, 1e-6, quant), quant, gamma=g, eps=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,tokens,nvec,dtype,quant,write_norm,moved", [
+    (2, 1, 1, torch.bfloat16, "none", True, False), (8, 67, 15, torch.bfloat16, "fp8_token", False, False), (4, 4103, 16, torch.float16, "int8_token", True, False),
+    (2, 6, 17, torch.float32, "fp8_token", True, False), (4, 259, 31, torch.float32, "none", True, False), (8, 4097, 32, torch.bfloat16, "fp8_static", False, False),
+    (2, 7201, 129, torch.bfloat16, "none", True, True), (2, 3702, 255, torch.float16, "int8_token", False, True), (4, 614, 1023, torch.float16, "fp8_static", True, True),
+    (8, 1026, 1021, torch.bfloat16, "fp8_token", False, True), (2, 2124, 253, torch.float32, "fp8_token", False, True), (8, 7346, 65, torch.float32, "none", True, True),
+])
+def test_traffic_skeletons_of_short_and_moved_rows(cuda_device, n, tokens, nvec, dtype, quant, write_norm, moved):
+    """As test_traffic_skeleton_touches_every_byte_once, where the launch it stands for moves its rows or lets them share a wavefront: its outputs are the
+    exclusive-or of all input rows."""
+    print("case", n, tokens, nvec, dtype, quant, flush=True)
+    hidden = nvec * 16 // dtype.itemsize
+    r = route(n, tokens, hidden, dtype, quant, write_norm=int(write_norm))
+    assert bool(r.moved_to_lines) == moved and (r.kernel == _capi.KERNEL_SHORT) == (not moved)
+    p, res, g = eager.make_inputs(n, tokens, hidden, dtype, 1.0, seed=nvec)
+    words = lambda t: t.contiguous().view(torch.int32).reshape(tokens, -1, 4)
+    x = words(res).clone()
+    for k in range(n):
+        x ^= words(p[k])
+    codes = (x[..., 0] ^ x[..., 1] ^ x[..., 2] ^ x[..., 3]) if dtype == torch.float32 else torch.stack([x[..., 0] ^ x[..., 2], x[..., 1] ^ x[..., 3]], dim=-1)
+    out = run_hip(p, res, g, 1e-6, quant, write_norm=write_norm, static_scale=0.03 if quant == "fp8_static" else 0.0, calls=[(("traffic",), 0)])
+    assert torch.equal(words(out["residual_out"]), x)
+    if write_norm or quant == "none":
+        assert torch.equal(words(out["norm_out"]), x)
+    if quant != "none":
+        assert torch.equal(out["q"].contiguous().view(torch.uint8).view(torch.int32).reshape(codes.shape), codes)

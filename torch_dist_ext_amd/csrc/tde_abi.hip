@@ -452,10 +452,8 @@ int vecs_per_thread_shifted(const tde_problem *p, int64_t nvec, int64_t t, int v
     return vpt;
 }
 
-// `launch`: what the geometry is for.
-enum Launch { kWhole, kNormAlone /* norms the rows of the stage */, kSkeleton /* the traffic probe: row_kernel's geometry */ };
-int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
-    const bool norm_alone = launch == kNormAlone;
+// `norm_alone`: the geometry of a launch that only norms the rows of the stage.
+int validate(const tde_problem *p, tde::Geometry *geo, bool norm_alone = false) {
     if (p == nullptr) return TDE_EINVAL;
     const int eb = elem_bytes(p->dtype);
     if (eb == 0) return TDE_EDTYPE;
@@ -485,7 +483,7 @@ int validate(const tde_problem *p, tde::Geometry *geo, Launch launch = kWhole) {
     }
     if (p->tune_rows_per_block < 0) return TDE_EINVAL;
     if (p->tune_workgroups_per_cu < -1 || p->tune_workgroups_per_cu > 8 || p->reserved != 0) return TDE_EINVAL;
-    const bool short_rows = launch != kSkeleton && p->tune_vecs_per_thread == 0 && p->tune_rows_per_block == 0 && share_a_wavefront(p, nvec, t, norm_alone);
+    const bool short_rows = p->tune_vecs_per_thread == 0 && p->tune_rows_per_block == 0 && share_a_wavefront(p, nvec, t, norm_alone);
     const int64_t lanes = (nvec + vpt - 1) / vpt;
     const int tpr = short_rows ? (nvec <= 16 ? 16 : 32) : (int)((lanes + 63) / 64 * 64);
     // pack short rows so a workgroup has at least four wavefronts (two of two rows each: 1 % faster than four)
@@ -809,7 +807,7 @@ bool phases_overlap(const tde_problem *p, const tde_buffers *b) {
 
 int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int phases, int probe_parts = 7) {
     tde::Geometry g{};
-    const int st = validate(p, &g, phases == kTrafficOnly ? kSkeleton : kWhole);
+    const int st = validate(p, &g);
     if (st != TDE_OK) return st;
     if (b == nullptr) return TDE_EINVAL;
     if (p->tokens == 0) return TDE_OK; // nothing to do; empty buffers may be null
@@ -853,7 +851,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     // been stored; so do partials that only a device table knows (RowArgs has no room for the table beside the stage, and no torch operator makes such a call).
     const bool one_launch = staged && both && !from_table && !phases_overlap(p, b);
     if (staged && !one_launch) {
-        const int alone = validate(p, &g, kNormAlone);
+        const int alone = validate(p, &g, true);
         if (alone != TDE_OK) return alone;
     }
 
@@ -883,7 +881,7 @@ int run_phases(const tde_problem *p, const tde_buffers *b, void *hip_stream, int
     a.static_scale = p->static_scale;
     a.chunked_blocks = tde::chunked_blocks(g.grid, (uint32_t)g.xcd_chunk);
     a.owner = (uint8_t)p->rank;
-    a.line_mask = (uint8_t)(traffic ? 0 : g.line_mask);
+    a.line_mask = (uint8_t)g.line_mask;
 
     int n = p->nranks;
     hipError_t e = hipSuccess;

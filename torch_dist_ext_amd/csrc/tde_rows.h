@@ -1445,6 +1445,7 @@ hipError_t launch_reduce_f32(int n, const RowArgs &a, uint64_t table, int64_t ro
 // Rows of up to 32 vectors, several to a wavefront (tde_short_rows.hip; not doubles).  The normed rows go where the arguments have a
 // buffer for them.
 constexpr int kShortRowVecs = 32;
+constexpr uint32_t kPastEnd = 0x7ffffff0u; // an offset beyond every resource of theirs: loads give zeros, stores are dropped
 inline size_t short_rows_lds_bytes(int block_threads, int rows_per_block, int vec_floats) {
     return ((size_t)block_threads * vec_floats + (size_t)rows_per_block * 32) * sizeof(float);
 }

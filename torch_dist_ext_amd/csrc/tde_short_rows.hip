@@ -15,8 +15,6 @@ namespace tde {
 
 namespace {
 
-constexpr uint32_t kPastEnd = 0x7ffffff0u; // beyond every resource here: loads give zeros, stores are dropped
-
 // Lane n of each 16-lane row, in all of them.
 template <int n>
 __device__ __forceinline__ float row16_lane(float v) {
