@@ -1036,7 +1036,10 @@ template <> struct Arithmetic<ElemF16, kFormLong> { typedef ElemF16Unmixed type;
 
 template <class E, int N, int VPT, int Q, bool WN, int FORM = kFormPlain, bool SHIFTED = false>
 __global__ void __launch_bounds__(1024 / VPT)
-    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? 5 : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))), FORM == kFormWide ? 2 : 8)))
+    // Owned rows of eight partials with two vectors per thread fit eight wavefronts per SIMD without being told, but for fp16: with the mixed
+    // instructions it takes 68 registers and seven, and rows of 513 to 575 vectors (29 launches) were 1.2 % behind conversions on average, single ones
+    // 4 to 5; with 60 registers and eight 0 to 0.2 %.
+    __attribute__((amdgpu_waves_per_eu(VPT == 1 ? 8 : (VPT == 2 ? (E::MIXED && N == 8 && FORM == kFormOwned ? 8 : 5) : (FORM == kFormWide ? 2 : (FORM == kFormOwned ? 4 : 3))), FORM == kFormWide ? 2 : 8)))
     row_kernel(const RowArgs a) {
     constexpr bool WIDE = FORM == kFormWide, OWNED = FORM == kFormOwned;
     constexpr int VEC = E::VEC;
