@@ -39,7 +39,7 @@ def test_converted_rows_are_converted(tokens, hidden, quant, algo):
     kw = dict(algo=algo, write_norm=hidden < 6000, vecs_per_thread=4, rows_per_block=1)
     r = route(4, tokens, hidden, torch.float16, quant, **kw)
     assert r.kernel == (_capi.KERNEL_ROWS if tokens == 8191 else _capi.KERNEL_LONG if hidden == 6656 else _capi.KERNEL_CONVERTED) # beyond each end
-    assert bool(r.moved_to_lines) == (hidden % 64 != 0 and (4 + 2) * tokens * hidden // 8 >> 16 >= 28)
+    assert bool(r.moved_to_lines) == (hidden % 64 != 0 and (4 + 2) * tokens * hidden // 8 >> 16 >= 56)
 
 
 @pytest.mark.parametrize("n,tokens,hidden,dtype,quant,kw,kernel,lanes", [
@@ -118,3 +118,13 @@ def test_traffic_skeletons_of_short_and_moved_rows(cuda_device, n, tokens, nvec,
         assert torch.equal(words(out["norm_out"]), x)
     if quant != "none":
         assert torch.equal(out["q"].contiguous().view(torch.uint8).view(torch.int32).reshape(codes.shape), codes)
+
+
+@pytest.mark.parametrize("n,nvec,tokens,quant,algo,vpt,moved", [
+    # a wavefront to a row with four vectors per thread, up to four partials: moved from 56 MB on; longer rows from 28
+    (2, 217, 2999, "none", _capi.ALGO_AUTO, 4, False), (2, 217, 4227, "none", _capi.ALGO_AUTO, 4, False), (2, 217, 4230, "none", _capi.ALGO_AUTO, 4, True),
+    (4, 255, 2390, "none", _capi.ALGO_STAGED, 4, False), (4, 255, 2400, "none", _capi.ALGO_STAGED, 4, True), (8, 217, 1000, "none", _capi.ALGO_AUTO, 4, True),
+    (2, 259, 1800, "none", _capi.ALGO_AUTO, 4, True), (2, 217, 3000, "none", _capi.ALGO_AUTO, 2, True),
+])
+def test_where_moving_begins(n, nvec, tokens, quant, algo, vpt, moved):
+    assert bool(route(n, tokens, nvec * 8, torch.bfloat16, quant, algo=algo, vecs_per_thread=vpt).moved_to_lines) == moved

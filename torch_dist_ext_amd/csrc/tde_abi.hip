@@ -411,7 +411,8 @@ int line_vectors(const tde_problem *p) { return p->quant == TDE_QUANT_NONE ? 8 :
 // time in memory.  From 3000 launches of 5 to 2200 MB in place and shifted, the same vectors per thread: 10 MB +1.5 %, 20 MB
 // 0 to +0.5 %, 40 MB -1.5 % (single ones up to +3.5 % with two and four partials of one vector per thread), 100 MB -2.2 %,
 // from 300 MB on -3.3 % (2 x [31779, 3256] bf16 -> static fp8 and T-typed rows 198.4 -> 183.3 us, 4 x [26096, 962] doubles staged
-// 285 -> 255, 2 x [30413, 4008] fp32 -> int8 375 -> 323).  Two wavefronts a row: 0 to -0.5 %, 2-byte types nothing.  Eight partials of a 2-byte type, one
+// 285 -> 255, 2 x [30413, 4008] fp32 -> int8 375 -> 323).  Two and four partials of a 2-byte type, four vectors per thread and one wavefront to
+// a row: +0.4 to +1.6 % from 28 to 45 MB (2 x [2999, 1776] fp16 10.1 us against 9.9).  Two wavefronts a row: 0 to -0.5 %, 2-byte types nothing.  Eight partials of a 2-byte type, one
 // vector per thread: owned rows +0.2 %, up to four wavefronts a row with workgroups limited per unit +0.3 %.
 // Rows of whole T-typed lines whose codes start inside lines: two partials -1 to -3 %, others nothing.
 bool rows_are_shifted(const tde_problem *p, int64_t nvec, int64_t t, int vpt) {
@@ -422,7 +423,7 @@ bool rows_are_shifted(const tde_problem *p, int64_t nvec, int64_t t, int vpt) {
     if (elem_bytes(p->dtype) > 2) return mb >= (nvec <= 128 ? 56 : 32);
     if (nvec <= 128) return false;
     if (!few && vpt == 1 && (owned || (nvec <= 256 && t >= kLimitFromWorkgroupsPerCu8 * 256))) return false;
-    return mb >= (owned || (vpt == 1 && few) ? 56 : 28);
+    return mb >= (owned || (few && (vpt == 1 || (vpt == 4 && nvec <= 256))) ? 56 : 28);
 }
 
 // Vectors per thread where rows are shifted and the lengths that vecs_per_thread was swept at do not speak for them (same launches; against
