@@ -1164,10 +1164,12 @@ __global__ void __launch_bounds__(1024 / VPT)
         constexpr bool RANK_MAJOR = !OWNED && (N >= 4 && (VPT >= 4 || VPT == 1));
         u32x4 sraw[VPT]; // the row's sums, rounded to T
         if constexpr (OWNED) {
-            // Decided by a scalar where T-typed rows alone are stored: as a mask of lanes the compiler lets the two ways of loading share registers, and
-            // four partials of fp16 with four vectors per thread then waited for the residual ahead of the partials: 4 x [283, 6272] 6.4 us
-            // against 5.8.  (Beside codes that wait happens to pay, 1.5 % on average.)
-            const bool sum_here = Q == TDE_QUANT_NONE ? __builtin_amdgcn_readfirstlane((int)sum_is_new) != 0 : sum_is_new;
+            // Four partials of fp16 with four vectors per thread: decided by a scalar where T-typed rows alone are stored.  As a mask of lanes the
+            // compiler lets the two ways of loading share registers, and these kernels then waited for the residual ahead of the partials: 58 launches
+            // 0.3 % slower on average, of 250 to 500 rows 3 to 13 % (4 x [283, 6272] 6.29 us against 5.62).  Beside codes the same wait happens to pay,
+            // 1.5 % on average; of other types and row lengths nothing waits, and a scalar moves single launches by up to 11 % either way.
+            constexpr bool SCALAR = E::MIXED && N == 4 && VPT == 4 && Q == TDE_QUANT_NONE;
+            const bool sum_here = SCALAR ? __builtin_amdgcn_readfirstlane((int)sum_is_new) != 0 : sum_is_new;
             if (sum_here) {
                 // At most four partials in flight per vector: each one's registers are loaded with the partial four
                 // ranks on as soon as it has been added.  That keeps the kernel within 128 registers, four wavefronts
