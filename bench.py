@@ -40,8 +40,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E published peak
 # They describe the kernels whose sources hash to `sources_sha256`; with any other kernel source the bench line reports
 # traffic as null.
 TRAFFIC = {
-    "sources_sha256": "e0d444b6d27db3d251b1636357d2d20598985d914095467479702250b6047b73",
-    "bytes": {"c2": 11670726, "c3": 352603386, "c4": 765409876, "c5": 2181210598},
+    "sources_sha256": "5a9e0ca58b9ed43f67064f3c31b7ac40862d8c9f1e33796c76577947c8982c0c",
+    "bytes": {"c2": 11671245, "c3": 352606687, "c4": 765406551, "c5": 2181231436},
 }
 
 BENCH_CONFIGS = {
